@@ -248,10 +248,10 @@ KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao
     const S uf = u0.v * h0 + u1.v * h1 + u2.v * h2;
     const S ufq = uf * q.v;
     const S fz1 = h0 + u0.v * ufq, fz2 = h1 + u1.v * ufq, fz3 = h2 + u2.v * ufq;
-    const S ft = uf * (1.0 / G.lapse);
-    const S fr_ = fz1 * (1.0 / G.sgrr);
-    const S fth = fz3 * (-1.0 / G.sgthth);
-    const S fph = fz2 * (1.0 / G.sgpp) + G.omega * ft;
+    const S ft = uf * G.ilapse;
+    const S fr_ = fz1 * G.isgrr;
+    const S fth = fz3 * (-G.isgthth);
+    const S fph = fz2 * G.isgpp + G.omega * ft;
     const S* p = G.pu;
     const S C1 = a * G.st * G.st, C2 = G.r * G.r + a * a, act = a * G.ct;
     const S A = p[0] * fr_ - p[1] * ft + C1 * (p[1] * fph - p[3] * fr_);
@@ -271,9 +271,9 @@ KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao
     const S fphb = Ab * (C1 * p[1]) - Bws * (C2 * p[2]);
     const S ftb = Bws * (a * p[2]) - Ab * p[1] + fphb * G.omega;
     const S frb = Ab * (p[0] - C1 * p[3]);
-    const S z1b = frb * (1.0 / G.sgrr), z2b = fphb * (1.0 / G.sgpp), z3b = fthb * (-1.0 / G.sgthth);
+    const S z1b = frb * G.isgrr, z2b = fphb * G.isgpp, z3b = fthb * (-G.isgthth);
     const S ufqb = z1b * u0.v + z2b * u1.v + z3b * u2.v;
-    const S ufb = ftb * (1.0 / G.lapse) + ufqb * q.v;
+    const S ufb = ftb * G.ilapse + ufqb * q.v;
     const S qb = ufqb * uf;
     const S fb0 = (z1b + ufb * u0.v) * ifn, fb1 = (z2b + ufb * u1.v) * ifn, fb2 = (z3b + ufb * u2.v) * ifn;
     // f = k x bh: kbar = bh x fbar, bhbar = fbar x k

@@ -77,6 +77,15 @@ KS_DEV float hw_log2(float x) {
     return log2f(x);
 #endif
 }
+// sine and cosine on v_sin_f32 / v_cos_f32 (absolute error about 1e-6 plus the phase's rounding)
+KS_DEV void hw_sincos(float x, float& s, float& c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float rev = __builtin_amdgcn_fractf(x * 0.15915494f);
+    s = __builtin_amdgcn_sinf(rev); c = __builtin_amdgcn_cosf(rev);
+#else
+    s = sinf(x); c = cosf(x);
+#endif
+}
 KS_DEV float hw_pow(float x, float y) {
     const float p = hw_exp2(y * hw_log2(x));
     return y == 0.0f ? 1.0f : p;

@@ -31,9 +31,9 @@ KS_DEV TransCtxT<S> make_ctx(double a, double rp, double rm, double thetao_sin, 
 // The Gaussian exponent at (t, x, y, z) of a splat whose centre follows knots (trajectories.jl:93-128): the offset
 // from the knot-interpolated centre (knot_centre), no pattern rotation.
 template <class S>
-KS_DEV S knot_gexp(const TransCtxT<S>& c, const SplatCT<S>& sc, S t, S x, S y, S z) {
+KS_DEV S knot_gexp(const S* __restrict__ knots, const S* __restrict__ ktimes, const SplatCT<S>& sc, S t, S x, S y, S z) {
     S cx, cy, cz;
-    knot_centre(sc, c.knots, c.ktimes, t, cx, cy, cz);
+    knot_centre(sc, knots, ktimes, t, cx, cy, cz);
     S d0 = x - cx, d1 = y - cy, d2 = z - cz;
     S u0 = sc.R[0] * d0 + sc.R[3] * d1 + sc.R[6] * d2;
     S u1 = sc.R[1] * d0 + sc.R[4] * d1 + sc.R[7] * d2;
@@ -43,14 +43,64 @@ KS_DEV S knot_gexp(const TransCtxT<S>& c, const SplatCT<S>& sc, S t, S x, S y, S
     return q0 * q0 + q1 * q1 + q2 * q2 + tt * tt;
 }
 
+// A splat's Gaussian weight at (t, x, y, z), zero where the transport does not count it (outside its support sphere,
+// or below the weight cutoff).
+template <int KIND, class S>
+KS_DEV S splat_weight(const SplatCT<S>& sc, const S* __restrict__ knots, const S* __restrict__ ktimes, S t, S x, S y, S z) {
+    S gexp;
+    if (KIND == MODEL_KNOT || sc.nk > 0) {
+        gexp = knot_gexp(knots, ktimes, sc, t, x, y, z);
+    } else {
+        S sph, cph;
+        if (outside_support(sc, t, x, y, z, sph, cph)) return S(0.0);
+        gexp = gauss_exponent(sc, t, x, y, z, sph, cph);
+    }
+    if (gexp > GEXP_SKIP) return S(0.0);
+    const S G_ = exp(-0.5 * gexp);
+    return G_ > WEIGHT_CUTOFF ? G_ : S(0.0);
+}
+
+// One splat's share of a sample of geometry G, given its weight G_ > 0: the invariant j (c[0..3]), alpha (c[4..7]) and
+// rho (c[8..10]) in screen axes; false when it has none (element and screen_coefficients, transport.jl:223-276).
+template <int KIND, class S>
+KS_DEV bool splat_contribution(const SplatCT<S>& sc, const GeoT<S>& G, S aS, S alpha, S beta, S thetao_sin, S nu, S G_, S c[11]) {
+    const FrameT<S> fr = local_frame(G, aS, alpha, beta, thetao_sin, sc.u, sc.bh);
+    const S nuf = nu / fr.g;
+    const S cb = dmin(dmax(fr.cosB, -1.0), 1.0);
+    S sth, cth;
+    // FP64 takes cos = cb and the product form of the sine; the FP32 path keeps acos and sincos: with the
+    // product form, or with the sine taken in FP64 from cb, its images moved further from the FP64 images
+    // (9.0e-7 against 6.2e-7 of peak I, 16 x 16 pixels, N = 256, 4 thermal splats), which the sine's
+    // accuracy alone does not explain
+    if constexpr (std::is_same<S, double>::value) pitch_sincos(cb, sth, cth);
+    else sincos(acos(cb), &sth, &cth);
+    const S ne = exp(sc.lnA) * G_;
+    CoefT<S> cf;
+    if constexpr (KIND == MODEL_THERMAL || KIND == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
+    else if constexpr (KIND == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
+    else if constexpr (KIND == MODEL_KAPPA) cf = kappa_coefs(KappaGet<S>{sc.kk}, ne, nuf, sth, cth);
+    else if (sc.kind == MODEL_THERMAL || sc.kind == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
+    else if (sc.kind == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
+    else cf = kappa_coefs(KappaGet<S>{sc.kk}, ne, nuf, sth, cth);
+    if (!(cf.jI > 0.0 || cf.aI > 0.0 || cf.rQ != 0.0 || cf.rV != 0.0)) return false;
+    const S fe = cap_factor(cf.jI, cf.jQ, cf.jV), fa = cap_factor(cf.aI, cf.aQ, cf.aV);
+    const S nh = nuf * (1.0 / NU0);
+    const S i2 = 1.0 / (nh * nh);
+    S s2c, c2c; sincos(2.0 * fr.chi, &s2c, &c2c);
+    const S jQ = fe * cf.jQ * i2, aQ = fa * cf.aQ * nh, rQ = cf.rQ * nh;
+    c[0] = cf.jI * i2; c[1] = jQ * c2c; c[2] = jQ * s2c; c[3] = fe * cf.jV * i2;
+    c[4] = cf.aI * nh; c[5] = aQ * c2c; c[6] = aQ * s2c; c[7] = fa * cf.aV * nh;
+    c[8] = rQ * c2c; c[9] = rQ * s2c; c[10] = cf.rV * nh;
+    return true;
+}
+
 // The splat sum of one sample (accumulate_elements, transport.jl:254-276): invariant j, alpha, rho in
-// screen axes; false when no splat contributes. One instantiation per population and scalar.
-// With a candidate list (ascending splat indices, the per-tile cull) only those splats are visited; the
-// others lie outside their support at every sample of the tile and would add exact zeros. With gout the sample's
-// geometry (in S) is returned when the sample contributes.
+// screen axes; false when no splat contributes. One instantiation per population and scalar. One sample at a time, for
+// the march fused with the transport; the transfer over stored samples packs the pairs of a wavefront's samples
+// instead (transfer_task). With a candidate list only those splats are visited.
 template <int KIND, class S>
 KS_DEV bool sample_coefficients(const TransCtxT<S>& c, double st, double r, double th, bool nur, bool nuth, S x, S y, S z,
-                                S j4[4], S a4[4], S r3[3], const uint16_t* cand = nullptr, int ncand = 0, GeoT<S>* gout = nullptr) {
+                                S j4[4], S a4[4], S r3[3], const uint16_t* cand = nullptr, int ncand = 0) {
     const S t = S(c.t_obs - st);
     for (int i = 0; i < 4; ++i) { j4[i] = S(0.0); a4[i] = S(0.0); }
     r3[0] = r3[1] = r3[2] = S(0.0);
@@ -58,56 +108,50 @@ KS_DEV bool sample_coefficients(const TransCtxT<S>& c, double st, double r, doub
     GeoT<S> G;
     const int nloop = cand ? ncand : c.ns;
     for (int ci = 0; ci < nloop; ++ci) {
-        const int i = cand ? (int)cand[ci] : ci;
-        const SplatCT<S>& sc = c.sp[i];
-        S gexp;
-        if (KIND == MODEL_KNOT || sc.nk > 0) {
-            gexp = knot_gexp(c, sc, t, x, y, z);
-        } else {
-            S sph, cph;
-            if (outside_support(sc, t, x, y, z, sph, cph)) continue;
-            gexp = gauss_exponent(sc, t, x, y, z, sph, cph);
-        }
-        if (gexp > GEXP_SKIP) continue;
-        S G_ = exp(-0.5 * gexp);
-        if (!(G_ > WEIGHT_CUTOFF)) continue;
+        const SplatCT<S>& sc = c.sp[cand ? (int)cand[ci] : ci];
+        const S G_ = splat_weight<KIND>(sc, c.knots, c.ktimes, t, x, y, z);
+        if (!(G_ > 0.0)) continue;
         if (!geo_ready) {
             Geo Gd;
             make_geo(c.a, r, th, c.eta, c.lam, nur, nuth, Gd);
             G = geo_as<S>(Gd);
             geo_ready = true;
         }
-        FrameT<S> fr = local_frame(G, c.aS, c.alpha, c.beta, c.thetao_sin, sc.u, sc.bh);
-        S nuf = c.nu / fr.g;
-        S cb = dmin(dmax(fr.cosB, -1.0), 1.0);
-        S sth, cth;
-        // FP64 takes cos = cb and the product form of the sine; the FP32 path keeps acos and sincos: with the
-        // product form, or with the sine taken in FP64 from cb, its images moved further from the FP64 images
-        // (9.0e-7 against 6.2e-7 of peak I, 16 x 16 pixels, N = 256, 4 thermal splats), which the sine's
-        // accuracy alone does not explain
-        if constexpr (std::is_same<S, double>::value) pitch_sincos(cb, sth, cth);
-        else sincos(acos(cb), &sth, &cth);
-        S ne = exp(sc.lnA) * G_;
-        CoefT<S> cf;
-        if constexpr (KIND == MODEL_THERMAL || KIND == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
-        else if constexpr (KIND == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
-        else if constexpr (KIND == MODEL_KAPPA) cf = kappa_coefs(KappaGet<S>{sc.kk}, ne, nuf, sth, cth);
-        else if (sc.kind == MODEL_THERMAL || sc.kind == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
-        else if (sc.kind == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
-        else cf = kappa_coefs(KappaGet<S>{sc.kk}, ne, nuf, sth, cth);
-        if (!(cf.jI > 0.0 || cf.aI > 0.0 || cf.rQ != 0.0 || cf.rV != 0.0)) continue;
-        S fe = cap_factor(cf.jI, cf.jQ, cf.jV), fa = cap_factor(cf.aI, cf.aQ, cf.aV);
-        S nh = nuf * (1.0 / NU0);
-        S i2 = 1.0 / (nh * nh);
-        S s2c, c2c; sincos(2.0 * fr.chi, &s2c, &c2c);
-        S jQ = fe * cf.jQ * i2, aQ = fa * cf.aQ * nh, rQ = cf.rQ * nh;
-        j4[0] += cf.jI * i2; j4[1] += jQ * c2c; j4[2] += jQ * s2c; j4[3] += fe * cf.jV * i2;
-        a4[0] += cf.aI * nh; a4[1] += aQ * c2c; a4[2] += aQ * s2c; a4[3] += fa * cf.aV * nh;
-        r3[0] += rQ * c2c; r3[1] += rQ * s2c; r3[2] += cf.rV * nh;
+        S v[11];
+        if (!splat_contribution<KIND>(sc, G, c.aS, c.alpha, c.beta, c.thetao_sin, c.nu, G_, v)) continue;
+        for (int q = 0; q < 4; ++q) { j4[q] += v[q]; a4[q] += v[4 + q]; }
+        for (int q = 0; q < 3; ++q) r3[q] += v[8 + q];
         active = true;
     }
-    if (gout && active) *gout = G;
     return active;
+}
+
+// Whether a splat may pass the weight cutoff at a sample, in FP32 on the hardware's sine and cosine, for both
+// precisions: false only when splat_weight is zero. The Gaussian exponent is taken to within 2 d (5.3 + d) of its value
+// near the cutoff (27.63 = 5.26^2), where d = pm0 + pm1 |t| bounds the error of the splat's scaled coordinates; a bound
+// that is not finite lets every sample through. About 45 instructions against 150 to 400 for the weight and 400 to 3000
+// for the contribution, which then run on the passing pairs alone, 64 at a time.
+template <int KIND>
+KS_DEV bool may_weigh(const SplatCf& c, const f32* __restrict__ knots, const f32* __restrict__ ktimes, float t, float x, float y, float z) {
+    float e0, e1, e2;
+    if (KIND == MODEL_KNOT || c.nk > 0) {
+        f32 cx, cy, cz;
+        knot_centre(c, knots, ktimes, f32(t), cx, cy, cz);
+        e0 = x - cx.v; e1 = y - cy.v; e2 = z - cz.v;
+    } else {
+        float sp, cp;
+        hw_sincos(c.omega.v * (t - c.t0.v), sp, cp);
+        // Rz(-ph) (X - Rz(ph) c) = Rz(-ph) X - c
+        e0 = x * cp + y * sp - c.x.v; e1 = y * cp - x * sp - c.y.v; e2 = z - c.z.v;
+    }
+    float g = (t - c.t0.v) * c.iw.v;
+    g = g * g;
+    for (int b = 0; b < 3; ++b) {
+        const float q = (c.R[b].v * e0 + c.R[3 + b].v * e1 + c.R[6 + b].v * e2) * c.is[b].v;
+        g += q * q;
+    }
+    const float d = c.pm1.v * fabsf(t) + c.pm0.v;
+    return !(g > 27.641f + 2.0f * d * (5.3f + d));
 }
 
 // thin splats (Splats.jl:113-128): sum_i j_i g^2 Sigma dtau with the ZAMO redshift g

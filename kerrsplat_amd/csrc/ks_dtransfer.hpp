@@ -64,6 +64,7 @@ template <class S> struct SplatCT {
     S g[6];               // power law: Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12);
                           // kappa: Gamma(k-4/3), Gamma(k-2), Gamma(k/4-1/3), Gamma(k/4+4/3), Gamma(2+k/2), K0/(K2+1e-40) at 1/w
     S kc[3], kr;          // splats whose centre follows knots: a sphere holding every knot (centre, radius; kr = 0 without)
+    S pm0, pm1;           // the FP32 prefilter's error in the splat's scaled coordinates, pm0 + pm1 |t| (may_weigh)
     KappaK<S> kk;         // kappa: the fits' per-splat factors (kappa_consts)
     int knot0, nk, kt0;   // splats whose centre follows knots (nk > 0): the first of its nk knots (xyz triples) and of their
                           // times in the model's arrays
@@ -191,6 +192,7 @@ KS_DEV void knot_centre(const SplatCT<S>& sc, const S* __restrict__ knots, const
 // ---- metric, ZAMO tetrad, photon momentum ----------------------------------------------------------------------
 template <class T> struct GeoT {   // everything of a sample the splats share
     T r, th, st, ct, S, Dl, Xi, lapse, omega, sgrr, sgthth, sgpp;
+    T ilapse, isgrr, isgthth, isgpp;    // their reciprocals, once per sample for all its splats
     T pu[4];        // contravariant BL photon momentum
     T pz[4];        // ZAMO components (t, r, phi, -theta)
 };
@@ -207,6 +209,7 @@ KS_DEV void make_geo(Q a, Q r, Q th, Q eta, Q lam, bool nur, bool nuth, GeoT<Q>&
     g.sgrr = sqrt(g.S / g.Dl);
     g.sgthth = sqrt(g.S);
     g.sgpp = g.st * sqrt(g.Xi / g.S);
+    g.ilapse = 1.0 / g.lapse; g.isgrr = 1.0 / g.sgrr; g.isgthth = 1.0 / g.sgthth; g.isgpp = 1.0 / g.sgpp;
     Q w = r * r + a * a - a * lam;
     Q R = w * w - g.Dl * (eta + (lam - a) * (lam - a));
     Q Th = eta + a * a * g.ct * g.ct - lam * lam * g.ct * g.ct / (g.st * g.st);
@@ -226,23 +229,23 @@ KS_DEV void make_geo(Q a, Q r, Q th, Q eta, Q lam, bool nur, bool nuth, GeoT<Q>&
     g.pz[3] = -g.sgthth * g.pu[2];
 }
 // The fields of a sample's geometry that the frames use (local_frame, frame_jacobian), stored field-major at
-// w[f * st] (f < 16): pz, pu, lapse, sgrr, sgthth, sgpp, omega, r, st, ct. geo_load leaves th, S, Dl and Xi unset.
+// w[f * st] (f < 16): pz, pu, 1 / lapse, 1 / sgrr, 1 / sgthth, 1 / sgpp, omega, r, st, ct. geo_load leaves the rest unset.
 template <class T> KS_DEV void geo_store(const GeoT<T>& g, T* w, int64_t st) {
     for (int i = 0; i < 4; ++i) { w[i * st] = g.pz[i]; w[(4 + i) * st] = g.pu[i]; }
-    w[8 * st] = g.lapse; w[9 * st] = g.sgrr; w[10 * st] = g.sgthth; w[11 * st] = g.sgpp; w[12 * st] = g.omega;
+    w[8 * st] = g.ilapse; w[9 * st] = g.isgrr; w[10 * st] = g.isgthth; w[11 * st] = g.isgpp; w[12 * st] = g.omega;
     w[13 * st] = g.r; w[14 * st] = g.st; w[15 * st] = g.ct;
 }
 template <class T> KS_DEV void geo_load(const T* o, int64_t st, GeoT<T>& g) {
     for (int i = 0; i < 4; ++i) { g.pz[i] = o[i * st]; g.pu[i] = o[(4 + i) * st]; }
-    g.lapse = o[8 * st]; g.sgrr = o[9 * st]; g.sgthth = o[10 * st]; g.sgpp = o[11 * st]; g.omega = o[12 * st];
+    g.ilapse = o[8 * st]; g.isgrr = o[9 * st]; g.isgthth = o[10 * st]; g.isgpp = o[11 * st]; g.omega = o[12 * st];
     g.r = o[13 * st]; g.st = o[14 * st]; g.ct = o[15 * st];
-    g.th = T(0.0); g.S = T(0.0); g.Dl = T(0.0); g.Xi = T(0.0);
 }
 // the FP64 geometry of a sample in another scalar (built once per sample, shared by the splats)
 template <class T> KS_DEV GeoT<T> geo_as(const Geo& g) {
     GeoT<T> o;
     o.r = T(g.r); o.th = T(g.th); o.st = T(g.st); o.ct = T(g.ct); o.S = T(g.S); o.Dl = T(g.Dl); o.Xi = T(g.Xi);
     o.lapse = T(g.lapse); o.omega = T(g.omega); o.sgrr = T(g.sgrr); o.sgthth = T(g.sgthth); o.sgpp = T(g.sgpp);
+    o.ilapse = T(g.ilapse); o.isgrr = T(g.isgrr); o.isgthth = T(g.isgthth); o.isgpp = T(g.isgpp);
     for (int i = 0; i < 4; ++i) { o.pu[i] = T(g.pu[i]); o.pz[i] = T(g.pz[i]); }
     return o;
 }
@@ -276,10 +279,10 @@ KS_DEV FrameT<T> local_frame(const GeoT<S>& G, S a, S alpha, S beta, S thetao_si
     T ufq = uf * q;
     T fz1 = f0 + u[0] * ufq, fz2 = f1 + u[1] * ufq, fz3 = f2 + u[2] * ufq;
     // ZAMO -> BL contravariant
-    T ft = uf * (1.0 / G.lapse);
-    T fr_ = fz1 * (1.0 / G.sgrr);
-    T fth = fz3 * (-1.0 / G.sgthth);
-    T fph = fz2 * (1.0 / G.sgpp) + G.omega * ft;
+    T ft = uf * G.ilapse;
+    T fr_ = fz1 * G.isgrr;
+    T fth = fz3 * (-G.isgthth);
+    T fph = fz2 * G.isgpp + G.omega * ft;
     const S* p = G.pu;
     T A = p[0] * fr_ - p[1] * ft + (a * G.st * G.st) * (p[1] * fph - p[3] * fr_);
     T Bw = ((G.r * G.r + a * a) * (p[3] * fth - p[2] * fph) - a * (p[0] * fth - p[2] * ft)) * G.st;

@@ -72,6 +72,7 @@ template <class T> inline void splat_as(const SplatC& a, SplatCT<T>& b) {
     for (int i = 0; i < 6; ++i) b.g[i] = T(a.g[i]);
     for (int i = 0; i < 3; ++i) b.kc[i] = T(a.kc[i]);
     b.kr = T(a.kr);
+    b.pm0 = T(a.pm0); b.pm1 = T(a.pm1);
     for (int f = 0; f < KK_N; ++f) b.kk.v[f] = T(a.kk.v[f]);
     b.knot0 = a.knot0; b.nk = a.nk; b.kt0 = a.kt0; b.kind = a.kind;
 }
@@ -90,7 +91,7 @@ template <class T> inline void adj_as(const SplatAdj& a, SplatAdjT<T>& b) {
 // and 2F1 factors, kappa's fit factors, the knot sphere) and those of the adjoint (SplatAdj, with the partials of
 // the per-splat tables in the population rows). kind is the model's population (ModelKind).
 inline void host_splat_constants(int kind, int nrows, int i, const double* p, double gamma_max, bool with_knots,
-                                 const double* knots, int nknots, SplatC& c, SplatAdj& sa) {
+                                 const double* knots, const double* knot_times, int nknots, SplatC& c, SplatAdj& sa) {
     const double SR2 = -2.0 * std::log(1e-6);
     std::memset((void*)&sa, 0, sizeof sa);
     std::memset((void*)&c, 0, sizeof c);
@@ -124,6 +125,28 @@ inline void host_splat_constants(int kind, int nrows, int i, const double* p, do
             r2 = std::max(r2, d2);
         }
         c.kr = std::sqrt(r2) * (1.0 + 1e-12);
+    }
+    {
+        // may_weigh's error bound. FP32 rounds a position of size R by R 6e-8 in each of a few operations (1e-6 R covers
+        // them), a time by |t| 6e-8 twice, and the centre moves by v per unit of time; the hardware's sine and cosine are
+        // within 4e-6. Each error enters the scaled coordinate times the largest inverse scale.
+        const double is = std::max(std::max(c.is[0], c.is[1]), c.is[2]);
+        const double rho = std::hypot(c.x, c.y);
+        double R = rho + std::fabs(c.z), v = std::fabs(c.omega) * rho, tmax = std::fabs(c.t0);
+        if (with_knots) {
+            R = std::sqrt(c.kc[0] * c.kc[0] + c.kc[1] * c.kc[1] + c.kc[2] * c.kc[2]) + c.kr;
+            v = 0.0;
+            const double* K = knots + (size_t)3 * nknots * i;
+            for (int k = 0; k < nknots; ++k) tmax = std::max(tmax, std::fabs(knot_times[k]));
+            for (int k = 0; k + 1 < nknots; ++k) {
+                double d2 = 0.0;
+                for (int a_ = 0; a_ < 3; ++a_) d2 += (K[3 * k + 3 + a_] - K[3 * k + a_]) * (K[3 * k + 3 + a_] - K[3 * k + a_]);
+                v = std::max(v, std::sqrt(d2) / (knot_times[k + 1] - knot_times[k]));
+            }
+        }
+        R += std::sqrt(c.rsup2);
+        c.pm0 = 2.0 * is * (1e-6 * R + 4e-6 * rho + 6e-7 * v * tmax) + 6e-7 * std::fabs(c.t0) * c.iw;
+        c.pm1 = 2.0 * is * 6e-7 * v + 6e-7 * c.iw;
     }
     if (kind == MODEL_THIN) return;
     int rB = (kind == MODEL_THERMAL || kind == MODEL_KNOT) ? 14 : 15;

@@ -8,41 +8,78 @@ namespace ksd {
 
 // ---- the dual-sweep adjoint (dual_gradient.jl:125-249) over stored samples -------------------------------------
 // Per item: from the chunk maps (P_m, S_m), the tail behind each chunk T_out[m] = S_{m+1} + P_{m+1} T_out[m+1]
-// (T_out[last] = 0), the image nu-hat^3 T_in[0], and the adjoint in front of each chunk
-// w_in[m] = (P_0 ... P_{m-1})^T w_1 with w_1 = nu-hat^3 dstokes (dual_gradient.jl:162).
-// wT[(8 m + q) nitems + item] = w_in, wT[(8 m + 4 + q) nitems + item] = T_out; the image only when out is given.
-__global__ void ks_adj_combine(int64_t npix, int N, int chunk, int nt, const double* __restrict__ nus, int nnu, const double* __restrict__ seg,
-                               const double* __restrict__ dstokes, double* __restrict__ wT, double* __restrict__ out) {
+// (T_out[last] = 0), and the adjoint in front of each chunk w_in[m] = (P_0 ... P_{m-1})^T w_1 with w_1 = nu-hat^3
+// dstokes (dual_gradient.jl:162). wT[(8 m + q) nitems + item] = w_in, wT[(8 m + 4 + q) nitems + item] = T_out.
+// A workgroup takes 64 items, each of its wavefronts a run of their chunks: first the run's own map, then through LDS
+// the tail behind the run and the adjoint in front of it, then the run's chunks (ks_seg_combine has the same split).
+template <class G>
+__global__ void __launch_bounds__(64 * COMBINE_WAVES)
+ks_adj_combine(int64_t npix, int N, int chunk, int nt, const double* __restrict__ nus, int nnu, const G* __restrict__ seg,
+               const double* __restrict__ dstokes, double* __restrict__ wT) {
+    __shared__ double s_map[COMBINE_WAVES][SEG_FIELDS][64];
     const int64_t nitems = npix * nt * nnu;
-    const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (item >= nitems) return;
-    const int inu = (int)((item / npix) / nt);
+    const int lane = (int)(threadIdx.x % 64), wv = (int)(threadIdx.x / 64);
+    const int64_t item = (int64_t)blockIdx.x * 64 + lane;
     const int nseg = (N + chunk - 1) / chunk;
-    const double nh = nus[inu] * (1.0 / NU0);
-    const double s3 = nh * nh * nh;
+    const int per = (nseg + COMBINE_WAVES - 1) / COMBINE_WAVES;
+    const int m0 = wv * per, m1 = m0 + per < nseg ? m0 + per : nseg;
+    {
+        double P[16], Sv[4] = {0, 0, 0, 0};
+        for (int i = 0; i < 16; ++i) P[i] = (i % 5 == 0) ? 1.0 : 0.0;
+        if (item < nitems)
+            for (int m = m0; m < m1; ++m) {
+                double Pm[16], Sm[4];
+                seg_load(seg, m, nitems, item, Pm, Sm);
+                seg_append(P, Sv, Pm, Sm);
+            }
+        for (int q = 0; q < 16; ++q) s_map[wv][q][lane] = P[q];
+        for (int q = 0; q < 4; ++q) s_map[wv][16 + q][lane] = Sv[q];
+    }
+    __syncthreads();
+    if (item >= nitems) return;
     double T[4] = {0, 0, 0, 0};
-    for (int m = nseg - 1; m >= 0; --m) {
-        const double* g = seg + (int64_t)SEG_FIELDS * m * nitems + item;
-        for (int q = 0; q < 4; ++q) wT[(8 * (int64_t)m + 4 + q) * nitems + item] = T[q];
+    for (int w = COMBINE_WAVES - 1; w > wv; --w) {
         double Tn[4];
         for (int i = 0; i < 4; ++i) {
-            double v = g[(16 + i) * nitems];
-            for (int q = 0; q < 4; ++q) v += g[(4 * i + q) * nitems] * T[q];
+            double v = s_map[w][16 + i][lane];
+            for (int q = 0; q < 4; ++q) v += s_map[w][4 * i + q][lane] * T[q];
             Tn[i] = v;
         }
         for (int i = 0; i < 4; ++i) T[i] = Tn[i];
     }
-    if (out)
-        for (int q = 0; q < 4; ++q) out[4 * item + q] = T[q] * s3;
+    const double nh = nus[(item / npix) / nt] * (1.0 / NU0);
+    const double s3 = nh * nh * nh;
     double w[4];
     for (int q = 0; q < 4; ++q) w[q] = dstokes[4 * item + q] * s3;
-    for (int m = 0; m < nseg; ++m) {
-        const double* g = seg + (int64_t)SEG_FIELDS * m * nitems + item;
+    for (int v = 0; v < wv; ++v) {
+        double wn[4];
+        for (int c = 0; c < 4; ++c) {
+            double acc = 0.0;
+            for (int i = 0; i < 4; ++i) acc += s_map[v][4 * i + c][lane] * w[i];
+            wn[c] = acc;
+        }
+        for (int q = 0; q < 4; ++q) w[q] = wn[q];
+    }
+    for (int m = m1 - 1; m >= m0; --m) {
+        double Pm[16], Sm[4];
+        seg_load(seg, m, nitems, item, Pm, Sm);
+        for (int q = 0; q < 4; ++q) wT[(8 * (int64_t)m + 4 + q) * nitems + item] = T[q];
+        double Tn[4];
+        for (int i = 0; i < 4; ++i) {
+            double v = Sm[i];
+            for (int q = 0; q < 4; ++q) v += Pm[4 * i + q] * T[q];
+            Tn[i] = v;
+        }
+        for (int i = 0; i < 4; ++i) T[i] = Tn[i];
+    }
+    for (int m = m0; m < m1; ++m) {
+        double Pm[16], Sm[4];
+        seg_load(seg, m, nitems, item, Pm, Sm);
         for (int q = 0; q < 4; ++q) wT[(8 * (int64_t)m + q) * nitems + item] = w[q];
         double wn[4];
         for (int c = 0; c < 4; ++c) {
             double v = 0.0;
-            for (int i = 0; i < 4; ++i) v += g[(4 * i + c) * nitems] * w[i];
+            for (int i = 0; i < 4; ++i) v += Pm[4 * i + c] * w[i];
             wn[c] = v;
         }
         for (int q = 0; q < 4; ++q) w[q] = wn[q];
@@ -408,10 +445,11 @@ __global__ void __launch_bounds__(64) ks_adj_reduce(const double* __restrict__ p
 }
 
 // ---- launchers ----
-hipError_t launch_adj_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const double* seg,
-                              const double* dstokes, double* wT, double* out) {
-    const int64_t items = npix * nt * nnu;
-    hipLaunchKernelGGL(ks_adj_combine, dim3(grid_for(items, 128)), dim3(128), 0, s, npix, N, chunk, nt, nus, nnu, seg, dstokes, wT, out);
+hipError_t launch_adj_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const void* seg, int seg32,
+                              const double* dstokes, double* wT) {
+    const dim3 grid(grid_for(npix * nt * nnu, 64)), block(64 * COMBINE_WAVES);
+    if (seg32) hipLaunchKernelGGL(ks_adj_combine<f32>, grid, block, 0, s, npix, N, chunk, nt, nus, nnu, (const f32*)seg, dstokes, wT);
+    else hipLaunchKernelGGL(ks_adj_combine<double>, grid, block, 0, s, npix, N, chunk, nt, nus, nnu, (const double*)seg, dstokes, wT);
     return hipGetLastError();
 }
 hipError_t launch_adj_segment(hipStream_t s, int N, int chunk, int64_t nitems, const double* wT, const double* rec, double* bar,

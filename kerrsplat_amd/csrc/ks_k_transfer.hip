@@ -10,8 +10,8 @@
 namespace ksd {
 
 // ---- polarized transport from stored samples (transport.jl:263-290) ----------------------------------------
-// Work items (chunk m, item), item = j + npix (it + nt inu) fastest: samples m chunk + 1 .. of the
-// item's ray, composed into the chunk's map seg[(20 m + f) nitems + item]. With rec != nullptr the
+// Work items (slice m, item), item = j + npix (it + nt inu) fastest: samples m chunk + 1 .. of the
+// item's ray, composed into the slice's map seg[(20 m + f) nitems + item]. With rec != nullptr the
 // adjoint records (RecField) of every step-taking sample are written, and aflg[(k - 1) nitems + item]
 // = 1 when the sample takes a step. A task is one workgroup's 128 consecutive slots (slot = item slot +
 // nitems m); the item slots run over the cache's wavefront patches (slot_item).
@@ -26,13 +26,44 @@ struct TransferArgs {
     const double* nus; int nnu;
     double L;
     const int* kstop;
-    double* seg;
     uint8_t* aflg;
+    const SplatCf* spf; const f32* knots_f; const f32* ktimes_f;     // the FP32 copies (may_weigh)
 };
 KS_DEV int64_t npix_items(const TransferArgs& A) { return A.npix * A.nt * A.nnu; }
+// A wavefront's workspace in LDS, field-major over its 64 lanes: the geometry of its rays' current sample, the sums of
+// the sample's contributions and whether it has any, the rays' screen coordinates and frequency, the pair queue (lane |
+// splat << 6), the slice's candidate splats. 7.8 KB in FP32 and 15.6 KB in FP64: as many wavefronts as the registers
+// allow fit a compute unit.
+constexpr int QCAP = 128;              // the queue holds < 64 pending pairs and up to 64 pushes of one splat
+template <class S>
+struct WaveWork {
+    S geo[GEO_FIELDS * 64], sum[11 * 64], alpha[64], beta[64], nu[64];
+    uint64_t mask[CAND_MAX / 64];
+    int q[QCAP], act[64];
+};
+// Values written by some lanes of the wavefront are read by others: the LDS operations of a wavefront run in order, and
+// the compiler keeps theirs across this.
+KS_DEV void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+KS_DEV uint64_t uniform64(uint64_t x) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+}
+// One wavefront: 64 items x one slice. Sample by sample, the lanes test their ray's sample against the candidate splats
+// (may_weigh) and queue the pairs that pass; whenever 64 are queued, or the candidates are through, the queued pairs'
+// weights, frames and coefficients run one pair a lane (splat_contribution), and each adds its 11 values to its
+// sample's sums in LDS, the pairs of one splat at a time: a sample's contributions are added in ascending splat order,
+// whatever wavefront it sits in. Then every lane takes its sample's step. Before, each lane visited its own sample's
+// splats, with 43 to 71% of the lanes in a splat's support, over slices four times as long, and 5 to 40% of the vector
+// issue slots used. MI355X, whole call, before and after: FP64 image of 6 thermal splats (50 x 37 x 301) 1.17 -> 0.37 ms,
+// FP64 march and image of 32 thermal splats (128^2 x 1024) 13.9 -> 9.2 ms, FP64 gradient of 48 power-law splats
+// (102 x 67 x 333, 2 frames) 28.4 -> 14.0 ms, FP64 fit iteration of 1024 kappa splats (112 x 96 x 512) 780 -> 351 ms, mixed
+// (256^2 x 1024) 1084 -> 953 ms, mixed movie of 128 splats (36,864 points x 512 x 12 frames) 113 -> 76 ms.
+// The queue, not the lanes, decides what runs: all lanes take part in every collective, and each loop exit is uniform.
 template <int KIND, class S, bool CULL>
 __device__ __forceinline__ void transfer_task(const TransferArgs& A, const SplatCT<S>* __restrict__ sp, const S* __restrict__ knots,
-                                    const S* __restrict__ ktimes, S* __restrict__ rec, int64_t task, uint16_t* s_cand) {
+                                    const S* __restrict__ ktimes, S* __restrict__ seg, S* __restrict__ rec, int64_t task, WaveWork<S>& W) {
     const int64_t npix = A.npix;
     const int N = A.N;
     const int64_t nitems = npix * A.nt * A.nnu;
@@ -48,68 +79,135 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
     const double a = A.a;
     const Spin Sp = make_spin(a);
     const double dtau = A.soa[(int64_t)PF_TAUTOT * npix + j] / (double)(N + 1);
-    const TransCtxT<S> c = make_ctx<S>(a, Sp.rp, Sp.rm, sin(A.thetao), A.soa[(int64_t)PF_ALPHA * npix + j], A.soa[(int64_t)PF_BETA * npix + j],
-                                       A.soa[(int64_t)PF_ETA * npix + j], A.soa[(int64_t)PF_LAM * npix + j], sp, A.ns, knots, ktimes, A.nknots,
-                                       A.times[it], A.nus[inu], A.L);
+    const S aS = S(a), tos = S(sin(A.thetao));
+    const double t_obs = A.times[it], nu = A.nus[inu];
     const int ks = A.kstop ? A.kstop[j] : N + 1;
     const double hor = Sp.rp * (1.0 + 1e-3);
     const int kbeg = m * A.chunk + 1, kend = kbeg + A.chunk - 1 < N ? kbeg + A.chunk - 1 : N;
     const int64_t st = (int64_t)N * nitems;
-    // the per-tile cull: the splats that can reach the wavefront's samples of this chunk, in ascending
-    // order, as a candidate list in LDS (the rest add exact zeros to every sample of the tile)
-    constexpr bool cull = CULL;     // the launcher picks CULL for CULL_MIN_NS <= ns <= CAND_MAX
-    const int wv = (int)(threadIdx.x / 64), lane = (int)(threadIdx.x % 64);
-    int ncand = 0;
-    if constexpr (cull) {
+    const int lane = (int)(threadIdx.x % 64);
+    W.alpha[lane] = S(A.soa[(int64_t)PF_ALPHA * npix + j]);
+    W.beta[lane] = S(A.soa[(int64_t)PF_BETA * npix + j]);
+    W.nu[lane] = S(nu);
+    // the per-tile cull: the splats that can reach the wavefront's samples of this slice, a bit each (the rest add exact
+    // zeros to every sample of the tile); every splat without it
+    const int nblk = (A.ns + 63) / 64;
+    if constexpr (CULL) {     // the launcher picks CULL for CULL_MIN_NS <= ns <= CAND_MAX
         double lo[4] = {INFINITY, INFINITY, INFINITY, INFINITY}, hi[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
         if (live)
             for (int k = kbeg; k <= kend; ++k) {
                 const int64_t o = (int64_t)(k - 1) * npix + j;
                 if ((smp.fl[o] & 1) && smp.r[o] > hor && k < ks) {
-                    const double v[4] = {smp.x[o], smp.y[o], smp.z[o], c.t_obs - smp.t[o]};
+                    const double v[4] = {smp.x[o], smp.y[o], smp.z[o], t_obs - smp.t[o]};
                     for (int q = 0; q < 4; ++q) { lo[q] = fmin(lo[q], v[q]); hi[q] = fmax(hi[q], v[q]); }
                 }
             }
         double px = 0.0, py = 0.0, pz = 0.0, R = 0.0, tmin = 0.0, tmax = 0.0;
         const bool any = wave_region(lo, hi, px, py, pz, R, tmin, tmax);
-        for (int i0 = 0; i0 < A.ns; i0 += 64) {
-            const int i = i0 + lane;
-            const bool hit = any && i < A.ns && splat_may_reach(sp[i], px, py, pz, R, tmin, tmax, knots, ktimes);
-            const uint64_t mk = __ballot(hit);
-            if (hit) s_cand[wv * CAND_MAX + ncand + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u))] = (uint16_t)i;
-            ncand += __popcll(mk);
+        for (int b = 0; b < nblk; ++b) {
+            const int i = b * 64 + lane;
+            const uint64_t mk = __ballot(any && i < A.ns && splat_may_reach(sp[i], px, py, pz, R, tmin, tmax, knots, ktimes));
+            if (lane == 0) W.mask[b] = mk;
         }
     }
-    if constexpr (cull) __syncthreads();
-    if (!live) return;
+    wave_sync();
     SegMapT<S> sm;
     sm.init();
-    for (int k = kbeg; k <= kend; ++k) {
-        const int64_t o = (int64_t)(k - 1) * npix + j;
+    for (int s = 0; s < A.chunk; ++s) {
+        const int k = kbeg + s;
+        const bool in = live && k <= kend;
+        const int64_t o = (int64_t)((in ? k : 1) - 1) * npix + j;
         const uint8_t fl = smp.fl[o];
-        bool step = false;
         const double r = smp.r[o];
-        if ((fl & 1) && r > hor && k < ks) {
-            const double th = smp.th[o];
-            S j4[4], a4[4], r3[3];
-            GeoT<S> G;
-            if (sample_coefficients<KIND, S>(c, smp.t[o], r, th, (fl & 2) != 0, (fl & 4) != 0, S(smp.x[o]), S(smp.y[o]), S(smp.z[o]),
-                                             j4, a4, r3, cull ? s_cand + wv * CAND_MAX : nullptr, ncand, rec ? &G : nullptr)) {
-                const S D = S(path_weight(A.L, A.nus[inu], a, r, th, dtau));
+        const bool valid = in && (fl & 1) && r > hor && k < ks;
+        bool step = false, ready = false;
+        if (__ballot(valid)) {
+            const S t = S(t_obs - smp.t[o]), x = S(smp.x[o]), y = S(smp.y[o]), z = S(smp.z[o]);
+            const float tf = (float)val(t), xf = (float)val(x), yf = (float)val(y), zf = (float)val(z);
+            S D(0.0);
+            int qh = 0, qn = 0, b = -1;
+            uint64_t mk = 0;
+            bool more = true;
+            for (;;) {
+                while (qn < 64) {
+                    while (mk == 0 && more) {
+                        if (++b >= nblk) more = false;
+                        else if constexpr (CULL) mk = uniform64(W.mask[b]);
+                        else mk = A.ns - 64 * b >= 64 ? ~0ull : (1ull << (A.ns - 64 * b)) - 1;
+                    }
+                    if (!more) break;
+                    const int i = b * 64 + __builtin_ctzll(mk);
+                    mk &= mk - 1;
+                    const bool hit = valid && may_weigh<KIND>(A.spf[i], A.knots_f, A.ktimes_f, tf, xf, yf, zf);
+                    const uint64_t hm = __ballot(hit);
+                    if (hit) W.q[(qh + qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u))) & (QCAP - 1)] = lane | (i << 6);
+                    qn += __popcll(hm);
+                }
+                if (qn == 0) break;
+                if (!ready) {            // the sample's geometry, in FP64, for its first queued pairs
+                    ready = true;
+                    for (int q = 0; q < 11; ++q) W.sum[64 * q + lane] = S(0.0);
+                    W.act[lane] = 0;
+                    if (valid) {
+                        Geo Gd;
+                        make_geo(a, r, smp.th[o], A.soa[(int64_t)PF_ETA * npix + j], A.soa[(int64_t)PF_LAM * npix + j], (fl & 2) != 0, (fl & 4) != 0, Gd);
+                        geo_store(geo_as<S>(Gd), W.geo + lane, 64);
+                        D = S(A.L / (nu * (1.0 / NU0)) * Gd.S * dtau);       // path_weight
+                    }
+                }
+                wave_sync();
+                const int cnt = qn < 64 ? qn : 64;
+                const bool on = lane < cnt;
+                const int e = W.q[(qh + lane) & (QCAP - 1)];
+                const int l = on ? e & 63 : lane, i = on ? e >> 6 : 0;
+                const S tt = lane_value(t, l), xx = lane_value(x, l), yy = lane_value(y, l), zz = lane_value(z, l);
+                bool act = false;
+                S c[11];
+                for (int q = 0; q < 11; ++q) c[q] = S(0.0);
+                if (on) {
+                    const SplatCT<S>& sc = sp[i];
+                    const S G_ = splat_weight<KIND>(sc, knots, ktimes, tt, xx, yy, zz);
+                    if (G_ > 0.0) {
+                        GeoT<S> G;
+                        geo_load(W.geo + l, 64, G);
+                        act = splat_contribution<KIND>(sc, G, aS, W.alpha[l], W.beta[l], tos, W.nu[l], G_, c);
+                    }
+                }
+                uint64_t todo = __ballot(act);
+                while (todo) {
+                    const int si = __builtin_amdgcn_readlane(i, __builtin_ctzll(todo));
+                    const bool mine = act && i == si;
+                    if (mine) {
+                        for (int q = 0; q < 11; ++q) W.sum[64 * q + l] += c[q];
+                        W.act[l] = 1;
+                    }
+                    wave_sync();
+                    todo &= ~__ballot(mine);
+                }
+                qh += cnt;
+                qn -= cnt;
+                if (!more && qn == 0) break;
+            }
+            wave_sync();
+            step = ready && W.act[lane] != 0;
+            if (step) {
+                S j4[4], a4[4], r3[3];
+                for (int q = 0; q < 4; ++q) { j4[q] = W.sum[64 * q + lane]; a4[q] = W.sum[64 * (4 + q) + lane]; }
+                for (int q = 0; q < 3; ++q) r3[q] = W.sum[64 * (8 + q) + lane];
                 map_step(sm, j4, a4, r3, D);
-                step = true;
                 if (rec) {
                     S* w = rec + (int64_t)(k - 1) * nitems + item;
-                    for (int i = 0; i < 4; ++i) { w[(REC_J + i) * st] = j4[i]; w[(REC_A + i) * st] = a4[i]; }
-                    for (int i = 0; i < 3; ++i) w[(REC_RHO + i) * st] = r3[i];
+                    for (int q = 0; q < 4; ++q) { w[(REC_J + q) * st] = j4[q]; w[(REC_A + q) * st] = a4[q]; }
+                    for (int q = 0; q < 3; ++q) w[(REC_RHO + q) * st] = r3[q];
                     w[REC_D * st] = D;
-                    geo_store(G, w + REC_GEO * st, st);
+                    for (int f = 0; f < GEO_FIELDS; ++f) w[(REC_GEO + f) * st] = W.geo[64 * f + lane];
                 }
             }
+            wave_sync();
         }
-        if (rec) A.aflg[(int64_t)(k - 1) * nitems + item] = step ? 1 : 0;
+        if (rec && in) A.aflg[(int64_t)(k - 1) * nitems + item] = step ? 1 : 0;
     }
-    sm.store(A.seg, m, nitems, item);
+    if (live) sm.store(seg, m, nitems, item);
 }
 
 // The launch forms share one kernel and one copy of the task body (so both give the same numbers bit for bit):
@@ -126,9 +224,9 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
 template <int KIND, class S, bool CULL>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(Waves<S>::transfer)))
 ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __restrict__ knots, const S* __restrict__ ktimes,
-                  S* __restrict__ rec, const int* __restrict__ tasks, int64_t ntasks, unsigned* __restrict__ head,
+                  S* __restrict__ seg, S* __restrict__ rec, const int* __restrict__ tasks, int64_t ntasks, unsigned* __restrict__ head,
                   uint32_t* __restrict__ cost) {
-    __shared__ uint16_t s_cand[2][CULL ? CAND_MAX : 1];
+    __shared__ WaveWork<S> s_w[2];
     __shared__ unsigned s_q;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
     int64_t next = blockIdx.x;
@@ -149,7 +247,7 @@ ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __
         if (q >= ntasks) break;
         const int64_t task = tasks ? (int64_t)tasks[q] : q;
         const uint64_t t0 = cost ? wall_clock64() : 0;
-        transfer_task<KIND, S, CULL>(A, sp, knots, ktimes, rec, task, &s_cand[0][0]);
+        transfer_task<KIND, S, CULL>(A, sp, knots, ktimes, seg, rec, task, s_w[wave]);
         if (cost) {
             __syncthreads();
             atomicMax(cost + task, (uint32_t)min<uint64_t>(wall_clock64() - t0, 0xffffffffull));
@@ -267,29 +365,41 @@ KS_DEV int item_segments(const double* soa, int64_t npix, int64_t j, int N, int 
     const int L = chunk > 0 ? chunk : segment_length(M, 1.0 - soa[(int64_t)PF_K * npix + j]);
     return (N + L - 1) / L;
 }
-// S = sum_m P_0 ... P_{m-1} S_m, the observed Stokes vector nu-hat^3 S (observed_stokes, transport.jl:311-316)
-__global__ void ks_seg_combine(const double* __restrict__ soa, int64_t npix, int N, int M, int chunk, int nt, const double* __restrict__ nus,
-                               int nnu, const double* __restrict__ seg, double* __restrict__ out) {
+// S = sum_m P_0 ... P_{m-1} S_m, the observed Stokes vector nu-hat^3 S (observed_stokes, transport.jl:311-316). A
+// workgroup takes 64 items, each of its COMBINE_WAVES wavefronts a run of their segments; the runs' maps are composed
+// in order through LDS (one wavefront over all segments left most of the chip idle: 65 us for 128^2 items of 32
+// segments, 256 wavefronts).
+template <class G>
+__global__ void __launch_bounds__(64 * COMBINE_WAVES)
+ks_seg_combine(const double* __restrict__ soa, int64_t npix, int N, int M, int chunk, int nt, const double* __restrict__ nus, int nnu,
+               const G* __restrict__ seg, double* __restrict__ out) {
+    __shared__ double s_map[COMBINE_WAVES][SEG_FIELDS][64];
     const int64_t nitems = npix * nt * nnu;
-    const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (item >= nitems) return;
-    const int64_t j = item % npix;
-    const int inu = (int)((item / npix) / nt);
-    const int nseg = item_segments(soa, npix, j, N, M, chunk);
+    const int lane = (int)(threadIdx.x % 64), wv = (int)(threadIdx.x / 64);
+    const int64_t item = (int64_t)blockIdx.x * 64 + lane;
     double P[16], Sv[4] = {0, 0, 0, 0};
     for (int i = 0; i < 16; ++i) P[i] = (i % 5 == 0) ? 1.0 : 0.0;
-    for (int m = 0; m < nseg; ++m) {
-        const double* g = seg + (int64_t)SEG_FIELDS * m * nitems + item;
-        double Pm[16], Sm[4];
-        for (int q = 0; q < 16; ++q) Pm[q] = g[q * nitems];
-        for (int q = 0; q < 4; ++q) Sm[q] = g[(16 + q) * nitems];
-        for (int i = 0; i < 4; ++i) Sv[i] += P[4 * i] * Sm[0] + P[4 * i + 1] * Sm[1] + P[4 * i + 2] * Sm[2] + P[4 * i + 3] * Sm[3];
-        double Pn[16];
-        for (int i = 0; i < 4; ++i)
-            for (int q = 0; q < 4; ++q) Pn[4 * i + q] = P[4 * i] * Pm[q] + P[4 * i + 1] * Pm[4 + q] + P[4 * i + 2] * Pm[8 + q] + P[4 * i + 3] * Pm[12 + q];
-        for (int i = 0; i < 16; ++i) P[i] = Pn[i];
+    if (item < nitems) {
+        const int nseg = item_segments(soa, npix, item % npix, N, M, chunk);
+        const int per = (nseg + COMBINE_WAVES - 1) / COMBINE_WAVES;
+        const int m1 = (wv + 1) * per < nseg ? (wv + 1) * per : nseg;
+        for (int m = wv * per; m < m1; ++m) {
+            double Pm[16], Sm[4];
+            seg_load(seg, m, nitems, item, Pm, Sm);
+            seg_append(P, Sv, Pm, Sm);
+        }
     }
-    const double nh = nus[inu] * (1.0 / NU0);
+    for (int q = 0; q < 16; ++q) s_map[wv][q][lane] = P[q];
+    for (int q = 0; q < 4; ++q) s_map[wv][16 + q][lane] = Sv[q];
+    __syncthreads();
+    if (wv != 0 || item >= nitems) return;
+    for (int w = 1; w < COMBINE_WAVES; ++w) {
+        double Pm[16], Sm[4];
+        for (int q = 0; q < 16; ++q) Pm[q] = s_map[w][q][lane];
+        for (int q = 0; q < 4; ++q) Sm[q] = s_map[w][16 + q][lane];
+        seg_append(P, Sv, Pm, Sm);
+    }
+    const double nh = nus[(item / npix) / nt] * (1.0 / NU0);
     const double s3 = nh * nh * nh;
     for (int q = 0; q < 4; ++q) out[4 * item + q] = Sv[q] * s3;
 }
@@ -304,14 +414,14 @@ hipError_t launch_fill_i32(hipStream_t s, int* p, int64_t n, int v) {
     return hipGetLastError();
 }
 template <int KIND, class S, bool CULL>
-static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* rec,
+static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* seg, S* rec,
                                    const TransferLaunch& tl) {
     const int64_t all = (npix_items(A) * A.nch + 127) / 128;
     const int64_t ntasks = tl.tasks ? tl.ntasks : all;
     if (ntasks <= 0) return hipSuccess;
     if (ntasks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
     if (!tl.queue) {
-        hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)ntasks), dim3(128), 0, s, A, sp, knots, ktimes, rec, tl.tasks,
+        hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)ntasks), dim3(128), 0, s, A, sp, knots, ktimes, seg, rec, tl.tasks,
                            ntasks, (unsigned*)nullptr, (uint32_t*)nullptr);
         return hipGetLastError();
     }
@@ -323,45 +433,44 @@ static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const S
     hipLaunchKernelGGL(ks_fill_i32, dim3(1), dim3(64), 0, s, tl.head, (int64_t)1, 0);
     if (tl.cost) hipLaunchKernelGGL(ks_fill_i32, dim3(grid_for(ntasks, 256)), dim3(256), 0, s, (int*)tl.cost, ntasks, 0);
     const int64_t grid = std::min<int64_t>(ntasks, (int64_t)groups * (tl.group_scale > 0 ? tl.group_scale : 1));
-    hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)grid), dim3(128), 0, s, A, sp, knots, ktimes, rec, tl.tasks,
+    hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)grid), dim3(128), 0, s, A, sp, knots, ktimes, seg, rec, tl.tasks,
                        ntasks, (unsigned*)tl.head, tl.cost);
     return hipGetLastError();
 }
 template <int KIND, class S>
-static hipError_t chunk_transfer_k(hipStream_t s, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* rec,
+static hipError_t chunk_transfer_k(hipStream_t s, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* seg, S* rec,
                                    const TransferLaunch& tl) {
     // the per-tile cull bounds pattern-rotating splats by their arc and knot splats by the sphere holding their knots
-    if (A.ns >= CULL_MIN_NS && A.ns <= CAND_MAX) return chunk_transfer_c<KIND, S, true>(s, A, sp, knots, ktimes, rec, tl);
-    return chunk_transfer_c<KIND, S, false>(s, A, sp, knots, ktimes, rec, tl);
+    if (A.ns >= CULL_MIN_NS && A.ns <= CAND_MAX) return chunk_transfer_c<KIND, S, true>(s, A, sp, knots, ktimes, seg, rec, tl);
+    return chunk_transfer_c<KIND, S, false>(s, A, sp, knots, ktimes, seg, rec, tl);
 }
 template <class S>
-static hipError_t chunk_transfer_s(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
-                                   const SplatCT<S>* sp, int ns, const S* knots, const S* ktimes, int nknots, const double* times, int nt,
-                                   const double* nus, int nnu, double L, const int* kstop, double* seg, S* rec, uint8_t* aflg,
-                                   const TransferLaunch& tl) {
+static hipError_t chunk_transfer_s(hipStream_t s, int kind, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* seg,
+                                   S* rec, const TransferLaunch& tl) {
     if (tl.chunk < 1) return hipErrorInvalidValue;
-    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, seg, aflg};
     switch (kind) {
-        case MODEL_THERMAL: return chunk_transfer_k<MODEL_THERMAL, S>(s, A, sp, knots, ktimes, rec, tl);
-        case MODEL_POWERLAW: return chunk_transfer_k<MODEL_POWERLAW, S>(s, A, sp, knots, ktimes, rec, tl);
-        case MODEL_KAPPA: return chunk_transfer_k<MODEL_KAPPA, S>(s, A, sp, knots, ktimes, rec, tl);
-        case MODEL_COMPOSITE: return chunk_transfer_k<MODEL_COMPOSITE, S>(s, A, sp, knots, ktimes, rec, tl);
-        default: return chunk_transfer_k<MODEL_KNOT, S>(s, A, sp, knots, ktimes, rec, tl);
+        case MODEL_THERMAL: return chunk_transfer_k<MODEL_THERMAL, S>(s, A, sp, knots, ktimes, seg, rec, tl);
+        case MODEL_POWERLAW: return chunk_transfer_k<MODEL_POWERLAW, S>(s, A, sp, knots, ktimes, seg, rec, tl);
+        case MODEL_KAPPA: return chunk_transfer_k<MODEL_KAPPA, S>(s, A, sp, knots, ktimes, seg, rec, tl);
+        case MODEL_COMPOSITE: return chunk_transfer_k<MODEL_COMPOSITE, S>(s, A, sp, knots, ktimes, seg, rec, tl);
+        default: return chunk_transfer_k<MODEL_KNOT, S>(s, A, sp, knots, ktimes, seg, rec, tl);
     }
 }
 hipError_t launch_chunk_transfer(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
-                                 const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots,
-                                 const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
-                                 double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl) {
-    return chunk_transfer_s<double>(s, kind, a, thetao, soa, npix, N, smp, sp, ns, knots, ktimes, nknots, times, nt, nus, nnu, L, kstop, seg, rec,
-                                    aflg, tl);
+                                 const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots, const SplatCf* spf,
+                                 const f32* knots_f, const f32* ktimes_f, const double* times, int nt, const double* nus, int nnu, double L,
+                                 const int* kstop, double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl) {
+    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg,
+                         spf, knots_f, ktimes_f};
+    return chunk_transfer_s<double>(s, kind, A, sp, knots, ktimes, seg, rec, tl);
 }
 hipError_t launch_chunk_transfer_f32(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                      const SplatCf* sp, int ns, const f32* knots, const f32* ktimes, int nknots,
                                      const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
-                                     double* seg, f32* rec, uint8_t* aflg, const TransferLaunch& tl) {
-    return chunk_transfer_s<f32>(s, kind, a, thetao, soa, npix, N, smp, sp, ns, knots, ktimes, nknots, times, nt, nus, nnu, L, kstop, seg, rec,
-                                 aflg, tl);
+                                     f32* seg, f32* rec, uint8_t* aflg, const TransferLaunch& tl) {
+    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg,
+                         sp, knots, ktimes};
+    return chunk_transfer_s<f32>(s, kind, A, sp, knots, ktimes, seg, rec, tl);
 }
 __global__ void ks_iota_i32(int* __restrict__ p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -409,9 +518,10 @@ hipError_t launch_thin_combine(hipStream_t s, int64_t npix, int nseg_max, const 
     return hipGetLastError();
 }
 hipError_t launch_seg_combine(hipStream_t s, const double* soa, int64_t npix, int N, int M, int chunk, int nt, const double* nus, int nnu,
-                              const double* seg, double* out) {
-    const int64_t items = npix * nt * nnu;
-    hipLaunchKernelGGL(ks_seg_combine, dim3(grid_for(items, 128)), dim3(128), 0, s, soa, npix, N, M, chunk, nt, nus, nnu, seg, out);
+                              const void* seg, int seg32, double* out) {
+    const dim3 grid(grid_for(npix * nt * nnu, 64)), block(64 * COMBINE_WAVES);
+    if (seg32) hipLaunchKernelGGL(ks_seg_combine<f32>, grid, block, 0, s, soa, npix, N, M, chunk, nt, nus, nnu, (const f32*)seg, out);
+    else hipLaunchKernelGGL(ks_seg_combine<double>, grid, block, 0, s, soa, npix, N, M, chunk, nt, nus, nnu, (const double*)seg, out);
     return hipGetLastError();
 }
 

@@ -20,6 +20,10 @@ namespace ksd {
 
 constexpr int PART_BLOCK = 256;    // block of the case partition
 constexpr int CHUNK = 32;          // samples per work item of the transfer from stored samples
+// A work item's samples are taken in slices by as many wavefronts, each with its own segment map: a quarter of the
+// work item (8 of 32 samples). The (sample, splat) pairs crowd into few items, and whole work items left most of the
+// chip idle behind the heaviest (0.3 to 1.6 wavefronts a SIMD in flight on average, up to 4 resident).
+__host__ __device__ inline int slice_length(int chunk) { return chunk < 8 ? 2 : chunk / 4; }
 constexpr int SEG_FIELDS = 20;     // a segment map: P (16, row-major), then Sv (4)
 // the populations an element-adjoint launch meets (a bit mask)
 constexpr int POP_THERMAL = 1, POP_POWERLAW = 2, POP_KNOTS = 4, POP_KAPPA = 8;
@@ -148,13 +152,33 @@ struct SegMapT {
             for (int q = 0; q < 4; ++q) P[4 * i + q] = acc[q];
         }
     }
-    KS_DEV void store(double* seg, int64_t m, int64_t nitems, int64_t item) const {
-        double* o = seg + SEG_FIELDS * m * nitems + item;
-        for (int q = 0; q < 16; ++q) o[q * nitems] = val(P[q]);
-        for (int q = 0; q < 4; ++q) o[(16 + q) * nitems] = val(Sv[q]);
+    KS_DEV void store(S* seg, int64_t m, int64_t nitems, int64_t item) const {
+        S* o = seg + SEG_FIELDS * m * nitems + item;
+        for (int q = 0; q < 16; ++q) o[q * nitems] = P[q];
+        for (int q = 0; q < 4; ++q) o[(16 + q) * nitems] = Sv[q];
     }
 };
 using SegMap = SegMapT<double>;
+
+// The composition of a ray's segment maps: wavefronts that share one ray's segments in the combine kernels.
+constexpr int COMBINE_WAVES = 4;
+template <class G>
+KS_DEV void seg_load(const G* __restrict__ seg, int64_t m, int64_t nitems, int64_t item, double P[16], double Sv[4]) {
+    const G* g = seg + (int64_t)SEG_FIELDS * m * nitems + item;
+    for (int q = 0; q < 16; ++q) P[q] = val(g[q * nitems]);
+    for (int q = 0; q < 4; ++q) Sv[q] = val(g[(16 + q) * nitems]);
+}
+// (P, S) <- (P Pm, S + P Sm): the segment (Pm, Sm) behind (P, S)
+KS_DEV void seg_append(double P[16], double Sv[4], const double Pm[16], const double Sm[4]) {
+    for (int i = 0; i < 4; ++i) Sv[i] += P[4 * i] * Sm[0] + P[4 * i + 1] * Sm[1] + P[4 * i + 2] * Sm[2] + P[4 * i + 3] * Sm[3];
+    double Pn[16];
+    for (int i = 0; i < 4; ++i)
+        for (int q = 0; q < 4; ++q) Pn[4 * i + q] = P[4 * i] * Pm[q] + P[4 * i + 1] * Pm[4 + q] + P[4 * i + 2] * Pm[8 + q] + P[4 * i + 3] * Pm[12 + q];
+    for (int i = 0; i < 16; ++i) P[i] = Pn[i];
+}
+// another lane's value (every lane takes part)
+KS_DEV double lane_value(double x, int lane) { return __shfl(x, lane, 64); }
+KS_DEV f32 lane_value(f32 x, int lane) { return f32(__shfl(x.v, lane, 64)); }
 
 // The half-orbit counter (WindingState, step.jl:362-398) over the valid samples outside the horizon
 // guard; kstop = the first sample beyond the nmax-th passage (N + 1 when there is none).
@@ -211,14 +235,16 @@ struct TransferLaunch {
 int64_t transfer_tasks(int64_t npix, int nt, int nnu, int N, int chunk);
 hipError_t launch_order_tasks(hipStream_t s, const uint32_t* cost, int64_t n, uint32_t* keys, int* ids, int* order, void* tmp, size_t& tmp_bytes);
 hipError_t launch_fill_i32(hipStream_t s, int* p, int64_t n, int v);
+// (spf, knots_f, ktimes_f: the FP32 copies, which the prefilter of both precisions reads; A.seg takes the maps in the
+// transfer's scalar)
 hipError_t launch_chunk_transfer(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
-                                 const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots,
-                                 const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
-                                 double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl);
+                                 const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots, const SplatCf* spf,
+                                 const f32* knots_f, const f32* ktimes_f, const double* times, int nt, const double* nus, int nnu, double L,
+                                 const int* kstop, double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl);
 hipError_t launch_chunk_transfer_f32(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                      const SplatCf* sp, int ns, const f32* knots, const f32* ktimes, int nknots,
                                      const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
-                                     double* seg, f32* rec, uint8_t* aflg, const TransferLaunch& tl);
+                                     f32* seg, f32* rec, uint8_t* aflg, const TransferLaunch& tl);
 hipError_t launch_seg_polarized(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, int M,
                                 const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots,
                                 const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
@@ -230,11 +256,11 @@ hipError_t launch_thin_parts(hipStream_t s, double a, double thetao, const doubl
                              const SplatC* sp, int ns, double t_obs, int nseg_max, double* part, double* res);
 hipError_t launch_thin_combine(hipStream_t s, int64_t npix, int nseg_max, const double* part, double* out);
 hipError_t launch_seg_combine(hipStream_t s, const double* soa, int64_t npix, int N, int M, int chunk, int nt, const double* nus, int nnu,
-                              const double* seg, double* out);
+                              const void* seg, int seg32, double* out);
 
 // ---- ks_k_adjoint.hip ----
-hipError_t launch_adj_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const double* seg,
-                              const double* dstokes, double* wT, double* out);
+hipError_t launch_adj_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const void* seg, int seg32,
+                              const double* dstokes, double* wT);
 hipError_t launch_adj_segment(hipStream_t s, int N, int chunk, int64_t nitems, const double* wT, const double* rec, double* bar,
                               const uint8_t* aflg, double* tails, Samples smp, int64_t npix);
 hipError_t launch_adj_segment_f32(hipStream_t s, int N, int chunk, int64_t nitems, const double* wT, const f32* rec, f32* bar,

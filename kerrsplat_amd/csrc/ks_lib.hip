@@ -141,7 +141,7 @@ struct ks_cache {
     Buf<double> bseed;                                 // binned χ²: the seed of every binned pixel
     Buf<int> ctri, cquad, coff, clegs;                 // closures: triangles, quadrangles, per-baseline term lists
     Buf<double> cdat, cterm;                           // closures: data and sigmas; per-term χ² and coefficients
-    double* seg = nullptr; int64_t seg_cap = 0;        // per-segment transfer maps
+    double* seg = nullptr; int64_t seg_cap = 0;        // per-segment transfer maps (FP32 ones on the mixed path), capacity in doubles
     double* dtn = nullptr; int64_t dtn_cap = 0;        // observation times then frequencies (device)
     std::vector<double> htn;                           // their host staging copy (outlives the async copy)
     double* segres = nullptr;                          // per-segment anchor residuals (2 x nseg_max x npix)
@@ -154,7 +154,7 @@ struct ks_cache {
     uint64_t fw_model = 0;                             // id of its model (0: no forward pass to reverse)
     int fw_nt = 0, fw_nnu = 0, fw_generation = -1, fw_precision = -1;
     std::vector<uint8_t> fw_seeded;                    // frames whose device seed a *_chi2_seed call wrote
-    int fw_chunk = CHUNK;                              // samples per chunk of its segment maps
+    int fw_chunk = 0;                                  // samples per slice of its segment maps
     std::vector<int> perm_host;
     // launch choices of the transfer over stored samples (ks_cache_tuning, ks_autotune): samples per work item,
     // the persistent work-queue form, the wavefront patch (patch_a x patch_b points of a screen part)
@@ -194,7 +194,7 @@ struct ks_model {
     // the same constants in FP32 (the mixed-precision transfer and adjoint)
     SplatCf* d_splats_f = nullptr; SplatAdjf* d_adj_f = nullptr; f32* d_knots_f = nullptr; f32* d_ktimes_f = nullptr;
     double gamma_max = 0.0;                            // of a single-population model: what its constants were made with
-    std::vector<double> h_knots;                       // and its knots (the per-splat constants bound the knot paths)
+    std::vector<double> h_knots, h_ktimes;             // and its knots (the per-splat constants bound the knot paths)
 };
 
 extern "C" {
@@ -487,14 +487,14 @@ int ks_model_create(ks_ctx* ctx, int kind, int nrows, int ns, const double* para
     std::vector<SplatC> h(ns > 0 ? ns : 1);
     std::vector<SplatAdj> ha(ns > 0 ? ns : 1);
     for (int i = 0; i < ns; ++i)
-        host_splat_constants(kind, nrows, i, params + (size_t)nrows * i, gamma_max, with_knots, knots, nknots, h[i], ha[i]);
+        host_splat_constants(kind, nrows, i, params + (size_t)nrows * i, gamma_max, with_knots, knots, knot_times, nknots, h[i], ha[i]);
     ks_model* m = new ks_model;
     m->id = next_model_id();
     m->ctx = ctx; m->kind = kind; m->nrows = nrows; m->ns = ns;
     m->hrows.assign((size_t)ns, nrows);
     m->pops = (kind == KS_MODEL_POWERLAW ? POP_POWERLAW : kind == KS_MODEL_KAPPA ? POP_KAPPA : POP_THERMAL) | (with_knots ? POP_KNOTS : 0);
     m->gamma_max = gamma_max;
-    if (with_knots) m->h_knots.assign(knots, knots + (size_t)3 * nknots * ns);
+    if (with_knots) { m->h_knots.assign(knots, knots + (size_t)3 * nknots * ns); m->h_ktimes.assign(knot_times, knot_times + nknots); }
     if (dalloc(&m->d_splats, h.size()) || dalloc(&m->d_adj, ha.size()) || dalloc(&m->d_splats_f, h.size()) || dalloc(&m->d_adj_f, ha.size())) {
         ks_model_destroy(m); return KS_ERR_HIP;
     }
@@ -631,8 +631,20 @@ static const double* stage_times(ks_cache* c, const double* times, int nt, const
     return c->dtn;
 }
 
-// Segment maps per item of the transfer: chunks of the stored samples or the pixel's anchor segments
-static int seg_count(const ks_cache* c, int chunk) { return std::max(max_segments(c->N), (c->N + chunk - 1) / chunk); }
+// Samples per slice of the transfer over stored samples, and whether its segment maps are FP32 (the mixed path's own
+// numbers, half the bytes of FP64 copies)
+static int slice_of(const ks_cache* c) { return slice_length(c->chunk); }
+static int seg_is32(const ks_cache* c) { return has_samples(c) && c->precision == KS_PRECISION_MIXED ? 1 : 0; }
+// room for the segment maps of `items` items: slices of the stored samples, or the pixel's anchor segments
+static int ensure_seg(ks_cache* c, int64_t items) {
+    const int64_t nseg = has_samples(c) ? (c->N + slice_of(c) - 1) / slice_of(c) : max_segments(c->N);
+    const int64_t need = ((int64_t)SEG_FIELDS * nseg * items * (seg_is32(c) ? 4 : 8) + 7) / 8;
+    if (c->seg_cap >= need) return KS_OK;
+    dfree(c->seg); c->seg_cap = 0;
+    if (dalloc(&c->seg, (size_t)need)) return KS_ERR_HIP;
+    c->seg_cap = need;
+    return KS_OK;
+}
 
 // The launch of the transfer over stored samples as the cache's tuning asks: one workgroup per task, or the
 // persistent work queue. The queue takes the tasks in the cost-descending order of an earlier launch of the same
@@ -641,9 +653,9 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, i
                            uint8_t* aflg, const TransferLaunch* sample) {
     ks_ctx* x = c->ctx;
     TransferLaunch tl;
-    tl.chunk = c->chunk;
+    tl.chunk = slice_of(c);
     tl.queue = (c->queue & KS_QUEUE_TRANSFER) ? 1 : 0;
-    const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, c->chunk);
+    const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c));
     bool order_after = false;
     if (sample) {
         tl.tasks = sample->tasks; tl.ntasks = sample->ntasks;
@@ -667,10 +679,11 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, i
     const int kind = m->kind;
     if (c->precision == KS_PRECISION_MIXED)
         HIPCHK(launch_chunk_transfer_f32(x->stream, kind, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats_f, m->ns,
-                                         m->d_knots_f, m->d_ktimes_f, m->nknots, d_tn, nt, d_tn + nt, nnu, L, kst, c->seg, (f32*)rec, aflg, tl));
+                                         m->d_knots_f, m->d_ktimes_f, m->nknots, d_tn, nt, d_tn + nt, nnu, L, kst, (f32*)c->seg, (f32*)rec, aflg, tl));
     else
         HIPCHK(launch_chunk_transfer(x->stream, kind, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->ns,
-                                     m->d_knots, m->d_ktimes, m->nknots, d_tn, nt, d_tn + nt, nnu, L, kst, c->seg, (double*)rec, aflg, tl));
+                                     m->d_knots, m->d_ktimes, m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_tn, nt, d_tn + nt, nnu, L, kst,
+                                     c->seg, (double*)rec, aflg, tl));
     if (order_after) {
         size_t bytes = 0;
         HIPCHK(launch_order_tasks(x->stream, c->qcost.p, ntasks, nullptr, nullptr, nullptr, nullptr, bytes));
@@ -690,12 +703,7 @@ static int launch_transfer(ks_cache* c, const ks_model* m, const double* d_tn, i
                            double* rec, uint8_t* aflg) {
     ks_ctx* x = c->ctx;
     const int64_t items = c->npix * nt * nnu;
-    const int nseg = seg_count(c, c->chunk);
-    if (c->seg_cap < (int64_t)SEG_FIELDS * nseg * items) {
-        dfree(c->seg);
-        if (dalloc(&c->seg, (size_t)SEG_FIELDS * nseg * items)) return KS_ERR_HIP;
-        c->seg_cap = (int64_t)SEG_FIELDS * nseg * items;
-    }
+    if (int rc = ensure_seg(c, items)) return rc;
     const int* kst = nullptr;
     if (nmax >= 0) {
         if (!c->kstop) { if (dalloc(&c->kstop, (size_t)c->npix)) return KS_ERR_HIP; }
@@ -733,7 +741,7 @@ int ks_render_device(ks_cache* c, const ks_model* m, const double* times, int nt
     int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, nullptr, nullptr);
     if (rc) return rc;
     const int64_t items = c->npix * frames;
-    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, has_samples(c) ? c->chunk : 0, nt, d_tn + nt, nnu, c->seg, c->out));
+    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, has_samples(c) ? slice_of(c) : 0, nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
     return KS_OK;
 }
 
@@ -850,13 +858,8 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                 if (chunks[ci] > std::max(c->N, 16)) continue;
                 c->chunk = chunks[ci];
                 if (records && ensure_adj(c, items, std::max(m->ns, 1))) return KS_ERR_HIP;
-                const int nseg = seg_count(c, c->chunk);
-                if (c->seg_cap < (int64_t)SEG_FIELDS * nseg * items) {
-                    dfree(c->seg);
-                    if (dalloc(&c->seg, (size_t)SEG_FIELDS * nseg * items)) return KS_ERR_HIP;
-                    c->seg_cap = (int64_t)SEG_FIELDS * nseg * items;
-                }
-                const int64_t all = transfer_tasks(c->npix, nt, nnu, c->N, c->chunk);
+                if (int rc = ensure_seg(c, items)) return rc;
+                const int64_t all = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c));
                 // a hashed Bernoulli sample of rate 1 / sample_every (a regular stride aliases with the screen: every k-th
                 // task can fall on one column of patches)
                 tasks.clear();
@@ -901,7 +904,7 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
         if (m->ns < 1) return fail(KS_ERR_ARG, "the element adjoints need splats");
         if (ensure_out(c, frames) || ensure_adj(c, items, m->ns)) return KS_ERR_HIP;
         if (int rc = launch_transfer(c, m, d_tn, nt, nnu, L, -1, 0.0, c->arec, c->aflg)) return rc;
-        c->fw_chunk = c->chunk;
+        c->fw_chunk = slice_of(c);
         HIPCHK(hipMemsetAsync(c->ads, 0, (size_t)4 * items * sizeof(double), x->stream));
         int best_q = c->queue;
         double best_ms = INFINITY;
@@ -949,7 +952,7 @@ static int64_t adj_unit_batch(int64_t nunits, int ns) {
 }
 
 static int ensure_adj(ks_cache* c, int64_t items, int ns) {
-    const int nseg = (c->N + c->chunk - 1) / c->chunk;
+    const int nseg = (c->N + slice_of(c) - 1) / slice_of(c);
     if (c->a_items < items) {
         dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->ads);
         c->a_items = 0;
@@ -991,7 +994,7 @@ static int reverse_launches(ks_cache* c, const ks_model* m, const double* d_tn, 
     ks_ctx* x = c->ctx;
     const int64_t items = c->npix * nt * nnu;
     const int ns = m->ns;
-    HIPCHK(launch_adj_combine(x->stream, c->npix, c->N, c->fw_chunk, nt, d_tn + nt, nnu, c->seg, c->ads, c->awT, nullptr));
+    HIPCHK(launch_adj_combine(x->stream, c->npix, c->N, c->fw_chunk, nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->ads, c->awT));
     HIPCHK(x->stage_begin(KS_STAGE_ADJ_STEPS));
     const bool mixed = c->precision == KS_PRECISION_MIXED;
     if (mixed) HIPCHK(launch_adj_segment_f32(x->stream, c->N, c->fw_chunk, items, c->awT, (const f32*)c->arec, (f32*)c->abar, c->aflg, (f32*)c->atail,
@@ -1048,9 +1051,9 @@ int ks_gradient_forward(ks_cache* c, const ks_model* m, const double* times, int
     if (!d_tn) return KS_ERR_HIP;
     int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, c->arec, c->aflg);
     if (rc) return rc;
-    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, c->chunk, nt, d_tn + nt, nnu, c->seg, c->out));
+    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, slice_of(c), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
     c->fw_model = m->id; c->fw_nt = nt; c->fw_nnu = nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
-    c->fw_chunk = c->chunk;
+    c->fw_chunk = slice_of(c);
     c->fw_seeded.assign((size_t)frames, 0);
     if (image) return ks_copy_stokes(c, frames, image, screen_order);
     return KS_OK;
@@ -1623,7 +1626,7 @@ static int graph_record(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpyAsync(m->d_adj_f, g->h_adf, ns * sizeof(SplatAdjf), hipMemcpyHostToDevice, s));
     const int nt = g->nt, nnu = g->nnu;
     if (int rc = launch_transfer(c, m, g->dtn.p, nt, nnu, g->L, -1, 0.0, c->arec, c->aflg)) return rc;
-    HIPCHK(launch_seg_combine(s, c->soa, c->npix, c->N, c->M, c->chunk, nt, g->dtn.p + nt, nnu, c->seg, c->out));
+    HIPCHK(launch_seg_combine(s, c->soa, c->npix, c->N, c->M, slice_of(c), nt, g->dtn.p + nt, nnu, c->seg, seg_is32(c), c->out));
     const int na = c->nalpha, nb = c->nbeta;
     for (int f = 0; f < g->frames; ++f) {
         if (g->loss == KS_LOSS_IMAGE) {
@@ -1672,7 +1675,7 @@ static int graph_capture(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpy(g->h_ad, m->d_adj, m->ns * sizeof(SplatAdj), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(g->h_spf, m->d_splats_f, m->ns * sizeof(SplatCf), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(g->h_adf, m->d_adj_f, m->ns * sizeof(SplatAdjf), hipMemcpyDeviceToHost));
-    c->fw_chunk = c->chunk;
+    c->fw_chunk = slice_of(c);
     if (int rc = graph_record(g, m)) return rc;
     HIPCHK(hipStreamSynchronize(x->stream));
     // the capture
@@ -1763,7 +1766,7 @@ int ks_fit_graph_step(ks_graph* g, const ks_model* m, const double* params, doub
         const bool with_knots = m->nknots >= 1 && !m->h_knots.empty();
         for (int i = 0; i < m->ns; ++i) {
             host_splat_constants(m->kind, m->nrows, i, params + (size_t)m->nrows * i, m->gamma_max, with_knots, with_knots ? m->h_knots.data() : nullptr,
-                                 m->nknots, g->h_sp[i], g->h_ad[i]);
+                                 with_knots ? m->h_ktimes.data() : nullptr, m->nknots, g->h_sp[i], g->h_ad[i]);
             splat_as(g->h_sp[i], g->h_spf[i]);
             adj_as(g->h_ad[i], g->h_adf[i]);
         }
@@ -1773,7 +1776,7 @@ int ks_fit_graph_step(ks_graph* g, const ks_model* m, const double* params, doub
     g->replays += 1;
     // the forward pass the graph ran is the cache's: images and seeds as after ks_gradient_forward + the seeds
     c->fw_model = m->id; c->fw_nt = g->nt; c->fw_nnu = g->nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
-    c->fw_chunk = c->chunk;
+    c->fw_chunk = slice_of(c);
     c->fw_seeded.assign((size_t)g->frames, 1);
     double s = 0.0;
     for (int f = 0; f < g->frames; ++f) s += g->h_chi[f];

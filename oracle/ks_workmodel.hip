@@ -113,7 +113,7 @@ extern "C" int kswm_count_slice(int kind, int nrows, int ns, const double* param
     std::vector<SplatC> h(ns);
     std::vector<SplatAdj> ha(ns);
     for (int i = 0; i < ns; ++i)
-        host_splat_constants(kind, nrows, i, params + (size_t)nrows * i, gamma_max, with_knots, knots, nknots, h[i], ha[i]);
+        host_splat_constants(kind, nrows, i, params + (size_t)nrows * i, gamma_max, with_knots, knots, knot_times, nknots, h[i], ha[i]);
     std::vector<SplatCT<Cnt>> sc(ns);
     std::vector<SplatAdjT<Cnt>> sa(ns);
     for (int i = 0; i < ns; ++i) { splat_as(h[i], sc[i]); adj_as(ha[i], sa[i]); }
