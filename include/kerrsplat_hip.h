@@ -97,10 +97,10 @@ int ks_cache_march_precision(ks_cache* cache, int precision);
 /* Launch choices of the transfer over stored samples and of the element adjoints. The reference fixes
  * them: one work item per pixel over all N samples, a workgroup of consecutive pixels (cache.jl:234-246
  * splits a screen into even tiles of consecutive pixels). Here: chunk = samples per work item of the
- * transfer (8:1024, default 32); queue = bits: KS_QUEUE_TRANSFER, the transfer as a persistent grid of
- * the resident workgroups taking tasks of 128 work items from a work queue (the tasks of a repeated
- * launch in descending order of the ticks each took the last time), else one workgroup per task;
- * KS_QUEUE_ADJOINT, the element adjoints as a persistent grid taking (unit, splat) blocks from per-XCD
+ * transfer (8:1024, default 32), which takes them in slices of a quarter, fewer where the launch is
+ * small; the transfer is a persistent grid of the resident workgroups taking tasks of 128 slices from a
+ * work queue; queue = bits: KS_QUEUE_TRANSFER, the tasks of a repeated launch in descending order of the
+ * ticks each took the last time, else in index order; KS_QUEUE_ADJOINT, the element adjoints as a persistent grid taking (unit, splat) blocks from per-XCD
  * queues, else one workgroup per block; patch_a x patch_b = the screen patch a wavefront's 64 work
  * items cover (default 8 x 8) within each screen part. The results do not depend on the patch or the
  * launch forms (bit for bit); the chunk length changes the order of the Stokes sums only. */
@@ -114,7 +114,7 @@ int ks_cache_get_tuning(const ks_cache* cache, int* chunk, int* queue, int* patc
  * one screen. The sum of the part sizes must be the cache's point count. */
 int ks_cache_set_parts(ks_cache* cache, int nparts, const int* n_alpha, const int* n_beta);
 /* The autotuner (no counterpart in the reference). Unless flags has KS_TUNE_KEEP_TRANSFER: times every launch
- * choice of the transfer (chunk 16, 32, 64, 128 x patch 8x8, 16x4, 4x16 x the two transfer launch forms) on
+ * choice of the transfer (chunk 16, 32, 64, 128 x patch 8x8, 16x4, 4x16 x the two orders of its queue) on
  * a hashed sample of 1 / sample_every of its tasks for (times, nus), with the dual sweep's records written
  * when flags has KS_TUNE_RECORDS, and keeps the fastest. With KS_TUNE_ADJOINT: one forward pass with the
  * records, then the reverse pass in each launch form of the element adjoints, and keeps the faster.

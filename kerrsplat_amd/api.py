@@ -425,7 +425,7 @@ def _set_parts(cache, camera):
 
 def tuning(cache, chunk=None, queue=None, patch=None, adjoint_queue=None):
     """The launch choices of the cache's transfer over stored samples and of its element adjoints: samples per work
-    item (chunk), the transfer's persistent work-queue form (queue), the element adjoints' persistent form
+    item (chunk), the cost order of the transfer's work queue (queue), the element adjoints' persistent form
     (adjoint_queue), the wavefront's screen patch (patch = (n_alpha, n_beta) points); arguments left at None keep
     their value. Returns the current choices as a dict."""
     lib = cache._lib

@@ -50,6 +50,10 @@ KS_DEV void wave_sync() {
 KS_DEV uint64_t uniform64(uint64_t x) {
     return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
 }
+// The slice of the q-th of n rows of tasks: the middle of the rays first, then outwards. A ray is nearest the hole around
+// its middle, where the splats crowd: in this order the tasks' costs fall (by five from the first sixteenth to the last),
+// and the queue's last ones are cheap.
+KS_DEV int slice_order(int q, int n) { return (q & 1) ? (n - 1) / 2 + (q + 1) / 2 : (n - 1) / 2 - q / 2; }
 // One wavefront: 64 items x one slice. Sample by sample, the lanes test their ray's sample against the candidate splats
 // (may_weigh) and queue the pairs that pass; whenever 64 are queued, or the candidates are through, the queued pairs'
 // weights, frames and coefficients run one pair a lane (splat_contribution), and each adds its 11 values to its
@@ -72,7 +76,7 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
     const int64_t slot = live ? tid : 0;
     const Samples& smp = A.smp;
     const int64_t item = slot_item(smp, slot % nitems, npix);     // wavefronts over compact patches of sky
-    const int m = (int)(slot / nitems);
+    const int m = slice_order((int)(slot / nitems), A.nch);
     const int64_t j = item % npix;
     const int64_t fr = item / npix;
     const int it = (int)(fr % A.nt), inu = (int)(fr / A.nt);
@@ -210,13 +214,13 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
     if (live) sm.store(seg, m, nitems, item);
 }
 
-// The launch forms share one kernel and one copy of the task body (so both give the same numbers bit for bit):
-//  * one workgroup per task (head == nullptr): workgroup b runs task q = b, or tasks[b] when a task list is given
-//    (the autotuner's sample of the work), ntasks = the grid;
-//  * the persistent work queue (head != nullptr): a grid sized to the resident workgroups, each taking the next
-//    ticket q from the queue head until ntasks are taken; task q is tasks[q] (a cost-descending order from an
-//    earlier launch's per-task times, or a sample of the work) or q itself (ntasks < 2^31).
-// With cost != nullptr the wall-clock ticks each task took go to cost[task] (zeroed by the launcher). The loop holds
+// The launch: a persistent grid of the resident workgroups, each taking the next ticket q from the queue head until
+// ntasks are taken; task q is tasks[q] when a task list is given (a cost-descending order from an earlier launch's
+// per-task times, or the autotuner's sample of the work), else q (ntasks < 2^31). With cost != nullptr the wall-clock
+// ticks each task took go to cost[task] (zeroed by the launcher). The tasks are heavy-tailed (1024 kappa splats, 256^2 x
+// 1024: median 0.6 ms, 99th percentile 31 ms), and dispatched one workgroup a task the hardware kept 1.7 of 4 wavefronts
+// a SIMD in flight: 340 ms, against 190 from the queue in index order and 166 in cost order (64 thermal splats,
+// 128^2 x 1024 x 4 frames: 21.2, 13.3, 12.7; FP64, 32 splats, 128^2 x 1024: 7.7, 5.8, 5.2). The loop holds
 // no lane-dependent branch outside the task: all 64 lanes of wavefront 0 execute the pop (lane 0 adds one, the others
 // zero), the first lane's ticket is shared through LDS, and every exit and back edge of the loop is a
 // wavefront-uniform (scalar) branch, so all lanes of the workgroup iterate together and each pass through the
@@ -229,21 +233,14 @@ ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __
     __shared__ WaveWork<S> s_w[2];
     __shared__ unsigned s_q;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
-    int64_t next = blockIdx.x;
     for (;;) {
-        int64_t q;
-        if (head) {
-            if (wave == 0) {
-                const unsigned ticket = atomicAdd(head, threadIdx.x == 0 ? 1u : 0u);
-                s_q = __builtin_amdgcn_readfirstlane(ticket);
-            }
-            __syncthreads();
-            q = (int64_t)__builtin_amdgcn_readfirstlane(s_q);
-            __syncthreads();             // every wavefront has read s_q before the next pop overwrites it
-        } else {
-            q = next;                    // one task, then the loop ends
-            next = ntasks;
+        if (wave == 0) {
+            const unsigned ticket = atomicAdd(head, threadIdx.x == 0 ? 1u : 0u);
+            s_q = __builtin_amdgcn_readfirstlane(ticket);
         }
+        __syncthreads();
+        const int64_t q = (int64_t)__builtin_amdgcn_readfirstlane(s_q);
+        __syncthreads();             // every wavefront has read s_q before the next pop overwrites it
         if (q >= ntasks) break;
         const int64_t task = tasks ? (int64_t)tasks[q] : q;
         const uint64_t t0 = cost ? wall_clock64() : 0;
@@ -420,11 +417,6 @@ static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const S
     const int64_t ntasks = tl.tasks ? tl.ntasks : all;
     if (ntasks <= 0) return hipSuccess;
     if (ntasks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
-    if (!tl.queue) {
-        hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)ntasks), dim3(128), 0, s, A, sp, knots, ktimes, seg, rec, tl.tasks,
-                           ntasks, (unsigned*)nullptr, (uint32_t*)nullptr);
-        return hipGetLastError();
-    }
     if (!tl.head) return hipErrorInvalidValue;
     static int groups = 0;       // per instantiation
     if (!groups) groups = resident_groups(ks_chunk_transfer<KIND, S, CULL>, 128);

@@ -23,7 +23,15 @@ constexpr int CHUNK = 32;          // samples per work item of the transfer from
 // A work item's samples are taken in slices by as many wavefronts, each with its own segment map: a quarter of the
 // work item (8 of 32 samples). The (sample, splat) pairs crowd into few items, and whole work items left most of the
 // chip idle behind the heaviest (0.3 to 1.6 wavefronts a SIMD in flight on average, up to 4 resident).
-__host__ __device__ inline int slice_length(int chunk) { return chunk < 8 ? 2 : chunk / 4; }
+// With few tasks (128 items x a slice each) the slices are halved, down to 2 samples: below SLICE_TASKS the last, dear
+// tasks leave the chip idle for longer than the further maps cost to compose (FP64 transfer of 1024 kappa splats,
+// 112 x 96 x 512: 131 ms with slices of 8, 5376 tasks; 111 of 4; 95 of 2).
+constexpr int64_t SLICE_TASKS = 8192;
+inline int slice_length(int chunk, int64_t nitems, int N) {
+    int len = chunk < 8 ? 2 : chunk / 4;
+    while (len >= 4 && (nitems * ((N + len - 1) / len) + 127) / 128 < SLICE_TASKS) len /= 2;
+    return len;
+}
 constexpr int SEG_FIELDS = 20;     // a segment map: P (16, row-major), then Sv (4)
 // the populations an element-adjoint launch meets (a bit mask)
 constexpr int POP_THERMAL = 1, POP_POWERLAW = 2, POP_KNOTS = 4, POP_KAPPA = 8;
@@ -221,16 +229,15 @@ hipError_t launch_unsort4(hipStream_t s, const double* src, const int* perm, int
 hipError_t launch_unsort1(hipStream_t s, const double* src, const int* perm, int64_t npix, double* dst);
 
 // ---- ks_k_transfer.hip ----
-// How the transfer from stored samples is launched: samples per work item (chunk), one workgroup per task or a
-// persistent grid over a work queue, and optionally a task list (the queue's order, or a sample of the work).
+// How the transfer from stored samples is launched: samples per slice (chunk), and optionally a task list (the cost
+// order, or a sample of the work).
 struct TransferLaunch {
     int chunk = CHUNK;
-    int queue = 0;                 // 1: persistent workgroups taking tasks from a queue
     const int* tasks = nullptr;    // tasks to run, in this order (null: every task, in index order)
     int64_t ntasks = 0;            // the list's length
     int* head = nullptr;           // the queue head (one int of device memory; zeroed by the launch)
-    uint32_t* cost = nullptr;      // queue form: per-task wall-clock ticks, indexed by task (null: not recorded)
-    int group_scale = 1;           // queue form: persistent workgroups = resident workgroups x group_scale
+    uint32_t* cost = nullptr;      // per-task wall-clock ticks, indexed by task (null: not recorded)
+    int group_scale = 1;           // persistent workgroups = resident workgroups x group_scale
 };
 int64_t transfer_tasks(int64_t npix, int nt, int nnu, int N, int chunk);
 hipError_t launch_order_tasks(hipStream_t s, const uint32_t* cost, int64_t n, uint32_t* keys, int* ids, int* order, void* tmp, size_t& tmp_bytes);

@@ -157,7 +157,7 @@ struct ks_cache {
     int fw_chunk = 0;                                  // samples per slice of its segment maps
     std::vector<int> perm_host;
     // launch choices of the transfer over stored samples (ks_cache_tuning, ks_autotune): samples per work item,
-    // the persistent work-queue form, the wavefront patch (patch_a x patch_b points of a screen part)
+    // the work queue's order, the wavefront patch (patch_a x patch_b points of a screen part)
     int chunk = CHUNK, queue = 0, patch_a = 8, patch_b = 8;
     // screen parts of the point list (ks_cache_set_parts): consecutive runs of points, each an n_alpha x n_beta
     // screen in screen order; empty: the whole camera is one nalpha x nbeta screen
@@ -633,11 +633,11 @@ static const double* stage_times(ks_cache* c, const double* times, int nt, const
 
 // Samples per slice of the transfer over stored samples, and whether its segment maps are FP32 (the mixed path's own
 // numbers, half the bytes of FP64 copies)
-static int slice_of(const ks_cache* c) { return slice_length(c->chunk); }
+static int slice_of(const ks_cache* c, int64_t items) { return slice_length(c->chunk, items, c->N); }
 static int seg_is32(const ks_cache* c) { return has_samples(c) && c->precision == KS_PRECISION_MIXED ? 1 : 0; }
 // room for the segment maps of `items` items: slices of the stored samples, or the pixel's anchor segments
 static int ensure_seg(ks_cache* c, int64_t items) {
-    const int64_t nseg = has_samples(c) ? (c->N + slice_of(c) - 1) / slice_of(c) : max_segments(c->N);
+    const int64_t nseg = has_samples(c) ? (c->N + slice_of(c, items) - 1) / slice_of(c, items) : max_segments(c->N);
     const int64_t need = ((int64_t)SEG_FIELDS * nseg * items * (seg_is32(c) ? 4 : 8) + 7) / 8;
     if (c->seg_cap >= need) return KS_OK;
     dfree(c->seg); c->seg_cap = 0;
@@ -646,23 +646,22 @@ static int ensure_seg(ks_cache* c, int64_t items) {
     return KS_OK;
 }
 
-// The launch of the transfer over stored samples as the cache's tuning asks: one workgroup per task, or the
-// persistent work queue. The queue takes the tasks in the cost-descending order of an earlier launch of the same
-// shape when there is one, records every task's ticks, and orders the tasks by them for the next launch.
+// The launch of the transfer over stored samples as the cache's tuning asks: the work queue in index order, or
+// (KS_QUEUE_TRANSFER) in the cost-descending order of an earlier launch of the same shape when there is one, recording
+// every task's ticks and ordering the tasks by them for the next launch.
 static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, int nt, int nnu, double L, const int* kst, void* rec,
                            uint8_t* aflg, const TransferLaunch* sample) {
     ks_ctx* x = c->ctx;
     TransferLaunch tl;
-    tl.chunk = slice_of(c);
-    tl.queue = (c->queue & KS_QUEUE_TRANSFER) ? 1 : 0;
-    const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c));
+    tl.chunk = slice_of(c, c->npix * nt * nnu);
+    if (c->qhead.grow(1)) return KS_ERR_HIP;
+    tl.head = c->qhead.p;
+    const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c, c->npix * nt * nnu));
     bool order_after = false;
     if (sample) {
         tl.tasks = sample->tasks; tl.ntasks = sample->ntasks;
     }
-    if (tl.queue) {
-        if (c->qhead.grow(1)) return KS_ERR_HIP;
-        tl.head = c->qhead.p;
+    if (c->queue & KS_QUEUE_TRANSFER) {
         if (!sample && x->capturing) {
             // a captured launch takes the order the last eager launch of this shape left, and records nothing
             const int64_t shape[6] = {ntasks, c->chunk, (int64_t)m->id, c->precision, rec ? 1 : 0, (int64_t)nt * 65536 + nnu};
@@ -741,7 +740,7 @@ int ks_render_device(ks_cache* c, const ks_model* m, const double* times, int nt
     int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, nullptr, nullptr);
     if (rc) return rc;
     const int64_t items = c->npix * frames;
-    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, has_samples(c) ? slice_of(c) : 0, nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
+    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, has_samples(c) ? slice_of(c, items) : 0, nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
     return KS_OK;
 }
 
@@ -859,7 +858,7 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                 c->chunk = chunks[ci];
                 if (records && ensure_adj(c, items, std::max(m->ns, 1))) return KS_ERR_HIP;
                 if (int rc = ensure_seg(c, items)) return rc;
-                const int64_t all = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c));
+                const int64_t all = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c, c->npix * nt * nnu));
                 // a hashed Bernoulli sample of rate 1 / sample_every (a regular stride aliases with the screen: every k-th
                 // task can fall on one column of patches)
                 tasks.clear();
@@ -904,7 +903,7 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
         if (m->ns < 1) return fail(KS_ERR_ARG, "the element adjoints need splats");
         if (ensure_out(c, frames) || ensure_adj(c, items, m->ns)) return KS_ERR_HIP;
         if (int rc = launch_transfer(c, m, d_tn, nt, nnu, L, -1, 0.0, c->arec, c->aflg)) return rc;
-        c->fw_chunk = slice_of(c);
+        c->fw_chunk = slice_of(c, items);
         HIPCHK(hipMemsetAsync(c->ads, 0, (size_t)4 * items * sizeof(double), x->stream));
         int best_q = c->queue;
         double best_ms = INFINITY;
@@ -952,7 +951,7 @@ static int64_t adj_unit_batch(int64_t nunits, int ns) {
 }
 
 static int ensure_adj(ks_cache* c, int64_t items, int ns) {
-    const int nseg = (c->N + slice_of(c) - 1) / slice_of(c);
+    const int nseg = (c->N + slice_of(c, items) - 1) / slice_of(c, items);
     if (c->a_items < items) {
         dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->ads);
         c->a_items = 0;
@@ -1051,9 +1050,9 @@ int ks_gradient_forward(ks_cache* c, const ks_model* m, const double* times, int
     if (!d_tn) return KS_ERR_HIP;
     int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, c->arec, c->aflg);
     if (rc) return rc;
-    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, slice_of(c), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
+    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, slice_of(c, items), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
     c->fw_model = m->id; c->fw_nt = nt; c->fw_nnu = nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
-    c->fw_chunk = slice_of(c);
+    c->fw_chunk = slice_of(c, items);
     c->fw_seeded.assign((size_t)frames, 0);
     if (image) return ks_copy_stokes(c, frames, image, screen_order);
     return KS_OK;
@@ -1626,7 +1625,7 @@ static int graph_record(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpyAsync(m->d_adj_f, g->h_adf, ns * sizeof(SplatAdjf), hipMemcpyHostToDevice, s));
     const int nt = g->nt, nnu = g->nnu;
     if (int rc = launch_transfer(c, m, g->dtn.p, nt, nnu, g->L, -1, 0.0, c->arec, c->aflg)) return rc;
-    HIPCHK(launch_seg_combine(s, c->soa, c->npix, c->N, c->M, slice_of(c), nt, g->dtn.p + nt, nnu, c->seg, seg_is32(c), c->out));
+    HIPCHK(launch_seg_combine(s, c->soa, c->npix, c->N, c->M, slice_of(c, c->npix * g->frames), nt, g->dtn.p + nt, nnu, c->seg, seg_is32(c), c->out));
     const int na = c->nalpha, nb = c->nbeta;
     for (int f = 0; f < g->frames; ++f) {
         if (g->loss == KS_LOSS_IMAGE) {
@@ -1675,7 +1674,7 @@ static int graph_capture(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpy(g->h_ad, m->d_adj, m->ns * sizeof(SplatAdj), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(g->h_spf, m->d_splats_f, m->ns * sizeof(SplatCf), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(g->h_adf, m->d_adj_f, m->ns * sizeof(SplatAdjf), hipMemcpyDeviceToHost));
-    c->fw_chunk = slice_of(c);
+    c->fw_chunk = slice_of(c, items);
     if (int rc = graph_record(g, m)) return rc;
     HIPCHK(hipStreamSynchronize(x->stream));
     // the capture
@@ -1776,7 +1775,7 @@ int ks_fit_graph_step(ks_graph* g, const ks_model* m, const double* params, doub
     g->replays += 1;
     // the forward pass the graph ran is the cache's: images and seeds as after ks_gradient_forward + the seeds
     c->fw_model = m->id; c->fw_nt = g->nt; c->fw_nnu = g->nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
-    c->fw_chunk = slice_of(c);
+    c->fw_chunk = slice_of(c, c->npix * g->frames);
     c->fw_seeded.assign((size_t)g->frames, 1);
     double s = 0.0;
     for (int f = 0; f < g->frames; ++f) s += g->h_chi[f];
