@@ -100,8 +100,9 @@ int ks_cache_march_precision(ks_cache* cache, int precision);
  * transfer (8:1024, default 32), which takes them in slices of a quarter, fewer where the launch is
  * small; the transfer is a persistent grid of the resident workgroups taking tasks of 128 slices from a
  * work queue; queue = bits: KS_QUEUE_TRANSFER, the tasks of a repeated launch in descending order of the
- * ticks each took the last time, else in index order; KS_QUEUE_ADJOINT, the element adjoints as a persistent grid taking (unit, splat) blocks from per-XCD
- * queues, else one workgroup per block; patch_a x patch_b = the screen patch a wavefront's 64 work
+ * ticks each took the last time, else in index order; KS_QUEUE_ADJOINT is kept for
+ * callers that set it (the element adjoints take their work list from per-XCD queues either way);
+ * patch_a x patch_b = the screen patch a wavefront's 64 work
  * items cover (default 8 x 8) within each screen part. The results do not depend on the patch or the
  * launch forms (bit for bit); the chunk length changes the order of the Stokes sums only. */
 #define KS_QUEUE_TRANSFER 1

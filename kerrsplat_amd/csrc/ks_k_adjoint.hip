@@ -3,6 +3,7 @@
 // per-sample adjoints inside each chunk, the per-splat element adjoints with a wavefront sum, and a
 // deterministic reduction over the item blocks.
 #include "ks_kernels.hpp"
+#include "ks_dsample.hpp"
 
 namespace ksd {
 
@@ -188,16 +189,24 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(Waves<
     }
 }
 
-// The region of each element-adjoint unit (64 items x ADJ_SLICE samples): the bounding sphere of its
-// step-taking samples and their emission times, ub[UB_FIELDS unit + f] (wave_region); one wavefront per unit.
-__global__ void __launch_bounds__(64) ks_unit_bounds(int64_t npix, int N, Samples smp, const double* __restrict__ times, int nt,
-                                                     int64_t nitems, const uint8_t* __restrict__ aflg, double* __restrict__ ub) {
-    const int64_t unit = blockIdx.x;
+// The work list of the element adjoints: a unit is 64 items x ADJ_SLICE samples, a block one (unit, splat) whose splat
+// can reach a step-taking sample of the unit (the bounding sphere of those samples and their emission times,
+// splat_may_reach). One wavefront per unit writes a bit per splat and their count; one workgroup gives every unit the
+// list position of its first block; one wavefront per unit then writes the list, and each mask word's position. The
+// units of a batch are listed XCD by XCD (unit u on XCD u % 8), so that all blocks of a unit run beside one L2, which
+// reads the unit's samples once. Blocks that are culled cost nothing further: before, each was a workgroup that
+// stored 22 zeros for the reduction to read (four in five of the 24 million of 1024 kappa splats at 256^2 x 1024).
+__global__ void __launch_bounds__(64) ks_unit_mask(int64_t npix, int N, Samples smp, const double* __restrict__ times, int nt,
+                                                   int64_t nitems, const uint8_t* __restrict__ aflg, const SplatC* __restrict__ sp, int ns,
+                                                   const double* __restrict__ knots, const double* __restrict__ ktimes, int64_t unit0,
+                                                   uint64_t* __restrict__ mask, int* __restrict__ count) {
+    const int64_t unit = unit0 + blockIdx.x;
     const int nslice = (N + ADJ_SLICE - 1) / ADJ_SLICE;
     const int64_t ib = unit / nslice;
     const int kfirst = (int)(unit % nslice) * ADJ_SLICE + 1;
     const int klast = kfirst + ADJ_SLICE - 1 < N ? kfirst + ADJ_SLICE - 1 : N;
-    const int64_t item = ib * 64 + threadIdx.x;
+    const int lane = (int)threadIdx.x;
+    const int64_t item = ib * 64 + lane;
     double lo[4] = {INFINITY, INFINITY, INFINITY, INFINITY}, hi[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     if (item < nitems) {
         const int64_t j = item % npix;
@@ -211,61 +220,98 @@ __global__ void __launch_bounds__(64) ks_unit_bounds(int64_t npix, int N, Sample
     }
     double px = 0.0, py = 0.0, pz = 0.0, R = 0.0, tmin = 0.0, tmax = 0.0;
     const bool any = wave_region(lo, hi, px, py, pz, R, tmin, tmax);
-    if (threadIdx.x == 0) {
-        double* o = ub + UB_FIELDS * unit;
-        o[0] = px; o[1] = py; o[2] = pz; o[3] = R; o[4] = tmin; o[5] = tmax; o[6] = any ? 1.0 : 0.0; o[7] = 0.0;
+    const int nw = (ns + 63) / 64;
+    int n = 0;
+    for (int b = 0; b < nw; ++b) {
+        const int i = 64 * b + lane;
+        const uint64_t m = __ballot(any && i < ns && splat_may_reach(sp[i], px, py, pz, R, tmin, tmax, knots, ktimes));
+        if (lane == 0) mask[(int64_t)blockIdx.x * nw + b] = m;
+        n += __popcll(m);
+    }
+    if (lane == 0) count[blockIdx.x] = n;
+}
+// the unit at position p of the list's order: XCD p / per, its units in ascending order (per = ceil(nb / 8); >= nb: none)
+KS_DEV int64_t listed_unit(int64_t p, int64_t per) { return (p % per) * 8 + p / per; }
+constexpr int LIST_THREADS = 1024;
+// first[u]: the list position of unit u's first block; xcd[0..8]: the ranges of the XCDs. Each thread sums a run of the
+// order, the runs' sums are scanned in LDS, and each thread then walks its run again.
+__global__ void __launch_bounds__(LIST_THREADS) ks_unit_first(int64_t nb, const int* __restrict__ count, int* __restrict__ first, int* __restrict__ xcd) {
+    __shared__ int s_sum[LIST_THREADS];
+    const int64_t per = (nb + 7) / 8, all = 8 * per, run = (all + LIST_THREADS - 1) / LIST_THREADS;
+    const int t = (int)threadIdx.x;
+    const int64_t p0 = t * run, p1 = p0 + run < all ? p0 + run : all;
+    int n = 0;
+    for (int64_t p = p0; p < p1; ++p) {
+        const int64_t u = listed_unit(p, per);
+        if (u < nb) n += count[u];
+    }
+    s_sum[t] = n;
+    __syncthreads();
+    for (int d = 1; d < LIST_THREADS; d *= 2) {
+        const int v = t >= d ? s_sum[t - d] : 0;
+        __syncthreads();
+        s_sum[t] += v;
+        __syncthreads();
+    }
+    int pos = s_sum[t] - n;
+    for (int64_t p = p0; p < p1; ++p) {
+        const int64_t u = listed_unit(p, per);
+        if (p % per == 0) xcd[p / per] = pos;
+        if (u < nb) { first[u] = pos; pos += count[u]; }
+    }
+    if (t == LIST_THREADS - 1) xcd[8] = s_sum[t];
+}
+// list[e] = (unit of the batch, splat); at[u nw + b] = the position of the first block of mask word b
+__global__ void __launch_bounds__(64) ks_unit_list(int ns, const uint64_t* __restrict__ mask, const int* __restrict__ first, int2* __restrict__ list,
+                                                   int* __restrict__ at) {
+    const int64_t u = blockIdx.x;
+    const int nw = (ns + 63) / 64, lane = (int)threadIdx.x;
+    int pos = first[u];
+    for (int b = 0; b < nw; ++b) {
+        const uint64_t m = mask[u * nw + b];
+        if (lane == 0) at[u * nw + b] = pos;
+        if ((m >> lane) & 1) list[pos + __popcll(m & ((1ull << lane) - 1))] = make_int2((int)u, 64 * b + lane);
+        pos += __popcll(m);
     }
 }
 
-// Per (64 consecutive items, slice of ADJ_SLICE samples, splat): the element adjoints of every
-// (item, sample) pair inside the splat's weight cutoff, 21 partial sums per lane, summed over the
-// wavefront; part[(u ns + i) 21 + r] for the unit u = ib nslice + slice. The slices bound the work of
+// Per block of the list (64 consecutive items, slice of ADJ_SLICE samples, splat): the element adjoints of every
+// (item, sample) pair inside the splat's weight cutoff, 22 partial sums per lane, summed over the
+// wavefront into part[22 e + r] for the block's list position e. The slices bound the work of
 // one wavefront: the pairs of a splat crowd into a few item blocks and stretches of the rays, and
 // whole-ray units left most of the chip idle behind the heaviest ones.
-// The wavefront first walks its items' samples with the cheap weight test, WALK samples at a time with
-// their loads issued together, and queues the pairs that pass (ballot + mbcnt into an LDS ring), then
-// runs the element adjoint 64 pairs at a time, so that lanes outside the splat's support do not idle
-// through it. Every pair of a wavefront belongs to
+// The wavefront walks its items' samples with the FP32 prefilter (may_weigh), WALK samples at a time with
+// their loads issued together, and queues the pairs that pass (ballot + mbcnt into an LDS ring); whenever 64 are queued,
+// or the samples are through, it runs the element adjoint of up to 64 pairs, so that lanes outside the splat's support
+// do not idle through it (one call site for both: a second inlined copy doubled the kernel's 60 KB of code).
+// MI355X, element adjoints of one pass, before and after (list, one call site, prefilter): FP64, 32 thermal splats at
+// 128^2 x 1024 9.4 -> 6.9 ms, 48 power-law splats 8.0 -> 6.0, 1024 kappa splats (112 x 96 x 512) 237 -> 167; mixed, 1024
+// kappa splats (256^2 x 1024) 583 -> 451, 64 thermal splats (4 frames of 128^2 x 1024) 22.7 -> 19.3.
+// Every pair of a wavefront belongs to
 // splat i, so the sums stay per lane in registers; the queue order is fixed, so the result is
 // deterministic.
 // POPS: the populations the launch meets, POP_THERMAL (thermal and knot splats), POP_POWERLAW, POP_KAPPA, and
 // POP_KNOTS (centres that follow knots); a launch of one population carries only its branch, whose registers would
 // otherwise cost it occupancy; mixed populations take a runtime branch on the splat's kind.
+// block-wide copy of a per-splat constant struct into LDS
+template <class T> KS_DEV void copy_to_lds(T* dst, const T* __restrict__ src, int lane) {
+    static_assert(sizeof(T) % 4 == 0, "copied in dwords");
+    for (int q = lane; q < (int)(sizeof(T) / 4); q += 64) ((int*)dst)[q] = ((const int*)src)[q];
+}
 template <class S, int POPS>
-__device__ __forceinline__ void adj_splats_block(int64_t blk, double a, double thetao, const double* __restrict__ soa, int64_t npix, int N,
+__device__ __forceinline__ void adj_splats_block(int64_t e, int64_t unit, int i, double a, double thetao, const double* __restrict__ soa, int64_t npix, int N,
                                                  Samples smp, const SplatCT<S>* __restrict__ sp, const SplatAdjT<S>* __restrict__ sadj,
-                                                 int ns, const S* __restrict__ knots, const S* __restrict__ ktimes,
+                                                 const SplatCf* __restrict__ spf, const f32* __restrict__ knots_f, const f32* __restrict__ ktimes_f,
+                                                 const S* __restrict__ knots, const S* __restrict__ ktimes,
                                                  const double* __restrict__ times, int nt, const double* __restrict__ nus, int64_t nitems,
                                                  const S* __restrict__ rec, const S* __restrict__ bar, const uint8_t* __restrict__ aflg,
-                                                 int64_t unit0, int64_t nb, const double* __restrict__ ub, double* __restrict__ part) {
+                                                 double* __restrict__ part) {
     constexpr int WALK = 8;                 // samples tested per group, their loads issued together
     constexpr int QCAP = 1024;              // ring capacity: < 64 pending + 64 per sample of a group
     static_assert(QCAP >= 64 * (WALK + 1) && (QCAP & (QCAP - 1)) == 0, "the ring must hold a group's pushes");
     __shared__ double s_alpha[64], s_beta[64], s_tobs[64], s_nu[64];
     __shared__ int64_t s_item[64];
     __shared__ int s_q[QCAP];   // entry = lane | k << 6
-    // XCD-aware order: the hardware deals consecutive blocks round-robin over the 8 XCDs, so block b runs on
-    // XCD b % 8; all ns splats of a unit go to one XCD (and its L2, which then reads the unit's samples once)
-    // this launch covers the units unit0 .. unit0 + nb - 1 (a batch: the partial sums of a batch are bounded by
-    // nb x ns x ADJ_ROWS doubles); `local` numbers the unit within the batch
-    int i;
-    int64_t unit, local;
-    {
-        const int64_t b = blk, q = b / 8, x = b % 8;
-        i = (int)(q % ns);
-        local = (q / ns) * 8 + x;
-        if (local >= nb) return;          // the padding of the last group of 8 units
-        unit = unit0 + local;
-    }
-    // the per-unit cull: a splat that cannot reach any step-taking sample of the unit adds zeros
-    {
-        const double* u = ub + UB_FIELDS * unit;
-        if (!(u[6] > 0.0) || !splat_may_reach(sp[i], u[0], u[1], u[2], u[3], u[4], u[5], knots, ktimes)) {
-            // every lane stores (lanes past the rows repeat the last row's zero): no lane-dependent branch
-            part[(local * ns + i) * ADJ_ROWS + min((int)threadIdx.x, ADJ_ROWS - 1)] = 0.0;
-            return;
-        }
-    }
     const int nslice = (N + ADJ_SLICE - 1) / ADJ_SLICE;
     const int64_t ib = unit / nslice;
     const int kfirst = (int)(unit % nslice) * ADJ_SLICE + 1;
@@ -277,7 +323,10 @@ __device__ __forceinline__ void adj_splats_block(int64_t blk, double a, double t
     // they outgrow the scalar file and spill into vector lanes
     __shared__ SplatCT<S> s_c;
     __shared__ SplatAdjT<S> s_sa;
-    if (lane == 0) { s_c = sp[i]; s_sa = sadj[i]; }
+    __syncthreads();                          // the last block's reads are done
+    copy_to_lds(&s_c, sp + i, lane);
+    copy_to_lds(&s_sa, sadj + i, lane);
+    const SplatCf& cf = spf[i];
     const SplatCT<S>& c = s_c;
     const SplatAdjT<S>& sa = s_sa;
     int64_t j = 0;
@@ -343,49 +392,43 @@ __device__ __forceinline__ void adj_splats_block(int64_t blk, double a, double t
         qhead = (qhead + cnt) & (QCAP - 1);
         qn -= cnt;
     };
-    for (int k0 = kfirst; k0 <= klast; k0 += WALK) {
-        uint8_t fl[WALK];
-        S tk[WALK], xk[WALK], yk[WALK], zk[WALK];     // t_obs - t~ and the position of each sample of the group
+    int k0 = kfirst;
+    for (;;) {
+        while (qn < 64 && k0 <= klast) {
+            uint8_t fl[WALK];
+            float tk[WALK], xk[WALK], yk[WALK], zk[WALK];     // t_obs - t~ and the position of each sample of the group
 #pragma unroll
-        for (int u = 0; u < WALK; ++u) {
-            const int k = k0 + u;
-            fl[u] = 0;
-            tk[u] = xk[u] = yk[u] = zk[u] = S(0.0);
-            if (valid && k <= klast) {
-                const int64_t so = (int64_t)(k - 1) * npix + j;
-                fl[u] = aflg[(int64_t)(k - 1) * nitems + item];
-                if constexpr (use_p4) {
-                    const float4 q = smp.p4[so];
-                    tk[u] = S((float)t_obs - q.w); xk[u] = S(q.x); yk[u] = S(q.y); zk[u] = S(q.z);
-                } else {
-                    tk[u] = S(t_obs - smp.t[so]); xk[u] = S(smp.x[so]); yk[u] = S(smp.y[so]); zk[u] = S(smp.z[so]);
+            for (int u = 0; u < WALK; ++u) {
+                const int k = k0 + u;
+                fl[u] = 0;
+                tk[u] = xk[u] = yk[u] = zk[u] = 0.0f;
+                if (valid && k <= klast) {
+                    const int64_t so = (int64_t)(k - 1) * npix + j;
+                    fl[u] = aflg[(int64_t)(k - 1) * nitems + item];
+                    if constexpr (use_p4) {
+                        const float4 q = smp.p4[so];
+                        tk[u] = (float)t_obs - q.w; xk[u] = q.x; yk[u] = q.y; zk[u] = q.z;
+                    } else {
+                        tk[u] = (float)(t_obs - smp.t[so]); xk[u] = (float)smp.x[so]; yk[u] = (float)smp.y[so]; zk[u] = (float)smp.z[so];
+                    }
                 }
             }
-        }
 #pragma unroll
-        for (int u = 0; u < WALK; ++u) {
-            bool act;
-            if constexpr ((POPS & POP_KNOTS) != 0)
-                act = fl[u] && (c.nk > 0 ? weight_active_knot(c, knots, ktimes, tk[u], xk[u], yk[u], zk[u])
-                                         : weight_active(c, tk[u], xk[u], yk[u], zk[u]));
-            else
-                act = fl[u] && weight_active(c, tk[u], xk[u], yk[u], zk[u]);
-            const uint64_t m = __ballot(act);
-            if (act) {
-                const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                s_q[(qhead + qn + rank) & (QCAP - 1)] = lane | ((k0 + u) << 6);
+            for (int u = 0; u < WALK; ++u) {
+                const bool act = fl[u] && may_weigh<MODEL_THERMAL>(cf, knots_f, ktimes_f, tk[u], xk[u], yk[u], zk[u]);
+                const uint64_t m = __ballot(act);
+                if (act) {
+                    const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    s_q[(qhead + qn + rank) & (QCAP - 1)] = lane | ((k0 + u) << 6);
+                }
+                qn += __popcll(m);
             }
-            qn += __popcll(m);
+            k0 += WALK;
         }
-        while (qn >= 64) {
-            __syncthreads();
-            run_batch(64);
-            __syncthreads();
-        }
-    }
-    if (qn > 0) {
+        if (qn == 0) break;
         __syncthreads();
-        run_batch(qn);
+        run_batch(qn < 64 ? qn : 64);
+        __syncthreads();
     }
     // wavefront sum (blockDim = 64 = one wavefront), in FP64
     double gsum[ADJ_ROWS];
@@ -397,51 +440,72 @@ __device__ __forceinline__ void adj_splats_block(int64_t blk, double a, double t
     // lane r < ADJ_ROWS stores row r (the lanes past the rows repeat the last row): selects, no lane-dependent branch
     double mine = gsum[ADJ_ROWS - 1];
     for (int r = 0; r < ADJ_ROWS - 1; ++r) mine = lane == r ? gsum[r] : mine;
-    part[(local * ns + i) * ADJ_ROWS + min(lane, ADJ_ROWS - 1)] = mine;
+    part[e * ADJ_ROWS + min(lane, ADJ_ROWS - 1)] = mine;
 }
 
-// The launch forms of the element adjoints: one workgroup (one wavefront) per block b of the XCD-aware numbering
-// (heads == nullptr), or a persistent grid of the resident workgroups (a multiple of 8, so workgroup w runs on XCD
-// w % 8) in which each workgroup takes tickets t from its XCD's queue heads[w % 8] and runs block b = 8 t + w % 8
-// until the blocks (nblocks) are taken: the blocks of a unit stay on one XCD as in the one-per-block form, and the
-// units whose splat is culled cost a ticket instead of a dispatch. The ticket is taken by all 64 lanes (lane 0 adds
-// one) and made scalar, so the loop's exit and back edge are uniform branches.
+// The launch: a persistent grid of the resident workgroups (a multiple of 8, so workgroup w runs on XCD w % 8), each
+// taking tickets from its XCD's queue heads[w % 8] over the XCD's range of the list, and from the other XCDs' once that
+// is through. The ticket is taken by all 64 lanes (lane 0 adds one) and made scalar, so the loop's exit and back edge
+// are uniform branches.
 template <class S, int POPS>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Waves<S>::adjelem)))
 ks_adj_splats(double a, double thetao, const double* __restrict__ soa, int64_t npix, int N, Samples smp, const SplatCT<S>* __restrict__ sp,
-              const SplatAdjT<S>* __restrict__ sadj, int ns, const S* __restrict__ knots, const S* __restrict__ ktimes,
+              const SplatAdjT<S>* __restrict__ sadj, const SplatCf* __restrict__ spf, const f32* __restrict__ knots_f,
+              const f32* __restrict__ ktimes_f, const S* __restrict__ knots, const S* __restrict__ ktimes,
               const double* __restrict__ times, int nt, const double* __restrict__ nus, int64_t nitems, const S* __restrict__ rec,
-              const S* __restrict__ bar, const uint8_t* __restrict__ aflg, int64_t unit0, int64_t nb, const double* __restrict__ ub,
-              double* __restrict__ part, int64_t nblocks, unsigned* __restrict__ heads) {
-    const int x = (int)(blockIdx.x % 8);
-    int64_t next = blockIdx.x;
+              const S* __restrict__ bar, const uint8_t* __restrict__ aflg, int64_t unit0, const int2* __restrict__ list,
+              const int* __restrict__ xcd, double* __restrict__ part, unsigned* __restrict__ heads) {
+    int x = (int)(blockIdx.x % 8), tried = 0;
     for (;;) {
-        int64_t blk;
-        if (heads) {
-            const unsigned t = __builtin_amdgcn_readfirstlane(atomicAdd(heads + x, threadIdx.x == 0 ? 1u : 0u));
-            blk = 8 * (int64_t)t + x;
+        const unsigned t = __builtin_amdgcn_readfirstlane(atomicAdd(heads + x, threadIdx.x == 0 ? 1u : 0u));
+        const int64_t e = (int64_t)xcd[x] + t;
+        if (e < xcd[x + 1]) {
+            const int2 b = list[e];
+            adj_splats_block<S, POPS>(e, unit0 + __builtin_amdgcn_readfirstlane(b.x), __builtin_amdgcn_readfirstlane(b.y), a, thetao, soa, npix, N, smp,
+                                      sp, sadj, spf, knots_f, ktimes_f, knots, ktimes, times, nt, nus, nitems, rec, bar, aflg, part);
         } else {
-            blk = next;
-            next = nblocks;
+            x = (x + 1) & 7;
+            ++tried;
         }
-        if (blk >= nblocks) break;
-        adj_splats_block<S, POPS>(blk, a, thetao, soa, npix, N, smp, sp, sadj, ns, knots, ktimes, times, nt, nus, nitems, rec, bar, aflg,
-                                  unit0, nb, ub, part);
+        if (tried == 8) break;
     }
 }
 
-// dparams[r + ADJ_ROWS i] = the sum over a batch's work units in a fixed order (deterministic): one wavefront per
-// (splat, row), lane l summing units l, l + 64, ..., then a fixed butterfly over the lanes; added to the sums of
-// the earlier batches when accumulate (the batches in order)
-__global__ void __launch_bounds__(64) ks_adj_reduce(const double* __restrict__ part, int64_t nunits, int ns, int accumulate,
-                                                    double* __restrict__ dparams) {
-    const int64_t t = blockIdx.x;
-    if (t >= (int64_t)ns * ADJ_ROWS) return;
-    const int i = (int)(t / ADJ_ROWS), r = (int)(t % ADJ_ROWS);
-    double s = 0.0;
-    for (int64_t b = threadIdx.x; b < nunits; b += 64) s += part[(b * ns + i) * ADJ_ROWS + r];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (threadIdx.x == 0) dparams[t] = accumulate ? dparams[t] + s : s;
+// dparams[r + ADJ_ROWS i] = the sum over a batch's blocks of splat i in a fixed order (deterministic): REDUCE_PARTS
+// workgroups a splat, each over a run of the units, lane l of its four wavefronts taking the run's units l, l + 256, ...
+// that hold a block of the splat; a fixed butterfly over the lanes, the wavefronts in order, then (ks_adj_reduce_parts)
+// the runs in order, added to the sums of the earlier batches when accumulate (the batches in order)
+constexpr int REDUCE_PARTS = 16;
+__global__ void __launch_bounds__(256) ks_adj_reduce(const double* __restrict__ part, int64_t nunits, int ns, const uint64_t* __restrict__ mask,
+                                                     const int* __restrict__ at, double* __restrict__ sums) {
+    const int i = (int)(blockIdx.x / REDUCE_PARTS), y = (int)(blockIdx.x % REDUCE_PARTS);
+    const int nw = (ns + 63) / 64, w = i / 64, bit = i % 64;
+    const int64_t per = (nunits + REDUCE_PARTS - 1) / REDUCE_PARTS;
+    const int64_t u1 = (y + 1) * per < nunits ? (y + 1) * per : nunits;
+    double s[ADJ_ROWS];
+    for (int r = 0; r < ADJ_ROWS; ++r) s[r] = 0.0;
+    for (int64_t u = y * per + threadIdx.x; u < u1; u += 256) {
+        const uint64_t m = mask[u * nw + w];
+        if (!((m >> bit) & 1)) continue;
+        const double* p = part + (int64_t)(at[u * nw + w] + __popcll(m & ((1ull << bit) - 1))) * ADJ_ROWS;
+        for (int r = 0; r < ADJ_ROWS; ++r) s[r] += p[r];
+    }
+    __shared__ double s_w[4][ADJ_ROWS];
+    for (int r = 0; r < ADJ_ROWS; ++r) {
+        double v = s[r];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        if (threadIdx.x % 64 == 0) s_w[threadIdx.x / 64][r] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < ADJ_ROWS) sums[(int64_t)blockIdx.x * ADJ_ROWS + threadIdx.x] = s_w[0][threadIdx.x] + s_w[1][threadIdx.x] + s_w[2][threadIdx.x] + s_w[3][threadIdx.x];
+}
+__global__ void ks_adj_reduce_parts(const double* __restrict__ sums, int ns, int accumulate, double* __restrict__ dparams) {
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t >= ns * ADJ_ROWS) return;
+    const int i = t / ADJ_ROWS, r = t % ADJ_ROWS;
+    double v = 0.0;
+    for (int y = 0; y < REDUCE_PARTS; ++y) v += sums[((int64_t)i * REDUCE_PARTS + y) * ADJ_ROWS + r];
+    dparams[t] = accumulate ? dparams[t] + v : v;
 }
 
 // ---- launchers ----
@@ -467,34 +531,18 @@ hipError_t launch_adj_segment_f32(hipStream_t s, int N, int chunk, int64_t nitem
     return hipGetLastError();
 }
 template <class S>
-static hipError_t adj_splats_k(hipStream_t s, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
-                               const SplatCT<S>* sp, const SplatAdjT<S>* sadj, int ns, const S* knots, const S* ktimes,
-                               const double* times, int nt, const double* nus, int64_t nitems, const S* rec, const S* bar,
-                               const uint8_t* aflg, int64_t unit0, int64_t nb, const double* ub, double* part, int* heads) {
-    const int64_t nblocks = (nb + 7) / 8 * 8 * ns;
-    dim3 grid((unsigned)nblocks), block(64);
-    unsigned* hq = nullptr;
-    if (heads) {
-        // the persistent grid: the resident workgroups of the launch's instantiation, a multiple of 8
-        int groups = 0;
-#define KS_ADJ_GROUPS(P) groups = resident_groups(ks_adj_splats<S, P>, 64)
-        switch (pops) {
-            case POP_THERMAL: KS_ADJ_GROUPS(POP_THERMAL); break;
-            case POP_THERMAL | POP_KNOTS: KS_ADJ_GROUPS(POP_THERMAL | POP_KNOTS); break;
-            case POP_POWERLAW: KS_ADJ_GROUPS(POP_POWERLAW); break;
-            case POP_POWERLAW | POP_KNOTS: KS_ADJ_GROUPS(POP_POWERLAW | POP_KNOTS); break;
-            case POP_KAPPA: KS_ADJ_GROUPS(POP_KAPPA); break;
-            case POP_KAPPA | POP_KNOTS: KS_ADJ_GROUPS(POP_KAPPA | POP_KNOTS); break;
-            default: KS_ADJ_GROUPS(POP_FLUIDS | POP_KNOTS); break;
-        }
-#undef KS_ADJ_GROUPS
-        if (groups < 8) return hipErrorInvalidValue;
-        grid = dim3((unsigned)std::min<int64_t>(groups / 8 * 8, nblocks));
-        if (hipError_t e = launch_fill_i32(s, heads, 8, 0)) return e;
-        hq = (unsigned*)heads;
-    }
-#define KS_ADJ_LAUNCH(P) hipLaunchKernelGGL((ks_adj_splats<S, P>), grid, block, 0, s, a, thetao, soa, npix, N, smp, sp, sadj, ns, knots, ktimes, \
-                                            times, nt, nus, nitems, rec, bar, aflg, unit0, nb, ub, part, nblocks, hq)
+static hipError_t adj_splats_k(hipStream_t s, const AdjWork& w, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
+                               const SplatCT<S>* sp, const SplatAdjT<S>* sadj, const SplatCf* spf, const f32* knots_f, const f32* ktimes_f,
+                               const S* knots, const S* ktimes, const double* times, int nt, const double* nus, int64_t nitems, const S* rec,
+                               const S* bar, const uint8_t* aflg, int64_t unit0, int64_t nb, int ns) {
+    if (hipError_t e = launch_fill_i32(s, w.heads, 8, 0)) return e;
+    // the resident workgroups of the launch's instantiation, a multiple of 8
+#define KS_ADJ_LAUNCH(P) do { static int groups = 0; \
+        if (!groups) groups = resident_groups(ks_adj_splats<S, P>, 64) / 8 * 8; \
+        if (groups < 8) return hipErrorInvalidValue; \
+        hipLaunchKernelGGL((ks_adj_splats<S, P>), dim3((unsigned)std::min<int64_t>(groups, (nb * ns + 7) / 8 * 8)), dim3(64), 0, s, a, thetao, soa, npix, N, \
+                           smp, sp, sadj, spf, knots_f, ktimes_f, knots, ktimes, times, nt, nus, nitems, rec, bar, aflg, unit0, (const int2*)w.list, w.xcd, \
+                           w.part, (unsigned*)w.heads); } while (0)
     switch (pops) {
         case POP_THERMAL: KS_ADJ_LAUNCH(POP_THERMAL); break;
         case POP_THERMAL | POP_KNOTS: KS_ADJ_LAUNCH(POP_THERMAL | POP_KNOTS); break;
@@ -507,29 +555,33 @@ static hipError_t adj_splats_k(hipStream_t s, int pops, double a, double thetao,
 #undef KS_ADJ_LAUNCH
     return hipGetLastError();
 }
-hipError_t launch_adj_splats(hipStream_t s, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
-                             const SplatC* sp, const SplatAdj* sadj, int ns, const double* knots, const double* ktimes,
-                             const double* times, int nt, const double* nus, int64_t nitems, const double* rec, const double* bar,
-                             const uint8_t* aflg, int64_t unit0, int64_t nb, const double* ub, double* part, int* heads) {
-    return adj_splats_k<double>(s, pops, a, thetao, soa, npix, N, smp, sp, sadj, ns, knots, ktimes, times, nt, nus, nitems, rec, bar, aflg, unit0,
-                                nb, ub, part, heads);
+hipError_t launch_adj_splats(hipStream_t s, const AdjWork& w, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
+                             const SplatC* sp, const SplatAdj* sadj, const SplatCf* spf, const f32* knots_f, const f32* ktimes_f, int ns,
+                             const double* knots, const double* ktimes, const double* times, int nt, const double* nus, int64_t nitems,
+                             const double* rec, const double* bar, const uint8_t* aflg, int64_t unit0, int64_t nb) {
+    return adj_splats_k<double>(s, w, pops, a, thetao, soa, npix, N, smp, sp, sadj, spf, knots_f, ktimes_f, knots, ktimes, times, nt, nus, nitems, rec,
+                                bar, aflg, unit0, nb, ns);
 }
-hipError_t launch_adj_splats_f32(hipStream_t s, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
+hipError_t launch_adj_splats_f32(hipStream_t s, const AdjWork& w, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                  const SplatCf* sp, const SplatAdjf* sadj, int ns, const f32* knots, const f32* ktimes,
                                  const double* times, int nt, const double* nus, int64_t nitems, const f32* rec, const f32* bar,
-                                 const uint8_t* aflg, int64_t unit0, int64_t nb, const double* ub, double* part, int* heads) {
+                                 const uint8_t* aflg, int64_t unit0, int64_t nb) {
     if (!smp.p4) return hipErrorInvalidValue;          // the FP32 element adjoints read the samples' FP32 copy
-    return adj_splats_k<f32>(s, pops, a, thetao, soa, npix, N, smp, sp, sadj, ns, knots, ktimes, times, nt, nus, nitems, rec, bar, aflg, unit0, nb,
-                             ub, part, heads);
+    return adj_splats_k<f32>(s, w, pops, a, thetao, soa, npix, N, smp, sp, sadj, sp, knots, ktimes, knots, ktimes, times, nt, nus, nitems, rec, bar,
+                             aflg, unit0, nb, ns);
 }
-hipError_t launch_unit_bounds(hipStream_t s, int64_t npix, int N, Samples smp, const double* times, int nt, int64_t nitems,
-                              const uint8_t* aflg, double* ub) {
-    hipLaunchKernelGGL(ks_unit_bounds, dim3((unsigned)adj_units(nitems, N)), dim3(64), 0, s, npix, N, smp, times, nt, nitems, aflg, ub);
+hipError_t launch_adj_list(hipStream_t s, const AdjWork& w, int64_t npix, int N, Samples smp, const double* times, int nt, int64_t nitems,
+                           const uint8_t* aflg, const SplatC* sp, int ns, const double* knots, const double* ktimes, int64_t unit0, int64_t nb) {
+    hipLaunchKernelGGL(ks_unit_mask, dim3((unsigned)nb), dim3(64), 0, s, npix, N, smp, times, nt, nitems, aflg, sp, ns, knots, ktimes, unit0, w.mask, w.count);
+    hipLaunchKernelGGL(ks_unit_first, dim3(1), dim3(LIST_THREADS), 0, s, nb, w.count, w.first, w.xcd);
+    hipLaunchKernelGGL(ks_unit_list, dim3((unsigned)nb), dim3(64), 0, s, ns, w.mask, w.first, (int2*)w.list, w.at);
     return hipGetLastError();
 }
-hipError_t launch_adj_reduce(hipStream_t s, const double* part, int64_t nunits, int ns, int accumulate, double* dparams) {
-    hipLaunchKernelGGL(ks_adj_reduce, dim3((unsigned)(ns * ADJ_ROWS)), dim3(64), 0, s, part, nunits, ns, accumulate, dparams);
+hipError_t launch_adj_reduce(hipStream_t s, const AdjWork& w, int64_t nunits, int ns, int accumulate, double* dparams) {
+    hipLaunchKernelGGL(ks_adj_reduce, dim3((unsigned)(ns * REDUCE_PARTS)), dim3(256), 0, s, w.part, nunits, ns, w.mask, w.at, w.sums);
+    hipLaunchKernelGGL(ks_adj_reduce_parts, dim3(grid_for((int64_t)ns * ADJ_ROWS, 256)), dim3(256), 0, s, w.sums, ns, accumulate, dparams);
     return hipGetLastError();
 }
+int adj_reduce_parts() { return REDUCE_PARTS; }
 
 }  // namespace ksd

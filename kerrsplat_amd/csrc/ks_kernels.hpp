@@ -40,7 +40,6 @@ constexpr int ADJ_ROWS = 22;       // gradient rows per splat (21 thermal and kn
 constexpr int ADJ_SLICE = 32;      // samples per work unit of the element adjoints
 constexpr int CAND_MAX = 1024;     // splats a tile's candidate list holds (more splats: no per-tile cull)
 constexpr int CULL_MIN_NS = 64;    // the transfer culls per tile from this many splats on (below, the per-sample test is cheaper)
-constexpr int UB_FIELDS = 8;       // a unit's region: centre (3), radius, emission times [min, max], any sample, pad
 // the minimum and maximum over a wavefront (butterfly: every lane ends with the wavefront's value)
 KS_DEV double wave_min(double v) { for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64)); return v; }
 KS_DEV double wave_max(double v) { for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64)); return v; }
@@ -272,17 +271,25 @@ hipError_t launch_adj_segment(hipStream_t s, int N, int chunk, int64_t nitems, c
                               const uint8_t* aflg, double* tails, Samples smp, int64_t npix);
 hipError_t launch_adj_segment_f32(hipStream_t s, int N, int chunk, int64_t nitems, const double* wT, const f32* rec, f32* bar,
                                   const uint8_t* aflg, f32* tails, Samples smp, int64_t npix);
-hipError_t launch_adj_splats_f32(hipStream_t s, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
+// The element adjoints' work list and sums of one batch of nb units and ns splats (nw = ceil(ns / 64)): a bit per (unit,
+// splat) (nb nw), blocks per unit (nb), list positions of the units (nb) and mask words (nb nw), the list (int2 each, up
+// to nb ns), the XCDs' ranges (9), their queue heads (8), the blocks' partial sums (22 each), the reduction's runs.
+struct AdjWork {
+    uint64_t* mask; int *count, *first, *at; void* list; int *xcd, *heads; double *part, *sums;
+};
+hipError_t launch_adj_list(hipStream_t s, const AdjWork& w, int64_t npix, int N, Samples smp, const double* times, int nt, int64_t nitems,
+                           const uint8_t* aflg, const SplatC* sp, int ns, const double* knots, const double* ktimes, int64_t unit0, int64_t nb);
+// (spf, knots_f, ktimes_f: the FP32 copies, which the prefilter of both precisions reads)
+hipError_t launch_adj_splats_f32(hipStream_t s, const AdjWork& w, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                  const SplatCf* sp, const SplatAdjf* sadj, int ns, const f32* knots, const f32* ktimes,
                                  const double* times, int nt, const double* nus, int64_t nitems, const f32* rec, const f32* bar,
-                                 const uint8_t* aflg, int64_t unit0, int64_t nb, const double* ub, double* part, int* heads);
-hipError_t launch_adj_splats(hipStream_t s, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
-                             const SplatC* sp, const SplatAdj* sadj, int ns, const double* knots, const double* ktimes,
-                             const double* times, int nt, const double* nus, int64_t nitems, const double* rec, const double* bar,
-                             const uint8_t* aflg, int64_t unit0, int64_t nb, const double* ub, double* part, int* heads);
-hipError_t launch_adj_reduce(hipStream_t s, const double* part, int64_t nunits, int ns, int accumulate, double* dparams);
-hipError_t launch_unit_bounds(hipStream_t s, int64_t npix, int N, Samples smp, const double* times, int nt, int64_t nitems,
-                              const uint8_t* aflg, double* ub);
+                                 const uint8_t* aflg, int64_t unit0, int64_t nb);
+hipError_t launch_adj_splats(hipStream_t s, const AdjWork& w, int pops, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
+                             const SplatC* sp, const SplatAdj* sadj, const SplatCf* spf, const f32* knots_f, const f32* ktimes_f, int ns,
+                             const double* knots, const double* ktimes, const double* times, int nt, const double* nus, int64_t nitems,
+                             const double* rec, const double* bar, const uint8_t* aflg, int64_t unit0, int64_t nb);
+hipError_t launch_adj_reduce(hipStream_t s, const AdjWork& w, int64_t nunits, int ns, int accumulate, double* dparams);
+int adj_reduce_parts();
 
 // ---- ks_k_vis.hip ----
 hipError_t launch_vis_tables(hipStream_t s, int nuv, int na, int nb, double psize, const double* u, const double* v, double* A2, double* B2);

@@ -148,8 +148,10 @@ struct ks_cache {
     int* kstop = nullptr;                              // half-orbit cutoff per pixel
     // adjoint workspace (grow-only): records, flags, tails, per-segment (w_in, T_out), seeds, partial sums
     double* arec = nullptr; double* abar = nullptr; uint8_t* aflg = nullptr; double* atail = nullptr; double* awT = nullptr; double* ads = nullptr;
-    double* apart = nullptr; double* adpar = nullptr; double* aub = nullptr;
-    int64_t a_items = 0, a_part = 0, a_dpar = 0, a_ub = 0, a_wT = 0;
+    double* apart = nullptr; double* adpar = nullptr;
+    int64_t a_items = 0, a_part = 0, a_dpar = 0, a_wT = 0;
+    Buf<uint64_t> amask; Buf<int> acount, afirst, aat, alist, axcd;      // the element adjoints' work list (AdjWork)
+    Buf<double> asums;
     // the last forward pass of the dual sweep (ks_gradient_forward): what ks_gradient_reverse needs
     uint64_t fw_model = 0;                             // id of its model (0: no forward pass to reverse)
     int fw_nt = 0, fw_nnu = 0, fw_generation = -1, fw_precision = -1;
@@ -307,7 +309,8 @@ int ks_cache_destroy(ks_cache* c) {
     c->imask.release();
     c->ctri.release(); c->cquad.release(); c->coff.release(); c->clegs.release(); c->cdat.release(); c->cterm.release();
     dfree(c->seg); dfree(c->segres); dfree(c->kstop); dfree(c->dtn);
-    dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->awT); dfree(c->ads); dfree(c->apart); dfree(c->adpar); dfree(c->aub);
+    dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->awT); dfree(c->ads); dfree(c->apart); dfree(c->adpar);
+    c->amask.release(); c->acount.release(); c->afirst.release(); c->aat.release(); c->alist.release(); c->axcd.release(); c->asums.release();
     c->qhead.release(); c->qorder.release(); c->qids.release(); c->aheads.release(); c->qcost.release(); c->qkeys.release(); c->qtmp.release();
     delete c;
     return KS_OK;
@@ -974,11 +977,10 @@ static int ensure_adj(ks_cache* c, int64_t items, int ns) {
         if (dalloc(&c->apart, (size_t)nb * ns * ADJ_ROWS)) return KS_ERR_HIP;
         c->a_part = nb * ns * ADJ_ROWS;
     }
-    if (c->a_ub < nunits) {
-        dfree(c->aub);
-        if (dalloc(&c->aub, (size_t)nunits * UB_FIELDS)) return KS_ERR_HIP;
-        c->a_ub = nunits;
-    }
+    const size_t nw = (size_t)(ns + 63) / 64;
+    if (c->amask.grow(nb * nw) || c->acount.grow(nb) || c->afirst.grow(nb) || c->aat.grow(nb * nw) || c->alist.grow((size_t)2 * nb * ns) ||
+        c->axcd.grow(9) || c->aheads.grow(8) || c->asums.grow((size_t)ns * adj_reduce_parts() * ADJ_ROWS))
+        return KS_ERR_HIP;
     if (c->a_dpar < (int64_t)ns * ADJ_ROWS) {
         dfree(c->adpar);
         if (dalloc(&c->adpar, (size_t)ns * ADJ_ROWS)) return KS_ERR_HIP;
@@ -1004,25 +1006,21 @@ static int reverse_launches(ks_cache* c, const ks_model* m, const double* d_tn, 
         if (mixed)
             if (int rc = ensure_p4(c)) return rc;
         HIPCHK(x->stage_begin(KS_STAGE_ADJ_ELEMENTS));
-        HIPCHK(launch_unit_bounds(x->stream, c->npix, c->N, samples_of(c), d_tn, nt, items, c->aflg, c->aub));
-        // the persistent form of the element adjoints with the cache's work-queue choice: per-XCD queue heads
-        int* heads = nullptr;
-        if (c->queue & KS_QUEUE_ADJOINT) {
-            if (c->aheads.grow(8)) return KS_ERR_HIP;
-            heads = c->aheads.p;
-        }
+        const AdjWork w{c->amask.p, c->acount.p, c->afirst.p, c->aat.p, c->alist.p, c->axcd.p, c->aheads.p, c->apart, c->asums.p};
         // the units in batches whose partial sums fit the workspace, each reduced into the running sums in order
         const int64_t nunits = adj_units(items, c->N), nbmax = adj_unit_batch(nunits, ns);
         for (int64_t u0 = 0; u0 < nunits; u0 += nbmax) {
             const int64_t nb = std::min(nbmax, nunits - u0);
+            HIPCHK(launch_adj_list(x->stream, w, c->npix, c->N, samples_of(c), d_tn, nt, items, c->aflg, m->d_splats, ns, m->d_knots, m->d_ktimes, u0, nb));
             if (mixed)
-                HIPCHK(launch_adj_splats_f32(x->stream, m->pops, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats_f, m->d_adj_f, ns,
+                HIPCHK(launch_adj_splats_f32(x->stream, w, m->pops, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats_f, m->d_adj_f, ns,
                                              m->d_knots_f, m->d_ktimes_f, d_tn, nt, d_tn + nt, items, (const f32*)c->arec, (const f32*)c->abar, c->aflg,
-                                             u0, nb, c->aub, c->apart, heads));
+                                             u0, nb));
             else
-                HIPCHK(launch_adj_splats(x->stream, m->pops, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->d_adj, ns, m->d_knots,
-                                         m->d_ktimes, d_tn, nt, d_tn + nt, items, c->arec, c->abar, c->aflg, u0, nb, c->aub, c->apart, heads));
-            HIPCHK(launch_adj_reduce(x->stream, c->apart, nb, ns, u0 > 0, c->adpar));
+                HIPCHK(launch_adj_splats(x->stream, w, m->pops, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->d_adj,
+                                         m->d_splats_f, m->d_knots_f, m->d_ktimes_f, ns, m->d_knots, m->d_ktimes, d_tn, nt, d_tn + nt, items, c->arec,
+                                         c->abar, c->aflg, u0, nb));
+            HIPCHK(launch_adj_reduce(x->stream, w, nb, ns, u0 > 0, c->adpar));
         }
         HIPCHK(x->stage_end(KS_STAGE_ADJ_ELEMENTS));
     }
@@ -1609,8 +1607,8 @@ static void graph_release_host(ks_graph* g) {
 
 // the cache buffers a captured iteration reads or writes
 static std::vector<const void*> graph_ptrs(const ks_cache* c) {
-    return {c->seg, c->out, c->arec, c->abar, c->aflg, c->atail, c->awT, c->ads, c->apart, c->adpar, c->aub, c->tmap, c->soa,
-            c->qhead.p, c->qorder.p, c->kstop, c->aheads.p, c->sp4};
+    return {c->seg, c->out, c->arec, c->abar, c->aflg, c->atail, c->awT, c->ads, c->apart, c->adpar, c->tmap, c->soa,
+            c->qhead.p, c->qorder.p, c->kstop, c->aheads.p, c->sp4, c->amask.p, c->acount.p, c->afirst.p, c->aat.p, c->alist.p, c->axcd.p, c->asums.p};
 }
 
 // the iteration's launches on the (capturing) stream
