@@ -95,9 +95,8 @@ KS_DEV bool splat_contribution(const SplatCT<S>& sc, const GeoT<S>& G, S aS, S a
 }
 
 // The splat sum of one sample (accumulate_elements, transport.jl:254-276): invariant j, alpha, rho in
-// screen axes; false when no splat contributes. One instantiation per population and scalar. One sample at a time, for
-// the march fused with the transport; the transfer over stored samples packs the pairs of a wavefront's samples
-// instead (transfer_task). With a candidate list only those splats are visited.
+// screen axes; false when no splat contributes. One sample at a time, for the work model; the transfer packs the pairs of
+// a wavefront's samples instead (transfer_task). With a candidate list only those splats are visited.
 template <int KIND, class S>
 KS_DEV bool sample_coefficients(const TransCtxT<S>& c, double st, double r, double th, bool nur, bool nuth, S x, S y, S z,
                                 S j4[4], S a4[4], S r3[3], const uint16_t* cand = nullptr, int ncand = 0) {
@@ -154,23 +153,14 @@ KS_DEV bool may_weigh(const SplatCf& c, const f32* __restrict__ knots, const f32
     return !(g > 27.641f + 2.0f * d * (5.3f + d));
 }
 
-// thin splats (Splats.jl:113-128): sum_i j_i g^2 Sigma dtau with the ZAMO redshift g
-KS_DEV double thin_sample(const SplatC* __restrict__ sp, int ns, double a, double lam, double t_obs, double st, double r, double th,
-                          double x, double y, double z, double dtau) {
-    const double t = t_obs - st;
-    double jt = 0.0;
-    for (int i = 0; i < ns; ++i) {
-        const SplatC& c = sp[i];
-        double sph, cph; sincos(c.omega * (t - c.t0), &sph, &cph);
-        jt += exp(c.lnA - 0.5 * gauss_exponent(c, t, x, y, z, sph, cph));
-    }
+// g^2 Sigma dtau of a thin sample, g the ZAMO redshift (Splats.jl:113-128)
+KS_DEV double thin_weight(double a, double lam, double r, double th, double dtau) {
     double s_, c_; sincos(th, &s_, &c_);
     double S_ = r * r + a * a * c_ * c_, Dl = r * r - 2.0 * r + a * a;
     double Xi = (r * r + a * a) * (r * r + a * a) - a * a * Dl * s_ * s_;
     double g = sqrt(Dl * S_ / Xi) / (1.0 - 2.0 * a * r / Xi * lam);
-    return g * g * jt * S_ * dtau;
+    return g * g * S_ * dtau;
 }
-
 
 // The FP64 step of an FP32 sample, out of line (the rare samples with a Faraday depth |rho| Delta above
 // FARADAY_FP64, where the step's polynomial in K' cancels strongly): O and E in FP64, rounded to FP32. The

@@ -84,6 +84,26 @@ KS_DEV void quasi_cartesian_ks(Q a, Q rp, Q rm, Q r, Q th, Q ph, Q& x, Q& y, Q& 
     x = r * st * cp; y = r * st * sp; z = r * ct;
 }
 
+// sine and cosine of a pattern phase: the phase less its nearest multiple of pi / 2 (two fused steps, exact to 1e-16 up to
+// 1e5 rad; the library beyond), then the Taylor series of both on |r| <= pi / 4, whose first dropped terms are below
+// 1e-19. About 35 instructions against the library's 100, whose large-argument reduction is inlined at every call.
+KS_COLD void sincos_large(double x, double* s, double* c) { ::sincos(x, s, c); }
+KS_DEV void phase_sincos(double x, double* s, double* c) {
+    if (!(::fabs(x) < 1e5)) { sincos_large(x, s, c); return; }
+    const double n = ::rint(x * 0.6366197723675814);
+    const double r = ::fma(-n, 6.123233995736766e-17, ::fma(-n, 1.5707963267948966, x));
+    const double q = r * r;
+    double ps = -1.0 / 6.0 + q * (1.0 / 120.0 + q * (-1.0 / 5040.0 + q * (1.0 / 362880.0 + q * (-1.0 / 39916800.0 +
+                q * (1.0 / 6227020800.0 + q * (-1.0 / 1307674368000.0 + q * (1.0 / 355687428096000.0)))))));
+    double pc = -0.5 + q * (1.0 / 24.0 + q * (-1.0 / 720.0 + q * (1.0 / 40320.0 + q * (-1.0 / 3628800.0 + q * (1.0 / 479001600.0 +
+                q * (-1.0 / 87178291200.0 + q * (1.0 / 20922789888000.0 + q * (-1.0 / 6402373705728000.0))))))));
+    const double sr = ::fma(r * q, ps, r), cr = ::fma(q, pc, 1.0);
+    const int m = (int)n;
+    const double sv = (m & 1) ? cr : sr, cv = (m & 1) ? sr : cr;
+    *s = (m & 2) ? -sv : sv;
+    *c = ((m + 1) & 2) ? -cv : cv;
+}
+
 // centre of a splat at time t under the pattern rotation and the squared distance (for the cull)
 template <class S>
 KS_DEV bool outside_support(const SplatCT<S>& s, S t, S x, S y, S z, S& sp, S& cp) {

@@ -132,26 +132,47 @@ __global__ void ks_res_reduce(int64_t npix, int nseg_max, const double* __restri
     rt[j] = r1; rp[j] = r2;
 }
 
-// from the march (fused caches) or from the stored samples (smp.r != nullptr)
-__global__ void __launch_bounds__(128) ks_wind_cutoff(double a, double thetao, const double* __restrict__ soa, int64_t npix, int N, int M,
-                                                      int nmax, double slab, Samples smp, int* __restrict__ kstop) {
-    int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// The half-orbit cutoff of every ray from its samples, WIND_GROUP of them loaded at a time: the counter is serial, and a
+// load a step left the ray's one thread waiting for memory (z = r cos theta is the sample's stored z).
+constexpr int WIND_GROUP = 16;
+__global__ void __launch_bounds__(64) ks_wind_cutoff(double a, int64_t npix, int N, int nmax, double slab, Samples smp, int* __restrict__ kstop) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= npix) return;
-    Spin S = make_spin(a);
-    WindF f{S.rp, slab, nmax, N + 1, NAN, 0, false, false};
-    if (smp.r) {
-        for (int k = 1; k <= N && f.kstop > N; ++k) {
-            const int64_t o = (int64_t)(k - 1) * npix + j;
-            const uint8_t fl = smp.fl[o];
-            Samp s{0.0, smp.r[o], smp.th[o], 0.0, (fl & 2) != 0, (fl & 4) != 0, (fl & 1) != 0};
-            f(k, s, 0.0);
+    WindF f{make_spin(a).rp, slab, nmax, N + 1, NAN, 0, false, false};
+    for (int k0 = 1; k0 <= N && f.kstop > N; k0 += WIND_GROUP) {
+        uint8_t fl[WIND_GROUP];
+        double r[WIND_GROUP], z[WIND_GROUP];
+#pragma unroll
+        for (int u = 0; u < WIND_GROUP; ++u) {
+            const int64_t o = (int64_t)((k0 + u <= N ? k0 + u : N) - 1) * npix + j;
+            fl[u] = smp.fl[o]; r[u] = smp.r[o]; z[u] = smp.z[o];
         }
-    } else {
-        PixC p = load_pixel(soa, npix, j);
-        double r1, r2;
-        march_ray(p, S, thetao, N, M, f, r1, r2);
+#pragma unroll
+        for (int u = 0; u < WIND_GROUP; ++u)
+            if (k0 + u <= N) f(k0 + u, (fl[u] & 1) != 0, r[u], z[u]);
     }
     kstop[j] = f.kstop;
+}
+
+// ---- tiles of a cache without stored samples ----------------------------------------------------------------------
+// The constants of the pixels at slots s0 .. s0 + n - 1 of the wavefront order, field-major over the tile; its images
+// and per-pixel values back to their sorted slots (dst[4 (tmap[s0 + s] + npix f) + q] = src[4 (s + n f) + q]).
+__global__ void ks_tile_gather(const double* __restrict__ soa, int64_t npix, const int* __restrict__ tmap, int64_t s0, int64_t n, double* __restrict__ dst) {
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int64_t j = tmap[s0 + s];
+    for (int f = 0; f < PF_COUNT; ++f) dst[f * n + s] = soa[f * npix + j];
+}
+__global__ void ks_tile_scatter4(const double* __restrict__ src, const int* __restrict__ tmap, int64_t s0, int64_t n, int64_t frames, int64_t npix,
+                                 double* __restrict__ dst) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n * frames) return;
+    const int64_t d = tmap[s0 + i % n] + npix * (i / n);
+    for (int q = 0; q < 4; ++q) dst[4 * d + q] = src[4 * i + q];
+}
+__global__ void ks_tile_scatter1(const double* __restrict__ src, const int* __restrict__ tmap, int64_t s0, int64_t n, double* __restrict__ dst) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[tmap[s0 + i]] = src[i];
 }
 
 // sorted -> screen: dst[4 (perm[j] + npix f) + q] = src[4 (j + npix f) + q]
@@ -198,9 +219,20 @@ hipError_t launch_res_reduce(hipStream_t s, int64_t npix, int nseg_max, const do
     hipLaunchKernelGGL(ks_res_reduce, dim3(grid_for(npix, 256)), dim3(256), 0, s, npix, nseg_max, res, rt, rp);
     return hipGetLastError();
 }
-hipError_t launch_wind_cutoff(hipStream_t s, double a, double thetao, const double* soa, int64_t npix, int N, int M, int nmax, double slab,
-                              Samples smp, int* kstop) {
-    hipLaunchKernelGGL(ks_wind_cutoff, dim3(grid_for(npix, 128)), dim3(128), 0, s, a, thetao, soa, npix, N, M, nmax, slab, smp, kstop);
+hipError_t launch_wind_cutoff(hipStream_t s, double a, int64_t npix, int N, int nmax, double slab, Samples smp, int* kstop) {
+    hipLaunchKernelGGL(ks_wind_cutoff, dim3(grid_for(npix, 64)), dim3(64), 0, s, a, npix, N, nmax, slab, smp, kstop);
+    return hipGetLastError();
+}
+hipError_t launch_tile_gather(hipStream_t s, const double* soa, int64_t npix, const int* tmap, int64_t s0, int64_t n, double* dst) {
+    hipLaunchKernelGGL(ks_tile_gather, dim3(grid_for(n, 128)), dim3(128), 0, s, soa, npix, tmap, s0, n, dst);
+    return hipGetLastError();
+}
+hipError_t launch_tile_scatter4(hipStream_t s, const double* src, const int* tmap, int64_t s0, int64_t n, int64_t frames, int64_t npix, double* dst) {
+    hipLaunchKernelGGL(ks_tile_scatter4, dim3(grid_for(n * frames, 256)), dim3(256), 0, s, src, tmap, s0, n, frames, npix, dst);
+    return hipGetLastError();
+}
+hipError_t launch_tile_scatter1(hipStream_t s, const double* src, const int* tmap, int64_t s0, int64_t n, double* dst) {
+    hipLaunchKernelGGL(ks_tile_scatter1, dim3(grid_for(n, 256)), dim3(256), 0, s, src, tmap, s0, n, dst);
     return hipGetLastError();
 }
 hipError_t launch_unsort4(hipStream_t s, const double* src, const int* perm, int64_t npix, int64_t nframes, double* dst) {

@@ -89,7 +89,7 @@ KS_DEV void tangent_item(int64_t item, double a, double thetao, double lnL, cons
         const SampT<D3> s = direct_sample(p, S, vis, dtau * (double)k);
         if (nmax >= 0) {
             const Samp sv{0.0, val(s.r), val(s.th), 0.0, s.nur, s.nuth, s.ok};
-            wf(k, sv, 0.0);
+            wf(k, sv.ok, sv.r, sv.r * cos(sv.th));
             if (wf.kstop <= k) break;
         }
         if (!(s.ok && s.r > rp * (1.0 + 1e-3))) continue;

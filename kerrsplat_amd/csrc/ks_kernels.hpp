@@ -192,9 +192,8 @@ KS_DEV f32 lane_value(f32 x, int lane) { return f32(__shfl(x.v, lane, 64)); }
 struct WindF {
     double rp, slab; int nmax, kstop;
     double zprev; int wn; bool inside, crossed;
-    KS_DEV void operator()(int k, const Samp& s, double) {
-        if (kstop <= k || !(s.ok && s.r > rp * (1.0 + 1e-3))) return;
-        double z = s.r * cos(s.th);
+    KS_DEV void operator()(int k, bool ok, double r, double z) {
+        if (kstop <= k || !(ok && r > rp * (1.0 + 1e-3))) return;
         if (isnan(zprev)) { zprev = z; inside = fabs(z) < slab; crossed = false; }
         else {
             bool inside_now = fabs(z) < slab;
@@ -221,8 +220,10 @@ hipError_t launch_pixel_constants(hipStream_t s, double a, double thetao, const 
 hipError_t launch_march_store(hipStream_t s, double a, double thetao, const double* soa, int64_t npix, int N, int M, int marcher, int nseg_max,
                               Samples smp, double* res, int fp32);
 hipError_t launch_res_reduce(hipStream_t s, int64_t npix, int nseg_max, const double* res, double* rt, double* rp);
-hipError_t launch_wind_cutoff(hipStream_t s, double a, double thetao, const double* soa, int64_t npix, int N, int M, int nmax, double slab,
-                              Samples smp, int* kstop);
+hipError_t launch_wind_cutoff(hipStream_t s, double a, int64_t npix, int N, int nmax, double slab, Samples smp, int* kstop);
+hipError_t launch_tile_gather(hipStream_t s, const double* soa, int64_t npix, const int* tmap, int64_t s0, int64_t n, double* dst);
+hipError_t launch_tile_scatter4(hipStream_t s, const double* src, const int* tmap, int64_t s0, int64_t n, int64_t frames, int64_t npix, double* dst);
+hipError_t launch_tile_scatter1(hipStream_t s, const double* src, const int* tmap, int64_t s0, int64_t n, double* dst);
 hipError_t launch_samples_f32(hipStream_t s, int64_t n, const double* x, const double* y, const double* z, const double* t, float4* p4);
 hipError_t launch_unsort4(hipStream_t s, const double* src, const int* perm, int64_t npix, int64_t nframes, double* dst);
 hipError_t launch_unsort1(hipStream_t s, const double* src, const int* perm, int64_t npix, double* dst);
@@ -251,18 +252,15 @@ hipError_t launch_chunk_transfer_f32(hipStream_t s, int kind, double a, double t
                                      const SplatCf* sp, int ns, const f32* knots, const f32* ktimes, int nknots,
                                      const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
                                      f32* seg, f32* rec, uint8_t* aflg, const TransferLaunch& tl);
-hipError_t launch_seg_polarized(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, int M,
-                                const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots,
-                                const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
-                                double* seg, double* res);
 hipError_t launch_ray_hits(hipStream_t s, double rp, int64_t npix, int N, Samples smp, const SplatC* sp, int ns, const double* times, int nt,
                            const int* kstop, uint8_t* hits, int* cnt);
 hipError_t launch_ray_fill(hipStream_t s, int64_t items, int64_t npix, int ns, int cap, const uint8_t* hits, const int* iperm, int32_t* ids);
-hipError_t launch_thin_parts(hipStream_t s, double a, double thetao, const double* soa, int64_t npix, int N, int M, Samples smp,
-                             const SplatC* sp, int ns, double t_obs, int nseg_max, double* part, double* res);
+int thin_chunks(int N);
+hipError_t launch_thin_parts(hipStream_t s, double a, const double* soa, int64_t npix, int N, Samples smp, const SplatC* sp, int ns, double t_obs,
+                             double* part);
 hipError_t launch_thin_combine(hipStream_t s, int64_t npix, int nseg_max, const double* part, double* out);
-hipError_t launch_seg_combine(hipStream_t s, const double* soa, int64_t npix, int N, int M, int chunk, int nt, const double* nus, int nnu,
-                              const void* seg, int seg32, double* out);
+hipError_t launch_seg_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const void* seg, int seg32,
+                              double* out);
 
 // ---- ks_k_adjoint.hip ----
 hipError_t launch_adj_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const void* seg, int seg32,

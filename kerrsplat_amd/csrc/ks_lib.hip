@@ -127,7 +127,10 @@ struct ks_cache {
     double *sx = nullptr, *sy = nullptr, *sz = nullptr;        // quasi-Cartesian position of each stored sample
     float4* sp4 = nullptr;                                     // their FP32 copy with t~ (x, y, z, t) for the FP32 element adjoints
     int64_t march_version = 0, p4_version = -1;                // marches into the samples; the march the copy was made from
-    double* thin_part = nullptr;                               // per-segment thin sums (max_segments x npix)
+    Buf<double> thin_part;                                     // per-chunk thin sums (thin_chunks x npix, or a tile's)
+    // caches without stored samples: one tile's samples, constants, anchor residuals (per segment, per pixel), half-orbit
+    // cutoff and images
+    Buf<double> ft, fr, fth, fph, fx, fy, fz, fsoa, fres, frt, frp, fout; Buf<uint8_t> ffl; Buf<int> fkstop;
     double *rt = nullptr, *rp = nullptr;
     double* out = nullptr; int64_t out_frames = 0;    // sorted-order Stokes images
     double* out_screen = nullptr;
@@ -301,12 +304,13 @@ int ks_cache_destroy(ks_cache* c) {
     (void)hipSetDevice(c->ctx->device);
     dfree(c->al); dfree(c->be); dfree(c->numreals); dfree(c->perm); dfree(c->tmap); dfree(c->iperm); dfree(c->bcount); dfree(c->soa);
     dfree(c->st); dfree(c->sr); dfree(c->sth); dfree(c->sph); dfree(c->sfl); dfree(c->rt); dfree(c->rp);
-    dfree(c->sx); dfree(c->sy); dfree(c->sz); dfree(c->thin_part); dfree(c->sp4);
+    dfree(c->sx); dfree(c->sy); dfree(c->sz); dfree(c->sp4);
     dfree(c->out); dfree(c->out_screen); dfree(c->img1);
     for (Buf<double>* b : {&c->vu, &c->vv, &c->vt, &c->vg, &c->vd, &c->vs, &c->vA2, &c->vB2, &c->vIm, &c->vC2, &c->vV, &c->vwq, &c->vE2,
-                           &c->vSd, &c->vSp, &c->vchi, &c->vsum, &c->idata, &c->isig, &c->bseed})
+                           &c->vSd, &c->vSp, &c->vchi, &c->vsum, &c->idata, &c->isig, &c->bseed, &c->thin_part, &c->ft, &c->fr, &c->fth, &c->fph,
+                           &c->fx, &c->fy, &c->fz, &c->fsoa, &c->fres, &c->frt, &c->frp, &c->fout})
         b->release();
-    c->imask.release();
+    c->imask.release(); c->ffl.release(); c->fkstop.release();
     c->ctri.release(); c->cquad.release(); c->coff.release(); c->clegs.release(); c->cdat.release(); c->cterm.release();
     dfree(c->seg); dfree(c->segres); dfree(c->kstop); dfree(c->dtn);
     dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->awT); dfree(c->ads); dfree(c->apart); dfree(c->adpar);
@@ -340,12 +344,6 @@ static int ensure_p4(ks_cache* c) {
     HIPCHK(launch_samples_f32(c->ctx->stream, n, c->sx, c->sy, c->sz, c->st, c->sp4));
     c->p4_version = c->march_version;
     return KS_OK;
-}
-static Samples no_samples() {
-    Samples S;
-    S.t = S.r = S.th = S.ph = S.x = S.y = S.z = nullptr; S.fl = nullptr;
-    S.tmap = nullptr;
-    return S;
 }
 // the cache's marcher into its sample storage (march!, cache.jl:182-190), anchor segments in parallel
 static int launch_store_march(ks_cache* c) {
@@ -634,14 +632,16 @@ static const double* stage_times(ks_cache* c, const double* times, int nt, const
     return c->dtn;
 }
 
-// Samples per slice of the transfer over stored samples, and whether its segment maps are FP32 (the mixed path's own
-// numbers, half the bytes of FP64 copies)
+// Samples per slice of the transfer, and whether its segment maps are FP32 (the mixed path's own numbers, half the bytes
+// of FP64 copies)
 static int slice_of(const ks_cache* c, int64_t items) { return slice_length(c->chunk, items, c->N); }
 static int seg_is32(const ks_cache* c) { return has_samples(c) && c->precision == KS_PRECISION_MIXED ? 1 : 0; }
-// room for the segment maps of `items` items: slices of the stored samples, or the pixel's anchor segments
+static int64_t seg_doubles(const ks_cache* c, int64_t items) {
+    const int64_t nseg = (c->N + slice_of(c, items) - 1) / slice_of(c, items);
+    return ((int64_t)SEG_FIELDS * nseg * items * (seg_is32(c) ? 4 : 8) + 7) / 8;
+}
 static int ensure_seg(ks_cache* c, int64_t items) {
-    const int64_t nseg = has_samples(c) ? (c->N + slice_of(c, items) - 1) / slice_of(c, items) : max_segments(c->N);
-    const int64_t need = ((int64_t)SEG_FIELDS * nseg * items * (seg_is32(c) ? 4 : 8) + 7) / 8;
+    const int64_t need = seg_doubles(c, items);
     if (c->seg_cap >= need) return KS_OK;
     dfree(c->seg); c->seg_cap = 0;
     if (dalloc(&c->seg, (size_t)need)) return KS_ERR_HIP;
@@ -698,31 +698,84 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, i
     return KS_OK;
 }
 
-// The transfer of every (pixel, time, frequency) item into the cache's segment maps: from the stored
-// samples when the cache holds them (one work item per chunk of samples), else fused with the march (one
-// work item per anchor segment). Records for the adjoint when rec != nullptr (stored samples only).
+// The transfer of every (pixel, time, frequency) item of the stored samples into the cache's segment maps, with the
+// adjoint's records when rec != nullptr.
 static int launch_transfer(ks_cache* c, const ks_model* m, const double* d_tn, int nt, int nnu, double L, int nmax, double slab,
                            double* rec, uint8_t* aflg) {
     ks_ctx* x = c->ctx;
-    const int64_t items = c->npix * nt * nnu;
-    if (int rc = ensure_seg(c, items)) return rc;
+    if (int rc = ensure_seg(c, c->npix * nt * nnu)) return rc;
     const int* kst = nullptr;
     if (nmax >= 0) {
         if (!c->kstop) { if (dalloc(&c->kstop, (size_t)c->npix)) return KS_ERR_HIP; }
-        HIPCHK(launch_wind_cutoff(x->stream, c->spin, c->thetao, c->soa, c->npix, c->N, c->M, nmax, slab,
-                                  has_samples(c) ? samples_of(c) : no_samples(), c->kstop));
+        HIPCHK(launch_wind_cutoff(x->stream, c->spin, c->npix, c->N, nmax, slab, samples_of(c), c->kstop));
         kst = c->kstop;
     }
     HIPCHK(x->stage_begin(KS_STAGE_TRANSFER));
-    if (has_samples(c)) {
-        if (int rc = transfer_launch(c, m, d_tn, nt, nnu, L, kst, rec, aflg, nullptr)) return rc;
-    } else
-        HIPCHK(launch_seg_polarized(x->stream, m->kind, c->spin, c->thetao, c->soa, c->npix, c->N, c->M, m->d_splats, m->ns,
-                                    m->d_knots, m->d_ktimes, m->nknots, d_tn, nt, d_tn + nt, nnu, L, kst, c->seg, c->segres));
+    if (int rc = transfer_launch(c, m, d_tn, nt, nnu, L, kst, rec, aflg, nullptr)) return rc;
     HIPCHK(x->stage_end(KS_STAGE_TRANSFER));
-    if (!has_samples(c)) {
-        HIPCHK(launch_res_reduce(x->stream, c->npix, max_segments(c->N), c->segres, c->rt, c->rp));
+    return KS_OK;
+}
+
+// Caches without stored samples march a tile of the pixels at a time into a workspace of at most FUSED_SAMPLES samples
+// (57 bytes each, 0.5 GB; at least FUSED_MIN pixels) and run the transfer of stored samples over it, the frames in
+// groups whose segment maps stay within FUSED_SEG bytes. A tile is a run of the wavefront order. Marched inside the
+// transport instead, every frame marched its own rays, one thread a segment of 64 samples with the pairs of its splats
+// in turn: 6.6 ms and 3.6 more for the half-orbit cutoff at 96 x 72 x 500 and 16 splats; the whole call now takes 1.9 ms
+(8.6 before). 200 kappa splats on knots, 96 x 72 x 400: 172 -> 12 ms.
+constexpr int64_t FUSED_SAMPLES = (int64_t)1 << 23, FUSED_MIN = 8, FUSED_SEG = (int64_t)1 << 29;
+static int64_t fused_tile(const ks_cache* c) {
+    const int64_t n = std::max(FUSED_SAMPLES / c->N, FUSED_MIN);
+    return std::min(n >= 128 ? n / 128 * 128 : n, c->npix);
+}
+// the samples and constants of the tile s0 .. s0 + n - 1; the anchor residuals to the cache's
+static int fused_march(ks_cache* c, int64_t s0, int64_t n, Samples& S) {
+    ks_ctx* x = c->ctx;
+    const size_t ns = (size_t)n * c->N, nseg = (size_t)max_segments(c->N);
+    if (c->ft.grow(ns) || c->fr.grow(ns) || c->fth.grow(ns) || c->fph.grow(ns) || c->fx.grow(ns) || c->fy.grow(ns) || c->fz.grow(ns) ||
+        c->ffl.grow(ns) || c->fsoa.grow((size_t)PF_COUNT * n) || c->fres.grow(2 * nseg * n) || c->frt.grow(n) || c->frp.grow(n))
+        return KS_ERR_HIP;
+    S.t = c->ft.p; S.r = c->fr.p; S.th = c->fth.p; S.ph = c->fph.p; S.x = c->fx.p; S.y = c->fy.p; S.z = c->fz.p; S.fl = c->ffl.p;
+    S.tmap = nullptr; S.p4 = nullptr;
+    HIPCHK(launch_tile_gather(x->stream, c->soa, c->npix, c->tmap, s0, n, c->fsoa.p));
+    HIPCHK(launch_march_store(x->stream, c->spin, c->thetao, c->fsoa.p, n, c->N, c->M, 1, (int)nseg, S, c->fres.p, 0));
+    HIPCHK(launch_res_reduce(x->stream, n, (int)nseg, c->fres.p, c->frt.p, c->frp.p));
+    HIPCHK(launch_tile_scatter1(x->stream, c->frt.p, c->tmap, s0, n, c->rt));
+    HIPCHK(launch_tile_scatter1(x->stream, c->frp.p, c->tmap, s0, n, c->rp));
+    return KS_OK;
+}
+static int fused_render(ks_cache* c, const ks_model* m, const double* d_tn, int nt, int nnu, double L, int nmax, double slab) {
+    ks_ctx* x = c->ctx;
+    const int64_t tile = fused_tile(c);
+    if (c->qhead.grow(1)) return KS_ERR_HIP;
+    HIPCHK(x->stage_begin(KS_STAGE_TRANSFER));
+    for (int64_t s0 = 0; s0 < c->npix; s0 += tile) {
+        const int64_t n = std::min(tile, c->npix - s0);
+        Samples S;
+        if (int rc = fused_march(c, s0, n, S)) return rc;
+        const int* kst = nullptr;
+        if (nmax >= 0) {
+            if (c->fkstop.grow(n)) return KS_ERR_HIP;
+            HIPCHK(launch_wind_cutoff(x->stream, c->spin, n, c->N, nmax, slab, S, c->fkstop.p));
+            kst = c->fkstop.p;
+        }
+        int group = nt;
+        while (group > 1 && 8 * seg_doubles(c, n * group) > FUSED_SEG) group = (group + 1) / 2;
+        for (int inu = 0; inu < nnu; ++inu)
+            for (int it = 0; it < nt; it += group) {
+                const int nf = std::min(group, nt - it);
+                if (ensure_seg(c, n * nf) || c->fout.grow((size_t)4 * n * nf)) return KS_ERR_HIP;
+                TransferLaunch tl;
+                tl.chunk = slice_of(c, n * nf);
+                tl.head = c->qhead.p;
+                const double* nu = d_tn + nt + inu;
+                HIPCHK(launch_chunk_transfer(x->stream, m->kind, c->spin, c->thetao, c->fsoa.p, n, c->N, S, m->d_splats, m->ns, m->d_knots, m->d_ktimes,
+                                             m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_tn + it, nf, nu, 1, L, kst, c->seg, nullptr, nullptr,
+                                             tl));
+                HIPCHK(launch_seg_combine(x->stream, n, c->N, tl.chunk, nf, nu, 1, c->seg, 0, c->fout.p));
+                HIPCHK(launch_tile_scatter4(x->stream, c->fout.p, c->tmap, s0, n, nf, c->npix, c->out + (int64_t)4 * c->npix * (it + (int64_t)nt * inu)));
+            }
     }
+    HIPCHK(x->stage_end(KS_STAGE_TRANSFER));
     return KS_OK;
 }
 
@@ -740,10 +793,10 @@ int ks_render_device(ks_cache* c, const ks_model* m, const double* times, int nt
     if (ensure_out(c, frames)) return KS_ERR_HIP;
     const double* d_tn = stage_times(c, times, nt, nus, nnu);
     if (!d_tn) return KS_ERR_HIP;
+    if (!has_samples(c)) return fused_render(c, m, d_tn, nt, nnu, L, nmax, slab);
     int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, nullptr, nullptr);
     if (rc) return rc;
-    const int64_t items = c->npix * frames;
-    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, has_samples(c) ? slice_of(c, items) : 0, nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
+    HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice_of(c, c->npix * frames), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
     return KS_OK;
 }
 
@@ -1048,7 +1101,7 @@ int ks_gradient_forward(ks_cache* c, const ks_model* m, const double* times, int
     if (!d_tn) return KS_ERR_HIP;
     int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, c->arec, c->aflg);
     if (rc) return rc;
-    HIPCHK(launch_seg_combine(x->stream, c->soa, c->npix, c->N, c->M, slice_of(c, items), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
+    HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice_of(c, items), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
     c->fw_model = m->id; c->fw_nt = nt; c->fw_nnu = nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
     c->fw_chunk = slice_of(c, items);
     c->fw_seeded.assign((size_t)frames, 0);
@@ -1131,13 +1184,23 @@ int ks_thin_image(ks_cache* c, const ks_model* m, double t_obs, double* out, int
     ks_ctx* x = c->ctx;
     HIPCHK(hipSetDevice(x->device));
     if (!c->img1) { if (dalloc(&c->img1, (size_t)2 * c->npix)) return KS_ERR_HIP; }
-    const int nseg = max_segments(c->N);
-    if (!c->thin_part) { if (dalloc(&c->thin_part, (size_t)nseg * c->npix)) return KS_ERR_HIP; }
-    // per segment sums from the stored samples (CHUNK samples) or fused with the march (anchor segments)
-    HIPCHK(launch_thin_parts(x->stream, c->spin, c->thetao, c->soa, c->npix, c->N, c->M, has_samples(c) ? samples_of(c) : no_samples(),
-                             m->d_splats, m->ns, t_obs, nseg, c->thin_part, c->segres));
-    HIPCHK(launch_thin_combine(x->stream, c->npix, nseg, c->thin_part, c->img1));
-    if (!has_samples(c)) HIPCHK(launch_res_reduce(x->stream, c->npix, nseg, c->segres, c->rt, c->rp));
+    const int nch = thin_chunks(c->N);
+    if (has_samples(c)) {
+        if (c->thin_part.grow((size_t)nch * c->npix)) return KS_ERR_HIP;
+        HIPCHK(launch_thin_parts(x->stream, c->spin, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->ns, t_obs, c->thin_part.p));
+        HIPCHK(launch_thin_combine(x->stream, c->npix, nch, c->thin_part.p, c->img1));
+    } else {
+        const int64_t tile = fused_tile(c);
+        for (int64_t s0 = 0; s0 < c->npix; s0 += tile) {
+            const int64_t n = std::min(tile, c->npix - s0);
+            Samples S;
+            if (int rc = fused_march(c, s0, n, S)) return rc;
+            if (c->thin_part.grow((size_t)nch * n) || c->fout.grow((size_t)n)) return KS_ERR_HIP;
+            HIPCHK(launch_thin_parts(x->stream, c->spin, c->fsoa.p, n, c->N, S, m->d_splats, m->ns, t_obs, c->thin_part.p));
+            HIPCHK(launch_thin_combine(x->stream, n, nch, c->thin_part.p, c->fout.p));
+            HIPCHK(launch_tile_scatter1(x->stream, c->fout.p, c->tmap, s0, n, c->img1));
+        }
+    }
     const double* src = c->img1;
     if (screen_order) {
         HIPCHK(launch_unsort1(x->stream, c->img1, c->perm, c->npix, c->img1 + c->npix));
@@ -1173,7 +1236,7 @@ int ks_ray_lists(ks_cache* c, const ks_model* m, const double* times, int nt, in
     const int* kst = nullptr;
     if (nmax >= 0) {
         if (!c->kstop) { if (dalloc(&c->kstop, (size_t)npix)) return KS_ERR_HIP; }
-        HIPCHK(launch_wind_cutoff(x->stream, c->spin, c->thetao, c->soa, npix, c->N, c->M, nmax, slab, samples_of(c), c->kstop));
+        HIPCHK(launch_wind_cutoff(x->stream, c->spin, npix, c->N, nmax, slab, samples_of(c), c->kstop));
         kst = c->kstop;
     }
     const double rp = 1.0 + sqrt(1.0 - c->spin * c->spin);
@@ -1623,7 +1686,7 @@ static int graph_record(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpyAsync(m->d_adj_f, g->h_adf, ns * sizeof(SplatAdjf), hipMemcpyHostToDevice, s));
     const int nt = g->nt, nnu = g->nnu;
     if (int rc = launch_transfer(c, m, g->dtn.p, nt, nnu, g->L, -1, 0.0, c->arec, c->aflg)) return rc;
-    HIPCHK(launch_seg_combine(s, c->soa, c->npix, c->N, c->M, slice_of(c, c->npix * g->frames), nt, g->dtn.p + nt, nnu, c->seg, seg_is32(c), c->out));
+    HIPCHK(launch_seg_combine(s, c->npix, c->N, slice_of(c, c->npix * g->frames), nt, g->dtn.p + nt, nnu, c->seg, seg_is32(c), c->out));
     const int na = c->nalpha, nb = c->nbeta;
     for (int f = 0; f < g->frames; ++f) {
         if (g->loss == KS_LOSS_IMAGE) {

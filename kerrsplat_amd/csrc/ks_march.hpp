@@ -288,12 +288,6 @@ KS_DEV void march_range(const PixC& p, const Spin& S, double thetao, int N, int 
     march_range<double, F>(p, S, thetao, N, M, kbeg, kend, f, resid_t, resid_ph);
 }
 
-// March one whole ray (samples 1..N). Returns the largest anchor residuals.
-template <class F>
-KS_DEV void march_ray(const PixC& p, const Spin& S, double thetao, int N, int M, F& f, double& resid_t, double& resid_ph) {
-    march_range(p, S, thetao, N, M, 1, N, f, resid_t, resid_ph);
-}
-
 // Segments of a ray for parallel marching: whole multiples of the anchor interval, at least SEG_MIN
 // samples (at most 2 SEG_MIN - 1, or the anchor interval itself when that is longer).
 constexpr int SEG_MIN = 32;
