@@ -256,7 +256,7 @@ ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __
 // m THIN_CHUNK + 1 .. of pixel j. A thread holds its samples in registers and takes the splats in turn, their constants
 // once for all of them; bound by the FP64 sine, cosine and exponential of every (sample, splat). Folded into the march
 // (one thread a 64-sample segment, one wavefront a SIMD for its registers) the sums ran at a fifth of the issue rate:
-300 splats, 96 x 72 x 400, fused march 12.5 -> 3.8 ms; 40 splats over stored samples 1.38 -> 0.51 ms.
+// 300 splats, 96 x 72 x 400, fused march 12.5 -> 3.8 ms; 40 splats over stored samples 1.38 -> 0.51 ms.
 constexpr int THIN_CHUNK = 4;
 __global__ void __launch_bounds__(128) ks_thin_parts(double a, const double* __restrict__ soa, int64_t npix, int N, Samples smp,
                                                      const SplatC* __restrict__ sp, int ns, double t_obs, double* __restrict__ part) {

@@ -721,7 +721,7 @@ static int launch_transfer(ks_cache* c, const ks_model* m, const double* d_tn, i
 // groups whose segment maps stay within FUSED_SEG bytes. A tile is a run of the wavefront order. Marched inside the
 // transport instead, every frame marched its own rays, one thread a segment of 64 samples with the pairs of its splats
 // in turn: 6.6 ms and 3.6 more for the half-orbit cutoff at 96 x 72 x 500 and 16 splats; the whole call now takes 1.9 ms
-(8.6 before). 200 kappa splats on knots, 96 x 72 x 400: 172 -> 12 ms.
+// (8.6 before). 200 kappa splats on knots, 96 x 72 x 400: 172 -> 12 ms.
 constexpr int64_t FUSED_SAMPLES = (int64_t)1 << 23, FUSED_MIN = 8, FUSED_SEG = (int64_t)1 << 29;
 static int64_t fused_tile(const ks_cache* c) {
     const int64_t n = std::max(FUSED_SAMPLES / c->N, FUSED_MIN);
