@@ -263,7 +263,7 @@ KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao
     // reverse: d chi = (ea d eb - eb d ea) / (ea^2 + eb^2)
     const S den = ea * ea + eb * eb;
     if (!(den > 0.0)) return o;
-    const S w = 1.0 / den;
+    const S w = sdiv(S(1.0), den);
     const S eab = -eb * w, ebb = ea * w;
     const S kk1b = beta * ebb - mu * eab, kk2b = beta * eab + mu * ebb;
     const S Ab = G.r * kk1b - act * kk2b, Bws = -(act * kk1b + G.r * kk2b) * G.st;
@@ -390,7 +390,7 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
     const bool jv = !(fabs(NhighV) < small * small);
     S rVr(0.0), pV(0.0), tV(1.0), PV(1.0);
     if (jv) {
-        rVr = NlowV / NhighV; pV = pow(rVr, XI); tV = 1.0 + pXI * pV; PV = pow(tV, MI);
+        rVr = sdiv(NlowV, NhighV); pV = pow(rVr, XI); tV = 1.0 + pXI * pV; PV = pow(tV, MI);
         c.jV = -(pref * NlowV * X13 * PV) * sgn;
     } else {
         c.jV = S(0.0);
@@ -407,7 +407,7 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
     const S v446 = pow_nonneg(u228, 0.446), s205 = sqrt(u205);
     const S NlowVA = CVA1 * v446 * Xm035;
     const S NhighVA = CVA2 * s205 / sX + small;
-    const S rVA = NlowVA / NhighVA, pVA = pow(rVA, XVA), pXVA = pow(X, EVA), tVA = 1.0 + pXVA * pVA, PVA = pow(tVA, MVA);
+    const S rVA = sdiv(NlowVA, NhighVA), pVA = pow(rVA, XVA), pXVA = pow(X, EVA), tVA = 1.0 + pXVA * pVA, PVA = pow(tVA, MVA);
     c.aV = -(apref * NlowVA * Xm53 * PVA) * sgn;
     const int i = (int)val(K(KK_IFIT));
     const S p084 = pow(X, 0.84), xm = 1.0 / sX;
@@ -456,9 +456,9 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
         bX += bpXVA * EVA * pXVA / X;
         bK[KK_EVA] += bpXVA * pXVA * lX;
         S brVA(0.0);
-        if (rVA > 0.0) { brVA = bpVA * XVA * pVA / rVA; bK[KK_XVA] += bpVA * pVA * log(rVA); }
-        bNlowVA += brVA / NhighVA;
-        const S bNhighVA = -(brVA * rVA / NhighVA);
+        if (rVA > 0.0) { brVA = sdiv(bpVA * XVA * pVA, rVA); bK[KK_XVA] += bpVA * pVA * log(rVA); }
+        bNlowVA += sdiv(brVA, NhighVA);
+        const S bNhighVA = -sdiv(brVA * rVA, NhighVA);
         bK[KK_CVA2] += bNhighVA * s205 / sX;
         const S bs205 = bNhighVA * CVA2 / sX;
         bsX += -(bNhighVA * CVA2 * s205 / (sX * sX));
@@ -506,9 +506,9 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
         bpXI += btV * pV;
         const S bpV = btV * pXI;
         S brV(0.0);
-        if (rVr > 0.0) { brV = bpV * XI * pV / rVr; bK[KK_XI] += bpV * pV * log(rVr); }
-        bNlowV += brV / NhighV;
-        const S bNhighV = -(brV * rVr / NhighV);
+        if (rVr > 0.0) { brV = sdiv(bpV * XI * pV, rVr); bK[KK_XI] += bpV * pV * log(rVr); }
+        bNlowV += sdiv(brV, NhighV);
+        const S bNhighV = -sdiv(brV * rVr, NhighV);
         bK[KK_CV2] += bNhighV * v44 / sX;
         const S bv44 = bNhighV * CV2 / sX;
         bsX += -(bNhighV * CV2 * v44 / (sX * sX));

@@ -381,7 +381,7 @@ KS_DEV CoefT<T> thermal(NE ne, T Th, T k0k2, T k1k2, T B, T nu, T sth, T cth) {
     c.jV = 2.0 * ne * EE * EE * nu * cth / sth / (3.0 * 1.7320508075688772 * CL * Th * Th * Th) *
            (1.81384 / xs + 3.42319 * xm23 + 0.0292545 / sqrt(xs) + 2.03773 * xm13) * e;
     T Bn = planck(nu, Th);
-    T ib = Bn > 0.0 ? 1.0 / Bn : T(0.0);
+    T ib = Bn > 0.0 ? sdiv(T(1.0), Bn) : T(0.0);
     c.aI = c.jI * ib; c.aQ = c.jQ * ib; c.aV = c.jV * ib;
     return c;
 }
@@ -527,14 +527,14 @@ KS_DEV CoefT<T> kappa_coefs(const KF& K, T ne, T nu, T sth, T cth) {
     T NhighV = K(KK_CV2) * pow_nonneg(expm1(-1.25 * ls2), 0.44) / sX - small;
     const double sgn = cth > 0.0 ? 1.0 : (cth < 0.0 ? -1.0 : 0.0);
     c.jV = fabs(NhighV) < small * small ? T(0.0)
-         : -(pref * NlowV * X13 * pow(1.0 + pXI * pow(NlowV / NhighV, K(KK_XI)), K(KK_MI))) * sgn;
+         : -(pref * NlowV * X13 * pow(1.0 + pXI * pow(sdiv(NlowV, NhighV), K(KK_XI)), K(KK_MI))) * sgn;
     T apref = ne * K(KK_APRE) / sth;
     T Xm53 = pow(X, -5.0 / 3.0);
     c.aI = apref * K(KK_LOWA) * Xm53 * pow(1.0 + pow(X, K(KK_EA)) * K(KK_RA), K(KK_MA));
     c.aQ = -(apref * K(KK_NLOWQA) * Xm53 * pow(1.0 + pow(X, K(KK_EQA)) * K(KK_RQA), K(KK_MQA)));
     T NlowVA = K(KK_CVA1) * pow_nonneg(expm1(-1.14 * ls2), 0.446) * Xm035;
     T NhighVA = K(KK_CVA2) * sqrt(expm1(-1.025 * ls2)) / sX + small;
-    c.aV = -(apref * NlowVA * Xm53 * pow(1.0 + pow(X, K(KK_EVA)) * pow(NlowVA / NhighVA, K(KK_XVA)), K(KK_MVA))) * sgn;
+    c.aV = -(apref * NlowVA * Xm53 * pow(1.0 + pow(X, K(KK_EVA)) * pow(sdiv(NlowVA, NhighVA), K(KK_XVA)), K(KK_MVA))) * sgn;
     const int i = (int)val(K(KK_IFIT));
     T p084 = pow(X, 0.84), xm = 1.0 / sX;
     T fQ = K(KK_FQ0) * kappa_rhoQ_x<T>(i, X, p084) + K(KK_FQ1) * kappa_rhoQ_x<T>(i + 1, X, p084);
@@ -678,8 +678,8 @@ KS_DEV void step_coefs_inv(T aI, T a2, T r2, T ar, S f, T o[4], T e4[4]) {
     T h = (a2 - r2) * 0.5;
     T root = sqrt(h * h + ar * ar);
     T L1sq, L2sq;
-    if (h >= 0.0) { L1sq = h + root; L2sq = L1sq > 0.0 ? ar * ar / L1sq : T(0.0); }
-    else { L2sq = root - h; L1sq = L2sq > 0.0 ? ar * ar / L2sq : T(0.0); }
+    if (h >= 0.0) { L1sq = h + root; L2sq = L1sq > 0.0 ? sdiv(ar * ar, L1sq) : T(0.0); }
+    else { L2sq = root - h; L1sq = L2sq > 0.0 ? sdiv(ar * ar, L2sq) : T(0.0); }
     T L1 = L1sq > 0.0 ? sqrt(L1sq) : T(0.0), L2 = L2sq > 0.0 ? sqrt(L2sq) : T(0.0);
     T b1 = L1 * f, b2 = L2 * f;
     T Th = L1sq + L2sq;
@@ -728,7 +728,7 @@ KS_DEV void step_coefs_inv(T aI, T a2, T r2, T ar, S f, T o[4], T e4[4]) {
         isc = M[1] - bb * (M[3] / 6.0 - bb * (M[5] / 120.0 - bb * (M[7] / 5040.0 - bb * M[9] / 362880.0)));
     } else {
         T sb = sin(b2);
-        T den = 1.0 / (a * a + b2 * b2);
+        T den = sdiv(T(1.0), a * a + b2 * b2);
         ivs = pa - (a - e * (a * cb2 - b2 * sb)) * den;
         isc = (1.0 - e * (a * sb / b2 + cb2)) * den;
     }
