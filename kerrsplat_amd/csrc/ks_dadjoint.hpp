@@ -27,15 +27,15 @@ template <class S> struct SplatAdjT {
     // power law, (kappa, ln w) for kappa: power law {dgPL0/dp, dgPL1/dp}; kappa {d2F1/dkappa, d2F1/d ln w,
     // dGamma(k-4/3)/dk, dGamma(k-2)/dk, dGamma(k/4-1/3)/dk, dGamma(k/4+4/3)/dk, dGamma(2+k/2)/dk, d(K0/K2)/d ln w}
     S dpop[8];
-    // kappa: the partials of the fits' per-splat factors (kappa_consts) in kappa, ln w and ln B
+    // kappa, power law: the partials of the fits' per-splat factors in the two population rows and ln B
     S dkk[3][KK_N];
 };
 using SplatAdj = SplatAdjT<double>;
 using SplatAdjf = SplatAdjT<f32>;
 
-// A kappa splat's per-splat factors as five-partial duals over (kappa, ln w, ln B, g, cos B): the values and their
-// partials in the three population rows, read as the fits use them
-template <class S> struct KappaDualGet {
+// A splat's fit factors as five-partial duals over (its two population rows, ln B, g, cos B): the values and their
+// partials in the three rows, read as the fits use them
+template <class S> struct FactorDual {
     const KappaK<S>& k;
     const SplatAdjT<S>& sa;
     KS_DEV DN<5, S> operator()(int f) const {
@@ -118,7 +118,7 @@ KS_DEV bool weight_active(const SplatCT<S>& c, S t, S x, S y, S z) {
     S sp, cp;
     if (outside_support(c, t, x, y, z, sp, cp)) return false;
     const S g = gauss_exponent(c, t, x, y, z, sp, cp);
-    return !(g > GEXP_SKIP) && exp(-0.5 * g) > WEIGHT_CUTOFF;
+    return !(g > GEXP_SKIP) && fexp(-0.5 * g) > WEIGHT_CUTOFF;
 }
 
 // rows 7-10 of d ln G: dlnG/dR[a][b] = e_a gu_b (R the rotation of the pattern offset e, gu = dlnG/du) through the
@@ -148,7 +148,7 @@ KS_DEV bool weight_active_knot(const SplatCT<S>& c, const S* knots, const S* kti
     for (int b = 0; b < 3; ++b) { const S q = (c.R[b] * e0 + c.R[3 + b] * e1 + c.R[6 + b] * e2) * c.is[b]; q2 += q * q; }
     const S tt = (t - c.t0) * c.iw;
     const S g = q2 + tt * tt;
-    return !(g > GEXP_SKIP) && exp(-0.5 * g) > WEIGHT_CUTOFF;
+    return !(g > GEXP_SKIP) && fexp(-0.5 * g) > WEIGHT_CUTOFF;
 }
 
 // d ln G of a splat whose centre follows knots (trajectories.jl:93-128) with respect to rows 1-12: the centre rows
@@ -162,7 +162,7 @@ KS_DEV S weight_dlog_knot(const SplatCT<S>& c, const SplatAdjT<S>& sa, const S* 
     S u[3], q[3];
     for (int b = 0; b < 3; ++b) { u[b] = c.R[b] * e[0] + c.R[3 + b] * e[1] + c.R[6 + b] * e[2]; q[b] = u[b] * c.is[b]; }
     const S tt = (t - c.t0) * c.iw;
-    const S G = exp(-0.5 * (q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + tt * tt));
+    const S G = fexp(-0.5 * (q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + tt * tt));
     if (!(G > WEIGHT_CUTOFF)) return S(0.0);
     S gu[3], ge[3];
     for (int b = 0; b < 3; ++b) { gu[b] = -q[b] * c.is[b]; dl[3 + b] = q[b] * q[b]; }
@@ -189,7 +189,7 @@ KS_DEV S weight_dlog(const SplatCT<S>& c, const SplatAdjT<S>& sa, S t, S x, S y,
     const S dt = t - c.t0;
     const S tt = dt * c.iw;
     const S gexp = q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + tt * tt;
-    const S G = exp(-0.5 * gexp);
+    const S G = fexp(-0.5 * gexp);
     if (!(G > WEIGHT_CUTOFF)) return S(0.0);
     // ln G = -(|q|^2 + tt^2) / 2, q_b = u_b exp(-s_b), u = R^T e, e = Rz(-ph) (X - c(ph))
     S gu[3], ge[3];
@@ -213,38 +213,34 @@ KS_DEV S weight_dlog(const SplatCT<S>& c, const SplatAdjT<S>& sa, S t, S x, S y,
 // the boost of the photon momentum (g, the wave vector k) forward in three-partial duals over u, cos B = k . bh
 // from those, and chi by one reverse sweep of its own chain (the polarisation direction f = k x bh, the
 // inverse boost, the Walker-Penrose constant, the screen angle) joined to the partials of k and of the boost's
-// q = 1 / (gamma + 1). chi depends on the unit direction h = f / |f| only, so the normalisation adds
-// nothing to its partials (hbar . h = 0, fbar = hbar / |f|).
-template <class S> struct FrameJ { S g, cosB, chi, dg[5], dcosB[5], dchi[5]; };
+// q = 1 / (gamma + 1). chi does not depend on the length of f, which is left as it is (local_frame).
+template <class S> struct FrameJ { S g, ig, cosB, c2, s2, dg[5], dcosB[5], dchi[5]; };   // c2, s2: cosine and sine of 2 chi
 
 template <class S>
-KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao_sin, const S uv[3], S sthB, S cthB, S sphB, S cphB) {
+KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao_sin, const S uv[3], S gamv, S qv, S sthB, S cthB, S sphB, S cphB) {
     using D3 = DN<3, S>;
     const S bh0 = sthB * cphB, bh1 = sthB * sphB, bh2 = cthB;
     const S bt0 = cthB * cphB, bt1 = cthB * sphB, bt2 = -sthB;     // d bh / d theta_B
     const S bp0 = -bh1, bp1 = bh0;                                  // d bh / d phi_B (third entry 0)
     const D3 u0 = D3::seed(uv[0], 0), u1 = D3::seed(uv[1], 1), u2 = D3::seed(uv[2], 2);
-    const D3 gam = sqrt(1.0 + (u0 * u0 + u1 * u1 + u2 * u2));
-    const D3 q = 1.0 / (gam + 1.0);
+    D3 gam(gamv), q(qv);
+    const S igam = 1.0 / gamv;
+    for (int i = 0; i < 3; ++i) { gam.d[i] = uv[i] * igam; q.d[i] = -(qv * qv) * gam.d[i]; }
     const D3 ud = u0 * G.pz[1] + u1 * G.pz[2] + u2 * G.pz[3];
     const D3 c1 = ud * q - G.pz[0];
-    const D3 g = 1.0 / (gam * G.pz[0] - ud);
+    const D3 ig = gam * G.pz[0] - ud, g = 1.0 / ig;
     const D3 k0 = (G.pz[1] + u0 * c1) * g, k1 = (G.pz[2] + u1 * c1) * g, k2 = (G.pz[3] + u2 * c1) * g;
     const D3 cosB = k0 * bh0 + k1 * bh1 + k2 * bh2;
     FrameJ<S> o;
-    o.g = g.v; o.cosB = cosB.v;
+    o.g = g.v; o.ig = ig.v; o.cosB = cosB.v;
     o.dg[0] = o.dg[1] = S(0.0);
     o.dcosB[0] = k0.v * bt0 + k1.v * bt1 + k2.v * bt2;
     o.dcosB[1] = k0.v * bp0 + k1.v * bp1;
     for (int i = 0; i < 3; ++i) { o.dg[2 + i] = g.d[i]; o.dcosB[2 + i] = cosB.d[i]; }
     for (int i = 0; i < 5; ++i) o.dchi[i] = S(0.0);
-    o.chi = S(0.0);
-    const S f0 = k1.v * bh2 - k2.v * bh1, f1 = k2.v * bh0 - k0.v * bh2, f2 = k0.v * bh1 - k1.v * bh0;
-    const S fn = sqrt(f0 * f0 + f1 * f1 + f2 * f2);
-    if (!(fn > 0.0)) return o;
+    o.c2 = S(1.0); o.s2 = S(0.0);
     // forward values (the expressions of local_frame)
-    const S ifn = 1.0 / fn;
-    const S h0 = f0 * ifn, h1 = f1 * ifn, h2 = f2 * ifn;
+    const S h0 = k1.v * bh2 - k2.v * bh1, h1 = k2.v * bh0 - k0.v * bh2, h2 = k0.v * bh1 - k1.v * bh0;
     const S uf = u0.v * h0 + u1.v * h1 + u2.v * h2;
     const S ufq = uf * q.v;
     const S fz1 = h0 + u0.v * ufq, fz2 = h1 + u1.v * ufq, fz3 = h2 + u2.v * ufq;
@@ -259,11 +255,12 @@ KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao
     const S kk1 = A * G.r - Bw * act, kk2 = -(A * act + Bw * G.r);
     const S mu = -(alpha + a * thetao_sin);
     const S ea = beta * kk2 - mu * kk1, eb = beta * kk1 + mu * kk2;
-    o.chi = atan2(-ea, eb);
     // reverse: d chi = (ea d eb - eb d ea) / (ea^2 + eb^2)
     const S den = ea * ea + eb * eb;
-    if (!(den > 0.0)) return o;
-    const S w = sdiv(S(1.0), den);
+    if (den == 0.0) return o;
+    const S w = 1.0 / den;
+    o.c2 = (eb - ea) * (eb + ea) * w;
+    o.s2 = -2.0 * ea * eb * w;
     const S eab = -eb * w, ebb = ea * w;
     const S kk1b = beta * ebb - mu * eab, kk2b = beta * eab + mu * ebb;
     const S Ab = G.r * kk1b - act * kk2b, Bws = -(act * kk1b + G.r * kk2b) * G.st;
@@ -275,7 +272,7 @@ KS_DEV FrameJ<S> frame_jacobian(const GeoT<S>& G, S a, S alpha, S beta, S thetao
     const S ufqb = z1b * u0.v + z2b * u1.v + z3b * u2.v;
     const S ufb = ftb * G.ilapse + ufqb * q.v;
     const S qb = ufqb * uf;
-    const S fb0 = (z1b + ufb * u0.v) * ifn, fb1 = (z2b + ufb * u1.v) * ifn, fb2 = (z3b + ufb * u2.v) * ifn;
+    const S fb0 = z1b + ufb * u0.v, fb1 = z2b + ufb * u1.v, fb2 = z3b + ufb * u2.v;
     // f = k x bh: kbar = bh x fbar, bhbar = fbar x k
     const S kb0 = bh1 * fb2 - bh2 * fb1, kb1 = bh2 * fb0 - bh0 * fb2, kb2 = bh0 * fb1 - bh1 * fb0;
     const S bb0 = fb1 * k2.v - fb2 * k1.v, bb1 = fb2 * k0.v - fb0 * k2.v, bb2 = fb0 * k1.v - fb1 * k0.v;
@@ -297,7 +294,7 @@ template <class S>
 KS_DEV void element_adjoint_thermal(const SplatCT<S>& c, const SplatAdjT<S>& sa, const GeoT<S>& G, S a, S alpha, S beta,
                                     S thetao_sin, S nu, const S bars[11], S Gw, const S dl[13], S grad[21]) {
     const S uv[3] = {c.u[0], c.u[1], c.u[2]};
-    const FrameJ<S> fr = frame_jacobian(G, a, alpha, beta, thetao_sin, uv, sa.sthB, sa.cthB, sa.sphB, sa.cphB);
+    const FrameJ<S> fr = frame_jacobian(G, a, alpha, beta, thetao_sin, uv, c.gam, c.q, sa.sthB, sa.cthB, sa.sphB, sa.cphB);
     // the contribution: partials ln Theta_e, ln B, g, cos B; chi enters only through the screen rotation,
     // q = A + Bc cos 2chi + Bs sin 2chi with A, Bc, Bs free of chi, so its derivative is written out
     using D4 = DN<4, S>;
@@ -306,18 +303,18 @@ KS_DEV void element_adjoint_thermal(const SplatCT<S>& c, const SplatAdjT<S>& sa,
     D4 k1k2(c.p3); k1k2.d[0] = sa.dk1k2;
     D4 Bm(c.Bmag); Bm.d[1] = c.Bmag;
     const D4 g = D4::seed(fr.g, 2), cosB = D4::seed(fr.cosB, 3);
-    D4 nuf = nu / g;
+    D4 nh(nu * (1.0 / NU0) * fr.ig), inh = (NU0 / nu) * g;
+    nh.d[2] = -(nh.v * fr.ig);
+    D4 iTh(c.g[0]); iTh.d[0] = -c.g[0];
     D4 cb = dmin(dmax(cosB, -1.0), 1.0);
     D4 sth, cth;
     pitch_sincos(cb, sth, cth);
-    const S ne = exp(c.lnA) * Gw;
-    CoefT<D4> cf = thermal(ne, Th, k0k2, k1k2, Bm, nuf, sth, cth);
+    const S ne = splat_density(c) * Gw;
+    CoefT<D4> cf = thermal(ne, Th, iTh, k0k2, k1k2, Bm, nh * NU0, nh, inh, sth, cth);
     if (!(cf.jI > 0.0 || cf.aI > 0.0 || cf.rQ.v != 0.0 || cf.rV.v != 0.0)) return;
     D4 fe = cap_factor(cf.jI, cf.jQ, cf.jV), fa = cap_factor(cf.aI, cf.aQ, cf.aV);
-    D4 nh = nuf * (1.0 / NU0);
-    D4 i2 = 1.0 / (nh * nh);
-    S s2c, c2c;
-    sincos(2.0 * fr.chi, &s2c, &c2c);
+    D4 i2 = inh * inh;
+    const S s2c = fr.s2, c2c = fr.c2;
     D4 jQ = fe * cf.jQ * i2, aQ = fa * cf.aQ * nh, rQ = cf.rQ * nh;
     D4 A = bars[0] * (cf.jI * i2) + bars[3] * (fe * cf.jV * i2) + bars[4] * (cf.aI * nh) + bars[7] * (fa * cf.aV * nh) + bars[10] * (cf.rV * nh);
     D4 Bc = bars[1] * jQ + bars[5] * aQ + bars[8] * rQ;
@@ -335,90 +332,104 @@ KS_DEV void element_adjoint_thermal(const SplatCT<S>& c, const SplatAdjT<S>& sa,
 
 // The X-dependent rotativity factors of kappa_coefs with their derivatives in X (kappa_rhoQ_x, kappa_rhoV_x).
 template <class S>
-KS_DEV void kappa_rhoQ_x_d(int n, S X, S p084, S& h, S& dh) {
-    const double d = n == 1 ? 30.0 : (n == 2 ? 18.0 : (n == 3 ? 12.0 : 8.0));
-    const double sd = n == 1 ? 10.0 : (n == 2 ? 6.0 : 4.0);         // sin(X / sd); the fourth fit takes sin(0.375 X)
-    const double is_ = n == 4 ? 0.375 : 1.0 / sd;
-    const double cc = n == 1 ? 1.5 : (n == 2 ? 1.75 : (n == 3 ? 2.0 : 2.25));
-    const double b = n == 1 ? 0.471 : (n == 2 ? 0.5 : (n == 3 ? 0.525 : 0.541));
-    const S xb = n == 2 ? sqrt(X) : pow(X, b);
-    const S e1 = exp(-p084 / d), E = exp(-cc * xb);
+KS_DEV void kappa_rhoQ_x_d(const KappaRho& k, S X, S iX, const PowBase<S>& xb, S p084, S& h, S& dh) {
+    const S xp = pow_of(xb, k.b);
+    const S e1 = fexp(p084 * k.d), E = fexp(-k.cc * xp);
     S sn, cs;
-    sincos(n == 4 ? 0.375 * X : X / sd, &sn, &cs);
+    sincos_small(dmin(X * k.sd, 1e5), &sn, &cs);
     h = 1.0 - e1 - sn * E;
-    dh = e1 * (0.84 / d) * p084 / X - E * (cs * is_ - sn * (cc * b) * xb / X);
+    dh = -(e1 * (0.84 * k.d) * p084 * iX) - E * (cs * k.sd - sn * (k.cc * k.b) * xp * iX);
 }
 template <class S>
-KS_DEV void kappa_rhoV_x_d(int n, S xm, S& h, S& dh) {
-    const double b = n == 1 ? 0.447 : (n == 2 ? 0.391 : (n == 3 ? 0.348 : 0.313));
-    h = 1.0 - 0.17 * log1p(b * xm);
-    dh = -0.17 * b / (1.0 + b * xm);
+KS_DEV void kappa_rhoV_x_d(const KappaRho& k, S xm, S& h, S& dh) {
+    h = 1.0 - 0.17 * log1p_pos(k.v * xm);
+    dh = (-0.17 * k.v) / (1.0 + k.v * xm);
 }
 
 // The kappa coefficients of one sample (kappa_coefs) with the reverse sweep of a scalar q of them: the forward
 // pass, then qbar(c, cbar), the caller's dq/dc of the coefficient values, then the partials of q in the splat's
 // factors (bK, added), the fluid-frame frequency (bnu) and the pitch angle's sine and cosine (bsth, bcth; zero when
-// the sine was floored). Where a base of a power is zero its partials are zero (pow_nonneg's choice).
+// the sine was floored). Where a base of a power is zero its partials are zero (pow_nonneg's choice). The logarithms
+// of the bases serve their powers and the powers' partials in the exponents; a quantity that several terms divide by is
+// inverted once.
 template <class S, class KF, class QBar>
-KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qbar, S bK[KK_N], S& bnu, S& bsth, S& bcth) {
+KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S inu, S sth, S cth, QBar&& qbar, S bK[KK_N], S& bnu, S& bsth, S& bcth) {
     bool floored = false;
     if (!(sth > 0.0)) { sth = S(sin_floor(sth)); floored = true; }
     const double small = 1e-40;
     // ---- forward (the operations of kappa_coefs)
-    const S NUW1 = K(KK_NUW1), JPRE = K(KK_JPRE), APRE = K(KK_APRE);
-    const S X = nu / (NUW1 * sth);
+    const S INUW1 = K(KK_INUW1), JPRE = K(KK_JPRE), APRE = K(KK_APRE);
+    const S ist = fdiv(S(1.0), sth);
+    const S X = nu * INUW1 * ist, iX = fdiv(S(1.0), X);
+    const PowBase<S> xb = pow_base(X);
     const S pref = ne * JPRE * sth;
     const S X13 = cbrt(X);
-    const S lX = log(X);
+    const S lX = ln_of(xb);
     const S EI = K(KK_EI), RI = K(KK_RI), MI = K(KK_MI), NLI = K(KK_NLOWI), XI = K(KK_XI);
-    const S pXI = pow(X, EI), tI = 1.0 + pXI * RI, PI_ = pow(tI, MI);
+    const S pXI = pow_of(xb, EI), tI = 1.0 + pXI * RI;
+    const PowBase<S> tIb = pow_base(tI);
+    const S PI_ = pow_of(tIb, MI), ltI = ln_of(tIb);
     CoefT<S> c;
     c.jI = pref * NLI * X13 * PI_;
     const S EQ = K(KK_EQ), RQ = K(KK_RQ), MQ = K(KK_MQ), NLQ = K(KK_NLOWQ);
-    const S pXQ = pow(X, EQ), tQ = 1.0 + pXQ * RQ, PQ = pow(tQ, MQ);
+    const S pXQ = pow_of(xb, EQ), tQ = 1.0 + pXQ * RQ;
+    const PowBase<S> tQb = pow_base(tQ);
+    const S PQ = pow_of(tQb, MQ), ltQ = ln_of(tQb);
     c.jQ = -(pref * NLQ * X13 * PQ);
     const S c2 = cth * cth;
     const bool near1 = c2 < 0.5;
     const S ls2 = near1 ? log1p(-c2) : 2.0 * log(sth);
     const S u24 = expm1(-1.2 * ls2), u25 = expm1(-1.25 * ls2), u228 = expm1(-1.14 * ls2), u205 = expm1(-1.025 * ls2);
-    const S Xm035 = pow(X, -0.35), sX = sqrt(X);
+    const S Xm035 = pow_of(xb, -0.35), xm = fdiv(S(1.0), S(sqrt(X)));
     const S CV1 = K(KK_CV1), CV2 = K(KK_CV2);
     const S v48 = pow_nonneg(u24, 0.48), v44 = pow_nonneg(u25, 0.44);
     const S NlowV = CV1 * v48 * Xm035;
-    const S NhighV = CV2 * v44 / sX - small;
+    const S NhighV = CV2 * v44 * xm - small;
     const double sgn = cth > 0.0 ? 1.0 : (cth < 0.0 ? -1.0 : 0.0);
     const bool jv = !(fabs(NhighV) < small * small);
-    S rVr(0.0), pV(0.0), tV(1.0), PV(1.0);
+    S rVr(0.0), lrV(0.0), pV(0.0), tV(1.0), ltV(0.0), PV(1.0);
     if (jv) {
-        rVr = sdiv(NlowV, NhighV); pV = pow(rVr, XI); tV = 1.0 + pXI * pV; PV = pow(tV, MI);
+        rVr = NlowV / NhighV;
+        const PowBase<S> rb = pow_base(rVr);
+        pV = pow_of(rb, XI); lrV = ln_of(rb); tV = 1.0 + pXI * pV;
+        const PowBase<S> tb = pow_base(tV);
+        PV = pow_of(tb, MI); ltV = ln_of(tb);
         c.jV = -(pref * NlowV * X13 * PV) * sgn;
     } else {
         c.jV = S(0.0);
     }
-    const S apref = ne * APRE / sth;
-    const S Xm53 = pow(X, -5.0 / 3.0);
+    const S apref = ne * APRE * ist;
+    const S Xm53 = pow_of(xb, -5.0 / 3.0);
     const S EA = K(KK_EA), RA = K(KK_RA), MA = K(KK_MA), LA = K(KK_LOWA);
-    const S pXA = pow(X, EA), tA = 1.0 + pXA * RA, PA = pow(tA, MA);
+    const S pXA = pow_of(xb, EA), tA = 1.0 + pXA * RA;
+    const PowBase<S> tAb = pow_base(tA);
+    const S PA = pow_of(tAb, MA), ltA = ln_of(tAb);
     c.aI = apref * LA * Xm53 * PA;
     const S EQA = K(KK_EQA), RQA = K(KK_RQA), MQA = K(KK_MQA), NLQA = K(KK_NLOWQA);
-    const S pXQA = pow(X, EQA), tQA = 1.0 + pXQA * RQA, PQA = pow(tQA, MQA);
+    const S pXQA = pow_of(xb, EQA), tQA = 1.0 + pXQA * RQA;
+    const PowBase<S> tQAb = pow_base(tQA);
+    const S PQA = pow_of(tQAb, MQA), ltQA = ln_of(tQAb);
     c.aQ = -(apref * NLQA * Xm53 * PQA);
     const S CVA1 = K(KK_CVA1), CVA2 = K(KK_CVA2), XVA = K(KK_XVA), EVA = K(KK_EVA), MVA = K(KK_MVA);
     const S v446 = pow_nonneg(u228, 0.446), s205 = sqrt(u205);
     const S NlowVA = CVA1 * v446 * Xm035;
-    const S NhighVA = CVA2 * s205 / sX + small;
-    const S rVA = sdiv(NlowVA, NhighVA), pVA = pow(rVA, XVA), pXVA = pow(X, EVA), tVA = 1.0 + pXVA * pVA, PVA = pow(tVA, MVA);
+    const S NhighVA = CVA2 * s205 * xm + small;
+    const S rVA = NlowVA / NhighVA;
+    const PowBase<S> rVAb = pow_base(rVA);
+    const S pVA = pow_of(rVAb, XVA), lrVA = ln_of(rVAb), pXVA = pow_of(xb, EVA), tVA = 1.0 + pXVA * pVA;
+    const PowBase<S> tVAb = pow_base(tVA);
+    const S PVA = pow_of(tVAb, MVA), ltVA = ln_of(tVAb);
     c.aV = -(apref * NlowVA * Xm53 * PVA) * sgn;
     const int i = (int)val(K(KK_IFIT));
-    const S p084 = pow(X, 0.84), xm = 1.0 / sX;
+    const KappaRho k0 = kappa_rho(i), k1 = kappa_rho(i + 1);
+    const S p084 = pow_of(xb, 0.84);
     S hq0, dhq0, hq1, dhq1, hv0, dhv0, hv1, dhv1;
-    kappa_rhoQ_x_d<S>(i, X, p084, hq0, dhq0);
-    kappa_rhoQ_x_d<S>(i + 1, X, p084, hq1, dhq1);
-    kappa_rhoV_x_d<S>(i, xm, hv0, dhv0);
-    kappa_rhoV_x_d<S>(i + 1, xm, hv1, dhv1);
+    kappa_rhoQ_x_d(k0, X, iX, xb, p084, hq0, dhq0);
+    kappa_rhoQ_x_d(k1, X, iX, xb, p084, hq1, dhq1);
+    kappa_rhoV_x_d(k0, xm, hv0, dhv0);
+    kappa_rhoV_x_d(k1, xm, hv1, dhv1);
     const S FQ0 = K(KK_FQ0), FQ1 = K(KK_FQ1), FV0 = K(KK_FV0), FV1 = K(KK_FV1), RHOQ = K(KK_RHOQ), RHOV = K(KK_RHOV);
     const S fQ = FQ0 * hq0 + FQ1 * hq1, fV = FV0 * hv0 + FV1 * hv1;
-    const S inu = 1.0 / nu;
     c.rQ = -(ne * RHOQ * sth * sth) * inu * inu * inu * fQ;
     c.rV = ne * RHOV * cth * inu * inu * fV;
     // ---- the caller's adjoints of the coefficients
@@ -426,7 +437,7 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
     qbar(c, cb);
     const S bjI = cb[0], bjQ = cb[1], bjV = cb[2], baI = cb[3], baQ = cb[4], baV = cb[5], brQ = cb[6], brV = cb[7];
     // ---- reverse
-    S bX(0.0), bs(0.0), bc(0.0), binu(0.0), bpref(0.0), bapref(0.0), bX13(0.0), bXm53(0.0), bXm035(0.0), bsX(0.0), bls2(0.0), bpXI(0.0);
+    S bX(0.0), bs(0.0), bc(0.0), binu(0.0), bpref(0.0), bapref(0.0), bX13(0.0), bXm53(0.0), bXm035(0.0), bxm(0.0), bls2(0.0), bpXI(0.0);
     {   // rV = ne RHOV cth inu^2 fV, rQ = -ne RHOQ sth^2 inu^3 fQ
         const S t = brV * ne, i2 = inu * inu;
         bK[KK_RHOV] += t * cth * i2 * fV;
@@ -439,10 +450,9 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
         binu += u * RHOQ * sth * sth * 3.0 * i2 * fQ;
         const S bfQ = u * RHOQ * sth * sth * i3;
         bK[KK_FV0] += bfV * hv0; bK[KK_FV1] += bfV * hv1;
-        const S bxm = bfV * (FV0 * dhv0 + FV1 * dhv1);
+        bxm += bfV * (FV0 * dhv0 + FV1 * dhv1);
         bK[KK_FQ0] += bfQ * hq0; bK[KK_FQ1] += bfQ * hq1;
         bX += bfQ * (FQ0 * dhq0 + FQ1 * dhq1);
-        bsX += bxm * (-(xm * xm));
     }
     {   // aV = -sgn apref NlowVA Xm53 PVA
         const S g0 = -(baV * sgn);
@@ -450,18 +460,19 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
         S bNlowVA = g0 * apref * Xm53 * PVA;
         bXm53 += g0 * apref * NlowVA * PVA;
         const S bPVA = g0 * apref * NlowVA * Xm53;
-        const S btVA = bPVA * MVA * PVA / tVA;
-        bK[KK_MVA] += bPVA * PVA * log(tVA);
+        const S btVA = fdiv(bPVA * MVA * PVA, tVA);
+        bK[KK_MVA] += bPVA * PVA * ltVA;
         const S bpXVA = btVA * pVA, bpVA = btVA * pXVA;
-        bX += bpXVA * EVA * pXVA / X;
+        bX += bpXVA * EVA * pXVA * iX;
         bK[KK_EVA] += bpXVA * pXVA * lX;
         S brVA(0.0);
-        if (rVA > 0.0) { brVA = sdiv(bpVA * XVA * pVA, rVA); bK[KK_XVA] += bpVA * pVA * log(rVA); }
-        bNlowVA += sdiv(brVA, NhighVA);
-        const S bNhighVA = -sdiv(brVA * rVA, NhighVA);
-        bK[KK_CVA2] += bNhighVA * s205 / sX;
-        const S bs205 = bNhighVA * CVA2 / sX;
-        bsX += -(bNhighVA * CVA2 * s205 / (sX * sX));
+        if (rVA > 0.0) { brVA = bpVA * XVA * pVA / rVA; bK[KK_XVA] += bpVA * pVA * lrVA; }
+        const S bn = brVA / NhighVA;
+        bNlowVA += bn;
+        const S bNhighVA = -(bn * rVA);
+        bK[KK_CVA2] += bNhighVA * s205 * xm;
+        const S bs205 = bNhighVA * CVA2 * xm;
+        bxm += bNhighVA * CVA2 * s205;
         const S bu205 = s205 > 0.0 ? bs205 * 0.5 / s205 : S(0.0);
         bK[KK_CVA1] += bNlowVA * v446 * Xm035;
         const S bv446 = bNlowVA * CVA1 * Xm035;
@@ -475,43 +486,44 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
         bK[KK_NLOWQA] += g0 * apref * Xm53 * PQA;
         bXm53 += g0 * apref * NLQA * PQA;
         const S bPQA = g0 * apref * NLQA * Xm53;
-        const S btQA = bPQA * MQA * PQA / tQA;
-        bK[KK_MQA] += bPQA * PQA * log(tQA);
+        const S btQA = fdiv(bPQA * MQA * PQA, tQA);
+        bK[KK_MQA] += bPQA * PQA * ltQA;
         const S bpXQA = btQA * RQA;
         bK[KK_RQA] += btQA * pXQA;
-        bX += bpXQA * EQA * pXQA / X;
+        bX += bpXQA * EQA * pXQA * iX;
         bK[KK_EQA] += bpXQA * pXQA * lX;
         bapref += baI * LA * Xm53 * PA;
         bK[KK_LOWA] += baI * apref * Xm53 * PA;
         bXm53 += baI * apref * LA * PA;
         const S bPA = baI * apref * LA * Xm53;
-        const S btA = bPA * MA * PA / tA;
-        bK[KK_MA] += bPA * PA * log(tA);
+        const S btA = fdiv(bPA * MA * PA, tA);
+        bK[KK_MA] += bPA * PA * ltA;
         const S bpXA = btA * RA;
         bK[KK_RA] += btA * pXA;
-        bX += bpXA * EA * pXA / X;
+        bX += bpXA * EA * pXA * iX;
         bK[KK_EA] += bpXA * pXA * lX;
     }
-    bX += bXm53 * (-5.0 / 3.0) * Xm53 / X;
-    bK[KK_APRE] += bapref * ne / sth;
-    bs += -(bapref * apref / sth);
+    bX += bXm53 * (-5.0 / 3.0) * Xm53 * iX;
+    bK[KK_APRE] += bapref * ne * ist;
+    bs += -(bapref * apref * ist);
     if (jv) {   // jV = -sgn pref NlowV X13 PV
         const S g0 = -(bjV * sgn);
         bpref += g0 * NlowV * X13 * PV;
         S bNlowV = g0 * pref * X13 * PV;
         bX13 += g0 * pref * NlowV * PV;
         const S bPV = g0 * pref * NlowV * X13;
-        const S btV = bPV * MI * PV / tV;
-        bK[KK_MI] += bPV * PV * log(tV);
+        const S btV = fdiv(bPV * MI * PV, tV);
+        bK[KK_MI] += bPV * PV * ltV;
         bpXI += btV * pV;
         const S bpV = btV * pXI;
         S brV(0.0);
-        if (rVr > 0.0) { brV = sdiv(bpV * XI * pV, rVr); bK[KK_XI] += bpV * pV * log(rVr); }
-        bNlowV += sdiv(brV, NhighV);
-        const S bNhighV = -sdiv(brV * rVr, NhighV);
-        bK[KK_CV2] += bNhighV * v44 / sX;
-        const S bv44 = bNhighV * CV2 / sX;
-        bsX += -(bNhighV * CV2 * v44 / (sX * sX));
+        if (rVr > 0.0) { brV = bpV * XI * pV / rVr; bK[KK_XI] += bpV * pV * lrV; }
+        const S bn = brV / NhighV;
+        bNlowV += bn;
+        const S bNhighV = -(bn * rVr);
+        bK[KK_CV2] += bNhighV * v44 * xm;
+        const S bv44 = bNhighV * CV2 * xm;
+        bxm += bNhighV * CV2 * v44;
         const S bu25 = u25 > 0.0 ? bv44 * 0.44 * v44 / u25 : S(0.0);
         bK[KK_CV1] += bNlowV * v48 * Xm035;
         const S bv48 = bNlowV * CV1 * Xm035;
@@ -519,38 +531,39 @@ KS_DEV CoefT<S> kappa_coefs_rev(const KF& K, S ne, S nu, S sth, S cth, QBar&& qb
         const S bu24 = u24 > 0.0 ? bv48 * 0.48 * v48 / u24 : S(0.0);
         bls2 += bu25 * (-1.25) * (u25 + 1.0) + bu24 * (-1.2) * (u24 + 1.0);
     }
-    bX += bsX * 0.5 / sX + bXm035 * (-0.35) * Xm035 / X;
+    bX += (bxm * (-0.5) * xm + bXm035 * (-0.35) * Xm035) * iX;
     if (near1) bc += bls2 * (-2.0) * cth / (1.0 - c2);
-    else bs += bls2 * 2.0 / sth;
+    else bs += bls2 * 2.0 * ist;
     {   // jQ = -pref NLQ X13 PQ, jI = pref NLI X13 PI
         const S g0 = -bjQ;
         bpref += g0 * NLQ * X13 * PQ;
         bK[KK_NLOWQ] += g0 * pref * X13 * PQ;
         bX13 += g0 * pref * NLQ * PQ;
         const S bPQ = g0 * pref * NLQ * X13;
-        const S btQ = bPQ * MQ * PQ / tQ;
-        bK[KK_MQ] += bPQ * PQ * log(tQ);
+        const S btQ = fdiv(bPQ * MQ * PQ, tQ);
+        bK[KK_MQ] += bPQ * PQ * ltQ;
         const S bpXQ = btQ * RQ;
         bK[KK_RQ] += btQ * pXQ;
-        bX += bpXQ * EQ * pXQ / X;
+        bX += bpXQ * EQ * pXQ * iX;
         bK[KK_EQ] += bpXQ * pXQ * lX;
         bpref += bjI * NLI * X13 * PI_;
         bK[KK_NLOWI] += bjI * pref * X13 * PI_;
         bX13 += bjI * pref * NLI * PI_;
         const S bPI = bjI * pref * NLI * X13;
-        const S btI = bPI * MI * PI_ / tI;
-        bK[KK_MI] += bPI * PI_ * log(tI);
+        const S btI = fdiv(bPI * MI * PI_, tI);
+        bK[KK_MI] += bPI * PI_ * ltI;
         bpXI += btI * RI;
         bK[KK_RI] += btI * pXI;
     }
-    bX += bpXI * EI * pXI / X;
+    bX += bpXI * EI * pXI * iX;
     bK[KK_EI] += bpXI * pXI * lX;
-    bX += bX13 * X13 / (3.0 * X);
+    bX += bX13 * X13 * (1.0 / 3.0) * iX;
     bK[KK_JPRE] += bpref * ne * sth;
     bs += bpref * ne * JPRE;
-    bnu = bX * X / nu + binu * (-(inu * inu));
-    bK[KK_NUW1] += -(bX * X / NUW1);
-    bs += -(bX * X / sth);
+    const S bXX = bX * X;
+    bnu = bXX * inu + binu * (-(inu * inu));
+    bK[KK_INUW1] += bX * nu * ist;
+    bs += -(bXX * ist);
     bsth = floored ? S(0.0) : bs;
     bcth = bc;
     return c;
@@ -567,17 +580,15 @@ template <class S>
 KS_DEV void element_adjoint_kappa(const SplatCT<S>& c, const SplatAdjT<S>& sa, const GeoT<S>& G, S a, S alpha, S beta, S thetao_sin,
                                   S nu, const S bars[11], S Gw, const S dl[13], S grad[22]) {
     const S uv[3] = {c.u[0], c.u[1], c.u[2]};
-    const FrameJ<S> fr = frame_jacobian(G, a, alpha, beta, thetao_sin, uv, sa.sthB, sa.cthB, sa.sphB, sa.cphB);
-    const S nuf = nu / fr.g;
+    const FrameJ<S> fr = frame_jacobian(G, a, alpha, beta, thetao_sin, uv, c.gam, c.q, sa.sthB, sa.cthB, sa.sphB, sa.cphB);
+    const S nh = nu * (1.0 / NU0) * fr.ig, inh = NU0 / nu * fr.g, nuf = nh * NU0, inu = inh * (1.0 / NU0);
     const bool clipped = !(fr.cosB > -1.0 && fr.cosB < 1.0);
     const S cb = dmin(dmax(fr.cosB, -1.0), 1.0);
     S sth, cth;
     pitch_sincos(cb, sth, cth);
-    const S ne = exp(c.lnA) * Gw;
-    const S nh = nuf * (1.0 / NU0);
-    const S i2 = 1.0 / (nh * nh);
-    S s2c, c2c;
-    sincos(2.0 * fr.chi, &s2c, &c2c);
+    const S ne = splat_density(c) * Gw;
+    const S i2 = inh * inh;
+    const S s2c = fr.s2, c2c = fr.c2;
     S q(0.0), qchi(0.0), bnh(0.0);
     bool on = true;
     // q = i2 (b0 jI + fe (b3 jV + Bj jQ)) + nh (b4 aI + fa (b7 aV + Ba aQ) + b10 rV + Br rQ), with the caps fe, fa
@@ -600,7 +611,7 @@ KS_DEV void element_adjoint_kappa(const SplatCT<S>& c, const SplatAdjT<S>& sa, c
         cbar[5] = nh * (fa * bars[7] + Wa * dfa[2]);
         cbar[6] = nh * Br;
         cbar[7] = nh * bars[10];
-        bnh = -2.0 * i2 / nh * qj + qa;
+        bnh = -2.0 * (i2 * inh) * qj + qa;
         // d q / d chi: the cos 2chi, sin 2chi parts
         const S Bc = bars[1] * fe * cf.jQ * i2 + bars[5] * fa * cf.aQ * nh + bars[8] * cf.rQ * nh;
         const S Bs = bars[2] * fe * cf.jQ * i2 + bars[6] * fa * cf.aQ * nh + bars[9] * cf.rQ * nh;
@@ -609,13 +620,13 @@ KS_DEV void element_adjoint_kappa(const SplatCT<S>& c, const SplatAdjT<S>& sa, c
     S bK[KK_N];
     for (int f = 0; f < KK_N; ++f) bK[f] = S(0.0);
     S bnu, bsth, bcth;
-    kappa_coefs_rev(KappaGet<S>{c.kk}, ne, nuf, sth, cth, qbar, bK, bnu, bsth, bcth);
+    kappa_coefs_rev(FactorGet<S>{c.kk}, ne, nuf, inu, sth, cth, qbar, bK, bnu, bsth, bcth);
     if (!on) return;
     S dk(0.0), dw(0.0), dB(0.0);
     for (int f = 0; f < KK_N; ++f) { dk += bK[f] * sa.dkk[0][f]; dw += bK[f] * sa.dkk[1][f]; dB += bK[f] * sa.dkk[2][f]; }
     // nu_f = nu / g: d/dg = -(nu_f / g) d/dnu_f; cos B: cth = cb, sth = sqrt((1 - cb)(1 + cb))
     const S dnuf = bnu + bnh * (1.0 / NU0);
-    const S dg = -(dnuf * nuf / fr.g);
+    const S dg = -(dnuf * nuf * fr.ig);
     const S dcb = clipped ? S(0.0) : bcth + (sth > 0.0 ? bsth * (-(cb / sth)) : S(0.0));
     const S sv = q;
     for (int r = 0; r < 12; ++r) grad[r] += sv * dl[r];
@@ -636,27 +647,20 @@ template <class S>
 KS_DEV void element_adjoint_pop(const SplatCT<S>& c, const SplatAdjT<S>& sa, const GeoT<S>& G, S a, S alpha, S beta, S thetao_sin,
                                 S nu, const S bars[11], S Gw, const S dl[13], S grad[22]) {
     const S uv[3] = {c.u[0], c.u[1], c.u[2]};
-    const FrameJ<S> fr = frame_jacobian(G, a, alpha, beta, thetao_sin, uv, sa.sthB, sa.cthB, sa.sphB, sa.cphB);
+    const FrameJ<S> fr = frame_jacobian(G, a, alpha, beta, thetao_sin, uv, c.gam, c.q, sa.sthB, sa.cthB, sa.sphB, sa.cphB);
     using D5 = DN<5, S>;
-    D5 Bm(c.Bmag); Bm.d[2] = c.Bmag;
     const D5 g = D5::seed(fr.g, 3), cosB = D5::seed(fr.cosB, 4);
-    D5 nuf = nu / g;
+    D5 nh(nu * (1.0 / NU0) * fr.ig), inh = (NU0 / nu) * g;
+    nh.d[3] = -(nh.v * fr.ig);
     D5 cb = dmin(dmax(cosB, -1.0), 1.0);
     D5 sth, cth;
     pitch_sincos(cb, sth, cth);
-    const D5 ne(exp(c.lnA) * Gw);
-    CoefT<D5> cf;
-    const D5 p = D5::seed(c.p1, 0);
-    D5 gmin(c.p2); gmin.d[1] = c.p2;
-    D5 gPL[2];
-    for (int k = 0; k < 2; ++k) { gPL[k] = D5(c.g[k]); gPL[k].d[0] = sa.dpop[k]; }
-    cf = powerlaw(ne, p, gmin, D5(c.p3), gPL, Bm, nuf, sth, cth);
+    const S ne = splat_density(c) * Gw;
+    const CoefT<D5> cf = power_coefs(FactorDual<S>{c.kk, sa}, ne, nh * NU0, inh * (1.0 / NU0), sth, cth);
     if (!(cf.jI > 0.0 || cf.aI > 0.0 || cf.rQ.v != 0.0 || cf.rV.v != 0.0)) return;
     D5 fe = cap_factor(cf.jI, cf.jQ, cf.jV), fa = cap_factor(cf.aI, cf.aQ, cf.aV);
-    D5 nh = nuf * (1.0 / NU0);
-    D5 i2 = 1.0 / (nh * nh);
-    S s2c, c2c;
-    sincos(2.0 * fr.chi, &s2c, &c2c);
+    D5 i2 = inh * inh;
+    const S s2c = fr.s2, c2c = fr.c2;
     D5 jQ = fe * cf.jQ * i2, aQ = fa * cf.aQ * nh, rQ = cf.rQ * nh;
     D5 A = bars[0] * (cf.jI * i2) + bars[3] * (fe * cf.jV * i2) + bars[4] * (cf.aI * nh) + bars[7] * (fa * cf.aV * nh) + bars[10] * (cf.rV * nh);
     D5 Bc = bars[1] * jQ + bars[5] * aQ + bars[8] * rQ;

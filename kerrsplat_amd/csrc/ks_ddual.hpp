@@ -35,26 +35,23 @@ KS_DEV double val(f32 x) { return (double)x.v; }
 KSF_BIN(+)
 KSF_BIN(-)
 KSF_BIN(*)
+KSF_BIN(/)
 #undef KSF_BIN
 // Division by the hardware reciprocal (v_rcp_f32, one ulp), one step on the residual, and v_div_fixup_f32 for zeros and
 // infinities: 5 instructions and correctly rounded but for rare last bits, where the compiler's division takes 9 for 2.5
-// ulp (it scales the operands for divisors below 1.2e-38 or above 8.5e37; where one can occur, sdiv is taken). The FP32
-// images of 64 x 56 x 400 rays are 25 % closer to the FP64 images (kappa 9.7e-7 -> 7.3e-7 of their norm, thermal
-// 1.11e-6 -> 9.3e-7); 1024 kappa splats at 256^2 x 1024, MI355X: adjoint pass 225.8 -> 216.5 ms, transfer
-// 189.4 -> 184.1 ms. Without the residual step the adjoint takes 202.8 ms, with errors as before.
-KS_DEV float hw_div(float a, float b) {
+// ulp (it scales the operands for divisors below 1.2e-38 or above 8.5e37). For the kappa and power-law fits and the duals: 1024 kappa
+// splats at 256^2 x 1024, MI355X: adjoint pass 225.8 -> 216.5 ms, transfer 189.4 -> 184.1 ms, the image of 64 kappa splats
+// 25 % closer to FP64. Without the residual step the adjoint takes 202.8 ms, with errors as before. The thermal fits and
+// the frames keep the operator: their rho_V turns the polarisation by up to thousands of radians.
+KS_DEV f32 fdiv(f32 a, f32 b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const float r = __builtin_amdgcn_rcpf(b), q = a * r;
-    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-b, q, a), r, q), b, a);
+    const float r = __builtin_amdgcn_rcpf(b.v), q = a.v * r;
+    return f32(__builtin_amdgcn_div_fixupf(fmaf(fmaf(-b.v, q, a.v), r, q), b.v, a.v));
 #else
-    return a / b;
+    return f32(a.v / b.v);
 #endif
 }
-KS_DEV f32 operator/(f32 a, f32 b) { return f32(hw_div(a.v, b.v)); }
-KS_DEV f32 operator/(f32 a, double b) { return f32(a.v * (float)(1.0 / b)); }
-KS_DEV f32 operator/(double a, f32 b) { return f32(hw_div((float)a, b.v)); }
-KS_DEV f32 sdiv(f32 a, f32 b) { return f32(a.v / b.v); }
-KS_DEV double sdiv(double a, double b) { return a / b; }
+KS_DEV double fdiv(double a, double b) { return a / b; }
 #define KSF_CMP(op)                                                                                \
     KS_DEV bool operator op(f32 a, f32 b) { return a.v op b.v; }                                   \
     KS_DEV bool operator op(f32 a, double b) { return a.v op (float)b; }                           \
@@ -151,6 +148,9 @@ template <int N, class S = double> struct DN {
     KS_DEV static DN seed(S x, int k) { DN r; r.v = x; for (int i = 0; i < N; ++i) r.d[i] = S(0.0); r.d[k] = S(1.0); return r; }
 };
 template <int N, class S> KS_DEV double val(const DN<N, S>& x) { return val(x.v); }
+KS_DEV double base(double x) { return x; }
+KS_DEV f32 base(f32 x) { return x; }
+template <int N, class S> KS_DEV S base(const DN<N, S>& x) { return x.v; }
 
 #define KSDD_T template <int N, class S>
 #define KSDD_LOOP _Pragma("unroll") for (int i = 0; i < N; ++i)
@@ -159,12 +159,12 @@ KSDD_T KS_DEV DN<N, S> operator-(const DN<N, S>& a, const DN<N, S>& b) { DN<N, S
 KSDD_T KS_DEV DN<N, S> operator*(const DN<N, S>& a, const DN<N, S>& b) { DN<N, S> r; r.v = a.v * b.v; KSDD_LOOP r.d[i] = a.d[i] * b.v + a.v * b.d[i]; return r; }
 // one reciprocal per dual division (the value then carries at most one more rounding)
 KSDD_T KS_DEV DN<N, S> operator/(const DN<N, S>& a, const DN<N, S>& b) {
-    DN<N, S> r; const S ib = 1.0 / b.v; r.v = a.v * ib;
+    DN<N, S> r; const S ib = fdiv(S(1.0), b.v); r.v = a.v * ib;
     KSDD_LOOP r.d[i] = (a.d[i] - r.v * b.d[i]) * ib;
     return r;
 }
-KSDD_T KS_DEV DN<N, S> sdiv(const DN<N, S>& a, const DN<N, S>& b) {
-    DN<N, S> r; const S ib = sdiv(S(1.0), b.v); r.v = a.v * ib;
+KSDD_T KS_DEV DN<N, S> fdiv(const DN<N, S>& a, const DN<N, S>& b) {
+    DN<N, S> r; const S ib = fdiv(S(1.0), b.v); r.v = a.v * ib;
     KSDD_LOOP r.d[i] = (a.d[i] - r.v * b.d[i]) * ib;
     return r;
 }
@@ -175,7 +175,7 @@ KSDD_T KS_DEV DN<N, S> operator-(double a, const DN<N, S>& b) { DN<N, S> r; r.v 
 KSDD_T KS_DEV DN<N, S> operator*(const DN<N, S>& a, double b) { DN<N, S> r; r.v = a.v * b; KSDD_LOOP r.d[i] = a.d[i] * b; return r; }
 KSDD_T KS_DEV DN<N, S> operator*(double a, const DN<N, S>& b) { return b * a; }
 KSDD_T KS_DEV DN<N, S> operator/(const DN<N, S>& a, double b) { return a * (1.0 / b); }
-KSDD_T KS_DEV DN<N, S> operator/(double a, const DN<N, S>& b) { DN<N, S> r; const S ib = 1.0 / b.v; r.v = a * ib; const S f = -r.v * ib; KSDD_LOOP r.d[i] = f * b.d[i]; return r; }
+KSDD_T KS_DEV DN<N, S> operator/(double a, const DN<N, S>& b) { DN<N, S> r; const S ib = fdiv(S(1.0), b.v); r.v = a * ib; const S f = -r.v * ib; KSDD_LOOP r.d[i] = f * b.d[i]; return r; }
 KSDD_T KS_DEV DN<N, S> operator-(const DN<N, S>& a) { DN<N, S> r; r.v = -a.v; KSDD_LOOP r.d[i] = -a.d[i]; return r; }
 KSDD_T KS_DEV DN<N, S>& operator+=(DN<N, S>& a, const DN<N, S>& b) { a = a + b; return a; }
 KSDD_T KS_DEV DN<N, S>& operator*=(DN<N, S>& a, const DN<N, S>& b) { a = a * b; return a; }
@@ -247,11 +247,11 @@ KSDD_T KS_DEV DN<N, S> atan2(const DN<N, S>& y, const DN<N, S>& x) {
 // d x^y / dx = y x^y / x: one power per dual power (x^(y - 1) is taken only at x = 0)
 KSDD_T KS_DEV DN<N, S> pow(const DN<N, S>& x, double y) {
     const S p = pow(x.v, y);
-    return chain(p, y == 0.0 ? S(0.0) : (x.v != 0.0 ? sdiv(S(y * p), x.v) : S(y * pow(x.v, y - 1.0))), x);
+    return chain(p, y == 0.0 ? S(0.0) : (x.v != 0.0 ? S(y * p / x.v) : S(y * pow(x.v, y - 1.0))), x);
 }
 KSDD_T KS_DEV DN<N, S> pow(const DN<N, S>& x, const DN<N, S>& y) {
     const S p = pow(x.v, y.v);
-    const S dx = y.v == 0.0 ? S(0.0) : (x.v != 0.0 ? sdiv(S(y.v * p), x.v) : S(y.v * pow(x.v, y.v - 1.0)));
+    const S dx = y.v == 0.0 ? S(0.0) : (x.v != 0.0 ? S(y.v * p / x.v) : S(y.v * pow(x.v, y.v - 1.0)));
     const S dy = x.v > 0.0 ? S(p * log(x.v)) : S(0.0);
     DN<N, S> r; r.v = p;
     KSDD_LOOP r.d[i] = dx * x.d[i] + dy * y.d[i];

@@ -56,7 +56,7 @@ KS_DEV S splat_weight(const SplatCT<S>& sc, const S* __restrict__ knots, const S
         gexp = gauss_exponent(sc, t, x, y, z, sph, cph);
     }
     if (gexp > GEXP_SKIP) return S(0.0);
-    const S G_ = exp(-0.5 * gexp);
+    const S G_ = fexp(-0.5 * gexp);
     return G_ > WEIGHT_CUTOFF ? G_ : S(0.0);
 }
 
@@ -64,8 +64,8 @@ KS_DEV S splat_weight(const SplatCT<S>& sc, const S* __restrict__ knots, const S
 // rho (c[8..10]) in screen axes; false when it has none (element and screen_coefficients, transport.jl:223-276).
 template <int KIND, class S>
 KS_DEV bool splat_contribution(const SplatCT<S>& sc, const GeoT<S>& G, S aS, S alpha, S beta, S thetao_sin, S nu, S G_, S c[11]) {
-    const FrameT<S> fr = local_frame(G, aS, alpha, beta, thetao_sin, sc.u, sc.bh);
-    const S nuf = nu / fr.g;
+    const FrameT<S> fr = local_frame(G, aS, alpha, beta, thetao_sin, nu, sc.u, sc.gam, sc.q, sc.bh);
+    const S nh = fr.nh, inh = fr.inh;
     const S cb = dmin(dmax(fr.cosB, -1.0), 1.0);
     S sth, cth;
     // FP64 takes cos = cb and the product form of the sine; the FP32 path keeps acos and sincos: with the
@@ -74,19 +74,18 @@ KS_DEV bool splat_contribution(const SplatCT<S>& sc, const GeoT<S>& G, S aS, S a
     // accuracy alone does not explain
     if constexpr (std::is_same<S, double>::value) pitch_sincos(cb, sth, cth);
     else sincos(acos(cb), &sth, &cth);
-    const S ne = exp(sc.lnA) * G_;
+    const S ne = splat_density(sc) * G_;
+    const S nuf = fr.nu, inu = inh * (1.0 / NU0);
     CoefT<S> cf;
-    if constexpr (KIND == MODEL_THERMAL || KIND == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
-    else if constexpr (KIND == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
-    else if constexpr (KIND == MODEL_KAPPA) cf = kappa_coefs(KappaGet<S>{sc.kk}, ne, nuf, sth, cth);
-    else if (sc.kind == MODEL_THERMAL || sc.kind == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
-    else if (sc.kind == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
-    else cf = kappa_coefs(KappaGet<S>{sc.kk}, ne, nuf, sth, cth);
+    if constexpr (KIND == MODEL_THERMAL || KIND == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.g[0], sc.p2, sc.p3, sc.Bmag, fr.nu, nh, inh, sth, cth);
+    else if constexpr (KIND == MODEL_POWERLAW) cf = power_coefs(FactorGet<S>{sc.kk}, ne, nuf, inu, sth, cth);
+    else if constexpr (KIND == MODEL_KAPPA) cf = kappa_coefs(FactorGet<S>{sc.kk}, ne, nuf, inu, sth, cth);
+    else if (sc.kind == MODEL_THERMAL || sc.kind == MODEL_KNOT) cf = thermal(ne, sc.p1, sc.g[0], sc.p2, sc.p3, sc.Bmag, fr.nu, nh, inh, sth, cth);
+    else if (sc.kind == MODEL_POWERLAW) cf = power_coefs(FactorGet<S>{sc.kk}, ne, nuf, inu, sth, cth);
+    else cf = kappa_coefs(FactorGet<S>{sc.kk}, ne, nuf, inu, sth, cth);
     if (!(cf.jI > 0.0 || cf.aI > 0.0 || cf.rQ != 0.0 || cf.rV != 0.0)) return false;
     const S fe = cap_factor(cf.jI, cf.jQ, cf.jV), fa = cap_factor(cf.aI, cf.aQ, cf.aV);
-    const S nh = nuf * (1.0 / NU0);
-    const S i2 = 1.0 / (nh * nh);
-    S s2c, c2c; sincos(2.0 * fr.chi, &s2c, &c2c);
+    const S i2 = inh * inh, s2c = fr.s2, c2c = fr.c2;
     const S jQ = fe * cf.jQ * i2, aQ = fa * cf.aQ * nh, rQ = cf.rQ * nh;
     c[0] = cf.jI * i2; c[1] = jQ * c2c; c[2] = jQ * s2c; c[3] = fe * cf.jV * i2;
     c[4] = cf.aI * nh; c[5] = aQ * c2c; c[6] = aQ * s2c; c[7] = fa * cf.aV * nh;

@@ -12,7 +12,7 @@
 // once per splat on the host instead of at every sample.
 #pragma once
 #include "ks_dgeo.hpp"
-#include "ks_ddual.hpp"
+#include "ks_dfun.hpp"
 
 namespace ksd {
 
@@ -32,7 +32,7 @@ enum ModelKind : int { MODEL_THIN = 0, MODEL_THERMAL = 1, MODEL_POWERLAW = 2, MO
 // The kappa fits' factors that depend on the splat alone (kappa, w, the 2F1 factor, the Gamma values, |B|), built
 // once per splat by kappa_consts; kappa_coefs evaluates the fits at one sample from them. Indices into KappaK::v:
 enum KappaField : int {
-    KK_NUW1,                       // (w kappa)^2 nu_c: nu_w = KK_NUW1 sin(theta), X = nu / nu_w
+    KK_INUW1,                      // 1 / ((w kappa)^2 nu_c): X = nu KK_INUW1 / sin(theta)
     KK_JPRE, KK_APRE,              // e^2 nu_c / c (emissivity prefactor / (n_e sin)), e / B (absorptivity's, x sin / n_e)
     KK_NLOWI, KK_RI, KK_EI, KK_MI, KK_XI,       // N_low; (N_low / N_high)^x; x (3k - 4) / 6; -1 / x; x   (j_I; x_V = x_I)
     KK_NLOWQ, KK_RQ, KK_EQ, KK_MQ,              // j_Q
@@ -45,7 +45,20 @@ enum KappaField : int {
     KK_IFIT,                       // the rotativity fit below kappa (1..3)
     KK_N
 };
+// The power-law fits' factors, in the same places (power_consts):
+enum PowerField : int {
+    PL_INUC, PL_P2,                // 1 / nu_c, -p / 2
+    PL_J, PL_JQ, PL_JV,            // j_I / (n_e sin X^((1 - p)/2)), j_Q / j_I, j_V sin sqrt(X) / (j_I cos)
+    PL_A, PL_AQ, PL_AV,            // alpha_I nu / (n_e X^(-1 - p/2)), alpha_Q / alpha_I, alpha_V's
+    PL_RQ, PL_RG, PL_H, PL_RV,     // rho_Q's, 1 / gamma_min^2, 1 - p / 2, rho_V's
+    PL_N
+};
 template <class T> struct KappaK { T v[KK_N]; };
+static_assert((int)PL_N <= (int)KK_N, "the power-law factors use kappa's places");
+template <class T> struct FactorGet {
+    const KappaK<T>& k;
+    KS_DEV T operator()(int f) const { return k.v[f]; }
+};
 
 // Per-splat constants, built on the host by ks_model_create in both precisions (SplatC, SplatCf);
 // a kernel reads them with wave-uniform addresses.
@@ -61,15 +74,19 @@ template <class S> struct SplatCT {
     S u[3];               // fluid spatial 4-velocity (ZAMO axes)
     S p1, p2, p3;         // thermal: Theta_e, K0/K2, K1/K2 at 1/Theta_e; power law: p, gamma_min, gamma_max;
                           // kappa: kappa, w, hyp
-    S g[6];               // power law: Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12);
+    S g[6];               // thermal: 1 / Theta_e; power law: Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12);
                           // kappa: Gamma(k-4/3), Gamma(k-2), Gamma(k/4-1/3), Gamma(k/4+4/3), Gamma(2+k/2), K0/(K2+1e-40) at 1/w
     S kc[3], kr;          // splats whose centre follows knots: a sphere holding every knot (centre, radius; kr = 0 without)
     S pm0, pm1;           // the FP32 prefilter's error in the splat's scaled coordinates, pm0 + pm1 |t| (may_weigh)
-    KappaK<S> kk;         // kappa: the fits' per-splat factors (kappa_consts)
+    S eA;                 // exp(lnA)
+    S gam, q;             // sqrt(1 + u^2), 1 / (gam + 1)
+    KappaK<S> kk;         // kappa, power law: the fits' per-splat factors (kappa_consts, power_consts)
     int knot0, nk, kt0;   // splats whose centre follows knots (nk > 0): the first of its nk knots (xyz triples) and of their
                           // times in the model's arrays
     int kind;             // the splat's population (MODEL_THERMAL, MODEL_POWERLAW, MODEL_KAPPA, ...)
 };
+// exp(lnA); FP32: of the rounded lnA
+template <class S> KS_DEV S splat_density(const SplatCT<S>& c) { if constexpr (std::is_same<S, f32>::value) return exp(c.lnA); else return c.eA; }
 using SplatC = SplatCT<double>;
 using SplatCf = SplatCT<f32>;
 
@@ -84,31 +101,11 @@ KS_DEV void quasi_cartesian_ks(Q a, Q rp, Q rm, Q r, Q th, Q ph, Q& x, Q& y, Q& 
     x = r * st * cp; y = r * st * sp; z = r * ct;
 }
 
-// sine and cosine of a pattern phase: the phase less its nearest multiple of pi / 2 (two fused steps, exact to 1e-16 up to
-// 1e5 rad; the library beyond), then the Taylor series of both on |r| <= pi / 4, whose first dropped terms are below
-// 1e-19. About 35 instructions against the library's 100, whose large-argument reduction is inlined at every call.
-KS_COLD void sincos_large(double x, double* s, double* c) { ::sincos(x, s, c); }
-KS_DEV void phase_sincos(double x, double* s, double* c) {
-    if (!(::fabs(x) < 1e5)) { sincos_large(x, s, c); return; }
-    const double n = ::rint(x * 0.6366197723675814);
-    const double r = ::fma(-n, 6.123233995736766e-17, ::fma(-n, 1.5707963267948966, x));
-    const double q = r * r;
-    double ps = -1.0 / 6.0 + q * (1.0 / 120.0 + q * (-1.0 / 5040.0 + q * (1.0 / 362880.0 + q * (-1.0 / 39916800.0 +
-                q * (1.0 / 6227020800.0 + q * (-1.0 / 1307674368000.0 + q * (1.0 / 355687428096000.0)))))));
-    double pc = -0.5 + q * (1.0 / 24.0 + q * (-1.0 / 720.0 + q * (1.0 / 40320.0 + q * (-1.0 / 3628800.0 + q * (1.0 / 479001600.0 +
-                q * (-1.0 / 87178291200.0 + q * (1.0 / 20922789888000.0 + q * (-1.0 / 6402373705728000.0))))))));
-    const double sr = ::fma(r * q, ps, r), cr = ::fma(q, pc, 1.0);
-    const int m = (int)n;
-    const double sv = (m & 1) ? cr : sr, cv = (m & 1) ? sr : cr;
-    *s = (m & 2) ? -sv : sv;
-    *c = ((m + 1) & 2) ? -cv : cv;
-}
-
 // centre of a splat at time t under the pattern rotation and the squared distance (for the cull)
 template <class S>
 KS_DEV bool outside_support(const SplatCT<S>& s, S t, S x, S y, S z, S& sp, S& cp) {
     S ph = s.omega * (t - s.t0);
-    sincos(ph, &sp, &cp);
+    phase_sincos(ph, &sp, &cp);
     S cx = s.x * cp - s.y * sp, cy = s.x * sp + s.y * cp;
     S dx = x - cx, dy = y - cy, dz = z - s.z;
     return dx * dx + dy * dy + dz * dz > s.rsup2;
@@ -270,16 +267,27 @@ template <class T> KS_DEV GeoT<T> geo_as(const Geo& g) {
     return o;
 }
 
-template <class T> struct FrameT { T g, cosB, chi; };
+// redshift g, cos B, cosine and sine of twice the screen angle chi; the fluid-frame frequency nu, nh = nu / NU0, inh = 1 / nh
+template <class T> struct FrameT { T g, cosB, c2, s2, nu, nh, inh; };
 using Frame = FrameT<double>;
+template <class T> struct base_scalar { using type = T; };
+template <int N, class S> struct base_scalar<DN<N, S>> { using type = S; };
+// whether T is the FP32 scalar or duals over it. The rotation angles of hot, thin parcels are up to thousands of radians,
+// so a change of 1e-7 in a splat's rho_V (a constant rounded another way) moves an FP32 gradient by 1e-4: what enters
+// rho_V keeps its operations there (ne, g, the thermal fits), and only FP64 takes the shorter forms.
+template <class T> constexpr bool is_fp32 = std::is_same<typename base_scalar<T>::type, f32>::value;
 
-// frames.jl:108-128 for one splat: its boost built from the fluid velocity u, the field direction bh
-// (unit); T = the scalar S of the geometry, or duals over it in u and bh for the adjoint
+// frames.jl:108-128 for one splat: its boost built from the fluid velocity u (FP64: gam = sqrt(1 + u^2) and
+// q = 1 / (gam + 1) from the splat's constants), the field direction bh (unit); T = the scalar S of the geometry, or duals
+// over it. The screen angle chi = atan2(-ea, eb) enters the coefficients through cos 2chi = (eb^2 - ea^2) / (ea^2 + eb^2)
+// and sin 2chi = -2 ea eb / (ea^2 + eb^2), which do not depend on the length of the polarisation vector f: neither its norm
+// nor the angle is taken (atan2 and sincos were 280 instructions of a thermal pair, the norm 40).
 template <class T, class S>
-KS_DEV FrameT<T> local_frame(const GeoT<S>& G, S a, S alpha, S beta, S thetao_sin, const T u[3], const T bh[3]) {
-    T u2 = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-    T gam = sqrt(1.0 + u2);
-    T q = 1.0 / (gam + 1.0);
+KS_DEV FrameT<T> local_frame(const GeoT<S>& G, S a, S alpha, S beta, S thetao_sin, S nu, const T u[3], T gam, T q, const T bh[3]) {
+    if constexpr (is_fp32<T>) {
+        gam = sqrt(1.0 + (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]));
+        q = 1.0 / (gam + 1.0);
+    }
     // p_f = Lambda p_z
     T ud = u[0] * G.pz[1] + u[1] * G.pz[2] + u[2] * G.pz[3];
     T pf0 = gam * G.pz[0] - ud;
@@ -287,13 +295,18 @@ KS_DEV FrameT<T> local_frame(const GeoT<S>& G, S a, S alpha, S beta, S thetao_si
     T pf1 = G.pz[1] + u[0] * c1, pf2 = G.pz[2] + u[1] * c1, pf3 = G.pz[3] + u[2] * c1;
     FrameT<T> fr;
     fr.g = 1.0 / pf0;
+    if constexpr (is_fp32<T>) {
+        fr.nu = nu / fr.g;
+        fr.nh = fr.nu * (1.0 / NU0);
+        fr.inh = 1.0 / fr.nh;
+    } else {
+        fr.nu = nu * pf0;
+        fr.nh = nu * (1.0 / NU0) * pf0;
+        fr.inh = NU0 / nu * fr.g;
+    }
     T k0 = pf1 * fr.g, k1 = pf2 * fr.g, k2 = pf3 * fr.g;
     fr.cosB = k0 * bh[0] + k1 * bh[1] + k2 * bh[2];
     T f0 = k1 * bh[2] - k2 * bh[1], f1 = k2 * bh[0] - k0 * bh[2], f2 = k0 * bh[1] - k1 * bh[0];
-    T fn = sqrt(f0 * f0 + f1 * f1 + f2 * f2);
-    if (!(fn > 0.0)) { fr.chi = T(0.0); return fr; }
-    T ifn = 1.0 / fn;
-    f0 = f0 * ifn; f1 = f1 * ifn; f2 = f2 * ifn;
     // inverse boost of (0, f): time part = u.f, spatial f + u (u.f) q
     T uf = u[0] * f0 + u[1] * f1 + u[2] * f2;
     T ufq = uf * q;
@@ -309,7 +322,11 @@ KS_DEV FrameT<T> local_frame(const GeoT<S>& G, S a, S alpha, S beta, S thetao_si
     T kk1 = A * G.r - Bw * (a * G.ct), kk2 = -(A * (a * G.ct) + Bw * G.r);
     S mu = -(alpha + a * thetao_sin);
     T ea = beta * kk2 - mu * kk1, eb = beta * kk1 + mu * kk2;
-    fr.chi = atan2(-ea, eb);
+    T den = ea * ea + eb * eb;
+    if (den == 0.0) { fr.c2 = T(1.0); fr.s2 = T(0.0); return fr; }     // a photon along the field: chi = 0
+    T w = 1.0 / den;
+    fr.c2 = (eb - ea) * (eb + ea) * w;
+    fr.s2 = -2.0 * ea * eb * w;
     return fr;
 }
 
@@ -331,13 +348,10 @@ template <int N, class S> KS_DEV double sin_floor(const DN<N, S>&) { return sin_
 // cancellation of the difference (which rounds to zero, and leaves the partials of x^e at zero unbounded, when the
 // sine rounds to one); directly elsewhere
 template <class T> KS_DEV T sin_pow_m1(T sth, T cth, double p) {
-    if (cth * cth < 0.5) return expm1((-0.5 * p) * log1p(-(cth * cth)));
-    return pow(sth, -p) - 1.0;
+    const T c2 = cth * cth;
+    if (c2 < 0.5) return expm1((-0.5 * p) * log1p(-c2));
+    return pow_of(pow_base(sth), -p) - 1.0;
 }
-// x^e (0 < e < 1) of x >= 0, zero with zero partials at x = 0, where the derivative is unbounded (the reference's
-// safe_sqrt makes the same choice for the square root, frames.jl:83-97)
-template <class T> KS_DEV T pow_nonneg(T x, double e) { return x > 0.0 ? pow(x, e) : T(0.0); }
-
 template <class T> struct CoefT { T jI, jQ, jV, aI, aQ, aV, rQ, rV; };
 using Coef = CoefT<double>;
 
@@ -349,67 +363,136 @@ template <class T> KS_DEV T planck(T nu, T Th) {
     return pref / expm1(x);
 }
 
-// thermal (coefficients.jl:101-151) with the splat's Bessel ratios k0/k2, k1/k2 (k2 > 0 in practice);
-// ne enters linearly and stays a plain number in the adjoint
+// 1 / B_nu at nu = nh NU0 and h nu / k T = x, inh3 = nh^-3, zero where B_nu underflows
+template <class T> KS_DEV T inv_planck(T x, T inh3) {
+    const T em = x < 2e-3 ? x * (1.0 / 24.0) * (24.0 + x * (12.0 + x * (4.0 + x))) : expm1(x);
+    const T ib = em * inh3 * (1.0 / PLANCK0);
+    return isfinite_(ib) ? ib : T(0.0);
+}
+// cos(x / 2) of the thermal rotativity fit, which multiplies exp(-x^1.2 / 2.73): that factor is zero in FP64 beyond
+// x = 570, so a larger x is taken as 1e4 there
+template <class T> KS_DEV T cos_bounded(const T& x) {
+    T s, c;
+    sincos_small(dmin(x, 1e4) * 0.5, &s, &c);
+    return c;
+}
+
+// thermal (coefficients.jl:101-151) with the splat's Bessel ratios k0/k2, k1/k2 (k2 > 0 in practice) and 1 / Theta_e, at
+// nu = nh NU0, inh = 1 / nh (FP32 takes nu alone, in the operations it had: is_fp32); ne enters linearly and stays a plain number in the adjoint. The powers of x share one
+// logarithm, the four divisions left are nu / nu_s, its cube root's, cos / sin and the logistic's (which takes the place of
+// (1 + tanh) / 2 and is below 1e-21 for x < 10, where the term it multiplies is left out).
 template <class T, class NE>
-KS_DEV CoefT<T> thermal(NE ne, T Th, T k0k2, T k1k2, T B, T nu, T sth, T cth) {
+KS_DEV CoefT<T> thermal(NE ne, T Th, T iTh, T k0k2, T k1k2, T B, T nu, T nh, T inh, T sth, T cth) {
     CoefT<T> c;
-    T w = 2.0 * PI * nu;
-    T w0w = EE * B / (ME * CL) / w;
-    T wp2w2 = (4.0 * PI * ne * EE * EE / ME) / (w * w);
-    if (!(sth > 0.0)) {
-        c.jI = c.jQ = c.jV = c.aI = c.aQ = c.aV = c.rQ = T(0.0);
-        c.rV = w / CL * (wp2w2 * w0w * k0k2 * cth);
+    if constexpr (is_fp32<T>) {
+        T w = 2.0 * PI * nu;
+        T w0w = EE * B / (ME * CL) / w;
+        T wp2w2 = (4.0 * PI * ne * EE * EE / ME) / (w * w);
+        if (!(sth > 0.0)) {
+            c.jI = c.jQ = c.jV = c.aI = c.aQ = c.aV = c.rQ = T(0.0);
+            c.rV = w / CL * (wp2w2 * w0w * k0k2 * cth);
+            return c;
+        }
+        T x = Th * sqrt(1.4142135623730951 * sth * (1e3 * w0w));
+        T lx = log(x);
+        T extraterm = (0.011 * exp(-x / 47.2) - 0.7937005259840998 / 67.44733739010397 * PI * 1e4 * exp(-8.0 / 3.0 * log(x + 1e-16))) *
+                      (0.5 + 0.5 * tanh((lx - 4.787491742782046) / 0.1));
+        T jffunc = 2.011 * exp(-exp(1.035 * lx) / 4.7) - cos(x * 0.5) * exp(-exp(1.2 * lx) / 2.73) - 0.011 * exp(-x / 47.2) + extraterm;
+        T eps11m22 = jffunc * wp2w2 * w0w * w0w * (k1k2 + 6.0 * Th) * sth * sth;
+        c.rQ = w / (2.0 * CL) * eps11m22;
+        T ff = k0k2 * (1.0 - 0.11 * log1p(0.035 * x));
+        c.rV = w / CL * (wp2w2 * w0w * ff * cth);
+        T nus = 3.0 * EE * B * sth / (4.0 * PI * ME * CL) * Th * Th + 1.0;
+        T xs = nu / nus;
+        T x13 = cbrt(xs), xm13 = 1.0 / x13, xm23 = xm13 * xm13;
+        T e = exp(-1.8899 * x13);
+        T pref = ne * EE * EE * nu / (2.0 * 1.7320508075688772 * CL * Th * Th);
+        c.jI = pref * 2.5651 * (1.0 + 1.92 * xm13 + 0.9977 * xm23) * e;
+        c.jQ = pref * 2.5651 * (1.0 + 0.93193 * xm13 + 0.499873 * xm23) * e;
+        c.jV = 2.0 * ne * EE * EE * nu * cth / sth / (3.0 * 1.7320508075688772 * CL * Th * Th * Th) *
+               (1.81384 / xs + 3.42319 * xm23 + 0.0292545 / sqrt(xs) + 2.03773 * xm13) * e;
+        T Bn = planck(nu, Th);
+        T ib = Bn > 0.0 ? 1.0 / Bn : T(0.0);
+        c.aI = c.jI * ib; c.aQ = c.jQ * ib; c.aV = c.jV * ib;
         return c;
     }
-    T x = Th * sqrt(1.4142135623730951 * sth * (1e3 * w0w));
-    T lx = log(x);
-    T extraterm = (0.011 * exp(-x / 47.2) - 0.7937005259840998 / 67.44733739010397 * PI * 1e4 * exp(-8.0 / 3.0 * log(x + 1e-16))) *
-                  (0.5 + 0.5 * tanh((lx - 4.787491742782046) / 0.1));
-    T jffunc = 2.011 * exp(-exp(1.035 * lx) / 4.7) - cos(x * 0.5) * exp(-exp(1.2 * lx) / 2.73) - 0.011 * exp(-x / 47.2) + extraterm;
-    T eps11m22 = jffunc * wp2w2 * w0w * w0w * (k1k2 + 6.0 * Th) * sth * sth;
-    c.rQ = w / (2.0 * CL) * eps11m22;
-    T ff = k0k2 * (1.0 - 0.11 * log1p(0.035 * x));
-    c.rV = w / CL * (wp2w2 * w0w * ff * cth);
-    T nus = 3.0 * EE * B * sth / (4.0 * PI * ME * CL) * Th * Th + 1.0;
-    T xs = nu / nus;
-    T x13 = cbrt(xs), xm13 = 1.0 / x13, xm23 = xm13 * xm13;
-    T e = exp(-1.8899 * x13);
-    T pref = ne * EE * EE * nu / (2.0 * 1.7320508075688772 * CL * Th * Th);
-    c.jI = pref * 2.5651 * (1.0 + 1.92 * xm13 + 0.9977 * xm23) * e;
-    c.jQ = pref * 2.5651 * (1.0 + 0.93193 * xm13 + 0.499873 * xm23) * e;
-    c.jV = 2.0 * ne * EE * EE * nu * cth / sth / (3.0 * 1.7320508075688772 * CL * Th * Th * Th) *
-           (1.81384 / xs + 3.42319 * xm23 + 0.0292545 / sqrt(xs) + 2.03773 * xm13) * e;
-    T Bn = planck(nu, Th);
-    T ib = Bn > 0.0 ? sdiv(T(1.0), Bn) : T(0.0);
+    // omega_p^2 / omega^2 (omega_B / omega) omega / c at nu = NU0 per n_e B, and omega_B / omega per B: the constants of
+    // a product are joined before they are rounded to the scalar (a constant's rounding biases every sample alike)
+    const double W0 = 2.0 * PI * NU0, WB = EE / (ME * CL) / W0, WV = 4.0 * PI * EE * EE / ME / (W0 * CL) * WB;
+    T i2 = inh * inh;
+    T rv = ne * B * i2 * cth * WV;
+    if (!(sth > 0.0)) {
+        c.jI = c.jQ = c.jV = c.aI = c.aQ = c.aV = c.rQ = T(0.0);
+        c.rV = rv * k0k2;
+        return c;
+    }
+    T x = Th * sqrt((1414.2135623730951 * WB) * (sth * B * inh));
+    const PowBase<T> xb = pow_base(x);
+    T e472 = fexp(x * (-1.0 / 47.2));
+    T jffunc = 2.011 * fexp(pow_of(xb, 1.035) * (-1.0 / 4.7)) - cos_bounded(x) * fexp(pow_of(xb, 1.2) * (-1.0 / 2.73)) - 0.011 * e472;
+    if (x > 10.0)
+        jffunc += (0.011 * e472 - 0.7937005259840998 / 67.44733739010397 * PI * 1e4 * pow_of(xb, -8.0 / 3.0)) /
+                  (1.0 + fexp((4.787491742782046 - ln_of(xb)) * 20.0));
+    c.rQ = ne * (0.5 * WV * WB) * (B * B) * (i2 * inh) * (jffunc * (k1k2 + 6.0 * Th)) * (sth * sth);
+    T ff = k0k2 * (1.0 - 0.11 * log1p_pos(0.035 * x));
+    c.rV = rv * ff;
+    T nus = 3.0 * EE / (4.0 * PI * ME * CL) / NU0 * B * sth * Th * Th + 1.0 / NU0;
+    T xs = nh / nus;
+    T x13 = cbrt(xs), xm13 = 1.0 / x13, xm23 = xm13 * xm13, xm1 = xm13 * xm23;
+    T e = fexp(-1.8899 * x13);
+    T pref = ne * (2.5651 * EE * EE * NU0 / (2.0 * 1.7320508075688772 * CL)) * nh * (iTh * iTh);
+    c.jI = pref * (1.0 + 1.92 * xm13 + 0.9977 * xm23) * e;
+    c.jQ = pref * (1.0 + 0.93193 * xm13 + 0.499873 * xm23) * e;
+    c.jV = pref * iTh * (4.0 / 3.0 / 2.5651) * (cth / sth) * (1.81384 * xm1 + 3.42319 * xm23 + 0.0292545 * sqrt(xm1) + 2.03773 * xm13) * e;
+    T ib = inv_planck((HPL * NU0 / (ME * CL * CL)) * nh * iTh, i2 * inh);
     c.aI = c.jI * ib; c.aQ = c.jQ * ib; c.aV = c.jV * ib;
     return c;
 }
 
-// power law (coefficients.jl:208-256); gPL = {Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12)}
+// power law (coefficients.jl:208-256), split as kappa's: its per-splat factors from p, gamma_min, gamma_max and
+// gPL = {Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12)} (power_consts, once per splat), and its
+// evaluation at one sample (power_coefs) from one power X^(-p/2) of X = nu / (nu_c sin), where eleven powers were taken
+// at every pair, seven of them of the splat's numbers alone.
 template <class T>
-KS_DEV CoefT<T> powerlaw(T ne, T p, T gmin, T gmax, const T* gPL, T B, T nu, T sth, T cth) {
+KS_DEV void power_consts(T p, T gmin, T gmax, const T* gPL, T B, KappaK<T>& K) {
+    const T nuc = EE * B / (2.0 * PI * ME * CL);
+    const T gspan = pow(gmin, 1.0 - p) - pow(gmax, 1.0 - p);
+    const T h = 0.5 * p - 1.0, lg = log(gmin);
+    K.v[PL_INUC] = 1.0 / nuc;
+    K.v[PL_P2] = -0.5 * p;
+    K.v[PL_J] = EE * EE * nuc / CL * pow(3.0, p * 0.5) * (p - 1.0) / (2.0 * (p + 1.0) * gspan) * gPL[0];
+    K.v[PL_JQ] = (p + 1.0) / (p + 7.0 / 3.0);
+    K.v[PL_JV] = (171.0 / 250.0) * 1.7320508075688772 * pow(p, 0.49);
+    K.v[PL_A] = EE * EE / (ME * CL) * pow(3.0, (p + 1.0) * 0.5) * (p - 1.0) / (4.0 * gspan) * gPL[1];
+    K.v[PL_AQ] = pow((17.0 / 500.0) * p - 43.0 / 1250.0, 43.0 / 500.0);
+    K.v[PL_AV] = pow(0.71 * p + 22.0 / 625.0, 197.0 / 500.0);
+    const T rp = EE * EE * (p - 1.0) / (ME * CL * nuc * gspan);
+    K.v[PL_RQ] = rp * pow(gmin, 2.0 - p) / h;
+    K.v[PL_RG] = 1.0 / (gmin * gmin);
+    K.v[PL_H] = -h;
+    K.v[PL_RV] = 2.0 * (p + 2.0) / (p + 1.0) * rp * pow(gmin, -(p + 1.0)) * lg;
+}
+template <class T, class NE, class KF>
+KS_DEV CoefT<T> power_coefs(const KF& K, NE ne, T nu, T inu, T sth, T cth) {
     CoefT<T> c;
     if (!(sth > 0.0)) sth = T(sin_floor(sth));
-    T nuc = EE * B / (2.0 * PI * ME * CL);
-    T gspan = pow(gmin, 1.0 - p) - pow(gmax, 1.0 - p);
-    T pref = ne * EE * EE * nuc / CL;
-    T X = nu / (nuc * sth);
-    c.jI = pref * (pow(3.0, p * 0.5) * (p - 1.0) * sth) / (2.0 * (p + 1.0) * gspan) * gPL[0] * pow(X, -(p - 1.0) * 0.5);
-    c.jQ = (p + 1.0) / (p + 7.0 / 3.0) * c.jI;
-    c.jV = (171.0 / 250.0) * pow(p, 0.49) * cth / sth * pow(nu / (3.0 * nuc * sth), -0.5) * c.jI;
-    T apref = ne * EE * EE / (nu * ME * CL);
-    c.aI = apref * pow(3.0, (p + 1.0) * 0.5) * (p - 1.0) / (4.0 * gspan) * gPL[1] * pow(X, -(p + 2.0) * 0.5);
-    c.aQ = c.aI * pow((17.0 / 500.0) * p - 43.0 / 1250.0, 43.0 / 500.0);
-    T term6 = pow_nonneg(3.1 * sin_pow_m1(sth, cth, 48.0 / 25.0), 64.0 / 125.0);
+    const T ist = fdiv(T(1.0), sth);
+    const T X = nu * K(PL_INUC) * ist, iX = fdiv(T(1.0), X), isX = sqrt(iX);
+    const PowBase<T> xb = pow_base(X);
+    const T s = pow_of(xb, K(PL_P2));
+    c.jI = ne * K(PL_J) * sth * (X * isX) * s;
+    c.jQ = K(PL_JQ) * c.jI;
+    c.jV = K(PL_JV) * cth * ist * isX * c.jI;
+    c.aI = ne * inu * K(PL_A) * s * iX;
+    c.aQ = c.aI * K(PL_AQ);
+    const T term6 = pow_nonneg(3.1 * sin_pow_m1(sth, cth, 48.0 / 25.0), 64.0 / 125.0);
     const double sgn = cth > 0.0 ? 1.0 : (cth < 0.0 ? -1.0 : 0.0);
-    c.aV = c.aI * pow(0.71 * p + 22.0 / 625.0, 197.0 / 500.0) * term6 * pow(X, -0.5) * sgn;
-    T nuB = nuc * sth;
-    T rperp = ne * EE * EE * (p - 1.0) / (ME * CL * nuB * gspan);
-    T numin = gmin * gmin * nuB;
-    T rb = nuB / nu;
-    c.rQ = -rperp * rb * rb * rb * pow(gmin, 2.0 - p) * (1.0 - pow(numin / nu, p * 0.5 - 1.0)) / (p * 0.5 - 1.0);
-    c.rV = 2.0 * (p + 2.0) / (p + 1.0) * rperp * rb * rb * pow(gmin, -(p + 1.0)) * log(gmin) * cth / sth;
+    c.aV = c.aI * K(PL_AV) * term6 * isX * sgn;
+    // 1 - (gamma_min^2 nu_B / nu)^(p/2 - 1)
+    const T m = 1.0 - pow_of(pow_base(X * K(PL_RG)), K(PL_H));
+    const T ri = ne * ist * iX * iX;
+    c.rQ = -(ri * K(PL_RQ)) * iX * m;
+    c.rV = ri * K(PL_RV) * cth * ist;
     return c;
 }
 
@@ -419,7 +502,7 @@ template <class T>
 KS_DEV void kappa_consts(T kap, T w, T hyp, const T* gK, T B, KappaK<T>& K) {
     const double small = 1e-40;
     T nuc = EE * B / (2.0 * PI * ME * CL);
-    K.v[KK_NUW1] = (w * kap) * (w * kap) * nuc;
+    K.v[KK_INUW1] = 1.0 / ((w * kap) * (w * kap) * nuc);
     K.v[KK_JPRE] = EE * EE * nuc / CL;
     K.v[KK_APRE] = EE / B;
     T g43 = gK[0], g2 = gK[1], gq = gK[2], gp = gK[3], gk2 = gK[4];
@@ -494,66 +577,72 @@ KS_DEV void kappa_consts(T kap, T w, T hyp, const T* gK, T B, KappaK<T>& K) {
     K.v[KK_RHOV] = 2.0 * EE * EE * nuc / (ME * CL) * gK[5];
     K.v[KK_IFIT] = T((double)i);
 }
-// the X-dependent factors of the rotativity fits n = 1..4 (kappa.jl:72-97); p084 = X^0.84, xm = X^-1/2
-template <class T>
-KS_DEV T kappa_rhoQ_x(int n, T X, T p084) {
-    if (n == 1) return 1.0 - exp(-p084 / 30.0) - sin(X / 10.0) * exp(-1.5 * pow(X, 0.471));
-    if (n == 2) return 1.0 - exp(-p084 / 18.0) - sin(X / 6.0) * exp(-1.75 * sqrt(X));
-    if (n == 3) return 1.0 - exp(-p084 / 12.0) - sin(X / 4.0) * exp(-2.0 * pow(X, 0.525));
-    return 1.0 - exp(-p084 / 8.0) - sin(0.375 * X) * exp(-2.25 * pow(X, 0.541));
+// the X-dependent factors of the rotativity fits n = 1..4 (kappa.jl:72-97); p084 = X^0.84, xm = X^-1/2. Each is
+// 1 - exp(-p084 d) - sin(sd X) exp(-cc X^b): the four share one piece of code, since a wavefront's pairs hold splats of
+// several kappa. The second exponential is zero in FP64 beyond X = 6e5, so a larger phase is taken as 1e5.
+struct KappaRho { double d, sd, cc, b, v; };
+KS_DEV KappaRho kappa_rho(int n) {
+    KappaRho k;
+    k.d = n == 1 ? -1.0 / 30.0 : (n == 2 ? -1.0 / 18.0 : (n == 3 ? -1.0 / 12.0 : -1.0 / 8.0));
+    k.sd = n == 1 ? 1.0 / 10.0 : (n == 2 ? 1.0 / 6.0 : (n == 3 ? 1.0 / 4.0 : 0.375));
+    k.cc = n == 1 ? 1.5 : (n == 2 ? 1.75 : (n == 3 ? 2.0 : 2.25));
+    k.b = n == 1 ? 0.471 : (n == 2 ? 0.5 : (n == 3 ? 0.525 : 0.541));
+    k.v = n == 1 ? 0.447 : (n == 2 ? 0.391 : (n == 3 ? 0.348 : 0.313));
+    return k;
 }
 template <class T>
-KS_DEV T kappa_rhoV_x(int n, T xm) {
-    const double b = n == 1 ? 0.447 : (n == 2 ? 0.391 : (n == 3 ? 0.348 : 0.313));
-    return 1.0 - 0.17 * log1p(b * xm);
+KS_DEV T kappa_rhoQ_x(const KappaRho& k, const T& X, const PowBase<T>& xb, const T& p084) {
+    T s, c;
+    sincos_small(dmin(X * k.sd, 1e5), &s, &c);
+    return 1.0 - fexp(p084 * k.d) - s * fexp(-k.cc * pow_of(xb, k.b));
 }
+template <class T> KS_DEV T kappa_rhoV_x(const KappaRho& k, const T& xm) { return 1.0 - 0.17 * log1p_pos(k.v * xm); }
 // One sample's kappa coefficients from the splat's factors: K(f) gives factor f (a value, or a dual carrying its
-// partials in the splat's rows); ne the density, nu the fluid-frame frequency, (sth, cth) the pitch angle.
+// partials in the splat's rows); ne the density, nu the fluid-frame frequency (inu = 1 / nu), (sth, cth) the pitch angle.
 template <class T, class KF>
-KS_DEV CoefT<T> kappa_coefs(const KF& K, T ne, T nu, T sth, T cth) {
+KS_DEV CoefT<T> kappa_coefs(const KF& K, T ne, T nu, T inu, T sth, T cth) {
     CoefT<T> c;
     if (!(sth > 0.0)) sth = T(sin_floor(sth));
     const double small = 1e-40;
-    T X = nu / (K(KK_NUW1) * sth);
+    const T ist = fdiv(T(1.0), sth);
+    T X = nu * K(KK_INUW1) * ist;
+    const PowBase<T> xb = pow_base(X);
     T pref = ne * K(KK_JPRE) * sth;
     T X13 = cbrt(X);
-    T pXI = pow(X, K(KK_EI));
-    c.jI = pref * K(KK_NLOWI) * X13 * pow(1.0 + pXI * K(KK_RI), K(KK_MI));
-    c.jQ = -(pref * K(KK_NLOWQ) * X13 * pow(1.0 + pow(X, K(KK_EQ)) * K(KK_RQ), K(KK_MQ)));
+    T pXI = pow_of(xb, K(KK_EI));
+    c.jI = pref * K(KK_NLOWI) * X13 * pow_of(pow_base(1.0 + pXI * K(KK_RI)), K(KK_MI));
+    c.jQ = -(pref * K(KK_NLOWQ) * X13 * pow_of(pow_base(1.0 + pow_of(xb, K(KK_EQ)) * K(KK_RQ)), K(KK_MQ)));
     // the sin^-p - 1 factors from one logarithm of sin^2 (sin_pow_m1)
     T ls2 = cth * cth < 0.5 ? log1p(-(cth * cth)) : 2.0 * log(sth);
-    T Xm035 = pow(X, -0.35), sX = sqrt(X);
+    T Xm035 = pow_of(xb, -0.35), xm = fdiv(T(1.0), T(sqrt(X)));
     T NlowV = K(KK_CV1) * pow_nonneg(expm1(-1.2 * ls2), 0.48) * Xm035;
-    T NhighV = K(KK_CV2) * pow_nonneg(expm1(-1.25 * ls2), 0.44) / sX - small;
+    T NhighV = K(KK_CV2) * pow_nonneg(expm1(-1.25 * ls2), 0.44) * xm - small;
     const double sgn = cth > 0.0 ? 1.0 : (cth < 0.0 ? -1.0 : 0.0);
     c.jV = fabs(NhighV) < small * small ? T(0.0)
-         : -(pref * NlowV * X13 * pow(1.0 + pXI * pow(sdiv(NlowV, NhighV), K(KK_XI)), K(KK_MI))) * sgn;
-    T apref = ne * K(KK_APRE) / sth;
-    T Xm53 = pow(X, -5.0 / 3.0);
-    c.aI = apref * K(KK_LOWA) * Xm53 * pow(1.0 + pow(X, K(KK_EA)) * K(KK_RA), K(KK_MA));
-    c.aQ = -(apref * K(KK_NLOWQA) * Xm53 * pow(1.0 + pow(X, K(KK_EQA)) * K(KK_RQA), K(KK_MQA)));
+         : -(pref * NlowV * X13 * pow_of(pow_base(1.0 + pXI * pow_of(pow_base(NlowV / NhighV), K(KK_XI))), K(KK_MI))) * sgn;
+    T apref = ne * K(KK_APRE) * ist;
+    T Xm53 = pow_of(xb, -5.0 / 3.0);
+    c.aI = apref * K(KK_LOWA) * Xm53 * pow_of(pow_base(1.0 + pow_of(xb, K(KK_EA)) * K(KK_RA)), K(KK_MA));
+    c.aQ = -(apref * K(KK_NLOWQA) * Xm53 * pow_of(pow_base(1.0 + pow_of(xb, K(KK_EQA)) * K(KK_RQA)), K(KK_MQA)));
     T NlowVA = K(KK_CVA1) * pow_nonneg(expm1(-1.14 * ls2), 0.446) * Xm035;
-    T NhighVA = K(KK_CVA2) * sqrt(expm1(-1.025 * ls2)) / sX + small;
-    c.aV = -(apref * NlowVA * Xm53 * pow(1.0 + pow(X, K(KK_EVA)) * pow(sdiv(NlowVA, NhighVA), K(KK_XVA)), K(KK_MVA))) * sgn;
+    T NhighVA = K(KK_CVA2) * sqrt(expm1(-1.025 * ls2)) * xm + small;
+    c.aV = -(apref * NlowVA * Xm53 *
+             pow_of(pow_base(1.0 + pow_of(xb, K(KK_EVA)) * pow_of(pow_base(NlowVA / NhighVA), K(KK_XVA))), K(KK_MVA))) * sgn;
     const int i = (int)val(K(KK_IFIT));
-    T p084 = pow(X, 0.84), xm = 1.0 / sX;
-    T fQ = K(KK_FQ0) * kappa_rhoQ_x<T>(i, X, p084) + K(KK_FQ1) * kappa_rhoQ_x<T>(i + 1, X, p084);
-    T fV = K(KK_FV0) * kappa_rhoV_x<T>(i, xm) + K(KK_FV1) * kappa_rhoV_x<T>(i + 1, xm);
-    T inu = 1.0 / nu;
+    const KappaRho k0 = kappa_rho(i), k1 = kappa_rho(i + 1);
+    T p084 = pow_of(xb, 0.84);
+    T fQ = K(KK_FQ0) * kappa_rhoQ_x(k0, X, xb, p084) + K(KK_FQ1) * kappa_rhoQ_x(k1, X, xb, p084);
+    T fV = K(KK_FV0) * kappa_rhoV_x(k0, xm) + K(KK_FV1) * kappa_rhoV_x(k1, xm);
     c.rQ = -(ne * K(KK_RHOQ) * sth * sth) * inu * inu * inu * fQ;
     c.rV = ne * K(KK_RHOV) * cth * inu * inu * fV;
     return c;
 }
-template <class T> struct KappaGet {
-    const KappaK<T>& k;
-    KS_DEV T operator()(int f) const { return k.v[f]; }
-};
 // the whole evaluation from the splat's population values (the spacetime tangent's path)
 template <class T>
-KS_DEV CoefT<T> kappa(T ne, T kap, T w, T hyp, const T* gK, T B, T nu, T sth, T cth) {
+KS_DEV CoefT<T> kappa(T ne, T kap, T w, T hyp, const T* gK, T B, T nu, T inu, T sth, T cth) {
     KappaK<T> K;
     kappa_consts(kap, w, hyp, gK, B, K);
-    return kappa_coefs(KappaGet<T>{K}, ne, nu, sth, cth);
+    return kappa_coefs(FactorGet<T>{K}, ne, nu, inu, sth, cth);
 }
 
 // ---- cap, invariants, rotation -----------------------------------------------------------------------------------
@@ -569,31 +658,39 @@ KS_DEV f32 pow2_below(f32 x) {
 }
 // a power of two has no derivative: the duals' partials stay on f = D / Dp
 template <int N, class S> KS_DEV DN<N, S> pow2_below(const DN<N, S>& x) { return DN<N, S>(pow2_below(x.v)); }
+// 2^-e of a value 2^e m, m in [1/2, 1): scales the caps' squares into range
+KS_DEV double cap_scale(double x) { int e; frexp_split(x, e); return ldexp(1.0, -e); }
+KS_DEV f32 cap_scale(f32 x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return f32(ldexpf(1.0f, -__builtin_amdgcn_frexp_expf(x.v)));
+#else
+    int e; frexpf(x.v, &e); return f32(ldexpf(1.0f, -e));
+#endif
+}
+// 0.99 I / sqrt(Q^2 + V^2) where that is below one; the root is taken only there
 template <class T> KS_DEV T cap_factor(T I, T Q, T V) {
     const double fmax = 0.99;
     if (!(I > 0.0)) return (val(Q) == 0.0 && val(V) == 0.0) ? T(1.0) : T(0.0);
-    const double s = pow2_below(dmax(dmax(fabs(val(I)), fabs(val(Q))), fabs(val(V))));
-    const double is = 1.0 / s;
+    const auto is = cap_scale(dmax(dmax(fabs(base(I)), fabs(base(Q))), fabs(base(V))));
     T Ih = I * is, q = Q * is, v = V * is;
     T pp = q * q + v * v;
-    T p = pp > 0.0 ? sqrt(pp) : T(0.0);
-    return p > fmax * Ih ? fmax * Ih / p : T(1.0);
+    if (!(pp > (fmax * fmax) * (Ih * Ih))) return T(1.0);
+    return fmax * Ih / sqrt(pp);
 }
 // cap_factor and its partials in (I, Q, V): f = fmax I / sqrt(Q^2 + V^2) where the cap acts, else a constant
 template <class T> KS_DEV void cap_factor_d(T I, T Q, T V, T& f, T df[3]) {
     const double fmax = 0.99;
     df[0] = df[1] = df[2] = T(0.0);
     if (!(I > 0.0)) { f = (val(Q) == 0.0 && val(V) == 0.0) ? T(1.0) : T(0.0); return; }
-    const double s = pow2_below(dmax(dmax(fabs(val(I)), fabs(val(Q))), fabs(val(V))));
-    const double is = 1.0 / s;
+    const T is = cap_scale(dmax(dmax(fabs(I), fabs(Q)), fabs(V)));
     T Ih = I * is, q = Q * is, v = V * is;
     T pp = q * q + v * v;
-    T p = pp > 0.0 ? sqrt(pp) : T(0.0);
-    if (!(p > fmax * Ih)) { f = T(1.0); return; }
-    f = fmax * Ih / p;
-    df[0] = fmax * is / p;
-    df[1] = -(f * q / pp) * is;
-    df[2] = -(f * v / pp) * is;
+    if (!(pp > (fmax * fmax) * (Ih * Ih))) { f = T(1.0); return; }
+    const T ip = 1.0 / sqrt(pp);
+    f = fmax * Ih * ip;
+    df[0] = fmax * is * ip;
+    df[1] = -(f * q * (ip * ip)) * is;
+    df[2] = -(f * v * (ip * ip)) * is;
 }
 
 // ---- the exact 4x4 step -------------------------------------------------------------------------------------------
@@ -613,8 +710,6 @@ KS_DEV constexpr double moment_coef(int n, int m) {
     for (int i = 2; i <= m; ++i) f *= i;
     return ((m & 1) ? -1.0 : 1.0) / (f * (n + m + 1));
 }
-template <class T> struct base_scalar { using type = T; };
-template <int N, class S> struct base_scalar<DN<N, S>> { using type = S; };
 template <int NMAX, class T> KS_DEV void moments(T a, T M[10]) {
     if (fabs(val(a)) < 1.0) {
         if constexpr (std::is_same<typename base_scalar<T>::type, double>::value) {
@@ -678,8 +773,8 @@ KS_DEV void step_coefs_inv(T aI, T a2, T r2, T ar, S f, T o[4], T e4[4]) {
     T h = (a2 - r2) * 0.5;
     T root = sqrt(h * h + ar * ar);
     T L1sq, L2sq;
-    if (h >= 0.0) { L1sq = h + root; L2sq = L1sq > 0.0 ? sdiv(ar * ar, L1sq) : T(0.0); }
-    else { L2sq = root - h; L1sq = L2sq > 0.0 ? sdiv(ar * ar, L2sq) : T(0.0); }
+    if (h >= 0.0) { L1sq = h + root; L2sq = L1sq > 0.0 ? ar * ar / L1sq : T(0.0); }
+    else { L2sq = root - h; L1sq = L2sq > 0.0 ? ar * ar / L2sq : T(0.0); }
     T L1 = L1sq > 0.0 ? sqrt(L1sq) : T(0.0), L2 = L2sq > 0.0 ? sqrt(L2sq) : T(0.0);
     T b1 = L1 * f, b2 = L2 * f;
     T Th = L1sq + L2sq;
@@ -728,7 +823,7 @@ KS_DEV void step_coefs_inv(T aI, T a2, T r2, T ar, S f, T o[4], T e4[4]) {
         isc = M[1] - bb * (M[3] / 6.0 - bb * (M[5] / 120.0 - bb * (M[7] / 5040.0 - bb * M[9] / 362880.0)));
     } else {
         T sb = sin(b2);
-        T den = sdiv(T(1.0), a * a + b2 * b2);
+        T den = 1.0 / (a * a + b2 * b2);
         ivs = pa - (a - e * (a * cb2 - b2 * sb)) * den;
         isc = (1.0 - e * (a * sb / b2 + cb2)) * den;
     }

@@ -73,6 +73,7 @@ template <class T> inline void splat_as(const SplatC& a, SplatCT<T>& b) {
     for (int i = 0; i < 3; ++i) b.kc[i] = T(a.kc[i]);
     b.kr = T(a.kr);
     b.pm0 = T(a.pm0); b.pm1 = T(a.pm1);
+    b.eA = T(a.eA); b.gam = T(a.gam); b.q = T(a.q);
     for (int f = 0; f < KK_N; ++f) b.kk.v[f] = T(a.kk.v[f]);
     b.knot0 = a.knot0; b.nk = a.nk; b.kt0 = a.kt0; b.kind = a.kind;
 }
@@ -156,12 +157,16 @@ inline void host_splat_constants(int kind, int nrows, int i, const double* p, do
     sa.qn[0] = w; sa.qn[1] = x; sa.qn[2] = y; sa.qn[3] = z; sa.iqn = 1.0 / nq;
     sa.sthB = st; sa.cthB = ct; sa.sphB = sp; sa.cphB = cp;
     c.u[0] = p[rB + 3]; c.u[1] = p[rB + 4]; c.u[2] = p[rB + 5];
+    c.eA = std::exp(c.lnA);
+    c.gam = std::sqrt(1.0 + c.u[0] * c.u[0] + c.u[1] * c.u[1] + c.u[2] * c.u[2]);
+    c.q = 1.0 / (c.gam + 1.0);
     if (kind == MODEL_THERMAL || kind == MODEL_KNOT) {
         double Th = std::exp(p[13]);
         double k0, k1;
         const double xb = 1.0 / Th;
         double k2 = host_besselk(xb, k0, k1);
         c.p1 = Th;
+        c.g[0] = 1.0 / Th;
         c.p2 = k2 > 0.0 ? k0 / k2 : 1.0;
         c.p3 = k2 > 0.0 ? k1 / k2 : 1.0;
         // d/d ln Theta = -x d/dx at x = 1/Theta, with K0' = -K1, K1' = -K0 - K1/x, K2 = K0 + 2 K1/x
@@ -174,6 +179,18 @@ inline void host_splat_constants(int kind, int nrows, int i, const double* p, do
         // d/dp of the Gamma products: Gamma'(x) = Gamma(x) psi(x), dx/dp = 1/4
         sa.dpop[0] = c.g[0] * 0.25 * (host_digamma((3 * pp - 1) / 12.0) + host_digamma((3 * pp + 19) / 12.0));
         sa.dpop[1] = c.g[1] * 0.25 * (host_digamma((3 * pp + 2) / 12.0) + host_digamma((3 * pp + 22) / 12.0));
+        // the fits' per-splat factors with their partials in (p, ln gamma_min, ln B), by three-partial duals
+        using D3 = DN<3, double>;
+        const D3 pd = D3::seed(pp, 0);
+        D3 gm(c.p2), Bd(c.Bmag), gd[2];
+        gm.d[1] = c.p2; Bd.d[2] = c.Bmag;
+        for (int k = 0; k < 2; ++k) { gd[k] = D3(c.g[k]); gd[k].d[0] = sa.dpop[k]; }
+        KappaK<D3> Kd;
+        power_consts(pd, gm, D3(gamma_max), gd, Bd, Kd);
+        for (int f = 0; f < PL_N; ++f) {
+            c.kk.v[f] = Kd.v[f].v;
+            for (int q = 0; q < 3; ++q) sa.dkk[q][f] = Kd.v[f].d[q];
+        }
     } else {
         double kap = p[13], wk = std::exp(p[14]);
         // the 2F1 factor and its partials in kappa and ln w, by two-partial duals through its series

@@ -16,9 +16,10 @@ KS_DEV SplatCT<D3> splat_dual(const SplatC& s) {
     o.x = D3(s.x); o.y = D3(s.y); o.z = D3(s.z);
     for (int i = 0; i < 9; ++i) o.R[i] = D3(s.R[i]);
     for (int i = 0; i < 3; ++i) { o.is[i] = D3(s.is[i]); o.bh[i] = D3(s.bh[i]); o.u[i] = D3(s.u[i]); }
-    o.t0 = D3(s.t0); o.iw = D3(s.iw); o.omega = D3(s.omega); o.rsup2 = D3(s.rsup2); o.lnA = D3(s.lnA); o.Bmag = D3(s.Bmag);
+    o.t0 = D3(s.t0); o.iw = D3(s.iw); o.omega = D3(s.omega); o.rsup2 = D3(s.rsup2); o.lnA = D3(s.lnA); o.eA = D3(s.eA); o.gam = D3(s.gam); o.q = D3(s.q); o.Bmag = D3(s.Bmag);
     o.p1 = D3(s.p1); o.p2 = D3(s.p2); o.p3 = D3(s.p3);
     for (int i = 0; i < 6; ++i) o.g[i] = D3(s.g[i]);
+    for (int f = 0; f < PL_N; ++f) o.kk.v[f] = D3(s.kk.v[f]);       // the power law's factors (kappa's are built from the above)
     o.knot0 = s.knot0; o.nk = s.nk; o.kt0 = s.kt0; o.kind = s.kind;
     return o;
 }
@@ -42,22 +43,20 @@ KS_DEV bool tangent_coefficients(const SplatC* __restrict__ sp, int ns, const D3
         const D3 G_ = exp(-0.5 * gexp);
         if (!(G_ > WEIGHT_CUTOFF)) continue;
         if (!geo_ready) { make_geo(a, s.r, s.th, eta, lam, s.nur, s.nuth, G); geo_ready = true; }
-        const FrameT<D3> fr = local_frame(G, a, alpha, beta, tsin, sc.u, sc.bh);
-        const D3 nuf = nu / fr.g;
+        const FrameT<D3> fr = local_frame(G, a, alpha, beta, tsin, D3(nu), sc.u, sc.gam, sc.q, sc.bh);
+        const D3 nh = fr.nh, inh = fr.inh, nuf = fr.nu, inu = inh * (1.0 / NU0);
         const D3 cb = dmin(dmax(fr.cosB, -1.0), 1.0);
         D3 sth, cth;
         pitch_sincos(cb, sth, cth);
-        const D3 ne = exp(sc.lnA) * G_;
+        const D3 ne = sc.eA * G_;
         CoefT<D3> cf;
         const int kind = KIND == MODEL_COMPOSITE ? sc.kind : KIND;
-        if (kind == MODEL_THERMAL) cf = thermal(ne, sc.p1, sc.p2, sc.p3, sc.Bmag, nuf, sth, cth);
-        else if (kind == MODEL_POWERLAW) cf = powerlaw(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
-        else cf = kappa(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, sth, cth);
+        if (kind == MODEL_THERMAL) cf = thermal(ne, sc.p1, sc.g[0], sc.p2, sc.p3, sc.Bmag, nuf, nh, inh, sth, cth);
+        else if (kind == MODEL_POWERLAW) cf = power_coefs(FactorGet<D3>{sc.kk}, ne, nuf, inu, sth, cth);
+        else cf = kappa(ne, sc.p1, sc.p2, sc.p3, sc.g, sc.Bmag, nuf, inu, sth, cth);
         if (!(cf.jI > 0.0 || cf.aI > 0.0 || cf.rQ != 0.0 || cf.rV != 0.0)) continue;
         const D3 fe = cap_factor(cf.jI, cf.jQ, cf.jV), fa = cap_factor(cf.aI, cf.aQ, cf.aV);
-        const D3 nh = nuf * (1.0 / NU0);
-        const D3 i2 = 1.0 / (nh * nh);
-        D3 s2c, c2c; sincos(2.0 * fr.chi, &s2c, &c2c);
+        const D3 i2 = inh * inh, s2c = fr.s2, c2c = fr.c2;
         const D3 jQ = fe * cf.jQ * i2, aQ = fa * cf.aQ * nh, rQ = cf.rQ * nh;
         j4[0] += cf.jI * i2; j4[1] += jQ * c2c; j4[2] += jQ * s2c; j4[3] += fe * cf.jV * i2;
         a4[0] += cf.aI * nh; a4[1] += aQ * c2c; a4[2] += aQ * s2c; a4[3] += fa * cf.aV * nh;

@@ -75,6 +75,19 @@ inline Cnt dmax(Cnt a, double b) { return a.v > b ? a : Cnt(b); }
 inline Cnt dmin(Cnt a, double b) { return a.v < b ? a : Cnt(b); }
 inline bool isfinite_(Cnt x) { return std::isfinite(x.v); }
 inline Cnt pow2_below(Cnt x) { return Cnt(pow2_below(x.v)); }
+// the fits' elementary functions: a base's logarithm and each of its powers count as one transcendental
+inline Cnt base(Cnt x) { return x; }
+inline Cnt cap_scale(Cnt x) { return Cnt(cap_scale(x.v)); }
+inline Cnt fdiv(Cnt a, Cnt b) { return a / b; }
+template <> struct PowBase<Cnt> { PowBase<double> b; };
+inline PowBase<Cnt> pow_base(Cnt x) { op_special(); return {pow_base(x.v)}; }
+inline Cnt pow_of(const PowBase<Cnt>& b, Cnt y) { op_special(); return Cnt(pow_of(b.b, y.v)); }
+inline Cnt pow_of(const PowBase<Cnt>& b, double y) { op_special(); return Cnt(pow_of(b.b, y)); }
+inline Cnt ln_of(const PowBase<Cnt>& b) { op(); return Cnt(ln_of(b.b)); }
+inline Cnt fexp(Cnt x) { return exp(x); }
+inline Cnt log1p_pos(Cnt x) { return log1p(x); }
+inline void sincos_small(Cnt x, Cnt* s, Cnt* c) { sincos(x, s, c); }
+inline void phase_sincos(Cnt x, Cnt* s, Cnt* c) { sincos(x, s, c); }
 // the scalar-dependent gates of the step and the pitch angle: those of the FP32 path or of the FP64 path
 inline bool& fp32_gates() { static bool g = true; return g; }
 inline double sin_floor(Cnt) { return fp32_gates() ? sin_floor(f32(0.0f)) : sin_floor(0.0); }
