@@ -3,6 +3,7 @@
 // segment map, and the path weight. Shared by the transfer kernels and the host-side work model.
 // Reference: transport.jl:254-290, polarized.jl:110-150, populations.jl:13-104, trajectories.jl:93-128.
 #pragma once
+#include <cstddef>
 #include "ks_kernels.hpp"
 
 namespace ksd {
@@ -31,9 +32,7 @@ KS_DEV TransCtxT<S> make_ctx(double a, double rp, double rm, double thetao_sin, 
 // The Gaussian exponent at (t, x, y, z) of a splat whose centre follows knots (trajectories.jl:93-128): the offset
 // from the knot-interpolated centre (knot_centre), no pattern rotation.
 template <class S>
-KS_DEV S knot_gexp(const S* __restrict__ knots, const S* __restrict__ ktimes, const SplatCT<S>& sc, S t, S x, S y, S z) {
-    S cx, cy, cz;
-    knot_centre(sc, knots, ktimes, t, cx, cy, cz);
+KS_DEV S knot_gexp(const SplatCT<S>& sc, S cx, S cy, S cz, S t, S x, S y, S z) {
     S d0 = x - cx, d1 = y - cy, d2 = z - cz;
     S u0 = sc.R[0] * d0 + sc.R[3] * d1 + sc.R[6] * d2;
     S u1 = sc.R[1] * d0 + sc.R[4] * d1 + sc.R[7] * d2;
@@ -44,12 +43,16 @@ KS_DEV S knot_gexp(const S* __restrict__ knots, const S* __restrict__ ktimes, co
 }
 
 // A splat's Gaussian weight at (t, x, y, z), zero where the transport does not count it (outside its support sphere,
-// or below the weight cutoff).
+// or below the weight cutoff);
+// at: t among the splat's knot times, where the caller has it.
 template <int KIND, class S>
-KS_DEV S splat_weight(const SplatCT<S>& sc, const S* __restrict__ knots, const S* __restrict__ ktimes, S t, S x, S y, S z) {
+KS_DEV S splat_weight(const SplatCT<S>& sc, const S* __restrict__ knots, const S* __restrict__ ktimes, S t, S x, S y, S z, const KnotAt<S>* at = nullptr) {
     S gexp;
     if (KIND == MODEL_KNOT || sc.nk > 0) {
-        gexp = knot_gexp(knots, ktimes, sc, t, x, y, z);
+        const KnotAt<S> k = at ? *at : knot_at(ktimes + sc.kt0, sc.nk, t);
+        S cx, cy, cz;
+        knot_centre(knots + 3 * ((int64_t)sc.knot0 + k.kk), sc.nk < 2, k.w, cx, cy, cz);
+        gexp = knot_gexp(sc, cx, cy, cz, t, x, y, z);
     } else {
         S sph, cph;
         if (outside_support(sc, t, x, y, z, sph, cph)) return S(0.0);
@@ -129,27 +132,46 @@ KS_DEV bool sample_coefficients(const TransCtxT<S>& c, double st, double r, doub
 // near the cutoff (27.63 = 5.26^2), where d = pm0 + pm1 |t| bounds the error of the splat's scaled coordinates; a bound
 // that is not finite lets every sample through. About 45 instructions against 150 to 400 for the weight and 400 to 3000
 // for the contribution, which then run on the passing pairs alone, 64 at a time.
-template <int KIND>
-KS_DEV bool may_weigh(const SplatCf& c, const f32* __restrict__ knots, const f32* __restrict__ ktimes, float t, float x, float y, float z) {
-    float e0, e1, e2;
-    if (KIND == MODEL_KNOT || c.nk > 0) {
-        f32 cx, cy, cz;
-        knot_centre(c, knots, ktimes, f32(t), cx, cy, cz);
-        e0 = x - cx.v; e1 = y - cy.v; e2 = z - cz.v;
-    } else {
-        float sp, cp;
-        hw_sincos(c.omega.v * (t - c.t0.v), sp, cp);
-        // Rz(-ph) (X - Rz(ph) c) = Rz(-ph) X - c
-        e0 = x * cp + y * sp - c.x.v; e1 = y * cp - x * sp - c.y.v; e2 = z - c.z.v;
-    }
-    float g = (t - c.t0.v) * c.iw.v;
+// The sample's offset from the splat's centre in the splat's frame (pattern_offset, knot_offset) is apart from the test of
+// the offset, so that a caller can place the sample among the knot times once for all splats that share them.
+struct SplatTest { float x, y, z, R[9], is[3], t0, iw, omega, pm0, pm1; int knot0, nk, kt0, kind; };     // a SplatCf's first fields
+static_assert(sizeof(SplatTest) == 96 && offsetof(SplatCf, kind) + 4 == sizeof(SplatTest), "the prefilter's fields lead SplatCf");
+KS_DEV SplatTest splat_test(const SplatCf& c) { SplatTest t; __builtin_memcpy(&t, &c, sizeof t); return t; }
+KS_DEV void pattern_offset(const SplatTest& c, float t, float x, float y, float z, float e[3]) {
+    float sp, cp;
+    hw_sincos(c.omega * (t - c.t0), sp, cp);
+    // Rz(-ph) (X - Rz(ph) c) = Rz(-ph) X - c
+    e[0] = x * cp + y * sp - c.x; e[1] = y * cp - x * sp - c.y; e[2] = z - c.z;
+}
+KS_DEV void knot_offset(const f32* __restrict__ K, bool one, float w, float x, float y, float z, float e[3]) {
+    f32 cx, cy, cz;
+    knot_centre(K, one, f32(w), cx, cy, cz);
+    e[0] = x - cx.v; e[1] = y - cy.v; e[2] = z - cz.v;
+}
+KS_DEV bool offset_may_weigh(const SplatTest& c, float t, const float e[3]) {
+    float g = (t - c.t0) * c.iw;
     g = g * g;
     for (int b = 0; b < 3; ++b) {
-        const float q = (c.R[b].v * e0 + c.R[3 + b].v * e1 + c.R[6 + b].v * e2) * c.is[b].v;
+        const float q = (c.R[b] * e[0] + c.R[3 + b] * e[1] + c.R[6 + b] * e[2]) * c.is[b];
         g += q * q;
     }
-    const float d = c.pm1.v * fabsf(t) + c.pm0.v;
+    const float d = c.pm1 * fabsf(t) + c.pm0;
     return !(g > 27.641f + 2.0f * d * (5.3f + d));
+}
+template <int KIND>
+KS_DEV bool may_weigh(const SplatTest& c, const f32* __restrict__ knots, const f32* __restrict__ ktimes, float t, float x, float y, float z) {
+    float e[3];
+    if (KIND == MODEL_KNOT || c.nk > 0) {
+        const KnotAt<f32> a = knot_at(ktimes + c.kt0, c.nk, f32(t));
+        knot_offset(knots + 3 * ((int64_t)c.knot0 + a.kk), c.nk < 2, a.w.v, x, y, z, e);
+    } else {
+        pattern_offset(c, t, x, y, z, e);
+    }
+    return offset_may_weigh(c, t, e);
+}
+template <int KIND>
+KS_DEV bool may_weigh(const SplatCf& c, const f32* __restrict__ knots, const f32* __restrict__ ktimes, float t, float x, float y, float z) {
+    return may_weigh<KIND>(splat_test(c), knots, ktimes, t, x, y, z);
 }
 
 // g^2 Sigma dtau of a thin sample, g the ZAMO redshift (Splats.jl:113-128)

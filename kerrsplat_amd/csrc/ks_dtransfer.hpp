@@ -68,6 +68,11 @@ template <class S> struct SplatCT {
     S is[3];              // exp(-s_a)
     S t0, iw;             // t0 and exp(-logw)
     S omega;              // pattern angular velocity
+    S pm0, pm1;           // the FP32 prefilter's error in the splat's scaled coordinates, pm0 + pm1 |t| (may_weigh)
+    int knot0, nk, kt0;   // splats whose centre follows knots (nk > 0): the first of its nk knots (xyz triples) and of their
+                          // times in the model's arrays
+    int kind;             // the splat's population (MODEL_THERMAL, MODEL_POWERLAW, MODEL_KAPPA, ...)
+    // (the fields so far are the prefilter's, in one piece: SplatTest)
     S rsup2;              // support sphere radius^2 = -2 ln(cutoff) exp(2 max s)
     S lnA;                // thin: logA; others: logne
     S Bmag, bh[3];        // field magnitude and unit direction (ZAMO axes r, phi, -theta)
@@ -77,13 +82,9 @@ template <class S> struct SplatCT {
     S g[6];               // thermal: 1 / Theta_e; power law: Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12);
                           // kappa: Gamma(k-4/3), Gamma(k-2), Gamma(k/4-1/3), Gamma(k/4+4/3), Gamma(2+k/2), K0/(K2+1e-40) at 1/w
     S kc[3], kr;          // splats whose centre follows knots: a sphere holding every knot (centre, radius; kr = 0 without)
-    S pm0, pm1;           // the FP32 prefilter's error in the splat's scaled coordinates, pm0 + pm1 |t| (may_weigh)
     S eA;                 // exp(lnA)
     S gam, q;             // sqrt(1 + u^2), 1 / (gam + 1)
     KappaK<S> kk;         // kappa, power law: the fits' per-splat factors (kappa_consts, power_consts)
-    int knot0, nk, kt0;   // splats whose centre follows knots (nk > 0): the first of its nk knots (xyz triples) and of their
-                          // times in the model's arrays
-    int kind;             // the splat's population (MODEL_THERMAL, MODEL_POWERLAW, MODEL_KAPPA, ...)
 };
 // exp(lnA); FP32: of the rounded lnA
 template <class S> KS_DEV S splat_density(const SplatCT<S>& c) { if constexpr (std::is_same<S, f32>::value) return exp(c.lnA); else return c.eA; }
@@ -187,23 +188,34 @@ KS_DEV S gauss_exponent(const SplatCT<S>& s, S t, S x, S y, S z, S sp, S cp) {
     return q0 * q0 + q1 * q1 + q2 * q2 + tt * tt;
 }
 
-// The centre of a splat that follows knots at emission time t (trajectories.jl:93-111): linear interpolation
-// between the knots around t, held at the first and last knot outside their times.
+// Where emission time t lies among nk ascending knot times: the interval and the weight of its end, held at the first and
+// last knot outside their times (trajectories.jl:93-111). Every time is compared, so the loads do not wait for each other,
+// and are scalar where the times are the same for the whole wavefront.
+template <class S> struct KnotAt { int kk; S w; };
+template <class S>
+KS_DEV KnotAt<S> knot_at(const S* __restrict__ kt, int nk, S t) {
+    KnotAt<S> a;
+    a.kk = 0;
+    a.w = S(0.0);
+    if (nk < 2) return a;
+    for (int k = 1; k < nk - 1; ++k) a.kk += kt[k] <= t ? 1 : 0;
+    const S w = (t - kt[a.kk]) / (kt[a.kk + 1] - kt[a.kk]);
+    a.w = w < 0.0 ? S(0.0) : (w > 1.0 ? S(1.0) : w);
+    return a;
+}
+// the centre between the interval's knots, K the first of them (one: a splat of a single knot)
+template <class S>
+KS_DEV void knot_centre(const S* __restrict__ K, bool one, S w, S& cx, S& cy, S& cz) {
+    const S* E = one ? K : K + 3;
+    cx = (1.0 - w) * K[0] + w * E[0];
+    cy = (1.0 - w) * K[1] + w * E[1];
+    cz = (1.0 - w) * K[2] + w * E[2];
+}
+// the centre of a splat that follows knots at emission time t
 template <class S>
 KS_DEV void knot_centre(const SplatCT<S>& sc, const S* __restrict__ knots, const S* __restrict__ ktimes, S t, S& cx, S& cy, S& cz) {
-    const S* K = knots + 3 * (int64_t)sc.knot0;
-    const S* kt = ktimes + sc.kt0;
-    const int nk = sc.nk;
-    if (t <= kt[0]) { cx = K[0]; cy = K[1]; cz = K[2]; }
-    else if (t >= kt[nk - 1]) { cx = K[3 * (nk - 1)]; cy = K[3 * (nk - 1) + 1]; cz = K[3 * (nk - 1) + 2]; }
-    else {
-        int kk = 0;
-        while (kk < nk - 2 && kt[kk + 1] <= t) ++kk;
-        S w = (t - kt[kk]) / (kt[kk + 1] - kt[kk]);
-        cx = (1.0 - w) * K[3 * kk] + w * K[3 * (kk + 1)];
-        cy = (1.0 - w) * K[3 * kk + 1] + w * K[3 * (kk + 1) + 1];
-        cz = (1.0 - w) * K[3 * kk + 2] + w * K[3 * (kk + 1) + 2];
-    }
+    const KnotAt<S> a = knot_at(ktimes + sc.kt0, sc.nk, t);
+    knot_centre(knots + 3 * ((int64_t)sc.knot0 + a.kk), sc.nk < 2, a.w, cx, cy, cz);
 }
 
 // ---- metric, ZAMO tetrad, photon momentum ----------------------------------------------------------------------
@@ -378,13 +390,15 @@ template <class T> KS_DEV T cos_bounded(const T& x) {
 }
 
 // thermal (coefficients.jl:101-151) with the splat's Bessel ratios k0/k2, k1/k2 (k2 > 0 in practice) and 1 / Theta_e, at
-// nu = nh NU0, inh = 1 / nh (FP32 takes nu alone, in the operations it had: is_fp32); ne enters linearly and stays a plain number in the adjoint. The powers of x share one
-// logarithm, the four divisions left are nu / nu_s, its cube root's, cos / sin and the logistic's (which takes the place of
-// (1 + tanh) / 2 and is below 1e-21 for x < 10, where the term it multiplies is left out).
+// nu = nh NU0, inh = 1 / nh; ne enters linearly and stays a plain number in the adjoint. The FP32 transfer takes nu alone,
+// in the operations it had (is_fp32). Else the powers of x share one logarithm, the four divisions left are nu / nu_s, its
+// cube root's, cos / sin and the logistic's (which takes the place of (1 + tanh) / 2 and is below 1e-21 for x < 10, where
+// the term it multiplies is left out). MI355X, 32 splats at 128^2 x 1024, FP64, with the frames' shorter form (local_frame):
+// transfer 5.5 -> 4.9 ms, element adjoints 6.9 -> 6.0 ms; 64 splats, 4 frames, FP32 duals: adjoints 19.1 -> 17.4 ms.
 template <class T, class NE>
 KS_DEV CoefT<T> thermal(NE ne, T Th, T iTh, T k0k2, T k1k2, T B, T nu, T nh, T inh, T sth, T cth) {
     CoefT<T> c;
-    if constexpr (is_fp32<T>) {
+    if constexpr (std::is_same<T, f32>::value) {
         T w = 2.0 * PI * nu;
         T w0w = EE * B / (ME * CL) / w;
         T wp2w2 = (4.0 * PI * ne * EE * EE / ME) / (w * w);
@@ -452,7 +466,8 @@ KS_DEV CoefT<T> thermal(NE ne, T Th, T iTh, T k0k2, T k1k2, T B, T nu, T nh, T i
 // power law (coefficients.jl:208-256), split as kappa's: its per-splat factors from p, gamma_min, gamma_max and
 // gPL = {Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12)} (power_consts, once per splat), and its
 // evaluation at one sample (power_coefs) from one power X^(-p/2) of X = nu / (nu_c sin), where eleven powers were taken
-// at every pair, seven of them of the splat's numbers alone.
+// at every pair, seven of them of the splat's numbers alone. MI355X, FP64, 48 splats, 102 x 67 x 333, 2 frames: transfer
+// 3.57 -> 2.02 ms, element adjoints 6.10 -> 3.42 ms.
 template <class T>
 KS_DEV void power_consts(T p, T gmin, T gmax, const T* gPL, T B, KappaK<T>& K) {
     const T nuc = EE * B / (2.0 * PI * ME * CL);
@@ -580,6 +595,8 @@ KS_DEV void kappa_consts(T kap, T w, T hyp, const T* gK, T B, KappaK<T>& K) {
 // the X-dependent factors of the rotativity fits n = 1..4 (kappa.jl:72-97); p084 = X^0.84, xm = X^-1/2. Each is
 // 1 - exp(-p084 d) - sin(sd X) exp(-cc X^b): the four share one piece of code, since a wavefront's pairs hold splats of
 // several kappa. The second exponential is zero in FP64 beyond X = 6e5, so a larger phase is taken as 1e5.
+// MI355X, FP64, 1024 splats, 112 x 96 x 512, with the powers of X from one logarithm: transfer 95 -> 60 ms, element
+// adjoints 166 -> 121 ms.
 struct KappaRho { double d, sd, cc, b, v; };
 KS_DEV KappaRho kappa_rho(int n) {
     KappaRho k;

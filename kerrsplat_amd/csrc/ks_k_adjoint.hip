@@ -326,7 +326,7 @@ __device__ __forceinline__ void adj_splats_block(int64_t e, int64_t unit, int i,
     __syncthreads();                          // the last block's reads are done
     copy_to_lds(&s_c, sp + i, lane);
     copy_to_lds(&s_sa, sadj + i, lane);
-    const SplatCf& cf = spf[i];
+    const SplatTest test = splat_test(spf[i]);
     const SplatCT<S>& c = s_c;
     const SplatAdjT<S>& sa = s_sa;
     int64_t j = 0;
@@ -415,7 +415,7 @@ __device__ __forceinline__ void adj_splats_block(int64_t e, int64_t unit, int i,
             }
 #pragma unroll
             for (int u = 0; u < WALK; ++u) {
-                const bool act = fl[u] && may_weigh<MODEL_THERMAL>(cf, knots_f, ktimes_f, tk[u], xk[u], yk[u], zk[u]);
+                const bool act = fl[u] && may_weigh<MODEL_THERMAL>(test, knots_f, ktimes_f, tk[u], xk[u], yk[u], zk[u]);
                 const uint64_t m = __ballot(act);
                 if (act) {
                     const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));

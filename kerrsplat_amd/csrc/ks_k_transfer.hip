@@ -26,14 +26,13 @@ struct TransferArgs {
     double L;
     const int* kstop;
     uint8_t* aflg;
-    const SplatCf* spf; const f32* knots_f; const f32* ktimes_f;     // the FP32 copies (may_weigh)
 };
 KS_DEV int64_t npix_items(const TransferArgs& A) { return A.npix * A.nt * A.nnu; }
 // A wavefront's workspace in LDS, field-major over its 64 lanes: the geometry of its rays' current sample, the sums of
 // the sample's contributions and whether it has any, the rays' screen coordinates and frequency, the pair queue (lane |
 // splat << 6), the slice's candidate splats. 7.8 KB in FP32 and 15.6 KB in FP64: as many wavefronts as the registers
 // allow fit a compute unit.
-constexpr int QCAP = 128;              // the queue holds < 64 pending pairs and up to 64 pushes of one splat
+constexpr int QCAP = 256;              // the queue holds < 64 pending pairs and up to 64 pushes of each of two splats
 template <class S>
 struct WaveWork {
     S geo[GEO_FIELDS * 64], sum[11 * 64], alpha[64], beta[64], nu[64];
@@ -49,6 +48,35 @@ KS_DEV void wave_sync() {
 KS_DEV uint64_t uniform64(uint64_t x) {
     return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
 }
+// The prefilter's fields of two splats at wave-uniform addresses, held in scalar registers: four scalar loads in flight at
+// once. Left to the compiler, each field is loaded where it is used, and a splat's test waits for its loads one after
+// another (as vector loads, before the pointer said that nothing writes them: 56 % of the FP64 transfer's wavefront cycles
+// were such waits). MI355X, transfer of one pass: FP64, 32 thermal splats at 128^2 x 1024 4.9 -> 3.7 ms, 48 power-law splats
+// 2.04 -> 1.65, 1024 kappa splats on knots (112 x 96 x 512) 61 -> 50; FP32, the same at 256^2 x 1024 165 -> 121, 64 thermal
+// splats (4 frames of 128^2 x 1024) 12.4 -> 10.4, 128 mixed splats (36,864 points x 512 x 12) 69 -> 57.
+typedef int sgpr16 __attribute__((ext_vector_type(16), aligned(4)));
+typedef int sgpr8 __attribute__((ext_vector_type(8), aligned(4)));
+struct SplatTests {
+    sgpr16 p, r;
+    sgpr8 q, s;
+    __device__ __forceinline__ SplatTests(const SplatCf* __restrict__ u, const SplatCf* __restrict__ v) {
+        p = *(const sgpr16*)u; q = *(const sgpr8*)((const int*)u + 16);
+        r = *(const sgpr16*)v; s = *(const sgpr8*)((const int*)v + 16);
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+s"(p), "+s"(q), "+s"(r), "+s"(s));
+#endif
+    }
+    __device__ __forceinline__ static SplatTest of(sgpr16 p, sgpr8 q) {
+        SplatTest t;
+        int w[24];
+        for (int i = 0; i < 16; ++i) w[i] = p[i];
+        for (int i = 0; i < 8; ++i) w[16 + i] = q[i];
+        __builtin_memcpy(&t, w, sizeof t);
+        return t;
+    }
+    __device__ __forceinline__ SplatTest a() const { return of(p, q); }
+    __device__ __forceinline__ SplatTest b() const { return of(r, s); }
+};
 // The slice of the q-th of n rows of tasks: the middle of the rays first, then outwards. A ray is nearest the hole around
 // its middle, where the splats crowd: in this order the tasks' costs fall (by five from the first sixteenth to the last),
 // and the queue's last ones are cheap.
@@ -66,7 +94,8 @@ KS_DEV int slice_order(int q, int n) { return (q & 1) ? (n - 1) / 2 + (q + 1) / 
 // The queue, not the lanes, decides what runs: all lanes take part in every collective, and each loop exit is uniform.
 template <int KIND, class S, bool CULL>
 __device__ __forceinline__ void transfer_task(const TransferArgs& A, const SplatCT<S>* __restrict__ sp, const S* __restrict__ knots,
-                                    const S* __restrict__ ktimes, S* __restrict__ seg, S* __restrict__ rec, int64_t task, WaveWork<S>& W) {
+                                    const S* __restrict__ ktimes, S* __restrict__ seg, S* __restrict__ rec, const SplatCf* __restrict__ spf, const f32* __restrict__ knots_f,
+                                    int64_t task, WaveWork<S>& W) {
     const int64_t npix = A.npix;
     const int N = A.N;
     const int64_t nitems = npix * A.nt * A.nnu;
@@ -131,6 +160,32 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
             int qh = 0, qn = 0, b = -1;
             uint64_t mk = 0;
             bool more = true;
+            // the sample among the knot times (of part kt_c of the model's), and its interval where the lanes share one
+            int kt_c = -1, nk_c = 0, kk_u = -1;
+            KnotAt<S> at{0, S(0.0)};
+            auto may = [&](const SplatTest& c) {
+                float e3[3];
+                if (KIND == MODEL_KNOT || c.nk > 0) {
+                    if (c.kt0 != kt_c || c.nk != nk_c) {
+                        kt_c = c.kt0; nk_c = c.nk;
+                        at = knot_at(ktimes + kt_c, nk_c, t);
+                        const uint64_t vm = __ballot(valid);
+                        const int k0 = __builtin_amdgcn_readlane(at.kk, __builtin_ctzll(vm));
+                        kk_u = (__ballot(at.kk != k0) & vm) == 0 ? k0 : -1;
+                    }
+                    const float w = (float)val(at.w);
+                    if (kk_u >= 0) knot_offset(knots_f + 3 * ((int64_t)c.knot0 + kk_u), c.nk < 2, w, xf, yf, zf, e3);
+                    else knot_offset(knots_f + 3 * ((int64_t)c.knot0 + at.kk), c.nk < 2, w, xf, yf, zf, e3);
+                } else {
+                    pattern_offset(c, tf, xf, yf, zf, e3);
+                }
+                return valid && offset_may_weigh(c, tf, e3);
+            };
+            auto push = [&](bool hit, int i) {
+                const uint64_t hm = __ballot(hit);
+                if (hit) W.q[(qh + qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u))) & (QCAP - 1)] = lane | (i << 6);
+                qn += __popcll(hm);
+            };
             for (;;) {
                 while (qn < 64) {
                     while (mk == 0 && more) {
@@ -139,12 +194,16 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
                         else mk = A.ns - 64 * b >= 64 ? ~0ull : (1ull << (A.ns - 64 * b)) - 1;
                     }
                     if (!more) break;
+                    // two splats at a time (the last one of an odd count twice, its second test not counted)
                     const int i = b * 64 + __builtin_ctzll(mk);
                     mk &= mk - 1;
-                    const bool hit = valid && may_weigh<KIND>(A.spf[i], A.knots_f, A.ktimes_f, tf, xf, yf, zf);
-                    const uint64_t hm = __ballot(hit);
-                    if (hit) W.q[(qh + qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u))) & (QCAP - 1)] = lane | (i << 6);
-                    qn += __popcll(hm);
+                    const bool two = mk != 0;
+                    const int i2 = two ? b * 64 + __builtin_ctzll(mk) : i;
+                    mk &= mk - 1;
+                    const SplatTests tests(spf + i, spf + i2);
+                    const bool h1 = may(tests.a()), h2 = may(tests.b());
+                    push(h1, i);
+                    push(two && h2, i2);
                 }
                 if (qn == 0) break;
                 if (!ready) {            // the sample's geometry, in FP64, for its first queued pairs
@@ -163,13 +222,15 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
                 const bool on = lane < cnt;
                 const int e = W.q[(qh + lane) & (QCAP - 1)];
                 const int l = on ? e & 63 : lane, i = on ? e >> 6 : 0;
+                const KnotAt<S> al{__shfl(at.kk, l, 64), lane_value(at.w, l)};
                 const S tt = lane_value(t, l), xx = lane_value(x, l), yy = lane_value(y, l), zz = lane_value(z, l);
                 bool act = false;
                 S c[11];
                 for (int q = 0; q < 11; ++q) c[q] = S(0.0);
                 if (on) {
                     const SplatCT<S>& sc = sp[i];
-                    const S G_ = splat_weight<KIND>(sc, knots, ktimes, tt, xx, yy, zz);
+                    const bool have = (KIND == MODEL_KNOT || sc.nk > 0) && sc.kt0 == kt_c && sc.nk == nk_c;
+                    const S G_ = splat_weight<KIND>(sc, knots, ktimes, tt, xx, yy, zz, have ? &al : nullptr);
                     if (G_ > 0.0) {
                         GeoT<S> G;
                         geo_load(W.geo + l, 64, G);
@@ -227,8 +288,8 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
 template <int KIND, class S, bool CULL>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(Waves<S>::transfer)))
 ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __restrict__ knots, const S* __restrict__ ktimes,
-                  S* __restrict__ seg, S* __restrict__ rec, const int* __restrict__ tasks, int64_t ntasks, unsigned* __restrict__ head,
-                  uint32_t* __restrict__ cost) {
+                  S* __restrict__ seg, S* __restrict__ rec, const SplatCf* __restrict__ spf, const f32* __restrict__ knots_f,
+                  const int* __restrict__ tasks, int64_t ntasks, unsigned* __restrict__ head, uint32_t* __restrict__ cost) {
     __shared__ WaveWork<S> s_w[2];
     __shared__ unsigned s_q;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
@@ -243,7 +304,7 @@ ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __
         if (q >= ntasks) break;
         const int64_t task = tasks ? (int64_t)tasks[q] : q;
         const uint64_t t0 = cost ? wall_clock64() : 0;
-        transfer_task<KIND, S, CULL>(A, sp, knots, ktimes, seg, rec, task, s_w[wave]);
+        transfer_task<KIND, S, CULL>(A, sp, knots, ktimes, seg, rec, spf, knots_f, task, s_w[wave]);
         if (cost) {
             __syncthreads();
             atomicMax(cost + task, (uint32_t)min<uint64_t>(wall_clock64() - t0, 0xffffffffull));
@@ -353,7 +414,7 @@ hipError_t launch_fill_i32(hipStream_t s, int* p, int64_t n, int v) {
 }
 template <int KIND, class S, bool CULL>
 static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* seg, S* rec,
-                                   const TransferLaunch& tl) {
+                                   const SplatCf* spf, const f32* knots_f, const TransferLaunch& tl) {
     const int64_t all = (npix_items(A) * A.nch + 127) / 128;
     const int64_t ntasks = tl.tasks ? tl.ntasks : all;
     if (ntasks <= 0) return hipSuccess;
@@ -366,44 +427,42 @@ static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const S
     hipLaunchKernelGGL(ks_fill_i32, dim3(1), dim3(64), 0, s, tl.head, (int64_t)1, 0);
     if (tl.cost) hipLaunchKernelGGL(ks_fill_i32, dim3(grid_for(ntasks, 256)), dim3(256), 0, s, (int*)tl.cost, ntasks, 0);
     const int64_t grid = std::min<int64_t>(ntasks, (int64_t)groups * (tl.group_scale > 0 ? tl.group_scale : 1));
-    hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)grid), dim3(128), 0, s, A, sp, knots, ktimes, seg, rec, tl.tasks,
+    hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)grid), dim3(128), 0, s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl.tasks,
                        ntasks, (unsigned*)tl.head, tl.cost);
     return hipGetLastError();
 }
 template <int KIND, class S>
 static hipError_t chunk_transfer_k(hipStream_t s, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* seg, S* rec,
-                                   const TransferLaunch& tl) {
+                                   const SplatCf* spf, const f32* knots_f, const TransferLaunch& tl) {
     // the per-tile cull bounds pattern-rotating splats by their arc and knot splats by the sphere holding their knots
-    if (A.ns >= CULL_MIN_NS && A.ns <= CAND_MAX) return chunk_transfer_c<KIND, S, true>(s, A, sp, knots, ktimes, seg, rec, tl);
-    return chunk_transfer_c<KIND, S, false>(s, A, sp, knots, ktimes, seg, rec, tl);
+    if (A.ns >= CULL_MIN_NS && A.ns <= CAND_MAX) return chunk_transfer_c<KIND, S, true>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
+    return chunk_transfer_c<KIND, S, false>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
 }
 template <class S>
 static hipError_t chunk_transfer_s(hipStream_t s, int kind, const TransferArgs& A, const SplatCT<S>* sp, const S* knots, const S* ktimes, S* seg,
-                                   S* rec, const TransferLaunch& tl) {
+                                   S* rec, const SplatCf* spf, const f32* knots_f, const TransferLaunch& tl) {
     if (tl.chunk < 1) return hipErrorInvalidValue;
     switch (kind) {
-        case MODEL_THERMAL: return chunk_transfer_k<MODEL_THERMAL, S>(s, A, sp, knots, ktimes, seg, rec, tl);
-        case MODEL_POWERLAW: return chunk_transfer_k<MODEL_POWERLAW, S>(s, A, sp, knots, ktimes, seg, rec, tl);
-        case MODEL_KAPPA: return chunk_transfer_k<MODEL_KAPPA, S>(s, A, sp, knots, ktimes, seg, rec, tl);
-        case MODEL_COMPOSITE: return chunk_transfer_k<MODEL_COMPOSITE, S>(s, A, sp, knots, ktimes, seg, rec, tl);
-        default: return chunk_transfer_k<MODEL_KNOT, S>(s, A, sp, knots, ktimes, seg, rec, tl);
+        case MODEL_THERMAL: return chunk_transfer_k<MODEL_THERMAL, S>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
+        case MODEL_POWERLAW: return chunk_transfer_k<MODEL_POWERLAW, S>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
+        case MODEL_KAPPA: return chunk_transfer_k<MODEL_KAPPA, S>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
+        case MODEL_COMPOSITE: return chunk_transfer_k<MODEL_COMPOSITE, S>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
+        default: return chunk_transfer_k<MODEL_KNOT, S>(s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
     }
 }
 hipError_t launch_chunk_transfer(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                  const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots, const SplatCf* spf,
                                  const f32* knots_f, const f32* ktimes_f, const double* times, int nt, const double* nus, int nnu, double L,
                                  const int* kstop, double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl) {
-    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg,
-                         spf, knots_f, ktimes_f};
-    return chunk_transfer_s<double>(s, kind, A, sp, knots, ktimes, seg, rec, tl);
+    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg};
+    return chunk_transfer_s<double>(s, kind, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);
 }
 hipError_t launch_chunk_transfer_f32(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                      const SplatCf* sp, int ns, const f32* knots, const f32* ktimes, int nknots,
                                      const double* times, int nt, const double* nus, int nnu, double L, const int* kstop,
                                      f32* seg, f32* rec, uint8_t* aflg, const TransferLaunch& tl) {
-    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg,
-                         sp, knots, ktimes};
-    return chunk_transfer_s<f32>(s, kind, A, sp, knots, ktimes, seg, rec, tl);
+    const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg};
+    return chunk_transfer_s<f32>(s, kind, A, sp, knots, ktimes, seg, rec, sp, knots, tl);
 }
 __global__ void ks_iota_i32(int* __restrict__ p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
