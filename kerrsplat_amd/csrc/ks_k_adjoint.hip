@@ -448,7 +448,7 @@ __device__ __forceinline__ void adj_splats_block(int64_t e, int64_t unit, int i,
 // is through. The ticket is taken by all 64 lanes (lane 0 adds one) and made scalar, so the loop's exit and back edge
 // are uniform branches.
 template <class S, int POPS>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Waves<S>::adjelem)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu((adjelem_waves<S, POPS>))))
 ks_adj_splats(double a, double thetao, const double* __restrict__ soa, int64_t npix, int N, Samples smp, const SplatCT<S>* __restrict__ sp,
               const SplatAdjT<S>* __restrict__ sadj, const SplatCf* __restrict__ spf, const f32* __restrict__ knots_f,
               const f32* __restrict__ ktimes_f, const S* __restrict__ knots, const S* __restrict__ ktimes,

@@ -286,7 +286,7 @@ __device__ __forceinline__ void transfer_task(const TransferArgs& A, const Splat
 // wavefront-uniform (scalar) branch, so all lanes of the workgroup iterate together and each pass through the
 // barriers is a pass through the pop.
 template <int KIND, class S, bool CULL>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(Waves<S>::transfer)))
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu((transfer_waves<KIND, S>))))
 ks_chunk_transfer(TransferArgs A, const SplatCT<S>* __restrict__ sp, const S* __restrict__ knots, const S* __restrict__ ktimes,
                   S* __restrict__ seg, S* __restrict__ rec, const SplatCf* __restrict__ spf, const f32* __restrict__ knots_f,
                   const int* __restrict__ tasks, int64_t ntasks, unsigned* __restrict__ head, uint32_t* __restrict__ cost) {

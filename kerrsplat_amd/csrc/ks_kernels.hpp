@@ -82,6 +82,15 @@ inline int64_t adj_units(int64_t nitems, int N) { return ((nitems + 63) / 64) * 
 template <class S> struct Waves;
 template <> struct Waves<double> { static constexpr int transfer = KS_WAVES_TRANSFER64, adjstep = KS_WAVES_ADJSTEP64, adjelem = KS_WAVES_ADJELEM64; };
 template <> struct Waves<f32> { static constexpr int transfer = KS_WAVES_TRANSFER32, adjstep = KS_WAVES_ADJSTEP32, adjelem = KS_WAVES_ADJELEM32; };
+// The FP64 kernels by population: the transfer of thermal and power-law splats is faster within the registers of four
+// waves (128), though its LDS admits two, kappa's needs those of two (at four 61 -> 87 ms); the element adjoints of thermal
+// splats fit two waves, the others' one (kappa at two 121 -> 194 ms, power-law 3.4 -> 6.3). MI355X: transfer of 32 thermal
+// splats at 128^2 x 1024 3.72 -> 3.52 ms, of 6 (50 x 37 x 301) 0.108 -> 0.097, of 48 power-law splats (102 x 67 x 333,
+// 2 frames) 1.63 -> 1.50; element adjoints of the 32 thermal splats 5.92 -> 5.62.
+template <int KIND, class S> constexpr int transfer_waves =
+    std::is_same<S, double>::value && (KIND == MODEL_THERMAL || KIND == MODEL_KNOT || KIND == MODEL_POWERLAW) ? 2 * Waves<S>::transfer : Waves<S>::transfer;
+template <class S, int POPS> constexpr int adjelem_waves =
+    std::is_same<S, double>::value && POPS == POP_THERMAL ? 2 * Waves<S>::adjelem : Waves<S>::adjelem;
 
 // FP32 transfer and adjoint: samples whose Faraday depth |rho| Delta exceeds this take the FP64 step
 // (the step's polynomial in K' cancels strongly at large Faraday depth)
