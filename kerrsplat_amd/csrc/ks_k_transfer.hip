@@ -30,8 +30,8 @@ struct TransferArgs {
 KS_DEV int64_t npix_items(const TransferArgs& A) { return A.npix * A.nt * A.nnu; }
 // A wavefront's workspace in LDS, field-major over its 64 lanes: the geometry of its rays' current sample, the sums of
 // the sample's contributions and whether it has any, the rays' screen coordinates and frequency, the pair queue (lane |
-// splat << 6), the slice's candidate splats. 8.3 KB in FP32 and 16.1 KB in FP64: eight wavefronts a compute unit in FP64, and in FP32 as many as the registers
-// allow fit a compute unit.
+// splat << 6), the slice's candidate splats. 8.3 KB in FP32 and 16.1 KB in FP64: in FP32 as many wavefronts as the
+// registers allow fit a compute unit, in FP64 eight.
 constexpr int QCAP = 256;              // the queue holds < 64 pending pairs and up to 64 pushes of each of two splats
 template <class S>
 struct WaveWork {
