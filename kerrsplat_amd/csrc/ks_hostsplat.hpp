@@ -129,10 +129,12 @@ inline void host_splat_constants(int kind, int nrows, int i, const double* p, do
     }
     {
         // may_weigh's error bound. FP32 rounds a position of size R by R 6e-8 in each of a few operations (1e-6 R covers
-        // them), a time by |t| 6e-8 twice, and the centre moves by v per unit of time; the hardware's sine and cosine are
-        // within 4e-6. Each error enters the scaled coordinate times the largest inverse scale.
+        // them) and a time by |t| 6e-8 twice; the hardware's sine and cosine are within 4e-6. A knot splat's centre moves by
+        // v per unit of time. The test of a pattern splat turns the sample, which weighs up to the support radius beyond the
+        // centre's distance from the axis: that distance, not the centre's, carries the errors of the phase. Each error
+        // enters the scaled coordinate times the largest inverse scale.
         const double is = std::max(std::max(c.is[0], c.is[1]), c.is[2]);
-        const double rho = std::hypot(c.x, c.y);
+        const double rho = std::hypot(c.x, c.y) + (with_knots ? 0.0 : std::sqrt(c.rsup2));
         double R = rho + std::fabs(c.z), v = std::fabs(c.omega) * rho, tmax = std::fabs(c.t0);
         if (with_knots) {
             R = std::sqrt(c.kc[0] * c.kc[0] + c.kc[1] * c.kc[1] + c.kc[2] * c.kc[2]) + c.kr;
@@ -145,7 +147,7 @@ inline void host_splat_constants(int kind, int nrows, int i, const double* p, do
                 v = std::max(v, std::sqrt(d2) / (knot_times[k + 1] - knot_times[k]));
             }
         }
-        R += std::sqrt(c.rsup2);
+        if (with_knots) R += std::sqrt(c.rsup2);
         c.pm0 = 2.0 * is * (1e-6 * R + 4e-6 * rho + 6e-7 * v * tmax) + 6e-7 * std::fabs(c.t0) * c.iw;
         c.pm1 = 2.0 * is * 6e-7 * v + 6e-7 * c.iw;
     }
