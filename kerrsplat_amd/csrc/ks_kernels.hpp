@@ -27,10 +27,23 @@ constexpr int CHUNK = 32;          // samples per work item of the transfer from
 // tasks leave the chip idle for longer than the further maps cost to compose (FP64 transfer of 1024 kappa splats,
 // 112 x 96 x 512: 131 ms with slices of 8, 5376 tasks; 111 of 4; 95 of 2).
 constexpr int64_t SLICE_TASKS = 8192;
-inline int slice_length(int chunk, int64_t nitems, int N) {
+// The maps of one launch stay within MAPS_MAX bytes: slices of a quarter take four times the maps of whole work items (20
+// bytes a sample and frame in FP64 against 5, 10 in FP32, and 8 more behind the records of a dual sweep), which at the
+// largest launches is the card's memory. A render past it runs its frames in groups (frame_group); a launch that cannot be
+// split (one frame, a dual sweep) takes whole work items.
+constexpr int64_t MAPS_MAX = (int64_t)1 << 34;
+inline int64_t maps_bytes(int64_t nitems, int N, int len, int64_t per_map) { return nitems * ((N + len - 1) / len) * per_map; }
+// per_map: the bytes a slice of one item leaves; held: the items whose maps are held together
+inline int slice_length(int chunk, int64_t nitems, int N, int64_t held, int64_t per_map) {
     int len = chunk < 8 ? 2 : chunk / 4;
     while (len >= 4 && (nitems * ((N + len - 1) / len) + 127) / 128 < SLICE_TASKS) len /= 2;
-    return len;
+    return maps_bytes(held, N, len, per_map) > MAPS_MAX ? chunk : len;
+}
+// frames of one frequency in a launch of npix pixels, nt of them when their maps fit together
+inline int frame_group(int nt, int64_t npix, int N, int len, int64_t per_map) {
+    int g = nt;
+    while (g > 1 && maps_bytes(npix * g, N, len, per_map) > MAPS_MAX) g = (g + 1) / 2;
+    return g;
 }
 constexpr int SEG_FIELDS = 20;     // a segment map: P (16, row-major), then Sv (4)
 // the populations an element-adjoint launch meets (a bit mask)

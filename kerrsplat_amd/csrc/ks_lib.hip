@@ -632,16 +632,16 @@ static const double* stage_times(ks_cache* c, const double* times, int nt, const
     return c->dtn;
 }
 
-// Samples per slice of the transfer, and whether its segment maps are FP32 (the mixed path's own numbers, half the bytes
-// of FP64 copies)
-static int slice_of(const ks_cache* c, int64_t items) { return slice_length(c->chunk, items, c->N); }
+// Whether the segment maps are FP32 (the mixed path's own numbers, half the bytes of FP64 copies), and the bytes of a
+// slice's map, with what the reverse pass keeps beside it (w_in, T_out)
 static int seg_is32(const ks_cache* c) { return has_samples(c) && c->precision == KS_PRECISION_MIXED ? 1 : 0; }
-static int64_t seg_doubles(const ks_cache* c, int64_t items) {
-    const int64_t nseg = (c->N + slice_of(c, items) - 1) / slice_of(c, items);
-    return ((int64_t)SEG_FIELDS * nseg * items * (seg_is32(c) ? 4 : 8) + 7) / 8;
-}
-static int ensure_seg(ks_cache* c, int64_t items) {
-    const int64_t need = seg_doubles(c, items);
+static int64_t map_bytes(const ks_cache* c, bool records) { return SEG_FIELDS * (seg_is32(c) ? 4 : 8) + (records ? 64 : 0); }
+// Samples per slice of a launch of `items` (pixel, frame) items: a render's groups of frames hold one frame's maps at the
+// least, a dual sweep all of them
+static int render_slice(const ks_cache* c, int64_t items, int64_t npix) { return slice_length(c->chunk, items, c->N, npix, map_bytes(c, false)); }
+static int sweep_slice(const ks_cache* c, int64_t items) { return slice_length(c->chunk, items, c->N, items, map_bytes(c, true)); }
+static int ensure_seg(ks_cache* c, int64_t items, int slice) {
+    const int64_t need = (maps_bytes(items, c->N, slice, map_bytes(c, false)) + 7) / 8;
     if (c->seg_cap >= need) return KS_OK;
     dfree(c->seg); c->seg_cap = 0;
     if (dalloc(&c->seg, (size_t)need)) return KS_ERR_HIP;
@@ -652,14 +652,14 @@ static int ensure_seg(ks_cache* c, int64_t items) {
 // The launch of the transfer over stored samples as the cache's tuning asks: the work queue in index order, or
 // (KS_QUEUE_TRANSFER) in the cost-descending order of an earlier launch of the same shape when there is one, recording
 // every task's ticks and ordering the tasks by them for the next launch.
-static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, int nt, int nnu, double L, const int* kst, void* rec,
-                           uint8_t* aflg, const TransferLaunch* sample) {
+static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_times, int nt, const double* d_nus, int nnu, double L, int slice,
+                           const int* kst, void* rec, uint8_t* aflg, const TransferLaunch* sample) {
     ks_ctx* x = c->ctx;
     TransferLaunch tl;
-    tl.chunk = slice_of(c, c->npix * nt * nnu);
+    tl.chunk = slice;
     if (c->qhead.grow(1)) return KS_ERR_HIP;
     tl.head = c->qhead.p;
-    const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c, c->npix * nt * nnu));
+    const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, slice);
     bool order_after = false;
     if (sample) {
         tl.tasks = sample->tasks; tl.ntasks = sample->ntasks;
@@ -681,10 +681,10 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, i
     const int kind = m->kind;
     if (c->precision == KS_PRECISION_MIXED)
         HIPCHK(launch_chunk_transfer_f32(x->stream, kind, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats_f, m->ns,
-                                         m->d_knots_f, m->d_ktimes_f, m->nknots, d_tn, nt, d_tn + nt, nnu, L, kst, (f32*)c->seg, (f32*)rec, aflg, tl));
+                                         m->d_knots_f, m->d_ktimes_f, m->nknots, d_times, nt, d_nus, nnu, L, kst, (f32*)c->seg, (f32*)rec, aflg, tl));
     else
         HIPCHK(launch_chunk_transfer(x->stream, kind, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->ns,
-                                     m->d_knots, m->d_ktimes, m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_tn, nt, d_tn + nt, nnu, L, kst,
+                                     m->d_knots, m->d_ktimes, m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_times, nt, d_nus, nnu, L, kst,
                                      c->seg, (double*)rec, aflg, tl));
     if (order_after) {
         size_t bytes = 0;
@@ -698,21 +698,52 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_tn, i
     return KS_OK;
 }
 
-// The transfer of every (pixel, time, frequency) item of the stored samples into the cache's segment maps, with the
-// adjoint's records when rec != nullptr.
-static int launch_transfer(ks_cache* c, const ks_model* m, const double* d_tn, int nt, int nnu, double L, int nmax, double slab,
-                           double* rec, uint8_t* aflg) {
+// the half-orbit cutoff of every ray (null without one: nmax < 0)
+static int wind_cutoff(ks_cache* c, int nmax, double slab, const int** kst) {
+    *kst = nullptr;
+    if (nmax < 0) return KS_OK;
+    if (!c->kstop) { if (dalloc(&c->kstop, (size_t)c->npix)) return KS_ERR_HIP; }
+    HIPCHK(launch_wind_cutoff(c->ctx->stream, c->spin, c->npix, c->N, nmax, slab, samples_of(c), c->kstop));
+    *kst = c->kstop;
+    return KS_OK;
+}
+// The forward pass of a dual sweep: every (pixel, time, frequency) item of the stored samples into the cache's segment
+// maps with the adjoint's records, and the images
+static int sweep_forward(ks_cache* c, const ks_model* m, const double* d_times, int nt, const double* d_nus, int nnu, double L, int nmax, double slab) {
     ks_ctx* x = c->ctx;
-    if (int rc = ensure_seg(c, c->npix * nt * nnu)) return rc;
+    const int64_t items = c->npix * nt * nnu;
+    const int slice = sweep_slice(c, items);
+    if (int rc = ensure_seg(c, items, slice)) return rc;
     const int* kst = nullptr;
-    if (nmax >= 0) {
-        if (!c->kstop) { if (dalloc(&c->kstop, (size_t)c->npix)) return KS_ERR_HIP; }
-        HIPCHK(launch_wind_cutoff(x->stream, c->spin, c->npix, c->N, nmax, slab, samples_of(c), c->kstop));
-        kst = c->kstop;
-    }
+    if (int rc = wind_cutoff(c, nmax, slab, &kst)) return rc;
     HIPCHK(x->stage_begin(KS_STAGE_TRANSFER));
-    if (int rc = transfer_launch(c, m, d_tn, nt, nnu, L, kst, rec, aflg, nullptr)) return rc;
+    if (int rc = transfer_launch(c, m, d_times, nt, d_nus, nnu, L, slice, kst, c->arec, c->aflg, nullptr)) return rc;
     HIPCHK(x->stage_end(KS_STAGE_TRANSFER));
+    HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice, nt, d_nus, nnu, c->seg, seg_is32(c), c->out));
+    c->fw_chunk = slice;
+    return KS_OK;
+}
+// The images of the stored samples, in one launch or, where the segment maps of all frames pass MAPS_MAX, in groups of the
+// frames of one frequency. The slices are the whole render's, so the images do not depend on the groups.
+static int stored_render(ks_cache* c, const ks_model* m, const double* d_times, int nt, const double* d_nus, int nnu, double L, int nmax, double slab) {
+    ks_ctx* x = c->ctx;
+    const int64_t items = c->npix * nt * nnu;
+    const int slice = render_slice(c, items, c->npix);
+    const bool whole = maps_bytes(items, c->N, slice, map_bytes(c, false)) <= MAPS_MAX;
+    const int gt = whole ? nt : frame_group(nt, c->npix, c->N, slice, map_bytes(c, false)), gnu = whole ? nnu : 1;
+    if (int rc = ensure_seg(c, c->npix * gt * gnu, slice)) return rc;
+    const int* kst = nullptr;
+    if (int rc = wind_cutoff(c, nmax, slab, &kst)) return rc;
+    HIPCHK(x->stage_begin(KS_STAGE_TRANSFER));
+    for (int inu = 0; inu < nnu; inu += gnu)
+        for (int it = 0; it < nt; it += gt) {
+            const int nf = std::min(gt, nt - it);
+            if (int rc = transfer_launch(c, m, d_times + it, nf, d_nus + inu, gnu, L, slice, kst, nullptr, nullptr, nullptr)) return rc;
+            if (whole) HIPCHK(x->stage_end(KS_STAGE_TRANSFER));
+            HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice, nf, d_nus + inu, gnu, c->seg, seg_is32(c),
+                                      c->out + (int64_t)4 * c->npix * (it + (int64_t)nt * inu)));
+        }
+    if (!whole) HIPCHK(x->stage_end(KS_STAGE_TRANSFER));
     return KS_OK;
 }
 
@@ -759,13 +790,13 @@ static int fused_render(ks_cache* c, const ks_model* m, const double* d_tn, int 
             kst = c->fkstop.p;
         }
         int group = nt;
-        while (group > 1 && 8 * seg_doubles(c, n * group) > FUSED_SEG) group = (group + 1) / 2;
+        while (group > 1 && maps_bytes(n * group, c->N, render_slice(c, n * group, n), map_bytes(c, false)) > FUSED_SEG) group = (group + 1) / 2;
         for (int inu = 0; inu < nnu; ++inu)
             for (int it = 0; it < nt; it += group) {
                 const int nf = std::min(group, nt - it);
-                if (ensure_seg(c, n * nf) || c->fout.grow((size_t)4 * n * nf)) return KS_ERR_HIP;
                 TransferLaunch tl;
-                tl.chunk = slice_of(c, n * nf);
+                tl.chunk = render_slice(c, n * nf, n);
+                if (ensure_seg(c, n * nf, tl.chunk) || c->fout.grow((size_t)4 * n * nf)) return KS_ERR_HIP;
                 tl.head = c->qhead.p;
                 const double* nu = d_tn + nt + inu;
                 HIPCHK(launch_chunk_transfer(x->stream, m->kind, c->spin, c->thetao, c->fsoa.p, n, c->N, S, m->d_splats, m->ns, m->d_knots, m->d_ktimes,
@@ -794,10 +825,7 @@ int ks_render_device(ks_cache* c, const ks_model* m, const double* times, int nt
     const double* d_tn = stage_times(c, times, nt, nus, nnu);
     if (!d_tn) return KS_ERR_HIP;
     if (!has_samples(c)) return fused_render(c, m, d_tn, nt, nnu, L, nmax, slab);
-    int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, nullptr, nullptr);
-    if (rc) return rc;
-    HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice_of(c, c->npix * frames), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
-    return KS_OK;
+    return stored_render(c, m, d_tn, nt, d_tn + nt, nnu, L, nmax, slab);
 }
 
 int ks_cache_march_precision(ks_cache* c, int precision) {
@@ -904,6 +932,17 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
         const int old[4] = {c->chunk, c->queue, c->patch_a, c->patch_b};
         int best = -1;
         double best_ms = INFINITY;
+        // the frames whose work is sampled: all of them, or the first group of a render that takes them in groups, at the
+        // chunk with the most maps
+        int tnt = nt, tnnu = nnu;
+        if (!records) {
+            c->chunk = chunks[0];
+            const int slice = render_slice(c, items, c->npix);
+            if (maps_bytes(items, c->N, slice, map_bytes(c, false)) > MAPS_MAX) {
+                tnt = frame_group(nt, c->npix, c->N, slice, map_bytes(c, false));
+                tnnu = 1;
+            }
+        }
         std::vector<int> tasks;
         Buf<int> dtasks;
         for (int pc = 0; pc < 3; ++pc) {
@@ -913,8 +952,9 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                 if (chunks[ci] > std::max(c->N, 16)) continue;
                 c->chunk = chunks[ci];
                 if (records && ensure_adj(c, items, std::max(m->ns, 1))) return KS_ERR_HIP;
-                if (int rc = ensure_seg(c, items)) return rc;
-                const int64_t all = transfer_tasks(c->npix, nt, nnu, c->N, slice_of(c, c->npix * nt * nnu));
+                const int slice = records ? sweep_slice(c, items) : render_slice(c, items, c->npix);
+                if (int rc = ensure_seg(c, c->npix * tnt * tnnu, slice)) return rc;
+                const int64_t all = transfer_tasks(c->npix, tnt, tnnu, c->N, slice);
                 // a hashed Bernoulli sample of rate 1 / sample_every (a regular stride aliases with the screen: every k-th
                 // task can fall on one column of patches)
                 tasks.clear();
@@ -933,7 +973,8 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                     float ms = INFINITY;
                     for (int rep = 0; rep < 2; ++rep) {
                         HIPCHK(hipEventRecord(x->ev0, x->stream));
-                        int rc = transfer_launch(c, m, d_tn, nt, nnu, L, nullptr, records ? (void*)c->arec : nullptr, records ? c->aflg : nullptr, &smp);
+                        int rc = transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr,
+                                                 records ? c->aflg : nullptr, &smp);
                         if (rc) { dtasks.release(); return rc; }
                         HIPCHK(hipEventRecord(x->ev1, x->stream));
                         HIPCHK(hipEventSynchronize(x->ev1));
@@ -958,8 +999,7 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
     if (flags & KS_TUNE_ADJOINT) {
         if (m->ns < 1) return fail(KS_ERR_ARG, "the element adjoints need splats");
         if (ensure_out(c, frames) || ensure_adj(c, items, m->ns)) return KS_ERR_HIP;
-        if (int rc = launch_transfer(c, m, d_tn, nt, nnu, L, -1, 0.0, c->arec, c->aflg)) return rc;
-        c->fw_chunk = slice_of(c, items);
+        if (int rc = sweep_forward(c, m, d_tn, nt, d_tn + nt, nnu, L, -1, 0.0)) return rc;
         HIPCHK(hipMemsetAsync(c->ads, 0, (size_t)4 * items * sizeof(double), x->stream));
         int best_q = c->queue;
         double best_ms = INFINITY;
@@ -1007,7 +1047,7 @@ static int64_t adj_unit_batch(int64_t nunits, int ns) {
 }
 
 static int ensure_adj(ks_cache* c, int64_t items, int ns) {
-    const int nseg = (c->N + slice_of(c, items) - 1) / slice_of(c, items);
+    const int slice = sweep_slice(c, items), nseg = (c->N + slice - 1) / slice;
     if (c->a_items < items) {
         dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->ads);
         c->a_items = 0;
@@ -1099,11 +1139,8 @@ int ks_gradient_forward(ks_cache* c, const ks_model* m, const double* times, int
     if (ensure_out(c, frames) || ensure_adj(c, items, ns > 0 ? ns : 1)) return KS_ERR_HIP;
     const double* d_tn = stage_times(c, times, nt, nus, nnu);
     if (!d_tn) return KS_ERR_HIP;
-    int rc = launch_transfer(c, m, d_tn, nt, nnu, L, nmax, slab, c->arec, c->aflg);
-    if (rc) return rc;
-    HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice_of(c, items), nt, d_tn + nt, nnu, c->seg, seg_is32(c), c->out));
+    if (int rc = sweep_forward(c, m, d_tn, nt, d_tn + nt, nnu, L, nmax, slab)) return rc;
     c->fw_model = m->id; c->fw_nt = nt; c->fw_nnu = nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
-    c->fw_chunk = slice_of(c, items);
     c->fw_seeded.assign((size_t)frames, 0);
     if (image) return ks_copy_stokes(c, frames, image, screen_order);
     return KS_OK;
@@ -1685,8 +1722,7 @@ static int graph_record(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpyAsync(m->d_splats_f, g->h_spf, ns * sizeof(SplatCf), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(m->d_adj_f, g->h_adf, ns * sizeof(SplatAdjf), hipMemcpyHostToDevice, s));
     const int nt = g->nt, nnu = g->nnu;
-    if (int rc = launch_transfer(c, m, g->dtn.p, nt, nnu, g->L, -1, 0.0, c->arec, c->aflg)) return rc;
-    HIPCHK(launch_seg_combine(s, c->npix, c->N, slice_of(c, c->npix * g->frames), nt, g->dtn.p + nt, nnu, c->seg, seg_is32(c), c->out));
+    if (int rc = sweep_forward(c, m, g->dtn.p, nt, g->dtn.p + nt, nnu, g->L, -1, 0.0)) return rc;
     const int na = c->nalpha, nb = c->nbeta;
     for (int f = 0; f < g->frames; ++f) {
         if (g->loss == KS_LOSS_IMAGE) {
@@ -1735,7 +1771,6 @@ static int graph_capture(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpy(g->h_ad, m->d_adj, m->ns * sizeof(SplatAdj), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(g->h_spf, m->d_splats_f, m->ns * sizeof(SplatCf), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(g->h_adf, m->d_adj_f, m->ns * sizeof(SplatAdjf), hipMemcpyDeviceToHost));
-    c->fw_chunk = slice_of(c, items);
     if (int rc = graph_record(g, m)) return rc;
     HIPCHK(hipStreamSynchronize(x->stream));
     // the capture
@@ -1836,7 +1871,7 @@ int ks_fit_graph_step(ks_graph* g, const ks_model* m, const double* params, doub
     g->replays += 1;
     // the forward pass the graph ran is the cache's: images and seeds as after ks_gradient_forward + the seeds
     c->fw_model = m->id; c->fw_nt = g->nt; c->fw_nnu = g->nnu; c->fw_generation = c->generation; c->fw_precision = c->precision;
-    c->fw_chunk = slice_of(c, c->npix * g->frames);
+    c->fw_chunk = sweep_slice(c, c->npix * g->frames);
     c->fw_seeded.assign((size_t)g->frames, 1);
     double s = 0.0;
     for (int f = 0; f < g->frames; ++f) s += g->h_chi[f];
