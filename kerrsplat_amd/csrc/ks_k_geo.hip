@@ -58,7 +58,8 @@ struct StoreF {
     Samples S; int64_t j, npix; double a, rp, rm;
     KS_DEV void operator()(int k, const Samp& s, double) {
         const int64_t o = (int64_t)(k - 1) * npix + j;
-        S.t[o] = s.t; S.r[o] = s.r; S.th[o] = s.th; S.ph[o] = s.ph;
+        S.t[o] = s.t; S.r[o] = s.r; S.th[o] = s.th;
+        if (S.ph) S.ph[o] = s.ph;                   // (a tile's samples are kept without phi)
         S.fl[o] = (uint8_t)((s.ok ? 1 : 0) | (s.nur ? 2 : 0) | (s.nuth ? 4 : 0));
         double x, y, z;
         quasi_cartesian_ks(a, rp, rm, s.r, s.th, s.ph, x, y, z);

@@ -359,8 +359,18 @@ __global__ void __launch_bounds__(128) ks_thin_parts(double a, const double* __r
 __global__ void ks_thin_combine(int64_t npix, int nseg_max, const double* __restrict__ part, double* __restrict__ out) {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= npix) return;
+    // one thread a pixel: COMBINE_GROUP loads in flight, added in order (one at a time, 8192 pixels of 256 chunks took 76 us)
+    constexpr int COMBINE_GROUP = 16;
     double s = 0.0;
-    for (int m = 0; m < nseg_max; ++m) s += part[m * npix + j];
+    int m = 0;
+    for (; m + COMBINE_GROUP <= nseg_max; m += COMBINE_GROUP) {
+        double v[COMBINE_GROUP];
+#pragma unroll
+        for (int u = 0; u < COMBINE_GROUP; ++u) v[u] = part[(int64_t)(m + u) * npix + j];
+#pragma unroll
+        for (int u = 0; u < COMBINE_GROUP; ++u) s += v[u];
+    }
+    for (; m < nseg_max; ++m) s += part[(int64_t)m * npix + j];
     out[j] = s;
 }
 

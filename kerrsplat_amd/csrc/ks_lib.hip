@@ -128,9 +128,7 @@ struct ks_cache {
     float4* sp4 = nullptr;                                     // their FP32 copy with t~ (x, y, z, t) for the FP32 element adjoints
     int64_t march_version = 0, p4_version = -1;                // marches into the samples; the march the copy was made from
     Buf<double> thin_part;                                     // per-chunk thin sums (thin_chunks x npix, or a tile's)
-    // caches without stored samples: one tile's samples, constants, anchor residuals (per segment, per pixel), half-orbit
-    // cutoff and images
-    Buf<double> ft, fr, fth, fph, fx, fy, fz, fsoa, fres, frt, frp, fout; Buf<uint8_t> ffl; Buf<int> fkstop;
+    Buf<double> fws;                                           // caches without stored samples: one tile's workspace (FusedTile)
     double *rt = nullptr, *rp = nullptr;
     double* out = nullptr; int64_t out_frames = 0;    // sorted-order Stokes images
     double* out_screen = nullptr;
@@ -307,10 +305,9 @@ int ks_cache_destroy(ks_cache* c) {
     dfree(c->sx); dfree(c->sy); dfree(c->sz); dfree(c->sp4);
     dfree(c->out); dfree(c->out_screen); dfree(c->img1);
     for (Buf<double>* b : {&c->vu, &c->vv, &c->vt, &c->vg, &c->vd, &c->vs, &c->vA2, &c->vB2, &c->vIm, &c->vC2, &c->vV, &c->vwq, &c->vE2,
-                           &c->vSd, &c->vSp, &c->vchi, &c->vsum, &c->idata, &c->isig, &c->bseed, &c->thin_part, &c->ft, &c->fr, &c->fth, &c->fph,
-                           &c->fx, &c->fy, &c->fz, &c->fsoa, &c->fres, &c->frt, &c->frp, &c->fout})
+                           &c->vSd, &c->vSp, &c->vchi, &c->vsum, &c->idata, &c->isig, &c->bseed, &c->thin_part, &c->fws})
         b->release();
-    c->imask.release(); c->ffl.release(); c->fkstop.release();
+    c->imask.release();
     c->ctri.release(); c->cquad.release(); c->coff.release(); c->clegs.release(); c->cdat.release(); c->cterm.release();
     dfree(c->seg); dfree(c->segres); dfree(c->kstop); dfree(c->dtn);
     dfree(c->arec); dfree(c->abar); dfree(c->aflg); dfree(c->atail); dfree(c->awT); dfree(c->ads); dfree(c->apart); dfree(c->adpar);
@@ -748,62 +745,77 @@ static int stored_render(ks_cache* c, const ks_model* m, const double* d_times, 
 }
 
 // Caches without stored samples march a tile of the pixels at a time into a workspace of at most FUSED_SAMPLES samples
-// (57 bytes each, 0.5 GB; at least FUSED_MIN pixels) and run the transfer of stored samples over it, the frames in
-// groups whose segment maps stay within FUSED_SEG bytes. A tile is a run of the wavefront order. Marched inside the
+// (49 bytes each, 0.8 GB; at least FUSED_MIN pixels) and run the transfer of stored samples over it, the frames in
+// groups whose segment maps stay within FUSED_SEG bytes. A tile is a run of the wavefront order; with tiles of half the
+// samples the march's tail at each tile's end made thin images of large screens slower than one launch (256 x 256 x 1024,
+// 8 splats: 10.85 ms, 10.05 with these). Marched inside the
 // transport instead, every frame marched its own rays, one thread a segment of 64 samples with the pairs of its splats
 // in turn: 6.6 ms and 3.6 more for the half-orbit cutoff at 96 x 72 x 500 and 16 splats; the whole call now takes 1.9 ms
 // (8.6 before). 200 kappa splats on knots, 96 x 72 x 400: 172 -> 12 ms.
-constexpr int64_t FUSED_SAMPLES = (int64_t)1 << 23, FUSED_MIN = 8, FUSED_SEG = (int64_t)1 << 29;
+constexpr int64_t FUSED_SAMPLES = (int64_t)1 << 24, FUSED_MIN = 8, FUSED_SEG = (int64_t)1 << 30;
 static int64_t fused_tile(const ks_cache* c) {
     const int64_t n = std::max(FUSED_SAMPLES / c->N, FUSED_MIN);
     return std::min(n >= 128 ? n / 128 * 128 : n, c->npix);
 }
-// the samples and constants of the tile s0 .. s0 + n - 1; the anchor residuals to the cache's
-static int fused_march(ks_cache* c, int64_t s0, int64_t n, Samples& S) {
-    ks_ctx* x = c->ctx;
+// A tile's workspace, in one allocation made for the cache's largest tile (a call on a new cache waits for it): the samples
+// (phi is not kept), constants, anchor residuals per segment and per pixel, half-orbit cutoff, and the caller's doubles
+struct FusedTile {
+    Samples S;
+    double *soa, *res, *rt, *rp, *extra;
+    int* kstop;
+};
+static int fused_tile_buffers(ks_cache* c, int64_t n, int64_t extra, FusedTile& T) {
     const size_t ns = (size_t)n * c->N, nseg = (size_t)max_segments(c->N);
-    if (c->ft.grow(ns) || c->fr.grow(ns) || c->fth.grow(ns) || c->fph.grow(ns) || c->fx.grow(ns) || c->fy.grow(ns) || c->fz.grow(ns) ||
-        c->ffl.grow(ns) || c->fsoa.grow((size_t)PF_COUNT * n) || c->fres.grow(2 * nseg * n) || c->frt.grow(n) || c->frp.grow(n))
-        return KS_ERR_HIP;
-    S.t = c->ft.p; S.r = c->fr.p; S.th = c->fth.p; S.ph = c->fph.p; S.x = c->fx.p; S.y = c->fy.p; S.z = c->fz.p; S.fl = c->ffl.p;
-    S.tmap = nullptr; S.p4 = nullptr;
-    HIPCHK(launch_tile_gather(x->stream, c->soa, c->npix, c->tmap, s0, n, c->fsoa.p));
-    HIPCHK(launch_march_store(x->stream, c->spin, c->thetao, c->fsoa.p, n, c->N, c->M, 1, (int)nseg, S, c->fres.p, 0));
-    HIPCHK(launch_res_reduce(x->stream, n, (int)nseg, c->fres.p, c->frt.p, c->frp.p));
-    HIPCHK(launch_tile_scatter1(x->stream, c->frt.p, c->tmap, s0, n, c->rt));
-    HIPCHK(launch_tile_scatter1(x->stream, c->frp.p, c->tmap, s0, n, c->rp));
+    const size_t doubles = 6 * ns + (size_t)(PF_COUNT + 2 + 2 * nseg) * n + extra, ints = (size_t)n;
+    if (c->fws.grow(doubles + (ints + 1) / 2 + (ns + 7) / 8)) return KS_ERR_HIP;
+    double* p = c->fws.p;
+    T.S.t = p; T.S.r = p + ns; T.S.th = p + 2 * ns; T.S.x = p + 3 * ns; T.S.y = p + 4 * ns; T.S.z = p + 5 * ns;
+    T.S.ph = nullptr; T.S.tmap = nullptr; T.S.p4 = nullptr;
+    p += 6 * ns;
+    T.soa = p; p += PF_COUNT * n;
+    T.res = p; p += 2 * nseg * n;
+    T.rt = p; T.rp = p + n; T.extra = p + 2 * n;
+    T.kstop = (int*)(c->fws.p + doubles);
+    T.S.fl = (uint8_t*)(c->fws.p + doubles + (ints + 1) / 2);
+    return KS_OK;
+}
+// the samples and constants of the tile s0 .. s0 + n - 1; the anchor residuals to the cache's
+static int fused_march(ks_cache* c, int64_t s0, int64_t n, const FusedTile& T) {
+    ks_ctx* x = c->ctx;
+    const int nseg = max_segments(c->N);
+    HIPCHK(launch_tile_gather(x->stream, c->soa, c->npix, c->tmap, s0, n, T.soa));
+    HIPCHK(launch_march_store(x->stream, c->spin, c->thetao, T.soa, n, c->N, c->M, 1, nseg, T.S, T.res, 0));
+    HIPCHK(launch_res_reduce(x->stream, n, nseg, T.res, T.rt, T.rp));
+    HIPCHK(launch_tile_scatter1(x->stream, T.rt, c->tmap, s0, n, c->rt));
+    HIPCHK(launch_tile_scatter1(x->stream, T.rp, c->tmap, s0, n, c->rp));
     return KS_OK;
 }
 static int fused_render(ks_cache* c, const ks_model* m, const double* d_tn, int nt, int nnu, double L, int nmax, double slab) {
     ks_ctx* x = c->ctx;
     const int64_t tile = fused_tile(c);
-    if (c->qhead.grow(1)) return KS_ERR_HIP;
+    int group = nt;
+    while (group > 1 && maps_bytes(tile * group, c->N, render_slice(c, tile * group, tile), map_bytes(c, false)) > FUSED_SEG) group = (group + 1) / 2;
+    FusedTile T;
+    if (c->qhead.grow(1) || fused_tile_buffers(c, tile, 4 * tile * group, T)) return KS_ERR_HIP;
     HIPCHK(x->stage_begin(KS_STAGE_TRANSFER));
     for (int64_t s0 = 0; s0 < c->npix; s0 += tile) {
         const int64_t n = std::min(tile, c->npix - s0);
-        Samples S;
-        if (int rc = fused_march(c, s0, n, S)) return rc;
-        const int* kst = nullptr;
-        if (nmax >= 0) {
-            if (c->fkstop.grow(n)) return KS_ERR_HIP;
-            HIPCHK(launch_wind_cutoff(x->stream, c->spin, n, c->N, nmax, slab, S, c->fkstop.p));
-            kst = c->fkstop.p;
-        }
-        int group = nt;
-        while (group > 1 && maps_bytes(n * group, c->N, render_slice(c, n * group, n), map_bytes(c, false)) > FUSED_SEG) group = (group + 1) / 2;
+        if (int rc = fused_march(c, s0, n, T)) return rc;
+        if (nmax >= 0) HIPCHK(launch_wind_cutoff(x->stream, c->spin, n, c->N, nmax, slab, T.S, T.kstop));
+        const int* kst = nmax >= 0 ? T.kstop : nullptr;
         for (int inu = 0; inu < nnu; ++inu)
             for (int it = 0; it < nt; it += group) {
                 const int nf = std::min(group, nt - it);
                 TransferLaunch tl;
                 tl.chunk = render_slice(c, n * nf, n);
-                if (ensure_seg(c, n * nf, tl.chunk) || c->fout.grow((size_t)4 * n * nf)) return KS_ERR_HIP;
+                if (ensure_seg(c, n * nf, tl.chunk)) return KS_ERR_HIP;
                 tl.head = c->qhead.p;
                 const double* nu = d_tn + nt + inu;
-                HIPCHK(launch_chunk_transfer(x->stream, m->kind, c->spin, c->thetao, c->fsoa.p, n, c->N, S, m->d_splats, m->ns, m->d_knots, m->d_ktimes,
+                HIPCHK(launch_chunk_transfer(x->stream, m->kind, c->spin, c->thetao, T.soa, n, c->N, T.S, m->d_splats, m->ns, m->d_knots, m->d_ktimes,
                                              m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_tn + it, nf, nu, 1, L, kst, c->seg, nullptr, nullptr,
                                              tl));
-                HIPCHK(launch_seg_combine(x->stream, n, c->N, tl.chunk, nf, nu, 1, c->seg, 0, c->fout.p));
-                HIPCHK(launch_tile_scatter4(x->stream, c->fout.p, c->tmap, s0, n, nf, c->npix, c->out + (int64_t)4 * c->npix * (it + (int64_t)nt * inu)));
+                HIPCHK(launch_seg_combine(x->stream, n, c->N, tl.chunk, nf, nu, 1, c->seg, 0, T.extra));
+                HIPCHK(launch_tile_scatter4(x->stream, T.extra, c->tmap, s0, n, nf, c->npix, c->out + (int64_t)4 * c->npix * (it + (int64_t)nt * inu)));
             }
     }
     HIPCHK(x->stage_end(KS_STAGE_TRANSFER));
@@ -1228,14 +1240,15 @@ int ks_thin_image(ks_cache* c, const ks_model* m, double t_obs, double* out, int
         HIPCHK(launch_thin_combine(x->stream, c->npix, nch, c->thin_part.p, c->img1));
     } else {
         const int64_t tile = fused_tile(c);
+        FusedTile T;
+        if (fused_tile_buffers(c, tile, (nch + 1) * tile, T)) return KS_ERR_HIP;
+        double *part = T.extra, *img = T.extra + nch * tile;
         for (int64_t s0 = 0; s0 < c->npix; s0 += tile) {
             const int64_t n = std::min(tile, c->npix - s0);
-            Samples S;
-            if (int rc = fused_march(c, s0, n, S)) return rc;
-            if (c->thin_part.grow((size_t)nch * n) || c->fout.grow((size_t)n)) return KS_ERR_HIP;
-            HIPCHK(launch_thin_parts(x->stream, c->spin, c->fsoa.p, n, c->N, S, m->d_splats, m->ns, t_obs, c->thin_part.p));
-            HIPCHK(launch_thin_combine(x->stream, n, nch, c->thin_part.p, c->fout.p));
-            HIPCHK(launch_tile_scatter1(x->stream, c->fout.p, c->tmap, s0, n, c->img1));
+            if (int rc = fused_march(c, s0, n, T)) return rc;
+            HIPCHK(launch_thin_parts(x->stream, c->spin, T.soa, n, c->N, T.S, m->d_splats, m->ns, t_obs, part));
+            HIPCHK(launch_thin_combine(x->stream, n, nch, part, img));
+            HIPCHK(launch_tile_scatter1(x->stream, img, c->tmap, s0, n, c->img1));
         }
     }
     const double* src = c->img1;
