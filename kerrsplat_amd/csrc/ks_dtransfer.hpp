@@ -47,7 +47,7 @@ enum KappaField : int {
 };
 // The power-law fits' factors, in the same places (power_consts):
 enum PowerField : int {
-    PL_INUC, PL_P2,                // 1 / nu_c, -p / 2
+    PL_INUC, PL_EJ,                // 1 / nu_c, (1 - p) / 2
     PL_J, PL_JQ, PL_JV,            // j_I / (n_e sin X^((1 - p)/2)), j_Q / j_I, j_V sin sqrt(X) / (j_I cos)
     PL_A, PL_AQ, PL_AV,            // alpha_I nu / (n_e X^(-1 - p/2)), alpha_Q / alpha_I, alpha_V's
     PL_RQ, PL_RG, PL_H, PL_RV,     // rho_Q's, 1 / gamma_min^2, 1 - p / 2, rho_V's
@@ -468,7 +468,7 @@ KS_DEV CoefT<T> thermal(NE ne, T Th, T iTh, T k0k2, T k1k2, T B, T nu, T nh, T i
 
 // power law (coefficients.jl:208-256), split as kappa's: its per-splat factors from p, gamma_min, gamma_max and
 // gPL = {Gamma((3p-1)/12) Gamma((3p+19)/12), Gamma((3p+2)/12) Gamma((3p+22)/12)} (power_consts, once per splat), and its
-// evaluation at one sample (power_coefs) from one power X^(-p/2) of X = nu / (nu_c sin), where eleven powers were taken
+// evaluation at one sample (power_coefs) from one power X^((1-p)/2) of X = nu / (nu_c sin), where eleven powers were taken
 // at every pair, seven of them of the splat's numbers alone. MI355X, FP64, 48 splats, 102 x 67 x 333, 2 frames: transfer
 // 3.57 -> 2.02 ms, element adjoints 6.10 -> 3.42 ms.
 template <class T>
@@ -477,7 +477,7 @@ KS_DEV void power_consts(T p, T gmin, T gmax, const T* gPL, T B, KappaK<T>& K) {
     const T gspan = pow(gmin, 1.0 - p) - pow(gmax, 1.0 - p);
     const T h = 0.5 * p - 1.0, lg = log(gmin);
     K.v[PL_INUC] = 1.0 / nuc;
-    K.v[PL_P2] = -0.5 * p;
+    K.v[PL_EJ] = 0.5 - 0.5 * p;
     K.v[PL_J] = EE * EE * nuc / CL * pow(3.0, p * 0.5) * (p - 1.0) / (2.0 * (p + 1.0) * gspan) * gPL[0];
     K.v[PL_JQ] = (p + 1.0) / (p + 7.0 / 3.0);
     K.v[PL_JV] = (171.0 / 250.0) * 1.7320508075688772 * pow(p, 0.49);
@@ -497,20 +497,20 @@ KS_DEV CoefT<T> power_coefs(const KF& K, NE ne, T nu, T inu, T sth, T cth) {
     const T ist = fdiv(T(1.0), sth);
     const T X = nu * K(PL_INUC) * ist, iX = fdiv(T(1.0), X), isX = sqrt(iX);
     const PowBase<T> xb = pow_base(X);
-    const T s = pow_of(xb, K(PL_P2));
-    c.jI = ne * K(PL_J) * sth * (X * isX) * s;
+    const T s = pow_of(xb, K(PL_EJ));               // zero, not infinity times zero, where X passes the scalar's range
+    c.jI = ne * K(PL_J) * sth * s;
     c.jQ = K(PL_JQ) * c.jI;
     c.jV = K(PL_JV) * cth * ist * isX * c.jI;
-    c.aI = ne * inu * K(PL_A) * s * iX;
+    c.aI = ne * inu * K(PL_A) * s * (isX * iX);
     c.aQ = c.aI * K(PL_AQ);
     const T term6 = pow_nonneg(3.1 * sin_pow_m1(sth, cth, 48.0 / 25.0), 64.0 / 125.0);
     const double sgn = cth > 0.0 ? 1.0 : (cth < 0.0 ? -1.0 : 0.0);
     c.aV = c.aI * K(PL_AV) * term6 * isX * sgn;
     // 1 - (gamma_min^2 nu_B / nu)^(p/2 - 1)
     const T m = 1.0 - pow_of(pow_base(X * K(PL_RG)), K(PL_H));
-    const T ri = ne * ist * iX * iX;
-    c.rQ = -(ri * K(PL_RQ)) * iX * m;
-    c.rV = ri * K(PL_RV) * cth * ist;
+    const T ri = ist * iX * iX;
+    c.rQ = -((ne * K(PL_RQ)) * ri) * iX * m;
+    c.rV = (ne * K(PL_RV)) * ri * cth * ist;
     return c;
 }
 
