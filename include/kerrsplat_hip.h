@@ -99,14 +99,16 @@ int ks_cache_march_precision(ks_cache* cache, int precision);
 /* Launch choices of the transfer over stored samples and of the element adjoints. The reference fixes
  * them: one work item per pixel over all N samples, a workgroup of consecutive pixels (cache.jl:234-246
  * splits a screen into even tiles of consecutive pixels). Here: chunk = samples per work item of the
- * transfer (8:1024, default 32), which takes them in slices of a quarter, fewer where the launch is
- * small; the transfer is a persistent grid of the resident workgroups taking tasks of 128 slices from a
- * work queue; queue = bits: KS_QUEUE_TRANSFER, the tasks of a repeated launch in descending order of the
- * ticks each took the last time, else in index order; KS_QUEUE_ADJOINT is kept for
+ * transfer (8:1024, default 32), which takes them in slices: a quarter of them, fewer where the launch is
+ * small, all of them where the slices' maps would pass 16 GiB and the launch cannot be split (a render's
+ * frames go in groups then); the transfer is a persistent grid of the resident workgroups taking tasks of
+ * 128 slices from a work queue; queue = bits: KS_QUEUE_TRANSFER, the tasks of a repeated launch in
+ * descending order of the ticks each took the last time, else in index order; KS_QUEUE_ADJOINT is kept for
  * callers that set it (the element adjoints take their work list from per-XCD queues either way);
  * patch_a x patch_b = the screen patch a wavefront's 64 work
- * items cover (default 8 x 8) within each screen part. The results do not depend on the patch or the
- * launch forms (bit for bit); the chunk length changes the order of the Stokes sums only. */
+ * items cover (default 8 x 8) within each screen part. The results do not depend on the patch, the queue's
+ * order or a render's groups (bit for bit); the slices' length - the chunk, and the number of points, samples
+ * and frames of a call - changes the order of the Stokes sums only. */
 #define KS_QUEUE_TRANSFER 1
 #define KS_QUEUE_ADJOINT 2
 int ks_cache_tuning(ks_cache* cache, int chunk, int queue, int patch_a, int patch_b);
@@ -118,11 +120,13 @@ int ks_cache_get_tuning(const ks_cache* cache, int* chunk, int* queue, int* patc
 int ks_cache_set_parts(ks_cache* cache, int nparts, const int* n_alpha, const int* n_beta);
 /* The autotuner (no counterpart in the reference). Unless flags has KS_TUNE_KEEP_TRANSFER: times every launch
  * choice of the transfer (chunk 16, 32, 64, 128 x patch 8x8, 16x4, 4x16 x the two orders of its queue) on
- * a hashed sample of 1 / sample_every of its tasks for (times, nus), with the dual sweep's records written
- * when flags has KS_TUNE_RECORDS, and keeps the fastest. With KS_TUNE_ADJOINT: one forward pass with the
- * records, then the reverse pass in each launch form of the element adjoints, and keeps the faster.
+ * a hashed sample of 1 / sample_every of its tasks for (times, nus) - the first group of their frames where a
+ * render takes them in groups -, with the dual sweep's records written when flags has KS_TUNE_RECORDS, and
+ * keeps the fastest. The cost order is that of the sample's own ticks in index order, its recording and sorting
+ * counted. With KS_TUNE_ADJOINT: one forward pass with the records, then the reverse pass once (the element
+ * adjoints have one launch form; the cache's KS_QUEUE_ADJOINT bit stays).
  * table[5 q + {0..4}] = (chunk, patch_a, patch_b, queue bits, milliseconds) of candidate q (the element
- * adjoints' rows with chunk 0; at most cap rows); *ncand = the candidates timed. Leaves no forward pass
+ * adjoints' row with chunk 0; at most cap rows); *ncand = the candidates timed. Leaves no forward pass
  * to reverse. */
 #define KS_TUNE_RECORDS 1
 #define KS_TUNE_ADJOINT 2

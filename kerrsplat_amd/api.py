@@ -425,9 +425,9 @@ def _set_parts(cache, camera):
 
 def tuning(cache, chunk=None, queue=None, patch=None, adjoint_queue=None):
     """The launch choices of the cache's transfer over stored samples and of its element adjoints: samples per work
-    item (chunk), the cost order of the transfer's work queue (queue), the element adjoints' persistent form
-    (adjoint_queue), the wavefront's screen patch (patch = (n_alpha, n_beta) points); arguments left at None keep
-    their value. Returns the current choices as a dict."""
+    item (chunk), the cost order of the transfer's work queue (queue), adjoint_queue (kept for callers that set it: the
+    element adjoints have one launch form), the wavefront's screen patch (patch = (n_alpha, n_beta) points); arguments
+    left at None keep their value. Returns the current choices as a dict."""
     lib = cache._lib
     c, q, pa, pb = _i(), _i(), _i(), _i()
     _check(lib.ks_cache_get_tuning(cache._h, ctypes.byref(c), ctypes.byref(q), ctypes.byref(pa), ctypes.byref(pb)))
@@ -443,12 +443,11 @@ def tuning(cache, chunk=None, queue=None, patch=None, adjoint_queue=None):
 
 
 def autotune(cache, model, times, nus, L, records=True, sample_every=16, adjoint=False, transfer=True):
-    """The autotuner: times every launch choice of the transfer (chunk 16/32/64/128 x patch 8x8/16x4/4x16 x queue
-    off/on) on a hashed sample of 1 / sample_every of the transfer's tasks for (times, nus) (records = the dual
-    sweep's records written, as in gradient_forward) and keeps the fastest on the cache (transfer=False keeps the
-    cache's transfer choices); with adjoint, also times one reverse pass in each launch form of the element adjoints
-    and keeps the faster. Returns (choice, table), table = [(chunk, (patch_a, patch_b), queue bits, ms), ...] (the
-    element adjoints' rows with chunk 0)."""
+    """The autotuner: times every launch choice of the transfer (chunk 16/32/64/128 x patch 8x8/16x4/4x16 x the queue's
+    index and cost order) on a hashed sample of 1 / sample_every of the transfer's tasks for (times, nus) (records = the
+    dual sweep's records written, as in gradient_forward) and keeps the fastest on the cache (transfer=False keeps the
+    cache's transfer choices); with adjoint, also times one reverse pass. Returns (choice, table), table = [(chunk,
+    (patch_a, patch_b), queue bits, ms), ...] (the element adjoints' row with chunk 0)."""
     m = _as_model(model, "thermal")
     tv, nv = _f64(np.atleast_1d(times)), _f64(np.atleast_1d(nus))
     cap = 64

@@ -659,7 +659,7 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_times
     const int64_t ntasks = transfer_tasks(c->npix, nt, nnu, c->N, slice);
     bool order_after = false;
     if (sample) {
-        tl.tasks = sample->tasks; tl.ntasks = sample->ntasks;
+        tl.tasks = sample->tasks; tl.ntasks = sample->ntasks; tl.cost = sample->cost;
     }
     if (c->queue & KS_QUEUE_TRANSFER) {
         if (!sample && x->capturing) {
@@ -911,14 +911,22 @@ int ks_queue_costs(const ks_cache* c, int64_t* ntasks, uint32_t* cost, int cap) 
     return KS_OK;
 }
 
+// The tuner's own buffers (the cost order that an earlier launch left on the cache stays)
+struct TunerBufs {
+    Buf<int> tasks, ids, order;
+    Buf<uint32_t> cost, keys;
+    Buf<uint8_t> tmp;
+    ~TunerBufs() { tasks.release(); ids.release(); order.release(); cost.release(); keys.release(); tmp.release(); }
+};
 // The autotuner. Transfer (unless KS_TUNE_KEEP_TRANSFER): every candidate launch (samples per work item x wavefront
-// patch x launch form) timed with HIP events on a sample of the transfer's work (each task of the candidate's own
+// patch x the queue's order) timed with HIP events on a sample of the transfer's work (each task of the candidate's own
 // task list with probability 1 / sample_every, by a hash of its index: the same fraction of the (item, sample)
-// pairs for every candidate, spread over the whole screen), twice, the faster run counting. Element adjoints (with
-// KS_TUNE_ADJOINT): one forward pass with the records at the chosen transfer, then the reverse pass once in each
-// launch form of the element adjoints, timed by their stage events (zero seeds: the work does not depend on them).
-// The cache keeps the fastest of each; rows of the table: (chunk, patch_a, patch_b, queue bits, ms), the element
-// adjoints' rows with chunk = 0.
+// pairs for every candidate, spread over the whole screen), twice, the faster run counting. The cost order is timed as a
+// launch takes it: the sample's tasks in descending order of the ticks of a run in index order, recording its own ticks and
+// sorting them. Element adjoints (with KS_TUNE_ADJOINT): they have one launch form, whose reverse pass is timed once after
+// a forward pass with the records at the chosen transfer, by its stage events (zero seeds: the work does not depend on
+// them). The cache keeps the fastest transfer; rows of the table: (chunk, patch_a, patch_b, queue bits, ms), the element
+// adjoints' row with chunk = 0.
 int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, const double* nus, int nnu, double L, int flags, int sample_every,
                 double* table, int cap, int* ncand) {
     if (!c || !m || !times || !nus || !ncand) return fail(KS_ERR_ARG, "ks_autotune: null argument");
@@ -956,7 +964,10 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
             }
         }
         std::vector<int> tasks;
-        Buf<int> dtasks;
+        TunerBufs d;
+        auto run = [&](const TransferLaunch& smp, int slice) {
+            return transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr, records ? c->aflg : nullptr, &smp);
+        };
         for (int pc = 0; pc < 3; ++pc) {
             c->patch_a = patches[pc][0]; c->patch_b = patches[pc][1];
             if (int rc = build_tmap(c)) return rc;
@@ -976,18 +987,31 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                     if (h % (uint64_t)sample_every == 0) tasks.push_back((int)q);
                 }
                 if (tasks.empty()) tasks.push_back(0);
-                if (dtasks.grow(tasks.size())) return KS_ERR_HIP;
-                HIPCHK(hipMemcpy(dtasks.p, tasks.data(), tasks.size() * sizeof(int), hipMemcpyHostToDevice));
+                const size_t nsamp = tasks.size();
+                size_t bytes = 0;
+                HIPCHK(launch_order_tasks(x->stream, d.cost.p, (int64_t)nsamp, nullptr, nullptr, nullptr, nullptr, bytes));
+                if (d.tasks.grow(nsamp) || d.cost.grow((size_t)all) || d.keys.grow(nsamp) || d.ids.grow(nsamp) || d.order.grow(nsamp) ||
+                    d.tmp.grow(std::max<size_t>(bytes, 1)))
+                    return KS_ERR_HIP;
                 TransferLaunch smp;
-                smp.tasks = dtasks.p; smp.ntasks = (int64_t)tasks.size();
+                smp.tasks = d.tasks.p; smp.ntasks = (int64_t)nsamp;
                 for (int qu = 0; qu < 2; ++qu) {
-                    c->queue = qu | adj_bit;
+                    if (qu) {          // the ticks of a run in index order, and the sample sorted by them
+                        HIPCHK(launch_fill_i32(x->stream, (int*)d.cost.p, all, 0));
+                        smp.cost = d.cost.p;
+                        if (int rc = run(smp, slice)) return rc;
+                        std::vector<uint32_t> cost((size_t)all);
+                        HIPCHK(hipStreamSynchronize(x->stream));
+                        HIPCHK(hipMemcpy(cost.data(), d.cost.p, (size_t)all * sizeof(uint32_t), hipMemcpyDeviceToHost));
+                        std::stable_sort(tasks.begin(), tasks.end(), [&](int p, int q) { return cost[p] > cost[q]; });
+                    }
+                    HIPCHK(hipMemcpy(d.tasks.p, tasks.data(), nsamp * sizeof(int), hipMemcpyHostToDevice));
+                    c->queue = qu ? KS_QUEUE_TRANSFER | adj_bit : adj_bit;
                     float ms = INFINITY;
                     for (int rep = 0; rep < 2; ++rep) {
                         HIPCHK(hipEventRecord(x->ev0, x->stream));
-                        int rc = transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr,
-                                                 records ? c->aflg : nullptr, &smp);
-                        if (rc) { dtasks.release(); return rc; }
+                        if (int rc = run(smp, slice)) return rc;
+                        if (qu) HIPCHK(launch_order_tasks(x->stream, d.cost.p, (int64_t)nsamp, d.keys.p, d.ids.p, d.order.p, d.tmp.p, bytes));
                         HIPCHK(hipEventRecord(x->ev1, x->stream));
                         HIPCHK(hipEventSynchronize(x->ev1));
                         float t = 0.0f;
@@ -1000,7 +1024,6 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                 }
             }
         }
-        dtasks.release();
         if (best < 0) { c->chunk = old[0]; c->queue = old[1]; c->patch_a = old[2]; c->patch_b = old[3]; }
         else {
             c->chunk = (int)rows[5 * best]; c->patch_a = (int)rows[5 * best + 1]; c->patch_b = (int)rows[5 * best + 2];
@@ -1013,19 +1036,12 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
         if (ensure_out(c, frames) || ensure_adj(c, items, m->ns)) return KS_ERR_HIP;
         if (int rc = sweep_forward(c, m, d_tn, nt, d_tn + nt, nnu, L, -1, 0.0)) return rc;
         HIPCHK(hipMemsetAsync(c->ads, 0, (size_t)4 * items * sizeof(double), x->stream));
-        int best_q = c->queue;
-        double best_ms = INFINITY;
-        for (int qa = 0; qa < 2; ++qa) {
-            c->queue = (c->queue & KS_QUEUE_TRANSFER) | (qa ? KS_QUEUE_ADJOINT : 0);
-            if (int rc = reverse_launches(c, m, d_tn, nt, nnu)) return rc;
-            HIPCHK(hipStreamSynchronize(x->stream));
-            float ms = 0.0f;
-            HIPCHK(hipEventElapsedTime(&ms, x->evs[KS_STAGE_ADJ_ELEMENTS][0], x->evs[KS_STAGE_ADJ_ELEMENTS][1]));
-            rows.insert(rows.end(), {0.0, 0.0, 0.0, (double)c->queue, (double)ms});
-            ++n;
-            if (ms < best_ms) { best_ms = ms; best_q = c->queue; }
-        }
-        c->queue = best_q;
+        if (int rc = reverse_launches(c, m, d_tn, nt, nnu)) return rc;
+        HIPCHK(hipStreamSynchronize(x->stream));
+        float ms = 0.0f;
+        HIPCHK(hipEventElapsedTime(&ms, x->evs[KS_STAGE_ADJ_ELEMENTS][0], x->evs[KS_STAGE_ADJ_ELEMENTS][1]));
+        rows.insert(rows.end(), {0.0, 0.0, 0.0, (double)c->queue, (double)ms});
+        ++n;
     }
     c->fw_model = 0;
     *ncand = n;
