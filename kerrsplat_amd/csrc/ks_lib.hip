@@ -172,6 +172,7 @@ struct ks_cache {
     Buf<uint8_t> qtmp;
     int64_t q_shape[6] = {-1, -1, -1, -1, -1, -1};
     bool q_ordered = false;
+    const int* graph_order = nullptr;                  // while an iteration is captured: its own copy of the queue's order
 };
 
 // Binning (camera.jl:62-80) on the device: the points of every pixel as a list in ascending screen order
@@ -663,9 +664,10 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_times
     }
     if (c->queue & KS_QUEUE_TRANSFER) {
         if (!sample && x->capturing) {
-            // a captured launch takes the order the last eager launch of this shape left, and records nothing
+            // a captured launch takes a copy of the order that the eager iteration before it left (a later eager launch of
+            // another shape orders other tasks in the cache's), and records nothing
             const int64_t shape[6] = {ntasks, c->chunk, (int64_t)m->id, c->precision, rec ? 1 : 0, (int64_t)nt * 65536 + nnu};
-            if (c->q_ordered && std::equal(shape, shape + 6, c->q_shape)) { tl.tasks = c->qorder.p; tl.ntasks = ntasks; }
+            if (c->graph_order && c->q_ordered && std::equal(shape, shape + 6, c->q_shape)) { tl.tasks = c->graph_order; tl.ntasks = ntasks; }
         } else if (!sample) {
             const int64_t shape[6] = {ntasks, c->chunk, (int64_t)m->id, c->precision, rec ? 1 : 0, (int64_t)nt * 65536 + nnu};
             if (!std::equal(shape, shape + 6, c->q_shape)) { std::copy(shape, shape + 6, c->q_shape); c->q_ordered = false; }
@@ -1718,6 +1720,7 @@ struct ks_graph {
     int gen = -1, prec = -1, chunk = -1, queue = -1, pa = -1, pb = -1;
     hipGraph_t graph = nullptr; hipGraphExec_t exec = nullptr;
     int64_t replays = 0, captures = 0;
+    Buf<int> order;                                    // the work queue's order that the captured transfer takes
 };
 
 static void graph_release_capture(ks_graph* g) {
@@ -1737,7 +1740,7 @@ static void graph_release_host(ks_graph* g) {
 // the cache buffers a captured iteration reads or writes
 static std::vector<const void*> graph_ptrs(const ks_cache* c) {
     return {c->seg, c->out, c->arec, c->abar, c->aflg, c->atail, c->awT, c->ads, c->apart, c->adpar, c->tmap, c->soa,
-            c->qhead.p, c->qorder.p, c->kstop, c->aheads.p, c->sp4, c->amask.p, c->acount.p, c->afirst.p, c->aat.p, c->alist.p, c->axcd.p, c->asums.p};
+            c->qhead.p, c->kstop, c->aheads.p, c->sp4, c->amask.p, c->acount.p, c->afirst.p, c->aat.p, c->alist.p, c->axcd.p, c->asums.p};
 }
 
 // the iteration's launches on the (capturing) stream
@@ -1802,10 +1805,18 @@ static int graph_capture(ks_graph* g, const ks_model* m) {
     HIPCHK(hipMemcpy(g->h_adf, m->d_adj_f, m->ns * sizeof(SplatAdjf), hipMemcpyDeviceToHost));
     if (int rc = graph_record(g, m)) return rc;
     HIPCHK(hipStreamSynchronize(x->stream));
+    const bool ordered = (c->queue & KS_QUEUE_TRANSFER) && c->q_ordered;
+    if (ordered) {
+        if (g->order.grow((size_t)c->q_shape[0])) return KS_ERR_HIP;
+        HIPCHK(hipMemcpy(g->order.p, c->qorder.p, (size_t)c->q_shape[0] * sizeof(int), hipMemcpyDeviceToDevice));
+        HIPCHK(hipDeviceSynchronize());
+    }
     // the capture
     HIPCHK(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
     x->capturing = true;
+    c->graph_order = ordered ? g->order.p : nullptr;
     const int rc = graph_record(g, m);
+    c->graph_order = nullptr;
     x->capturing = false;
     hipGraph_t gr = nullptr;
     const hipError_t e = hipStreamEndCapture(x->stream, &gr);
@@ -1929,7 +1940,7 @@ int ks_fit_graph_destroy(ks_graph* g) {
     for (Buf<double>* b : {&g->dtn, &g->data, &g->sig, &g->chif, &g->u, &g->v, &g->t, &g->A2, &g->B2, &g->Im, &g->C2, &g->V, &g->wq, &g->E2,
                            &g->Sd, &g->Sp, &g->chi})
         b->release();
-    g->mask.release();
+    g->mask.release(); g->order.release();
     delete g;
     return KS_OK;
 }
