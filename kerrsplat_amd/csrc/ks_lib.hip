@@ -1719,6 +1719,7 @@ struct ks_graph {
     std::vector<const void*> ptrs;
     int gen = -1, prec = -1, chunk = -1, queue = -1, pa = -1, pb = -1;
     hipGraph_t graph = nullptr; hipGraphExec_t exec = nullptr;
+    int64_t march = -1;                                // the march whose FP32 samples (sp4) the mixed path's iteration reads
     int64_t replays = 0, captures = 0;
     Buf<int> order;                                    // the work queue's order that the captured transfer takes
 };
@@ -1826,7 +1827,7 @@ static int graph_capture(ks_graph* g, const ks_model* m) {
     HIPCHK(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
     g->m = m; g->m_id = m->id;
     g->ptrs = graph_ptrs(c);
-    g->gen = c->generation; g->prec = c->precision; g->chunk = c->chunk; g->queue = c->queue; g->pa = c->patch_a; g->pb = c->patch_b;
+    g->gen = c->generation; g->prec = c->precision; g->march = c->march_version; g->chunk = c->chunk; g->queue = c->queue; g->pa = c->patch_a; g->pb = c->patch_b;
     g->captures += 1;
     return KS_OK;
 }
@@ -1893,7 +1894,7 @@ int ks_fit_graph_step(ks_graph* g, const ks_model* m, const double* params, doub
     ks_ctx* x = c->ctx;
     HIPCHK(hipSetDevice(x->device));
     const bool stale = !g->exec || m != g->m || m->id != g->m_id || graph_ptrs(c) != g->ptrs || c->generation != g->gen ||
-                       c->precision != g->prec || c->chunk != g->chunk || c->queue != g->queue || c->patch_a != g->pa || c->patch_b != g->pb;
+                       c->precision != g->prec || (c->precision == KS_PRECISION_MIXED && c->march_version != g->march) || c->chunk != g->chunk || c->queue != g->queue || c->patch_a != g->pa || c->patch_b != g->pb;
     if (stale)
         if (int rc = graph_capture(g, m)) return rc;
     // the constants of the new parameters into the pinned staging the graph uploads from
