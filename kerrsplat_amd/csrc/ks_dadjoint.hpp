@@ -112,15 +112,6 @@ KS_DEV void sample_adjoint(const S j4[4], const S a4[4], const S r3[3], S D, con
     }
 }
 
-// whether the splat's weight at the sample passes the cutoff, by the same arithmetic as weight_dlog
-template <class S>
-KS_DEV bool weight_active(const SplatCT<S>& c, S t, S x, S y, S z) {
-    S sp, cp;
-    if (outside_support(c, t, x, y, z, sp, cp)) return false;
-    const S g = gauss_exponent(c, t, x, y, z, sp, cp);
-    return !(g > GEXP_SKIP) && fexp(-0.5 * g) > WEIGHT_CUTOFF;
-}
-
 // rows 7-10 of d ln G: dlnG/dR[a][b] = e_a gu_b (R the rotation of the pattern offset e, gu = dlnG/du) through the
 // normalised quaternion (w, x, y, z)
 template <class S>
@@ -135,20 +126,6 @@ KS_DEV void quat_dlog(const SplatAdjT<S>& sa, const S e[3], const S gu[3], S dl[
     gn[3] = 2.0 * (-2.0 * qz * GR[0] - qw * GR[1] + qx * GR[2] + qw * GR[3] - 2.0 * qz * GR[4] + qy * GR[5] + qx * GR[6] + qy * GR[7]);
     const S ng = qw * gn[0] + qx * gn[1] + qy * gn[2] + qz * gn[3];
     for (int i = 0; i < 4; ++i) dl[6 + i] = (gn[i] - sa.qn[i] * ng) * sa.iqn;
-}
-
-// whether a splat whose centre follows knots passes the weight cutoff at the sample, by the arithmetic of
-// weight_dlog_knot
-template <class S>
-KS_DEV bool weight_active_knot(const SplatCT<S>& c, const S* knots, const S* ktimes, S t, S x, S y, S z) {
-    S cx, cy, cz;
-    knot_centre(c, knots, ktimes, t, cx, cy, cz);
-    const S e0 = x - cx, e1 = y - cy, e2 = z - cz;
-    S q2(0.0);
-    for (int b = 0; b < 3; ++b) { const S q = (c.R[b] * e0 + c.R[3 + b] * e1 + c.R[6 + b] * e2) * c.is[b]; q2 += q * q; }
-    const S tt = (t - c.t0) * c.iw;
-    const S g = q2 + tt * tt;
-    return !(g > GEXP_SKIP) && fexp(-0.5 * g) > WEIGHT_CUTOFF;
 }
 
 // d ln G of a splat whose centre follows knots (trajectories.jl:93-128) with respect to rows 1-12: the centre rows

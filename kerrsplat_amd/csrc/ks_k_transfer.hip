@@ -30,8 +30,8 @@ struct TransferArgs {
 KS_DEV int64_t npix_items(const TransferArgs& A) { return A.npix * A.nt * A.nnu; }
 // A wavefront's workspace in LDS, field-major over its 64 lanes: the geometry of its rays' current sample, the sums of
 // the sample's contributions and whether it has any, the rays' screen coordinates and frequency, the pair queue (lane |
-// splat << 6), the slice's candidate splats. 8.3 KB in FP32 and 16.1 KB in FP64: in FP32 as many wavefronts as the
-// registers allow fit a compute unit, in FP64 eight.
+// splat << 6), the slice's candidate splats. 8.9 KB in FP32 and 16.4 KB in FP64: in FP32 as many wavefronts as the
+// registers allow fit a compute unit (160 KB), in FP64 nine (a workgroup's two: eight).
 constexpr int QCAP = 256;              // the queue holds < 64 pending pairs and up to 64 pushes of each of two splats
 template <class S>
 struct WaveWork {
@@ -39,6 +39,7 @@ struct WaveWork {
     uint64_t mask[CAND_MAX / 64];
     int q[QCAP], act[64];
 };
+static_assert(sizeof(WaveWork<f32>) == 9088 && sizeof(WaveWork<double>) == 16768, "the figures above");
 // Values written by some lanes of the wavefront are read by others: the LDS operations of a wavefront run in order, and
 // the compiler keeps theirs across this.
 KS_DEV void wave_sync() {
@@ -436,7 +437,7 @@ static hipError_t chunk_transfer_c(hipStream_t s, const TransferArgs& A, const S
     // the head and the per-task costs start at zero (fill kernels: no memset nodes in a captured graph)
     hipLaunchKernelGGL(ks_fill_i32, dim3(1), dim3(64), 0, s, tl.head, (int64_t)1, 0);
     if (tl.cost) hipLaunchKernelGGL(ks_fill_i32, dim3(grid_for(ntasks, 256)), dim3(256), 0, s, (int*)tl.cost, ntasks, 0);
-    const int64_t grid = std::min<int64_t>(ntasks, (int64_t)groups * (tl.group_scale > 0 ? tl.group_scale : 1));
+    const int64_t grid = std::min<int64_t>(ntasks, (int64_t)groups);
     hipLaunchKernelGGL((ks_chunk_transfer<KIND, S, CULL>), dim3((unsigned)grid), dim3(128), 0, s, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl.tasks,
                        ntasks, (unsigned*)tl.head, tl.cost);
     return hipGetLastError();
@@ -462,7 +463,7 @@ static hipError_t chunk_transfer_s(hipStream_t s, int kind, const TransferArgs& 
 }
 hipError_t launch_chunk_transfer(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                  const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots, const SplatCf* spf,
-                                 const f32* knots_f, const f32* ktimes_f, const double* times, int nt, const double* nus, int nnu, double L,
+                                 const f32* knots_f, const double* times, int nt, const double* nus, int nnu, double L,
                                  const int* kstop, double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl) {
     const TransferArgs A{a, thetao, soa, npix, N, tl.chunk, (N + tl.chunk - 1) / tl.chunk, smp, ns, nknots, times, nt, nus, nnu, L, kstop, aflg};
     return chunk_transfer_s<double>(s, kind, A, sp, knots, ktimes, seg, rec, spf, knots_f, tl);

@@ -1,11 +1,13 @@
 // Shared layouts of the device buffers and the host launchers of every kernel of libkerrsplat_hip.
 //
-// The kernels live in four translation units compiled separately for gfx950:
-//   ks_k_geo.hip       K0 root cases, the stable case partition, K1 pixel constants, the stored-sample
-//                      march (anchor segments in parallel), the half-orbit cutoff, sorted -> screen
-//   ks_k_transfer.hip  the polarized transfer from stored samples (chunks) or fused with the march
-//                      (anchor segments), thin images, the composition of the segment maps
+// The kernels live in five translation units compiled separately for gfx950:
+//   ks_k_geo.hip       K0 root cases, the stable case partition, K1 pixel constants, the march into samples (a cache's, or
+//                      a tile's of a cache that keeps none; anchor segments in parallel), the half-orbit cutoff, the tiles'
+//                      gather and scatter, sorted -> screen
+//   ks_k_transfer.hip  the polarized transfer of marched samples (slices from a work queue), thin images, the composition
+//                      of the segment maps, per-ray splat lists
 //   ks_k_adjoint.hip   the dual-sweep adjoint over stored samples
+//   ks_k_tangent.hip   the spacetime tangent in duals
 //   ks_k_vis.hip       visibilities
 // ks_lib.hip holds the C-ABI and calls the launchers declared here.
 #pragma once
@@ -259,16 +261,15 @@ struct TransferLaunch {
     int64_t ntasks = 0;            // the list's length
     int* head = nullptr;           // the queue head (one int of device memory; zeroed by the launch)
     uint32_t* cost = nullptr;      // per-task wall-clock ticks, indexed by task (null: not recorded)
-    int group_scale = 1;           // persistent workgroups = resident workgroups x group_scale
 };
 int64_t transfer_tasks(int64_t npix, int nt, int nnu, int N, int chunk);
 hipError_t launch_order_tasks(hipStream_t s, const uint32_t* cost, int64_t n, uint32_t* keys, int* ids, int* order, void* tmp, size_t& tmp_bytes);
 hipError_t launch_fill_i32(hipStream_t s, int* p, int64_t n, int v);
-// (spf, knots_f, ktimes_f: the FP32 copies, which the prefilter of both precisions reads; A.seg takes the maps in the
+// (spf, knots_f: the FP32 copies, which the prefilter of both precisions reads; seg takes the maps in the
 // transfer's scalar)
 hipError_t launch_chunk_transfer(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                  const SplatC* sp, int ns, const double* knots, const double* ktimes, int nknots, const SplatCf* spf,
-                                 const f32* knots_f, const f32* ktimes_f, const double* times, int nt, const double* nus, int nnu, double L,
+                                 const f32* knots_f, const double* times, int nt, const double* nus, int nnu, double L,
                                  const int* kstop, double* seg, double* rec, uint8_t* aflg, const TransferLaunch& tl);
 hipError_t launch_chunk_transfer_f32(hipStream_t s, int kind, double a, double thetao, const double* soa, int64_t npix, int N, Samples smp,
                                      const SplatCf* sp, int ns, const f32* knots, const f32* ktimes, int nknots,

@@ -683,7 +683,7 @@ static int transfer_launch(ks_cache* c, const ks_model* m, const double* d_times
                                          m->d_knots_f, m->d_ktimes_f, m->nknots, d_times, nt, d_nus, nnu, L, kst, (f32*)c->seg, (f32*)rec, aflg, tl));
     else
         HIPCHK(launch_chunk_transfer(x->stream, kind, c->spin, c->thetao, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->ns,
-                                     m->d_knots, m->d_ktimes, m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_times, nt, d_nus, nnu, L, kst,
+                                     m->d_knots, m->d_ktimes, m->nknots, m->d_splats_f, m->d_knots_f, d_times, nt, d_nus, nnu, L, kst,
                                      c->seg, (double*)rec, aflg, tl));
     if (order_after) {
         size_t bytes = 0;
@@ -814,7 +814,7 @@ static int fused_render(ks_cache* c, const ks_model* m, const double* d_tn, int 
                 tl.head = c->qhead.p;
                 const double* nu = d_tn + nt + inu;
                 HIPCHK(launch_chunk_transfer(x->stream, m->kind, c->spin, c->thetao, T.soa, n, c->N, T.S, m->d_splats, m->ns, m->d_knots, m->d_ktimes,
-                                             m->nknots, m->d_splats_f, m->d_knots_f, m->d_ktimes_f, d_tn + it, nf, nu, 1, L, kst, c->seg, nullptr, nullptr,
+                                             m->nknots, m->d_splats_f, m->d_knots_f, d_tn + it, nf, nu, 1, L, kst, c->seg, nullptr, nullptr,
                                              tl));
                 HIPCHK(launch_seg_combine(x->stream, n, c->N, tl.chunk, nf, nu, 1, c->seg, 0, T.extra));
                 HIPCHK(launch_tile_scatter4(x->stream, T.extra, c->tmap, s0, n, nf, c->npix, c->out + (int64_t)4 * c->npix * (it + (int64_t)nt * inu)));
