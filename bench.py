@@ -53,7 +53,7 @@ def parse():
     p.add_argument("--no-tune", action="store_true", help="keep the default launch choices (no autotuner)")
     p.add_argument("--launch", default=None,
                    help="fixed launch choices instead of the autotuner (profiling runs): chunk,queue,patch_a,patch_b,"
-                        "adjoint_queue_mixed,adjoint_queue_fp64, e.g. 16,1,8,8,0,1")
+                        "adjoint_queue_mixed,adjoint_queue_fp64, e.g. 16,1,8,8,0,0 (the last two choose nothing)")
     p.add_argument("--copy-probe", action="store_true",
                    help="also run device-to-device copies of 256 MiB (the reference for scaling HBM byte counters)")
     return p.parse_args()
@@ -215,7 +215,6 @@ def main():
 
     # the transfer's launch choices by the autotuner (on a hashed 1/16 sample of the first slice's tasks, the mixed
     # path with the adjoint records); both paths then run with them
-    # the element adjoints' launch form per path (one reverse pass in each form, on the first slice)
     tune = None
     if args.launch:
         ch, qu, pa, pb, aqm, aq64 = (int(x) for x in args.launch.split(","))
@@ -226,7 +225,7 @@ def main():
     elif not args.no_tune:
         K.precision(cache, "mixed")
         t0 = time.perf_counter()
-        choice, table = K.autotune(cache, model, [slices[0][0]], [slices[0][1]], L, records=True, sample_every=16, adjoint=True)
+        choice, table = K.autotune(cache, model, [slices[0][0]], [slices[0][1]], L, records=True, sample_every=16)
         tune = {"mixed": {"choice": choice, "seconds": time.perf_counter() - t0,
                           "table": [{"chunk": c_, "patch": list(p_), "queue": q_, "ms": m_} for c_, p_, q_, m_ in table]}}
         progress(f"autotune mixed ({tune['mixed']['seconds']:.1f} s): {choice}")
@@ -299,13 +298,6 @@ def main():
                      adjoint_queue=mixed_choice["adjoint_queue"])
             if prec == "fp64" and "fp64_adjoint_queue" in tune:
                 K.tuning(cache, adjoint_queue=tune["fp64_adjoint_queue"])
-            elif prec == "fp64":
-                # the FP64 path keeps the transfer's choices and takes its own element-adjoint form
-                t0 = time.perf_counter()
-                choice, table = K.autotune(cache, model, [slices[0][0]], [slices[0][1]], L, adjoint=True, transfer=False)
-                tune["fp64"] = {"choice": choice, "seconds": time.perf_counter() - t0,
-                                "table": [{"chunk": c_, "patch": list(p_), "queue": q_, "ms": m_} for c_, p_, q_, m_ in table]}
-                progress(f"autotune fp64 element adjoints ({tune['fp64']['seconds']:.1f} s): {choice}")
         tsl, wsl = plan[prec]
         if prec == "fp64" and "mixed" not in args.paths.split(","):
             tsl = mixed_timed[:k64]
@@ -424,10 +416,10 @@ def main():
 def batched_main(args):
     """The batched configuration: one forward cube (the polarized transfer of every point of a 256 x 256 screen in
     uneven 32^2-128^2 tiles plus 32 extra screens of U[48, 160]^2, 1024 samples per ray, 128 splats of the three
-    populations, 3 frequencies x 16 frames) in one launch of the mixed-precision transfer. The launch is timed as
-    one workgroup per task, as the persistent work queue (index order, then the cost order of the previous launch)
-    and with the autotuner's choice (timed on a sample of one slice's tasks); a step is one cube with the chosen
-    launch. The FP64 path renders the first slice for the error bar of the mixed cube. No adjoint: this
+    populations, 3 frequencies x 16 frames) on the mixed-precision transfer, its frames in groups whose segment maps
+    stay within the library's limit. The cube is timed in the index order of the work queue, in the cost order of its
+    previous launch, and with the autotuner's choice (timed on a sample of one slice's tasks); a step is one cube with
+    the chosen launch. The FP64 path renders the first slice for the error bar of the mixed cube. No adjoint: this
     configuration is a forward render."""
     import kerrsplat_amd as K
     from kerrsplat_amd import api, synthetic as syn
@@ -462,24 +454,17 @@ def batched_main(args):
 
     runs = {}
     K.tuning(cache, chunk=32, queue=False, patch=(8, 8))
-    runs["grid"] = cube_ms("one workgroup per task (warm-up)")
-    runs["grid"] = cube_ms("one workgroup per task")
+    cube_ms("index order (warm-up)")
+    runs["index_order"] = cube_ms("index order")
     K.tuning(cache, queue=True)
-    runs["queue_index_order"] = cube_ms("work queue, index order")
-    runs["queue_cost_order"] = cube_ms("work queue, cost order")
+    cube_ms("cost order (its first launch, in index order)")
+    runs["cost_order"] = cube_ms("cost order")
     t0 = time.perf_counter()
     choice, table = K.autotune(cache, model, [times[0]], [nus[1]], L, records=False, sample_every=4)
     tune_s = time.perf_counter() - t0
     progress(f"autotune ({tune_s:.1f} s): {choice}")
     steps = []
-    try:
-        w, tr = cube_ms("tuned cube (first)")
-    except api.KernelError as e:
-        # the segment maps of the whole cube at the tuned chunk length did not fit: the next longer chunk
-        progress(f"tuned launch failed ({e}); chunk {2 * choice['chunk']}")
-        K.tuning(cache, chunk=2 * choice["chunk"])
-        choice = K.tuning(cache)
-        w, tr = cube_ms("tuned cube (first)")
+    cube_ms("tuned cube (first)")
     for k in range(max(args.warmup, 0) + max(args.steps, 1)):
         w, tr = cube_ms(f"tuned cube {k + 1}")
         if k >= args.warmup:

@@ -26,8 +26,11 @@ constexpr int CHUNK = 32;          // samples per work item of the transfer from
 // work item (8 of 32 samples). The (sample, splat) pairs crowd into few items, and whole work items left most of the
 // chip idle behind the heaviest (0.3 to 1.6 wavefronts a SIMD in flight on average, up to 4 resident).
 // With few tasks (128 items x a slice each) the slices are halved, down to 2 samples: below SLICE_TASKS the last, dear
-// tasks leave the chip idle for longer than the further maps cost to compose (FP64 transfer of 1024 kappa splats,
-// 112 x 96 x 512: 131 ms with slices of 8, 5376 tasks; 111 of 4; 95 of 2).
+// tasks leave the chip idle for longer than the further maps cost to compose. Whole calls, MI355X, never halved / halved to
+// 4 / to 2: FP64 image of 6 thermal splats (50 x 37 x 301) 0.361 / 0.303 / 0.286 ms, FP64 gradient of 48 power-law splats
+// (102 x 67 x 333, 2 frames) 6.72 / 6.50 / 6.52, mixed captured fit of 16 splats (64 x 64 x 256, 4 frames) 2.35 / 2.19 / 2.19,
+// FP64 fit of 1024 kappa splats (112 x 96 x 512) 177 / 165 / 165; of four drawn calls 1.00 to 2.1 times as fast as never
+// halved, 0.97 to 1.40 as halved to 4.
 constexpr int64_t SLICE_TASKS = 8192;
 // The maps of one launch stay within MAPS_MAX bytes: slices of a quarter take four times the maps of whole work items (20
 // bytes a sample and frame in FP64 against 5, 10 in FP32, and 8 more behind the records of a dual sweep), which at the
