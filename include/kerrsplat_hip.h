@@ -118,16 +118,16 @@ int ks_cache_get_tuning(const ks_cache* cache, int* chunk, int* queue, int* patc
  * order; the wavefront patches then stay inside one part. nparts = 0: the camera of ks_regenerate is
  * one screen. The sum of the part sizes must be the cache's point count. */
 int ks_cache_set_parts(ks_cache* cache, int nparts, const int* n_alpha, const int* n_beta);
-/* The autotuner (no counterpart in the reference). Unless flags has KS_TUNE_KEEP_TRANSFER: times every launch
- * choice of the transfer (chunk 16, 32, 64, 128 x patch 8x8, 16x4, 4x16 x the two orders of its queue) on
- * a hashed sample of 1 / sample_every of its tasks for (times, nus) - the first group of their frames where a
- * render takes them in groups -, with the dual sweep's records written when flags has KS_TUNE_RECORDS, and
- * keeps the fastest. The cost order is that of the sample's own ticks in index order, its recording and sorting
- * counted. With KS_TUNE_ADJOINT: one forward pass with the records, then the reverse pass once (the element
- * adjoints have one launch form; the cache's KS_QUEUE_ADJOINT bit stays).
- * table[5 q + {0..4}] = (chunk, patch_a, patch_b, queue bits, milliseconds) of candidate q (the element
- * adjoints' row with chunk 0; at most cap rows); *ncand = the candidates timed. Leaves no forward pass
- * to reverse. */
+/* The autotuner (no counterpart in the reference). Unless flags has KS_TUNE_KEEP_TRANSFER: times the chunks and
+ * patches of the transfer (16, 32, 64, 128 x 8x8, 16x4, 4x16) in the index order of its queue on a hashed sample
+ * of 1 / sample_every of its tasks for (times, nus) - the first group of their frames where a render takes them
+ * in groups -, with the dual sweep's records written when flags has KS_TUNE_RECORDS, then the index and the cost
+ * order on whole launches of the fastest (five launches), and keeps the fastest choice. With KS_TUNE_ADJOINT: one
+ * forward pass with the records, then the reverse pass once (the element adjoints have one launch form; the
+ * cache's KS_QUEUE_ADJOINT bit stays).
+ * table[5 q + {0..4}] = (chunk, patch_a, patch_b, queue bits, milliseconds) of candidate q: 12 pairs, the cost
+ * order's milliseconds those of the index order in the ratio of the whole launches, then the element adjoints' row
+ * with chunk 0 (at most cap rows); *ncand = the candidates. Leaves no forward pass to reverse. */
 #define KS_TUNE_RECORDS 1
 #define KS_TUNE_ADJOINT 2
 #define KS_TUNE_KEEP_TRANSFER 4

@@ -443,11 +443,12 @@ def tuning(cache, chunk=None, queue=None, patch=None, adjoint_queue=None):
 
 
 def autotune(cache, model, times, nus, L, records=True, sample_every=16, adjoint=False, transfer=True):
-    """The autotuner: times every launch choice of the transfer (chunk 16/32/64/128 x patch 8x8/16x4/4x16 x the queue's
-    index and cost order) on a hashed sample of 1 / sample_every of the transfer's tasks for (times, nus) (records = the
-    dual sweep's records written, as in gradient_forward) and keeps the fastest on the cache (transfer=False keeps the
-    cache's transfer choices); with adjoint, also times one reverse pass. Returns (choice, table), table = [(chunk,
-    (patch_a, patch_b), queue bits, ms), ...] (the element adjoints' row with chunk 0)."""
+    """The autotuner: times the transfer's chunks and patches (16/32/64/128 x 8x8/16x4/4x16) on a hashed sample of
+    1 / sample_every of its tasks for (times, nus) (records = the dual sweep's records written, as in gradient_forward),
+    then the queue's index and cost order on whole launches of the fastest, and keeps the fastest choice on the cache
+    (transfer=False keeps the cache's transfer choices); with adjoint, also times one reverse pass. Returns (choice,
+    table), table = [(chunk, (patch_a, patch_b), queue bits, ms), ...] (the cost order's ms those of the index order in
+    the ratio of the whole launches; the element adjoints' row with chunk 0)."""
     m = _as_model(model, "thermal")
     tv, nv = _f64(np.atleast_1d(times)), _f64(np.atleast_1d(nus))
     cap = 64

@@ -188,7 +188,7 @@ KS_DEV S gauss_exponent(const SplatCT<S>& s, S t, S x, S y, S z, S sp, S cp) {
     return q0 * q0 + q1 * q1 + q2 * q2 + tt * tt;
 }
 
-// Where emission time t lies among nk ascending knot times: the interval and the weight of its end, held at the first and
+// Where emission time t lies among nk increasing knot times (in S too: knot_times_as): the interval and the weight of its end, held at the first and
 // last knot outside their times (trajectories.jl:93-111). Every time is compared, so the loads do not wait for each other,
 // and are scalar where the times are the same for the whole wavefront.
 template <class S> struct KnotAt { int kk; S w; };
@@ -199,11 +199,8 @@ KS_DEV KnotAt<S> knot_at(const S* __restrict__ kt, int nk, S t) {
     a.w = S(0.0);
     if (nk < 2) return a;
     for (int k = 1; k < nk - 1; ++k) a.kk += kt[k] <= t ? 1 : 0;
-    // (the ends by comparison: knot times that increase in FP64 may coincide in FP32, and 0 / 0 is no weight)
-    const bool first = t <= kt[0], last = t >= kt[nk - 1];
-    a.kk = first ? 0 : a.kk;
     const S w = (t - kt[a.kk]) / (kt[a.kk + 1] - kt[a.kk]);
-    a.w = first ? S(0.0) : (last ? S(1.0) : w);
+    a.w = w < 0.0 ? S(0.0) : (w > 1.0 ? S(1.0) : w);
     return a;
 }
 // the centre between the interval's knots, K the first of them (one: a splat of a single knot)

@@ -514,7 +514,7 @@ int ks_model_create(ks_ctx* ctx, int kind, int nrows, int ns, const double* para
         HIPCHK(hipMemcpy(m->d_ktimes, knot_times, (size_t)nknots * sizeof(double), hipMemcpyHostToDevice));
         std::vector<f32> kf((size_t)3 * nknots * ns), tf((size_t)nknots);
         for (size_t i = 0; i < kf.size(); ++i) kf[i] = f32(knots[i]);
-        for (size_t i = 0; i < tf.size(); ++i) tf[i] = f32(knot_times[i]);
+        knot_times_as(knot_times, nknots, tf.data());
         if (dalloc(&m->d_knots_f, kf.size()) || dalloc(&m->d_ktimes_f, tf.size())) { ks_model_destroy(m); return KS_ERR_HIP; }
         HIPCHK(hipMemcpy(m->d_knots_f, kf.data(), kf.size() * sizeof(f32), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(m->d_ktimes_f, tf.data(), tf.size() * sizeof(f32), hipMemcpyHostToDevice));
@@ -559,6 +559,7 @@ int ks_model_composite(ks_ctx* ctx, int nparts, const ks_model* const* parts, ks
     std::vector<SplatC> h(n);
     std::vector<SplatCf> hf(n);
     std::vector<double> kn((size_t)3 * nkn), kt((size_t)nkt);
+    std::vector<f32> ktf((size_t)nkt);
     size_t off = 0, okn = 0, okt = 0;
     for (int p = 0; p < nparts; ++p) {
         const ks_model* q = parts[p];
@@ -572,6 +573,7 @@ int ks_model_composite(ks_ctx* ctx, int nparts, const ks_model* const* parts, ks
         if (q->nkn > 0) {
             HIPCHK_M(hipMemcpy(kn.data() + 3 * okn, q->d_knots, (size_t)3 * q->nkn * sizeof(double), hipMemcpyDeviceToHost));
             HIPCHK_M(hipMemcpy(kt.data() + okt, q->d_ktimes, (size_t)q->nkt * sizeof(double), hipMemcpyDeviceToHost));
+            knot_times_as(kt.data() + okt, (int)q->nkt, ktf.data() + okt);
         }
         off += q->ns; okn += q->nkn; okt += q->nkt;
     }
@@ -580,9 +582,8 @@ int ks_model_composite(ks_ctx* ctx, int nparts, const ks_model* const* parts, ks
     HIPCHK_M(hipMemcpy(m->d_splats_f, hf.data(), n * sizeof(SplatCf), hipMemcpyHostToDevice));
     if (nkn > 0) {
         m->nknots = (int)nkt; m->nkn = nkn; m->nkt = nkt;
-        std::vector<f32> knf(kn.size()), ktf(kt.size());
+        std::vector<f32> knf(kn.size());
         for (size_t i = 0; i < kn.size(); ++i) knf[i] = f32(kn[i]);
-        for (size_t i = 0; i < kt.size(); ++i) ktf[i] = f32(kt[i]);
         if (dalloc(&m->d_knots, kn.size()) || dalloc(&m->d_ktimes, kt.size()) || dalloc(&m->d_knots_f, kn.size()) || dalloc(&m->d_ktimes_f, kt.size())) {
             ks_model_destroy(m); return KS_ERR_HIP;
         }
@@ -920,15 +921,17 @@ struct TunerBufs {
     Buf<uint8_t> tmp;
     ~TunerBufs() { tasks.release(); ids.release(); order.release(); cost.release(); keys.release(); tmp.release(); }
 };
-// The autotuner. Transfer (unless KS_TUNE_KEEP_TRANSFER): every candidate launch (samples per work item x wavefront
-// patch x the queue's order) timed with HIP events on a sample of the transfer's work (each task of the candidate's own
-// task list with probability 1 / sample_every, by a hash of its index: the same fraction of the (item, sample)
-// pairs for every candidate, spread over the whole screen), twice, the faster run counting. The cost order is timed as a
-// launch takes it: the sample's tasks in descending order of the ticks of a run in index order, recording its own ticks and
-// sorting them. Element adjoints (with KS_TUNE_ADJOINT): they have one launch form, whose reverse pass is timed once after
-// a forward pass with the records at the chosen transfer, by its stage events (zero seeds: the work does not depend on
-// them). The cache keeps the fastest transfer; rows of the table: (chunk, patch_a, patch_b, queue bits, ms), the element
-// adjoints' row with chunk = 0.
+// The autotuner. Transfer (unless KS_TUNE_KEEP_TRANSFER): every chunk and wavefront patch timed with HIP events on a sample
+// of the transfer's work (each task of the candidate's own task list with probability 1 / sample_every, by a hash of its
+// index: the same fraction of the (item, sample) pairs for every candidate, spread over the whole screen), in the queue's
+// index order, twice, the faster run counting. The order is decided on whole launches at the fastest candidate, since a
+// sample has the whole launch's longest tasks and a fraction of its work, and so the more to gain from taking them first (the
+// 512 x 512 x 2048 fit's 1/16 sample 66.7 -> 49.6 ms, its whole transfer 1006 -> 990): index order and cost order (an index-order
+// run's ticks, the recording and the sort counted), twice each; a gain below the two runs' own difference counts as none. The
+// candidates' rows in cost order are their index-order times in the ratio of those two launches. Element adjoints (with
+// KS_TUNE_ADJOINT): they have one launch form, whose reverse pass is timed once after a forward pass with the records at the
+// chosen transfer, by its stage events (zero seeds: the work does not depend on them). The cache keeps the fastest transfer;
+// rows of the table: (chunk, patch_a, patch_b, queue bits, ms), the element adjoints' row with chunk = 0.
 int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, const double* nus, int nnu, double L, int flags, int sample_every,
                 double* table, int cap, int* ncand) {
     if (!c || !m || !times || !nus || !ncand) return fail(KS_ERR_ARG, "ks_autotune: null argument");
@@ -967,9 +970,25 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
         }
         std::vector<int> tasks;
         TunerBufs d;
-        auto run = [&](const TransferLaunch& smp, int slice) {
-            return transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr, records ? c->aflg : nullptr, &smp);
+        // the faster of two runs of a launch, and (spread) how far the two differ
+        auto timed = [&](const TransferLaunch& tl, int slice, bool sort, size_t bytes, float& ms, float& spread) -> int {
+            float t[2];
+            for (float& v : t) {
+                HIPCHK(hipEventRecord(x->ev0, x->stream));
+                if (int rc = transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr,
+                                             records ? c->aflg : nullptr, &tl))
+                    return rc;
+                if (sort) HIPCHK(launch_order_tasks(x->stream, d.cost.p, tl.ntasks, d.keys.p, d.ids.p, d.order.p, d.tmp.p, bytes));
+                HIPCHK(hipEventRecord(x->ev1, x->stream));
+                HIPCHK(hipEventSynchronize(x->ev1));
+                HIPCHK(hipEventElapsedTime(&v, x->ev0, x->ev1));
+            }
+            ms = std::min(t[0], t[1]);
+            spread = std::fabs(t[0] - t[1]);
+            return KS_OK;
         };
+        auto slice_now = [&] { return records ? sweep_slice(c, items) : render_slice(c, items, c->npix); };
+        float ms = 0.0f, spread = 0.0f;
         for (int pc = 0; pc < 3; ++pc) {
             c->patch_a = patches[pc][0]; c->patch_b = patches[pc][1];
             if (int rc = build_tmap(c)) return rc;
@@ -977,7 +996,7 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                 if (chunks[ci] > std::max(c->N, 16)) continue;
                 c->chunk = chunks[ci];
                 if (records && ensure_adj(c, items, std::max(m->ns, 1))) return KS_ERR_HIP;
-                const int slice = records ? sweep_slice(c, items) : render_slice(c, items, c->npix);
+                const int slice = slice_now();
                 if (int rc = ensure_seg(c, c->npix * tnt * tnnu, slice)) return rc;
                 const int64_t all = transfer_tasks(c->npix, tnt, tnnu, c->N, slice);
                 // a hashed Bernoulli sample of rate 1 / sample_every (a regular stride aliases with the screen: every k-th
@@ -989,42 +1008,39 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                     if (h % (uint64_t)sample_every == 0) tasks.push_back((int)q);
                 }
                 if (tasks.empty()) tasks.push_back(0);
-                const size_t nsamp = tasks.size();
-                size_t bytes = 0;
-                HIPCHK(launch_order_tasks(x->stream, d.cost.p, (int64_t)nsamp, nullptr, nullptr, nullptr, nullptr, bytes));
-                if (d.tasks.grow(nsamp) || d.cost.grow((size_t)all) || d.keys.grow(nsamp) || d.ids.grow(nsamp) || d.order.grow(nsamp) ||
-                    d.tmp.grow(std::max<size_t>(bytes, 1)))
-                    return KS_ERR_HIP;
+                if (d.tasks.grow(tasks.size())) return KS_ERR_HIP;
+                HIPCHK(hipMemcpy(d.tasks.p, tasks.data(), tasks.size() * sizeof(int), hipMemcpyHostToDevice));
                 TransferLaunch smp;
-                smp.tasks = d.tasks.p; smp.ntasks = (int64_t)nsamp;
-                for (int qu = 0; qu < 2; ++qu) {
-                    if (qu) {          // the ticks of a run in index order, and the sample sorted by them
-                        HIPCHK(launch_fill_i32(x->stream, (int*)d.cost.p, all, 0));
-                        smp.cost = d.cost.p;
-                        if (int rc = run(smp, slice)) return rc;
-                        std::vector<uint32_t> cost((size_t)all);
-                        HIPCHK(hipStreamSynchronize(x->stream));
-                        HIPCHK(hipMemcpy(cost.data(), d.cost.p, (size_t)all * sizeof(uint32_t), hipMemcpyDeviceToHost));
-                        std::stable_sort(tasks.begin(), tasks.end(), [&](int p, int q) { return cost[p] > cost[q]; });
-                    }
-                    HIPCHK(hipMemcpy(d.tasks.p, tasks.data(), nsamp * sizeof(int), hipMemcpyHostToDevice));
-                    c->queue = qu ? KS_QUEUE_TRANSFER | adj_bit : adj_bit;
-                    float ms = INFINITY;
-                    for (int rep = 0; rep < 2; ++rep) {
-                        HIPCHK(hipEventRecord(x->ev0, x->stream));
-                        if (int rc = run(smp, slice)) return rc;
-                        if (qu) HIPCHK(launch_order_tasks(x->stream, d.cost.p, (int64_t)nsamp, d.keys.p, d.ids.p, d.order.p, d.tmp.p, bytes));
-                        HIPCHK(hipEventRecord(x->ev1, x->stream));
-                        HIPCHK(hipEventSynchronize(x->ev1));
-                        float t = 0.0f;
-                        HIPCHK(hipEventElapsedTime(&t, x->ev0, x->ev1));
-                        ms = std::min(ms, t);
-                    }
-                    rows.insert(rows.end(), {(double)c->chunk, (double)c->patch_a, (double)c->patch_b, (double)c->queue, (double)ms});
-                    if (ms < best_ms) { best_ms = ms; best = n; }
-                    ++n;
-                }
+                smp.tasks = d.tasks.p; smp.ntasks = (int64_t)tasks.size();
+                c->queue = adj_bit;
+                if (int rc = timed(smp, slice, false, 0, ms, spread)) return rc;
+                for (int qu = 0; qu < 2; ++qu)
+                    rows.insert(rows.end(), {(double)c->chunk, (double)c->patch_a, (double)c->patch_b, (double)(adj_bit | (qu ? KS_QUEUE_TRANSFER : 0)), (double)ms});
+                if (ms < best_ms) { best_ms = ms; best = n; }
+                n += 2;
             }
+        }
+        if (best >= 0) {
+            c->chunk = (int)rows[5 * best]; c->patch_a = (int)rows[5 * best + 1]; c->patch_b = (int)rows[5 * best + 2];
+            if (int rc = build_tmap(c)) return rc;
+            const int slice = slice_now();
+            if (int rc = ensure_seg(c, c->npix * tnt * tnnu, slice)) return rc;
+            const int64_t all = transfer_tasks(c->npix, tnt, tnnu, c->N, slice);
+            const size_t na = (size_t)all;
+            size_t bytes = 0;
+            HIPCHK(launch_order_tasks(x->stream, d.cost.p, all, nullptr, nullptr, nullptr, nullptr, bytes));
+            if (d.cost.grow(na) || d.keys.grow(na) || d.ids.grow(na) || d.order.grow(na) || d.tmp.grow(std::max<size_t>(bytes, 1))) return KS_ERR_HIP;
+            TransferLaunch whole;              // every task in index order
+            float mi = 0.0f, si = 0.0f, mc = 0.0f, sc = 0.0f;
+            if (int rc = timed(whole, slice, false, 0, mi, si)) return rc;
+            whole.ntasks = all;
+            whole.cost = d.cost.p;
+            if (int rc = timed(whole, slice, true, bytes, mc, sc)) return rc;      // the ticks and the order they give
+            whole.tasks = d.order.p;
+            if (int rc = timed(whole, slice, true, bytes, mc, sc)) return rc;
+            const double ratio = std::fabs(mc - mi) > std::max(si, sc) && mi > 0.0f ? (double)mc / mi : 1.0;
+            for (size_t q = 1; q < rows.size() / 5; q += 2) rows[5 * q + 4] *= ratio;
+            if (ratio < 1.0) ++best;
         }
         if (best < 0) { c->chunk = old[0]; c->queue = old[1]; c->patch_a = old[2]; c->patch_b = old[3]; }
         else {

@@ -1,14 +1,18 @@
-// Host check of knot_at: the knot interval and weight at a time, for ascending knot times that may coincide in FP32, give
-// the centre that holds the first knot up to its time, the last one from its time on, and interpolates in between, at
-// times on the knots, beside them and far outside. Exit status 0 when every centre is finite and agrees to rounding.
+// Host check of the knot interval (knot_at) at the times that a model keeps (knot_times_as): for knot times that FP32 may not
+// tell apart, the kept ones increase and stay within FP32's rounding and a step a knot of them, and the interval gives the
+// centre that holds the first knot up to its time, the last one from its time on, and interpolates in between, at times on
+// the knots, beside them and far outside. Exit status 0 when every centre is finite and agrees to rounding.
 #include <cmath>
 #include <cstdio>
 #include <random>
 #include <vector>
-#include "../../kerrsplat_amd/csrc/ks_dtransfer.hpp"
+#include "../../kerrsplat_amd/csrc/ks_hostsplat.hpp"
 using namespace ksd;
 template <class S> double centre(const std::vector<double>& kt, const std::vector<double>& K, double t, bool held) {
-    std::vector<S> ktS(kt.begin(), kt.end()), KS(3 * K.size());
+    std::vector<S> ktS(kt.size()), KS(3 * K.size());
+    knot_times_as(kt.data(), (int)kt.size(), ktS.data());
+    for (size_t k = 0; k < kt.size(); ++k)
+        if ((k && !(ktS[k] > ktS[k - 1])) || fabs(val(ktS[k]) - kt[k]) > 1.2e-7 * (k + 1) * fmax(fabs(kt[k]), 1.0)) return NAN;
     for (size_t k = 0; k < K.size(); ++k) KS[3 * k] = KS[3 * k + 1] = KS[3 * k + 2] = S(K[k]);
     const int nk = (int)kt.size();
     const S tS = S(t);
