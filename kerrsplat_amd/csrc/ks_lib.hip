@@ -919,12 +919,14 @@ struct TunerBufs {
     Buf<int> tasks, ids, order;
     Buf<uint32_t> cost, keys;
     Buf<uint8_t> tmp;
-    ~TunerBufs() { tasks.release(); ids.release(); order.release(); cost.release(); keys.release(); tmp.release(); }
+    Buf<double> out;
+    ~TunerBufs() { tasks.release(); ids.release(); order.release(); cost.release(); keys.release(); tmp.release(); out.release(); }
 };
 // The autotuner. Transfer (unless KS_TUNE_KEEP_TRANSFER): every chunk and wavefront patch timed with HIP events on a sample
 // of the transfer's work (each task of the candidate's own task list with probability 1 / sample_every, by a hash of its
 // index: the same fraction of the (item, sample) pairs for every candidate, spread over the whole screen), in the queue's
-// index order, twice, the faster run counting. The order is decided on whole launches at the fastest candidate, since a
+// index order, twice, the faster run counting, and the composition of the whole launch's maps in the same fraction (shorter
+// slices leave more of them). The order is decided on whole launches at the fastest candidate, since a
 // sample has the whole launch's longest tasks and a fraction of its work, and so the more to gain from taking them first (the
 // 512 x 512 x 2048 fit's 1/16 sample 66.7 -> 49.6 ms, its whole transfer 1006 -> 990): index order and cost order (an index-order
 // run's ticks, the recording and the sort counted), twice each; a gain below the two runs' own difference counts as none. The
@@ -970,15 +972,21 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
         }
         std::vector<int> tasks;
         TunerBufs d;
-        // the faster of two runs of a launch, and (spread) how far the two differ
-        auto timed = [&](const TransferLaunch& tl, int slice, bool sort, size_t bytes, float& ms, float& spread) -> int {
+        // the faster of two runs, and (spread) how far the two differ: of a launch, with the sort of its ticks (sort = its
+        // workspace), or of the composition of the maps
+        auto timed = [&](const TransferLaunch* tl, int slice, size_t sort, float& ms, float& spread) -> int {
             float t[2];
             for (float& v : t) {
                 HIPCHK(hipEventRecord(x->ev0, x->stream));
-                if (int rc = transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr,
-                                             records ? c->aflg : nullptr, &tl))
-                    return rc;
-                if (sort) HIPCHK(launch_order_tasks(x->stream, d.cost.p, tl.ntasks, d.keys.p, d.ids.p, d.order.p, d.tmp.p, bytes));
+                if (tl) {
+                    if (int rc = transfer_launch(c, m, d_tn, tnt, d_tn + nt, tnnu, L, slice, nullptr, records ? (void*)c->arec : nullptr,
+                                                 records ? c->aflg : nullptr, tl))
+                        return rc;
+                    if (sort) HIPCHK(launch_order_tasks(x->stream, d.cost.p, tl->ntasks, d.keys.p, d.ids.p, d.order.p, d.tmp.p, sort));
+                } else {
+                    HIPCHK(launch_seg_combine(x->stream, c->npix, c->N, slice, tnt, d_tn + nt, tnnu, c->seg, seg_is32(c), d.out.p));
+                    if (records) HIPCHK(launch_adj_combine(x->stream, c->npix, c->N, slice, tnt, d_tn + nt, tnnu, c->seg, seg_is32(c), c->ads, c->awT));
+                }
                 HIPCHK(hipEventRecord(x->ev1, x->stream));
                 HIPCHK(hipEventSynchronize(x->ev1));
                 HIPCHK(hipEventElapsedTime(&v, x->ev0, x->ev1));
@@ -1008,12 +1016,15 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
                     if (h % (uint64_t)sample_every == 0) tasks.push_back((int)q);
                 }
                 if (tasks.empty()) tasks.push_back(0);
-                if (d.tasks.grow(tasks.size())) return KS_ERR_HIP;
+                if (d.tasks.grow(tasks.size()) || d.out.grow((size_t)4 * c->npix * tnt * tnnu)) return KS_ERR_HIP;
                 HIPCHK(hipMemcpy(d.tasks.p, tasks.data(), tasks.size() * sizeof(int), hipMemcpyHostToDevice));
                 TransferLaunch smp;
                 smp.tasks = d.tasks.p; smp.ntasks = (int64_t)tasks.size();
                 c->queue = adj_bit;
-                if (int rc = timed(smp, slice, false, 0, ms, spread)) return rc;
+                float compose = 0.0f;
+                if (int rc = timed(&smp, slice, 0, ms, spread)) return rc;
+                if (int rc = timed(nullptr, slice, 0, compose, spread)) return rc;
+                ms += compose / (float)sample_every;
                 for (int qu = 0; qu < 2; ++qu)
                     rows.insert(rows.end(), {(double)c->chunk, (double)c->patch_a, (double)c->patch_b, (double)(adj_bit | (qu ? KS_QUEUE_TRANSFER : 0)), (double)ms});
                 if (ms < best_ms) { best_ms = ms; best = n; }
@@ -1032,12 +1043,12 @@ int ks_autotune(ks_cache* c, const ks_model* m, const double* times, int nt, con
             if (d.cost.grow(na) || d.keys.grow(na) || d.ids.grow(na) || d.order.grow(na) || d.tmp.grow(std::max<size_t>(bytes, 1))) return KS_ERR_HIP;
             TransferLaunch whole;              // every task in index order
             float mi = 0.0f, si = 0.0f, mc = 0.0f, sc = 0.0f;
-            if (int rc = timed(whole, slice, false, 0, mi, si)) return rc;
+            if (int rc = timed(&whole, slice, 0, mi, si)) return rc;
             whole.ntasks = all;
             whole.cost = d.cost.p;
-            if (int rc = timed(whole, slice, true, bytes, mc, sc)) return rc;      // the ticks and the order they give
+            if (int rc = timed(&whole, slice, bytes, mc, sc)) return rc;      // the ticks and the order they give
             whole.tasks = d.order.p;
-            if (int rc = timed(whole, slice, true, bytes, mc, sc)) return rc;
+            if (int rc = timed(&whole, slice, bytes, mc, sc)) return rc;
             const double ratio = std::fabs(mc - mi) > std::max(si, sc) && mi > 0.0f ? (double)mc / mi : 1.0;
             for (size_t q = 1; q < rows.size() / 5; q += 2) rows[5 * q + 4] *= ratio;
             if (ratio < 1.0) ++best;
