@@ -63,7 +63,8 @@ int ks_stage_ms(ks_ctx* ctx, int stage, float* ms);
 
 /* GeodesicCache(backend, camera, Val(N); store_samples) - cache.jl:106-125. Stored samples take 57 bytes per point and
  * sample. Without them the first image allocates a workspace of one tile, kept until ks_cache_destroy: 49 bytes a sample
- * and up to 2^24 samples (0.8 GB; less where the screen is smaller), and up to 1 GiB of transfer maps for polarized images. */
+ * and up to 2^24 samples (0.8 GB; less where the screen is smaller), and up to 1 GiB of transfer maps for polarized images
+ * (thin images of few splats take neither). */
 int ks_cache_create(ks_ctx* ctx, int64_t npix, int N, int store_samples, ks_cache** cache);
 int ks_cache_destroy(ks_cache* cache);
 /* npixels / nsamples / generation / length.(ranges) - cache.jl:127-141. */

@@ -357,6 +357,44 @@ __global__ void __launch_bounds__(128) ks_thin_parts(double a, const double* __r
     }
     part[(int64_t)m * npix + j] = acc;
 }
+// The same sums fused with the march, a thread an anchor segment, for the few splats (THIN_MARCH_TILE) whose sums the march's idle
+// issue slots take: part[m npix + j] = the sum over segment m of pixel j (0 past its last segment), res its anchor residuals.
+struct ThinF {
+    const SplatC* sp; int ns; double a, rp, rm, t_obs, lam, acc;
+    KS_DEV void operator()(int, const Samp& s, double dtau) {
+        if (!(s.ok && rp * (1.0 + 1e-3) < s.r && s.r < 1e3)) return;
+        double x, y, z, jt = 0.0;
+        quasi_cartesian_ks(a, rp, rm, s.r, s.th, s.ph, x, y, z);
+        for (int i = 0; i < ns; ++i) {
+            const SplatC& c = sp[i];
+            double sph, cph;
+            phase_sincos(c.omega * (t_obs - s.t - c.t0), &sph, &cph);
+            jt += exp(c.lnA - 0.5 * gauss_exponent(c, t_obs - s.t, x, y, z, sph, cph));
+        }
+        acc += thin_weight(a, lam, s.r, s.th, dtau) * jt;
+    }
+};
+__global__ void __launch_bounds__(128) ks_thin_march(double a, double thetao, const double* __restrict__ soa, int64_t npix, int N, int M,
+                                                     const SplatC* __restrict__ sp, int ns, double t_obs, int nseg_max, double* __restrict__ part,
+                                                     double* __restrict__ res) {
+    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (tid >= npix * nseg_max) return;
+    const int64_t j = tid % npix;
+    const int m = (int)(tid / npix);
+    const Spin S = make_spin(a);
+    const PixC p = load_pixel(soa, npix, j);
+    double acc = 0.0, r1 = 0.0, r2 = 0.0;
+    const int Lseg = segment_length(M, 1.0 - p.k);
+    const int kbeg = m * Lseg + 1;
+    if (kbeg <= N && kbeg * (p.tau_total / (double)(N + 1)) <= p.tau_h) {
+        const int kend = kbeg + Lseg - 1 < N ? kbeg + Lseg - 1 : N;
+        ThinF f{sp, ns, a, S.rp, S.rm, t_obs, p.lam, 0.0};
+        march_range(p, S, thetao, N, M, kbeg, kend, f, r1, r2);
+        acc = f.acc;
+    }
+    res[2 * (m * npix + j)] = r1; res[2 * (m * npix + j) + 1] = r2;
+    part[m * npix + j] = acc;
+}
 __global__ void ks_thin_combine(int64_t npix, int nseg_max, const double* __restrict__ part, double* __restrict__ out) {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= npix) return;
@@ -494,6 +532,12 @@ hipError_t launch_thin_parts(hipStream_t s, double a, const double* soa, int64_t
     hipLaunchKernelGGL(ks_thin_parts, dim3(grid_for(npix * thin_chunks(N), 128)), dim3(128), 0, s, a, soa, npix, N, smp, sp, ns, t_obs, part);
     return hipGetLastError();
 }
+hipError_t launch_thin_march(hipStream_t s, double a, double thetao, const double* soa, int64_t npix, int N, int M, const SplatC* sp, int ns,
+                             double t_obs, int nseg_max, double* part, double* res) {
+    hipLaunchKernelGGL(ks_thin_march, dim3(grid_for(npix * nseg_max, 128)), dim3(128), 0, s, a, thetao, soa, npix, N, M, sp, ns, t_obs, nseg_max, part,
+                       res);
+    return hipGetLastError();
+}
 hipError_t launch_thin_combine(hipStream_t s, int64_t npix, int nseg_max, const double* part, double* out) {
     hipLaunchKernelGGL(ks_thin_combine, dim3(grid_for(npix, 256)), dim3(256), 0, s, npix, nseg_max, part, out);
     return hipGetLastError();
@@ -512,7 +556,7 @@ hipError_t launch_seg_combine(hipStream_t s, int64_t npix, int N, int chunk, int
 // splat i's support sphere at the frame's time (outside_support), else 0; cnt[j + npix f] = the number of hits.
 // Splats outer: a splat's test stops at the ray's first samples inside its sphere, and each byte is written once. Bound by the
 // latency of the samples' loads, HIT_GROUP samples of which are in flight together (5 splats, 128 x 128 x 512: one at a time
-// 7.0 ms, 6.5 before the sine had its present form; 3.4 so. Leaving samples out first by their distance to the circle of the
+// 7.0 ms, 6.5 before the sine had its present form; 3.1 so. Leaving samples out first by their distance to the circle of the
 // splat's centre gained nothing.)
 constexpr int HIT_GROUP = 4;
 __global__ void __launch_bounds__(64) ks_ray_hits(double rp, int64_t npix, int N, Samples smp, const SplatC* __restrict__ sp, int ns,

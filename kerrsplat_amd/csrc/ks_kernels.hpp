@@ -281,9 +281,16 @@ hipError_t launch_chunk_transfer_f32(hipStream_t s, int kind, double a, double t
 hipError_t launch_ray_hits(hipStream_t s, double rp, int64_t npix, int N, Samples smp, const SplatC* sp, int ns, const double* times, int nt,
                            const int* kstop, uint8_t* hits, int* cnt);
 hipError_t launch_ray_fill(hipStream_t s, int64_t items, int64_t npix, int ns, int cap, const uint8_t* hits, const int* iperm, int32_t* ids);
+// Thin images of a cache without samples: up to this many splats fused with the march, more through a tile's samples, whose
+// writing and reading the sums of few splats do not pay for. MI355X, fused / by tiles, ms: one tile, 128 x 128 x 512, 1 splat
+// 1.53 / 1.60, 2 splats 1.60 / 1.61, 4 splats 1.74 / 1.65; several tiles, 512 x 512 x 256, 1 splat 8.2 / 10.2, 6 splats
+// 10.3 / 11.0, 12 splats 13.0 / 12.1, 200 x 150 x 700, 6 splats 3.72 / 3.59.
+constexpr int THIN_MARCH_TILE = 2, THIN_MARCH_TILES = 6;
 int thin_chunks(int N);
 hipError_t launch_thin_parts(hipStream_t s, double a, const double* soa, int64_t npix, int N, Samples smp, const SplatC* sp, int ns, double t_obs,
                              double* part);
+hipError_t launch_thin_march(hipStream_t s, double a, double thetao, const double* soa, int64_t npix, int N, int M, const SplatC* sp, int ns,
+                             double t_obs, int nseg_max, double* part, double* res);
 hipError_t launch_thin_combine(hipStream_t s, int64_t npix, int nseg_max, const double* part, double* out);
 hipError_t launch_seg_combine(hipStream_t s, int64_t npix, int N, int chunk, int nt, const double* nus, int nnu, const void* seg, int seg32,
                               double* out);

@@ -1283,6 +1283,12 @@ int ks_thin_image(ks_cache* c, const ks_model* m, double t_obs, double* out, int
         if (c->thin_part.grow((size_t)nch * c->npix)) return KS_ERR_HIP;
         HIPCHK(launch_thin_parts(x->stream, c->spin, c->soa, c->npix, c->N, samples_of(c), m->d_splats, m->ns, t_obs, c->thin_part.p));
         HIPCHK(launch_thin_combine(x->stream, c->npix, nch, c->thin_part.p, c->img1));
+    } else if (m->ns <= (fused_tile(c) < c->npix ? THIN_MARCH_TILES : THIN_MARCH_TILE)) {
+        const int nseg = max_segments(c->N);
+        if (c->thin_part.grow((size_t)nseg * c->npix)) return KS_ERR_HIP;
+        HIPCHK(launch_thin_march(x->stream, c->spin, c->thetao, c->soa, c->npix, c->N, c->M, m->d_splats, m->ns, t_obs, nseg, c->thin_part.p, c->segres));
+        HIPCHK(launch_thin_combine(x->stream, c->npix, nseg, c->thin_part.p, c->img1));
+        HIPCHK(launch_res_reduce(x->stream, c->npix, nseg, c->segres, c->rt, c->rp));
     } else {
         const int64_t tile = fused_tile(c);
         FusedTile T;
