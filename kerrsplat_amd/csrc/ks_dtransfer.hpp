@@ -790,8 +790,11 @@ KS_DEV void step_coefs_inv(T aI, T a2, T r2, T ar, S f, T o[4], T e4[4]) {
     T h = (a2 - r2) * 0.5;
     T root = sqrt(h * h + ar * ar);
     T L1sq, L2sq;
-    if (h >= 0.0) { L1sq = h + root; L2sq = L1sq > 0.0 ? ar * ar / L1sq : T(0.0); }
-    else { L2sq = root - h; L1sq = L2sq > 0.0 ? ar * ar / L2sq : T(0.0); }
+    // (FP32: an invariant below the normal range counts as zero, since its reciprocal is infinite; the step takes its Taylor
+    // form there, which does not use it)
+    const double lmin = is_fp32<T> ? 1.2e-38 : 0.0;
+    if (h >= 0.0) { L1sq = h + root; L2sq = L1sq > lmin ? ar * ar / L1sq : T(0.0); }
+    else { L2sq = root - h; L1sq = L2sq > lmin ? ar * ar / L2sq : T(0.0); }
     T L1 = L1sq > 0.0 ? sqrt(L1sq) : T(0.0), L2 = L2sq > 0.0 ? sqrt(L2sq) : T(0.0);
     T b1 = L1 * f, b2 = L2 * f;
     T Th = L1sq + L2sq;
